@@ -25,7 +25,9 @@
 // LDS buffers, one barrier per block.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "uk_device_common.h"
 #include "uk_hip_abi.h"
@@ -82,7 +84,8 @@ __device__ __forceinline__ v2u read_tr(uint32_t lds_addr) {
 // bytes of each of IL neighbouring rows, read as they lie and interleaved in
 // registers (v_perm_b32); neighbouring lanes take neighbouring columns, which
 // are neighbours in the tile.
-template <int EB, int V, int IL = 0>
+// NTS: the stores are non-temporal.
+template <int EB, int V, int IL, bool NTS>
 __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kernel(TrArgs a) {
   static_assert(IL == 0 || (V == 16 && (IL * EB == 2 || IL * EB == 4)), "interleaved rows of 2 or 4 bytes");
   static_assert(EB != 4 || (V == 16 && IL == 0), "4-byte elements: four rows per 16-byte vector");
@@ -98,8 +101,10 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
   constexpr int N1 = kBlockBytes / 16 / kThreads;  // 16-byte source vectors per thread
   constexpr int N2 = kBlockBytes / V / kThreads;   // destination vectors per thread
   constexpr int R = V / 8;                     // reads per destination vector
-  typedef v4u v4u_a4 __attribute__((aligned(4)));
+  typedef v4u v4u_a1 __attribute__((aligned(1)));
 
+  uk::load_arguments_now(a.src, a.dst, a.src_pitch, a.s0, a.s1, a.rows, a.row_bytes, a.outer0, a.outer1, a.lt0, a.lt1,
+                         a.nblk0, a.nblk1, a.strip, a.down, a.lds_pitch, a.lds_buf_bytes, a.pad32, gridDim.x);
   const uint32_t tid = threadIdx.x;
   // Row groups of one tile (its extent along the rows over what an item takes).
   const uint32_t lht = IL ? 0 : a.lt0 - (RPI == 16 ? 4 : RPI == 8 ? 3 : 2);  // log2
@@ -163,9 +168,8 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
 
   struct Block {
     uint32_t blk0, blk1, row_base, col_base_bytes;
-    const char* src;
     char* dst;
-    bool interior;
+    uint32_t interior;
   };
   auto block_at = [&](uint32_t blk) {
     Block b;
@@ -177,75 +181,58 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
     b.blk1 = st * a.strip + (rem - b.blk0 * width);
     b.row_base = b.blk0 * kBlockRows;
     b.col_base_bytes = b.blk1 * kBlockRowBytes;
-    b.src = a.src + (int64_t)b.row_base * a.src_pitch + b.col_base_bytes;
     b.dst = a.dst + (int64_t)(b.blk0 * tiles0) * a.s0 + (int64_t)(b.blk1 * tiles1) * a.s1;
-    b.interior = b.row_base + kBlockRows <= a.rows && b.col_base_bytes + kBlockRowBytes <= a.row_bytes &&
-                 (b.blk0 + 1) * tiles0 <= a.outer0 && (b.blk1 + 1) * tiles1 <= a.outer1;
+    b.interior = (b.row_base + kBlockRows <= a.rows) & (b.col_base_bytes + kBlockRowBytes <= a.row_bytes) &
+                 ((b.blk0 + 1) * tiles0 <= a.outer0) & ((b.blk1 + 1) * tiles1 <= a.outer1);
     return b;
   };
+  // The loads of a block, one block ahead of their use, straight-line code for
+  // every block (see stream_tiled_kernel): on the edges rows beyond the matrix
+  // stand on its last row and vectors that reach beyond their row on the row's
+  // last 16 bytes, which is put right when the block goes to LDS.
   v4u pre[N1];
-  auto prefetch = [&](const Block& b) {
-    if (b.interior) {
+  auto prefetch = [&](const Block& b) __attribute__((always_inline)) {
+    const uint32_t row0 = min(b.row_base, a.rows - 1), col0 = uk::clipped_offset<16>(b.col_base_bytes, a.row_bytes);
+    const char* base = a.src + (int64_t)row0 * a.src_pitch + col0;
+    uint32_t off[N1];
 #pragma unroll
-      for (int i = 0; i < N1; ++i) pre[i] = *reinterpret_cast<const v4u_a4*>(b.src + g1off[i]);
-      return;
+    for (int i = 0; i < N1; ++i) off[i] = g1off[i];
+    if (!b.interior) {
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        const uint32_t idx = tid + i * kThreads;
+        off[i] = (min(b.row_base + idx / VPR, a.rows - 1) - row0) * (uint32_t)a.src_pitch +
+                 (uk::clipped_offset<16>(b.col_base_bytes + (idx % VPR) * 16, a.row_bytes) - col0);
+      }
     }
-    // Edge block: vectors that lie wholly inside the matrix; the rest is dealt
-    // with when the block goes to LDS.
+#pragma unroll
+    for (int i = 0; i < N1; ++i) pre[i] = *reinterpret_cast<const v4u_a1*>(base + off[i]);
+  };
+  auto store = [&](char* p, auto v) __attribute__((always_inline)) {
+    if constexpr (NTS) __builtin_nontemporal_store(v, reinterpret_cast<decltype(v)*>(p));
+    else *reinterpret_cast<decltype(v)*>(p) = v;
+  };
+  // ---- matrix rows -> LDS ----
+  auto phase1_inside = [&](char* lbuf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < N1; ++i) *reinterpret_cast<v4u*>(lbuf + l1off[i]) = pre[i];
+  };
+  auto phase1_edge = [&](const Block& b, char* lbuf) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < N1; ++i) {
       const uint32_t idx = tid + i * kThreads;
       const uint32_t r = idx / VPR, cb = (idx % VPR) * 16;
-      if (b.row_base + r < a.rows && b.col_base_bytes + cb + 16 <= a.row_bytes)
-        pre[i] = *reinterpret_cast<const v4u_a4*>(b.src + g1off[i]);
+      const int32_t left = b.row_base + r < a.rows ? (int32_t)(a.row_bytes - (b.col_base_bytes + cb)) : 0;
+      uint32_t w[4] = {pre[i][0], pre[i][1], pre[i][2], pre[i][3]};
+      if (a.row_bytes < 16) uk::load_short_row<16>(w, a.src + (int64_t)(b.row_base + r) * a.src_pitch + cb, left);
+      uk::clip_piece<16>(w, left, a.pad32);
+      *reinterpret_cast<v4u*>(lbuf + l1off[i]) = v4u{w[0], w[1], w[2], w[3]};
     }
   };
-
-  const uint32_t nblocks = a.nblk0 * a.nblk1;
-  // Workgroups go to the eight XCDs round-robin; the workgroups of one XCD
-  // take consecutive blocks.
-  const uint32_t first_blk = (gridDim.x & 7) ? blockIdx.x
-                                             : (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  if (first_blk < nblocks) prefetch(block_at(first_blk));
-  uint32_t buf = 0;
-  for (uint32_t blk = first_blk; blk < nblocks; blk += gridDim.x, buf ^= 1) {
-    const Block b = block_at(blk);
-    char* lbuf = lds + buf * a.lds_buf_bytes;
-    // ---- matrix rows -> LDS ----
-    if (b.interior) {
-#pragma unroll
-      for (int i = 0; i < N1; ++i) *reinterpret_cast<v4u*>(lbuf + l1off[i]) = pre[i];
-    } else {
-#pragma unroll
-      for (int i = 0; i < N1; ++i) {
-        const uint32_t idx = tid + i * kThreads;
-        const uint32_t r = idx / VPR, cb = (idx % VPR) * 16;
-        const bool row_ok = b.row_base + r < a.rows;
-        v4u val;
-        if (row_ok && b.col_base_bytes + cb + 16 <= a.row_bytes) {
-          val = pre[i];
-        } else {
-          val = v4u{a.pad32, a.pad32, a.pad32, a.pad32};
-          if (row_ok && b.col_base_bytes + cb < a.row_bytes) {
-            // The row ends inside this vector: element by element.
-            __attribute__((aligned(16))) char reg[16];
-            *reinterpret_cast<v4u*>(reg) = val;
-            const char* gp = b.src + g1off[i];
-            const uint32_t left = a.row_bytes - (b.col_base_bytes + cb);
-            for (uint32_t bb = 0; bb + EB <= left && bb < 16; bb += EB) {
-              if constexpr (EB == 4) *reinterpret_cast<uint32_t*>(reg + bb) = *reinterpret_cast<const uint32_t*>(gp + bb);
-              else if constexpr (EB == 2) *reinterpret_cast<uint16_t*>(reg + bb) = *reinterpret_cast<const uint16_t*>(gp + bb);
-              else reg[bb] = gp[bb];
-            }
-            val = *reinterpret_cast<const v4u*>(reg);
-          }
-        }
-        *reinterpret_cast<v4u*>(lbuf + l1off[i]) = val;
-      }
-    }
-    if (blk + gridDim.x < nblocks) prefetch(block_at(blk + gridDim.x));
-    __syncthreads();
-
+  // ---- LDS -> tiles ----
+  auto phase2 = [&](const Block& b, uint32_t lds_off, auto inside_c) __attribute__((always_inline)) {
+    constexpr bool kInside = decltype(inside_c)::value;
+    const char* lbuf = lds + lds_off;
     if constexpr (IL != 0) {
       // ---- LDS rows, interleaved -> tiles ----
       v4u out[N2];
@@ -274,10 +261,10 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
       }
 #pragma unroll
       for (int i = 0; i < N2; ++i) {
-        if (!b.interior && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
-        __builtin_nontemporal_store(out[i], reinterpret_cast<v4u*>(b.dst + g2off[i]));
+        if (!kInside && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
+        store(b.dst + g2off[i], out[i]);
       }
-      continue;
+      return;
     }
     if constexpr (EB == 4) {
       // ---- LDS columns, word by word -> tiles ----
@@ -290,13 +277,13 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
       }
 #pragma unroll
       for (int i = 0; i < N2; ++i) {
-        if (!b.interior && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
-        __builtin_nontemporal_store(out[i], reinterpret_cast<v4u*>(b.dst + g2off[i]));
+        if (!kInside && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
+        store(b.dst + g2off[i], out[i]);
       }
-      continue;
+      return;
     }
     // ---- LDS, transposed -> tiles ----
-    const uint32_t lb = lds_base + buf * a.lds_buf_bytes;
+    const uint32_t lb = lds_base + lds_off;
     v2u got[N2][R];
 #pragma unroll
     for (int i = 0; i < N2; ++i)
@@ -313,20 +300,63 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
     static_assert(N2 * R == 8, "eight reads per thread and block");
 #pragma unroll
     for (int i = 0; i < N2; ++i) {
-      if (!b.interior && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
+      if (!kInside && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
       char* gp = b.dst + g2off[i];
-      // Non-temporal stores: the tiles are written once, in whole lines over a
-      // few instructions, and not read again by this kernel (f16 4096 x 4096:
-      // 11.4 -> 9.4 us; s8 8192 x 28672: 97 -> 67 us).
       if constexpr (V == 16) {
         const v4u val = v4u{got[i][0][0], got[i][0][1], got[i][1][0], got[i][1][1]};
-        __builtin_nontemporal_store(val, reinterpret_cast<v4u*>(gp));
+        store(gp, val);
       } else {
-        __builtin_nontemporal_store(got[i][0], reinterpret_cast<v2u*>(gp));
+        store(gp, got[i][0]);
       }
     }
-    // No second barrier: the next block uses the other buffer, and its barrier
-    // orders this block's reads before that buffer is written again.
+  };
+
+  const uint32_t nblocks = a.nblk0 * a.nblk1;
+  // Workgroups go to the eight XCDs round-robin; the workgroups of one XCD
+  // take consecutive blocks.
+  uint32_t blk = (gridDim.x & 7) ? blockIdx.x : (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (blk >= nblocks) return;
+  uint32_t buf = 0;
+  // No second barrier per block: the next block uses the other buffer, and its
+  // barrier orders this block's reads before that buffer is written again.
+  auto advance = [&]() __attribute__((always_inline)) {
+    blk += gridDim.x;
+    buf = a.lds_buf_bytes - buf;
+  };
+  Block b = block_at(blk);
+  if (a.row_bytes >= 16) prefetch(b);
+  // Interior blocks with a successor, in a loop of their own behind a first
+  // copy of its body (see stream_tiled_kernel: the waits at the loop's head are
+  // then for the loads alone).
+  auto steady = [&]() { return b.interior && blk + gridDim.x < nblocks; };
+  auto steady_body = [&]() __attribute__((always_inline)) {
+    phase1_inside(lds + buf);
+    const Block next = block_at(blk + gridDim.x);
+    prefetch(next);
+    __syncthreads();
+    phase2(b, buf, std::true_type{});
+    advance();
+    b = next;
+  };
+  while (true) {
+    if (steady()) {
+      steady_body();
+      while (steady()) steady_body();
+    }
+    if (b.interior) phase1_inside(lds + buf);
+    else phase1_edge(b, lds + buf);
+    const bool more = blk + gridDim.x < nblocks;
+    Block next = b;
+    if (more) {
+      next = block_at(blk + gridDim.x);
+      if (a.row_bytes >= 16) prefetch(next);
+    }
+    __syncthreads();
+    if (b.interior) phase2(b, buf, std::true_type{});
+    else phase2(b, buf, std::false_type{});
+    if (!more) return;
+    advance();
+    b = next;
   }
 }
 
@@ -340,28 +370,27 @@ bool is_pow2(int64_t x) { return x > 0 && (x & (x - 1)) == 0; }
 
 }  // namespace
 
-// Launches the transposing pack when it serves the call (true), else launches
-// nothing. `es`: bytes per element of the pack's type; src / dst with their
-// offsets applied.
-bool iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, const char* src, char* dst,
-                                hipStream_t stream) {
+// Launches the transposing pack when it serves the call and returns its name,
+// else launches nothing and returns NULL. `es`: bytes per element of the pack's
+// type; src / dst with their offsets applied.
+const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, const char* src, char* dst,
+                                       hipStream_t stream) {
   const bool ti = p->flags & IREE_UK_FLAG_PACK_TRANSPOSE_INNER;
   const bool to = p->flags & IREE_UK_FLAG_PACK_TRANSPOSE_OUTER;
-  if (p->in_stride1 != 1 || p->in_stride0 < 0) return false;
+  if (p->in_stride1 != 1 || p->in_stride0 < 0) return nullptr;
   // Element of the transposition and the tile's extents in such elements:
   // t0 along the matrix rows, t1 along its columns.
   int eb;
   int64_t t0, t1, size1;
   if (ti) {
-    if (es > 4) return false;
+    if (es > 4) return nullptr;
     eb = es; t0 = p->out_size3; t1 = p->out_size2; size1 = p->in_size1;
   } else {
     // Tile rows of one, two or four bytes: the row is the element.
-    if (p->out_size3 * es > 4) return false;
+    if (p->out_size3 * es > 4) return nullptr;
     eb = (int)(p->out_size3 * es);
-    if (eb != 1 && eb != 2 && eb != 4) return false;
-    if (p->in_size1 % p->out_size3 != 0) return false;  // (a last row of half padding)
-    t0 = p->out_size2; t1 = 1; size1 = p->in_size1 / p->out_size3;
+    if (eb != 1 && eb != 2 && eb != 4) return nullptr;
+    t0 = p->out_size2; t1 = 1; size1 = uk::ceil_div(p->in_size1, p->out_size3);
   }
   const int64_t tile_bytes = t0 * t1 * eb;
   const int64_t outer0 = to ? p->out_size1 : p->out_size0;  // tiles along the matrix rows
@@ -372,29 +401,34 @@ bool iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, const ch
   // against 25; 6144 x 6144: 49 against 67), beyond that the other one, with
   // its 64 KB blocks (12288 x 12288: 241 against 194 us, 288 against 225 under
   // TRANSPOSE_OUTER).
-  if (eb == 4 && p->in_size0 * size1 * eb + outer0 * outer1 * tile_bytes > (448ll << 20)) return false;
+  if (eb == 4 && p->in_size0 * size1 * eb + outer0 * outer1 * tile_bytes > (448ll << 20)) return nullptr;
   const int64_t bc = kBlockRowBytes / eb;
-  if (!is_pow2(t0) || !is_pow2(t1) || t0 > kBlockRows || t1 > bc) return false;
+  if (!is_pow2(t0) || !is_pow2(t1) || t0 > kBlockRows || t1 > bc) return nullptr;
   // Tiles less than eight bytes tall: rows interleaved in registers, a vector
   // of 16 / (t0 * eb) columns inside one tile.
   const int il = (t0 * eb == 2 || t0 * eb == 4) && t0 > 1 ? (int)t0 : 0;
-  if (il ? t1 * t0 * eb < 16 : (t0 * eb) % (eb == 4 ? 16 : 8) != 0) return false;
+  if (il ? t1 * t0 * eb < 16 : (t0 * eb) % (eb == 4 ? 16 : 8) != 0) return nullptr;
   const int V = il || (t0 * eb) % 16 == 0 ? 16 : 8;
   const int64_t s_outer = p->out_stride0 * es;
   const int64_t s0 = to ? tile_bytes : s_outer;
   const int64_t s1 = to ? s_outer : tile_bytes;
   const int64_t pitch = p->in_stride0 * es;
-  if (s_outer < 0) return false;
-  // Alignment: 4 bytes on the matrix side, the store width on the tiled side.
-  if (((uintptr_t)src | (uint64_t)pitch) & 3) return false;
-  if (((uintptr_t)dst | (uint64_t)s0 | (uint64_t)s1) & (uint64_t)(V - 1)) return false;
+  if (s_outer < 0) return nullptr;
+  // Alignment: none beyond the element's on the matrix side (rows of odd length
+  // are the ordinary case of a ragged matrix: bf16 777 x 1501 from [K][N] takes 4.2
+  // us here and 22 on the kernel for narrow alignments, f16 4095 x 6001 20 and
+  // 80), the store width on the tiled side.
+  if (((uintptr_t)dst | (uint64_t)s0 | (uint64_t)s1) & (uint64_t)(V - 1)) return nullptr;
   const int64_t tiles0 = kBlockRows / t0, tiles1 = bc / t1;
   // 32-bit offsets inside a block, 32-bit sizes.
-  if (pitch * kBlockRows >= (1ll << 31) || tiles0 * s0 + tiles1 * s1 >= (1ll << 31)) return false;
-  if (p->in_size0 >= (1ll << 31) || size1 * eb >= (1ll << 31) || outer0 >= (1ll << 24) || outer1 >= (1ll << 24)) return false;
+  if (pitch * kBlockRows >= (1ll << 31) || tiles0 * s0 + tiles1 * s1 >= (1ll << 31)) return nullptr;
+  if (p->in_size0 >= (1ll << 31) || size1 * eb >= (1ll << 31) || outer0 >= (1ll << 24) || outer1 >= (1ll << 24)) return nullptr;
   const int64_t nblk0 = uk::ceil_div(outer0, tiles0), nblk1 = uk::ceil_div(outer1, tiles1);
-  if (nblk0 * nblk1 >= (1ll << 31) || nblk0 * nblk1 == 0) return false;
+  if (nblk0 * nblk1 >= (1ll << 31) || nblk0 * nblk1 == 0) return nullptr;
 
+  // Rows that are not whole words apart, or that end inside a tile row.
+  const bool ragged = (((uintptr_t)src | (uint64_t)pitch) & 3) || (!ti && p->in_size1 % p->out_size3 != 0);
+  const char* name = ragged ? "pack_transposing_ragged" : "pack_transposing";
   TrArgs a{};
   a.src = src;
   a.dst = dst;
@@ -402,7 +436,7 @@ bool iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, const ch
   a.s0 = s0;
   a.s1 = s1;
   a.rows = (uint32_t)p->in_size0;
-  a.row_bytes = (uint32_t)(size1 * eb);
+  a.row_bytes = (uint32_t)(p->in_size1 * es);
   a.outer0 = (uint32_t)outer0;
   a.outer1 = (uint32_t)outer1;
   a.lt0 = log2_exact(t0);
@@ -423,18 +457,33 @@ bool iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, const ch
   a.pad32 = es == 1 ? (uint32_t)(pad * 0x01010101ull) : es == 2 ? (uint32_t)(pad * 0x00010001ull) : (uint32_t)pad;
   const uint32_t nblocks = (uint32_t)(nblk0 * nblk1);
   const size_t lds = 2 * (size_t)a.lds_buf_bytes;
-  const uint32_t grid = nblocks < 1024 ? nblocks : 1024;
+  // Two workgroups per compute unit, four where that leaves them two blocks or
+  // less each (f16 4096 x 4096: 13.7 against 14.2 us, f32 4096 x 4096 24.5
+  // against 23.6, s8 9000 x 9000 27.4 against 27.1).
+  const uint32_t grid = std::min<uint32_t>(nblocks, nblocks <= 2048 ? 1024 : 512);
+  // Non-temporal stores from 72 MB of tiles on. They make the pack itself the
+  // faster one from some 10 MB on (f16 4096 x 4096: 13.3 against 14.2 us), but
+  // what they write has to come from HBM again, and up to that size the next
+  // kernel finds it in the memory-side cache otherwise (the unpack that follows:
+  // 21.3 against 16.4 us; f32 4096 x 4096, 67 MB: 29.4 + 23.8 against 23.6 +
+  // 21.7; f16 6000 x 8192, 98 MB: 37.5 + 51.5 against 39.8 + 58).
+  const bool nts = outer0 * outer1 * tile_bytes >= (72ll << 20);
   const dim3 block(kBlockRows * kBlockRowBytes / 64);
-  if (il) {
-    if (eb == 2) uk::launch(0, pack_tr_kernel<2, 16, 2>, dim3(grid), block, lds, stream, a);
-    else if (il == 2) uk::launch(0, pack_tr_kernel<1, 16, 2>, dim3(grid), block, lds, stream, a);
-    else uk::launch(0, pack_tr_kernel<1, 16, 4>, dim3(grid), block, lds, stream, a);
-    return true;
-  }
-  if (eb == 4) uk::launch(0, pack_tr_kernel<4, 16>, dim3(grid), block, lds, stream, a);
-  else if (eb == 2 && V == 16) uk::launch(0, pack_tr_kernel<2, 16>, dim3(grid), block, lds, stream, a);
-  else if (eb == 2) uk::launch(0, pack_tr_kernel<2, 8>, dim3(grid), block, lds, stream, a);
-  else if (V == 16) uk::launch(0, pack_tr_kernel<1, 16>, dim3(grid), block, lds, stream, a);
-  else uk::launch(0, pack_tr_kernel<1, 8>, dim3(grid), block, lds, stream, a);
-  return true;
+  auto go = [&](auto eb_c, auto v_c, auto il_c) {
+    constexpr int EB = decltype(eb_c)::value, VV = decltype(v_c)::value, IL = decltype(il_c)::value;
+    if (nts) uk::launch(0, pack_tr_kernel<EB, VV, IL, true>, dim3(grid), block, lds, stream, a);
+    else uk::launch(0, pack_tr_kernel<EB, VV, IL, false>, dim3(grid), block, lds, stream, a);
+  };
+  using std::integral_constant;
+  typedef integral_constant<int, 0> I0; typedef integral_constant<int, 1> I1; typedef integral_constant<int, 2> I2;
+  typedef integral_constant<int, 4> I4; typedef integral_constant<int, 8> I8; typedef integral_constant<int, 16> I16;
+  if (il && eb == 2) go(I2{}, I16{}, I2{});
+  else if (il == 2) go(I1{}, I16{}, I2{});
+  else if (il) go(I1{}, I16{}, I4{});
+  else if (eb == 4) go(I4{}, I16{}, I0{});
+  else if (eb == 2 && V == 16) go(I2{}, I16{}, I0{});
+  else if (eb == 2) go(I2{}, I8{}, I0{});
+  else if (V == 16) go(I1{}, I16{}, I0{});
+  else go(I1{}, I8{}, I0{});
+  return name;
 }

@@ -161,6 +161,7 @@ struct TiledArgs {
   uint32_t lds_buf_bytes;           // one LDS buffer of the streaming kernels
   uint32_t mat_stride0_bytes32;     // == mat_stride0_bytes when it fits
   uint32_t sl0_bytes32, sl1_bytes32;
+  uint32_t band, grp;               // walk: bands of block rows, groups of block columns
   uint32_t streaming_stores;        // 16 KB-block streaming kernels: non-temporal stores
 };
 
@@ -432,7 +433,10 @@ __global__ __launch_bounds__(kThreads) void unpack_tiled_kernel(TiledArgs a) {
 //     thread and the block shape (global offsets inside a block, LDS offsets
 //     of every granule) is computed once, before the walk;
 //   * all loads of a phase are issued before any of their data is used, one
-//     or two blocks ahead of their use;
+//     block ahead of their use, and stay in flight across the barrier while
+//     the block before is stored (f32 12288 x 12289 unpack 254 -> 248 us, f16
+//     4096 x 4096 unpack 14.8 -> 13.5, f32 12288 x 12289 untransposed 229 / 255
+//     -> 210 / 229);
 //   * LDS is double-buffered, one barrier per block, so the stores of block b
 //     and the loads of the following blocks are in flight together;
 //   * interior blocks in which every thread has all of its items run without
@@ -448,9 +452,9 @@ template <> struct GBytes<4> { using type = uint32_t; };
 template <> struct GBytes<8> { using type = v2u; };
 template <> struct GBytes<16> { using type = v4u; };
 
-// Global accesses of the streaming kernels. Addresses are 4-byte aligned at
-// least; wider vectors at such addresses are legal on gfx950 under HSA
-// (unaligned access mode), and the types say so.
+// Global accesses of the streaming kernels. Addresses have the element's
+// alignment and no more; vectors at such addresses are legal on gfx950 under
+// HSA (unaligned access mode), and the types say so.
 // Plain (cache-allocating) accesses on purpose: what pack writes is read by
 // mmt4d next, and what unpack reads was just written by mmt4d, so for operands
 // up to the size of the memory-side cache the hand-over never reaches HBM.
@@ -458,27 +462,17 @@ template <> struct GBytes<16> { using type = v4u; };
 // kernel reads again (see TiledPlan::streaming_loads).
 template <int N, bool STREAMING = false>
 __device__ __forceinline__ typename GBytes<N>::type gload(const char* gptr) {
-  typedef typename GBytes<N>::type T4 __attribute__((aligned(4)));
-  if constexpr (STREAMING) return __builtin_nontemporal_load(reinterpret_cast<const T4*>(gptr));
-  else return *reinterpret_cast<const T4*>(gptr);
+  typedef typename GBytes<N>::type T1 __attribute__((aligned(1)));
+  if constexpr (STREAMING) return __builtin_nontemporal_load(reinterpret_cast<const T1*>(gptr));
+  else return *reinterpret_cast<const T1*>(gptr);
 }
 // STREAMING: a non-temporal store, for the 64 KB-block kernels, whose output is
 // larger than the memory-side cache anyway (measured 3 % on a plain copy).
 template <int N, bool STREAMING = false>
 __device__ __forceinline__ void gstore(char* gptr, typename GBytes<N>::type v) {
-  typedef typename GBytes<N>::type T4 __attribute__((aligned(4)));
-  if constexpr (STREAMING) __builtin_nontemporal_store(v, reinterpret_cast<T4*>(gptr));
-  else *reinterpret_cast<T4*>(gptr) = v;
-}
-
-// The non-temporal store chosen at run time, as assembly: beside a plain
-// store of the same value to the same address in the other branch, the
-// compiler merges the two into one plain store.
-template <int N>
-__device__ __forceinline__ void gstore_nt_asm(char* gptr, typename GBytes<N>::type v) {
-  if constexpr (N == 16) asm volatile("global_store_dwordx4 %0, %1, off nt" : : "v"(gptr), "v"(v) : "memory");
-  else if constexpr (N == 8) asm volatile("global_store_dwordx2 %0, %1, off nt" : : "v"(gptr), "v"(v) : "memory");
-  else asm volatile("global_store_dword %0, %1, off nt" : : "v"(gptr), "v"(v) : "memory");
+  typedef typename GBytes<N>::type T1 __attribute__((aligned(1)));
+  if constexpr (STREAMING) __builtin_nontemporal_store(v, reinterpret_cast<T1*>(gptr));
+  else *reinterpret_cast<T1*>(gptr) = v;
 }
 
 constexpr uint32_t kStreamBlockBytes = 16384;     // matrix bytes per block, streaming kernels
@@ -513,28 +507,7 @@ __device__ __forceinline__ void tiled_item(const TiledArgs& a, uint32_t idx,
   *tl1 = a.transpose_outer ? *run : *t;
 }
 
-template <int N>
-__device__ __forceinline__ void lds_store_pieces(char* dst, typename GBytes<N>::type v,
-                                                 uint32_t piece) {
-  if (piece >= N) {
-    *reinterpret_cast<typename GBytes<N>::type*>(dst) = v;
-  } else {
-    __attribute__((aligned(16))) char tmp[N];
-    *reinterpret_cast<typename GBytes<N>::type*>(tmp) = v;
-    store_pieces<N>(dst, tmp, piece);
-  }
-}
-template <int N>
-__device__ __forceinline__ typename GBytes<N>::type lds_load_pieces(const char* src,
-                                                                     uint32_t piece) {
-  if (piece >= N) return *reinterpret_cast<const typename GBytes<N>::type*>(src);
-  __attribute__((aligned(16))) char tmp[N];
-  load_pieces<N>(tmp, src, piece);
-  return *reinterpret_cast<const typename GBytes<N>::type*>(tmp);
-}
-
-// The same with the piece size known at compile time (P divides N, P >= 4):
-// the hot path of the streaming kernels picks P once per block.
+// A vector of N bytes to / from LDS in accesses of P bytes (P divides N, P >= 4).
 template <int N> struct Words { uint32_t w[N / 4]; };
 template <int N, int P>
 __device__ __forceinline__ void lds_store_static(char* dst, typename GBytes<N>::type v) {
@@ -613,52 +586,36 @@ __device__ __forceinline__ void scatter_granules(char* lbuf, const uint32_t (&of
         __builtin_bit_cast(typename GBytes<G>::type, y);
   }
 }
-// Calls f with the piece size as a compile-time constant (4, 8 or 16, capped
-// at N); false when `piece` is none of them.
-template <int N, typename F>
-__device__ __forceinline__ bool with_static_piece(uint32_t piece, F f) {
-  if (piece >= N) { f(std::integral_constant<int, N>{}); return true; }
-  if (N > 8 && piece == 8) { f(std::integral_constant<int, (N > 8 ? 8 : N)>{}); return true; }
-  if (N > 4 && piece == 4) { f(std::integral_constant<int, 4>{}); return true; }
-  return false;
-}
-
-template <int G, int VEC, int MV, bool UNPACK, int BLK, int NT = kThreads, int DEPTH = 2, bool NTL = false>
+// NTL / NTS: the loads / stores are non-temporal.
+template <int G, int VEC, int MV, bool UNPACK, int BLK, int NT, bool NTL, bool NTS>
 __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int N1 = BLK / MV / NT;   // 2-D side items per thread
   constexpr int N2 = BLK / VEC / NT;  // tiled side items per thread
   constexpr int NG = VEC / G;                             // granules per tiled vector
-  constexpr bool kStreamingStores = BLK > (int)kStreamBlockBytes;
+  constexpr int P = G < MV ? G : MV;                      // LDS access width on a row (rows are G-aligned)
   using MatVec = typename GBytes<MV>::type;
   using TileVec = typename GBytes<VEC>::type;
   static_assert(G >= 4, "streaming kernels move granules of at least 4 bytes");
 
-  // Non-temporal in the 64 KB-block kernels, and in the others when the host
-  // asks for it (outputs beyond the memory-side cache).
-  const bool nt_stores = kStreamingStores || a.streaming_stores;
-  auto store_tiled = [&](char* p, TileVec v) {
-    if constexpr (kStreamingStores) gstore<VEC, true>(p, v);
-    else if (nt_stores) gstore_nt_asm<VEC>(p, v);
-    else gstore<VEC, false>(p, v);
-  };
-  auto store_mat = [&](char* p, MatVec v) {
-    if constexpr (kStreamingStores) gstore<MV, true>(p, v);
-    else if (nt_stores) gstore_nt_asm<MV>(p, v);
-    else gstore<MV, false>(p, v);
-  };
+  uk::load_arguments_now(a.src, a.dst, a.mat_stride0_bytes, a.sl0_bytes, a.sl1_bytes, a.mat_size0, a.mat_size1, a.outer0,
+                         a.outer1, a.tile0, a.tile1, a.G0, a.G1, a.nblk1, a.lds_pitch, a.elem_bytes, a.block_rows,
+                         a.block_row_bytes, a.transpose_inner, a.transpose_outer, a.pad32, a.tile_bytes, a.num_runs,
+                         a.run_vecs, a.div_row_vecs.mul, a.div_run_vecs.mul, a.div_tile_bytes.mul, a.nblk0,
+                         a.lds_buf_bytes, a.mat_stride0_bytes32, a.sl0_bytes32, a.sl1_bytes32, a.band, a.grp, gridDim.x);
   const uint32_t tid = threadIdx.x;
   const uint32_t total1 = a.block_rows * a.div_row_vecs.d;
   const uint32_t total2 = a.num_runs * a.run_vecs;
-  const uint32_t piece = a.lds_piece < MV ? a.lds_piece : MV;
   const uint32_t size1_bytes = a.mat_size1 * a.elem_bytes;
 
   // ---- per-thread tables (block independent) ----------------------------
+  // Items beyond the block (blocks smaller than N1 x NT or N2 x NT vectors)
+  // stand on item 0: what they load exists and goes nowhere.
   uint32_t g1off[N1], l1off[N1];
 #pragma unroll
   for (int i = 0; i < N1; ++i) {
     uint32_t r, cb;
-    mat_item<MV>(a, tid + i * NT, &r, &cb);
+    mat_item<MV>(a, tid + i * NT < total1 ? tid + i * NT : 0, &r, &cb);
     g1off[i] = r * a.mat_stride0_bytes32 + cb;
     l1off[i] = r * a.lds_pitch + cb;
   }
@@ -666,7 +623,7 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
 #pragma unroll
   for (int i = 0; i < N2; ++i) {
     uint32_t run, t, in_tile, tl0, tl1;
-    tiled_item<VEC>(a, tid + i * NT, &run, &t, &in_tile, &tl0, &tl1);
+    tiled_item<VEC>(a, tid + i * NT < total2 ? tid + i * NT : 0, &run, &t, &in_tile, &tl0, &tl1);
     g2off[i] = tl0 * a.sl0_bytes32 + tl1 * a.sl1_bytes32 + in_tile;
     for_each_granule<G, VEC>(a, run, t, in_tile, [&](int k, uint32_t off) { l2off[i][k] = off; });
   }
@@ -692,92 +649,149 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
   }
 
   const uint32_t nblocks = a.nblk0 * a.nblk1;
-  // Every thread has all of its N1 and N2 items and the LDS piece size is one
-  // of the compile-time cases: interior blocks then run without per-item
-  // bounds checks and with the piece size resolved once per block.
-  const bool full = total1 == (uint32_t)N1 * NT && total2 == (uint32_t)N2 * NT &&
-                    (piece >= MV || piece == 8 || piece == 4);
+  // Every thread has all of its N1 and N2 items: interior blocks then run
+  // without per-item bounds checks.
+  const bool full = total1 == (uint32_t)N1 * NT && total2 == (uint32_t)N2 * NT;
 
-  // Block coordinates, base pointers and whether the whole block lies inside
-  // the matrix and the tile grid ("interior").
+  // Block coordinates and whether the whole block lies inside the matrix and
+  // the tile grid ("interior").
   struct Block {
     uint32_t blk0, blk1, row_base, col_base_bytes;
-    const char* mat_c;
-    const char* tiled_c;
-    bool interior;
+    uint32_t interior;
   };
   auto block_at = [&](uint32_t blk) {
     Block b;
-    b.blk0 = blk / a.nblk1;
-    b.blk1 = blk - b.blk0 * a.nblk1;
+    const uint32_t per_band = a.band * a.nblk1;
+    const uint32_t bd = blk / per_band, rem = blk - bd * per_band;
+    const uint32_t rows = min(a.band, a.nblk0 - bd * a.band);
+    const uint32_t per_grp = rows * a.grp, g = rem / per_grp, rem2 = rem - g * per_grp;
+    const uint32_t w = min(a.grp, a.nblk1 - g * a.grp), rr = rem2 / w;
+    b.blk0 = bd * a.band + rr;
+    b.blk1 = g * a.grp + (rem2 - rr * w);
     b.row_base = b.blk0 * a.block_rows;
     b.col_base_bytes = b.blk1 * a.block_row_bytes;
-    b.mat_c = (UNPACK ? a.dst : a.src) + (int64_t)b.row_base * a.mat_stride0_bytes + b.col_base_bytes;
-    b.tiled_c = (UNPACK ? a.src : a.dst) + (int64_t)(b.blk0 * a.G0) * a.sl0_bytes +
-                (int64_t)(b.blk1 * a.G1) * a.sl1_bytes;
-    b.interior = b.row_base + a.block_rows <= a.mat_size0 &&
-                 b.col_base_bytes + a.block_row_bytes <= size1_bytes &&
-                 (b.blk0 + 1) * a.G0 <= a.outer0 && (b.blk1 + 1) * a.G1 <= a.outer1;
+    b.interior = (b.row_base + a.block_rows <= a.mat_size0) &
+                 (b.col_base_bytes + a.block_row_bytes <= size1_bytes) &
+                 ((b.blk0 + 1) * a.G0 <= a.outer0) & ((b.blk1 + 1) * a.G1 <= a.outer1);
     return b;
   };
+  auto tiled_base = [&](const Block& b) {
+    return (int64_t)(b.blk0 * a.G0) * a.sl0_bytes + (int64_t)(b.blk1 * a.G1) * a.sl1_bytes;
+  };
+  // Whether item i's tile exists / how much of its row the matrix still holds.
+  auto tile_exists = [&](const Block& b, int i) {
+    uint32_t run, t, in_tile, tl0, tl1;
+    tiled_item<VEC>(a, tid + i * NT, &run, &t, &in_tile, &tl0, &tl1);
+    return tid + i * NT < total2 && b.blk0 * a.G0 + tl0 < a.outer0 && b.blk1 * a.G1 + tl1 < a.outer1;
+  };
 
-  // The global loads of an interior block are issued DEPTH (1 or 2) blocks
-  // ahead, into one of DEPTH register sets (with two: the parity of the
-  // block's turn), right after the set's previous contents have gone to LDS,
-  // so that a workgroup keeps DEPTH blocks of loads and a block of stores in
-  // flight.
-  static_assert(DEPTH == 1 || DEPTH == 2, "one or two register sets");
-  MatVec pre1[DEPTH][UNPACK ? 1 : N1];
-  TileVec pre2[DEPTH][UNPACK ? N2 : 1];
-  auto prefetch = [&](const Block& b, auto slot_c) {
-    constexpr int S = decltype(slot_c)::value % DEPTH;
-    if (!b.interior) {
-      // Edge block: only what exists is loaded (2-D side: vectors that lie
-      // wholly inside the matrix; tiled side: vectors of tiles that exist);
-      // phase 1 applies the same predicate before it uses a register.
-      if constexpr (!UNPACK) {
+  // The global loads of a block, issued one block ahead, right after the
+  // registers' previous contents have gone to LDS, so that a workgroup keeps a
+  // block of loads and a block of stores in flight. A block on the ragged edge
+  // differs in its addresses only: rows beyond the matrix stand on its last row,
+  // a vector that reaches beyond its row on the row's last bytes (phase 1 puts
+  // it right), tiles that do not exist on the block's first tile. The loads
+  // themselves are the same straight-line code for every block: with loads of
+  // their own in the branches of the two cases the compiler moved registers
+  // where the branches met, and had to wait for every load before the barrier,
+  // which left nothing in flight while a block was stored.
+  MatVec pre1[UNPACK ? 1 : N1];
+  TileVec pre2[UNPACK ? N2 : 1];
+  auto prefetch = [&](uint32_t blk) __attribute__((always_inline)) {
+    const Block b = block_at(blk);
+    if constexpr (!UNPACK) {
+      const uint32_t row0 = min(b.row_base, a.mat_size0 - 1), col0 = uk::clipped_offset<MV>(b.col_base_bytes, size1_bytes);
+      const char* base = a.src + (int64_t)row0 * a.mat_stride0_bytes + col0;
+      uint32_t off[N1];
+#pragma unroll
+      for (int i = 0; i < N1; ++i) off[i] = g1off[i];
+      if (!b.interior) {
 #pragma unroll
         for (int i = 0; i < N1; ++i) {
-          const uint32_t idx = tid + i * NT;
-          if (idx < total1) {
-            uint32_t r, cb;
-            mat_item<MV>(a, idx, &r, &cb);
-            if (b.row_base + r < a.mat_size0 && b.col_base_bytes + cb + MV <= size1_bytes)
-              pre1[S][i] = gload<MV>(b.mat_c + g1off[i]);
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < N2; ++i) {
-          const uint32_t idx = tid + i * NT;
-          if (idx < total2) {
-            uint32_t run, t, in_tile, tl0, tl1;
-            tiled_item<VEC>(a, idx, &run, &t, &in_tile, &tl0, &tl1);
-            if (b.blk0 * a.G0 + tl0 < a.outer0 && b.blk1 * a.G1 + tl1 < a.outer1)
-              pre2[S][i] = gload<VEC>(b.tiled_c + g2off[i]);
-          }
+          uint32_t r, cb;
+          mat_item<MV>(a, tid + i * NT < total1 ? tid + i * NT : 0, &r, &cb);
+          off[i] = (min(b.row_base + r, a.mat_size0 - 1) - row0) * a.mat_stride0_bytes32 +
+                   (uk::clipped_offset<MV>(b.col_base_bytes + cb, size1_bytes) - col0);
         }
       }
-      return;
-    }
-    if (full) {
-      if constexpr (!UNPACK) {
 #pragma unroll
-        for (int i = 0; i < N1; ++i) pre1[S][i] = gload<MV, NTL>(b.mat_c + g1off[i]);
-      } else {
+      for (int i = 0; i < N1; ++i) pre1[i] = gload<MV, NTL>(base + off[i]);
+    } else {
+      const char* base = a.src + tiled_base(b);
+      uint32_t off[N2];
 #pragma unroll
-        for (int i = 0; i < N2; ++i) pre2[S][i] = gload<VEC, NTL>(b.tiled_c + g2off[i]);
+      for (int i = 0; i < N2; ++i) off[i] = g2off[i];
+      if (!b.interior) {
+#pragma unroll
+        for (int i = 0; i < N2; ++i)
+          if (!tile_exists(b, i)) off[i] = 0;
       }
-      return;
+#pragma unroll
+      for (int i = 0; i < N2; ++i) pre2[i] = gload<VEC, NTL>(base + off[i]);
     }
+  };
+
+  // Phase 1 of a block that every thread has all items of: registers -> LDS.
+  auto phase1_full = [&](char* lbuf) __attribute__((always_inline)) {
     if constexpr (!UNPACK) {
 #pragma unroll
-      for (int i = 0; i < N1; ++i)
-        if (tid + i * NT < total1) pre1[S][i] = gload<MV>(b.mat_c + g1off[i]);
+      for (int i = 0; i < N1; ++i) lds_store_static<MV, P>(lbuf + l1off[i], pre1[i]);
     } else {
 #pragma unroll
+      for (int i = 0; i < N2; ++i) scatter_granules<VEC, G>(lbuf, l2off[i], pre2[i], rot);
+    }
+  };
+  auto phase1 = [&](const Block& b, char* lbuf) __attribute__((always_inline)) {
+    if constexpr (!UNPACK) {
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        uint32_t r, cb;
+        mat_item<MV>(a, tid + i * NT, &r, &cb);
+        const int32_t left =
+            b.row_base + r < a.mat_size0 ? (int32_t)(size1_bytes - (b.col_base_bytes + cb)) : 0;
+        Words<MV> w = __builtin_bit_cast(Words<MV>, pre1[i]);
+        uk::clip_piece<MV>(w.w, left, a.pad32);
+        if (tid + i * NT < total1) lds_store_static<MV, P>(lbuf + l1off[i], __builtin_bit_cast(MatVec, w));
+      }
+    } else {
+      // (what stands for tiles that do not exist lands beyond the matrix)
+#pragma unroll
       for (int i = 0; i < N2; ++i)
-        if (tid + i * NT < total2) pre2[S][i] = gload<VEC>(b.tiled_c + g2off[i]);
+        if (tid + i * NT < total2) scatter_granules<VEC, G>(lbuf, l2off[i], pre2[i], rot);
+    }
+  };
+  // Phase 2: LDS -> destination.
+  auto phase2 = [&](const Block& b, const char* lbuf, auto inside_c) __attribute__((always_inline)) {
+    constexpr bool kInside = decltype(inside_c)::value;  // interior block, all items
+    if constexpr (!UNPACK) {
+      char* base = a.dst + tiled_base(b);
+      TileVec reg[N2];
+#pragma unroll
+      for (int i = 0; i < N2; ++i) reg[i] = gather_granules<VEC, G>(lbuf, l2off[i], rot);
+#pragma unroll
+      for (int i = 0; i < N2; ++i)
+        if (kInside || tile_exists(b, i)) gstore<VEC, NTS>(base + g2off[i], reg[i]);
+    } else {
+      char* base = a.dst + (int64_t)b.row_base * a.mat_stride0_bytes + b.col_base_bytes;
+      MatVec reg[N1];
+#pragma unroll
+      for (int i = 0; i < N1; ++i) reg[i] = lds_load_static<MV, P>(lbuf + l1off[i]);
+#pragma unroll
+      for (int i = 0; i < N1; ++i) {
+        if constexpr (kInside) {
+          gstore<MV, NTS>(base + g1off[i], reg[i]);
+        } else {
+          uint32_t r, cb;
+          mat_item<MV>(a, tid + i * NT, &r, &cb);
+          if (tid + i * NT >= total1 || b.row_base + r >= a.mat_size0) continue;
+          const int32_t left = (int32_t)(size1_bytes - (b.col_base_bytes + cb));
+          if (left >= MV) {
+            gstore<MV, NTS>(base + g1off[i], reg[i]);
+          } else if (left > 0) {
+            uk::store_head<MV>(base + g1off[i], __builtin_bit_cast(Words<MV>, reg[i]).w, (uint32_t)left);
+          }
+        }
+      }
     }
   };
 
@@ -786,187 +800,49 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
   // of one block row first): neighbouring blocks share the cache lines that
   // their unaligned row segments straddle, and the L2 of the XCD then sees
   // both halves of such a line at about the same time.
-  const uint32_t first_blk = (gridDim.x & 7) ? blockIdx.x
-                                             : (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  bool have_pre[2] = {false, false};
-  auto process = [&](uint32_t blk, auto slot_c) {
-    constexpr int L = decltype(slot_c)::value;  // LDS buffer: parity of the turn
-    constexpr int S = L % DEPTH;                // register set
-    const Block b = block_at(blk);
-    const uint32_t blk0 = b.blk0, blk1 = b.blk1, row_base = b.row_base,
-                   col_base_bytes = b.col_base_bytes;
-    const char* mat_c = b.mat_c;
-    const char* tiled_c = b.tiled_c;
-    const bool interior = b.interior;
-    char* lbuf = lds + L * a.lds_buf_bytes;
-    if (!have_pre[S]) prefetch(b, slot_c);
-
-    if constexpr (!UNPACK) {
-      // ---- pack phase 1: 2-D rows -> LDS ----
-      if (interior && full) {
-        with_static_piece<MV>(piece, [&](auto pc) {
-          constexpr int P = decltype(pc)::value;
-#pragma unroll
-          for (int i = 0; i < N1; ++i) lds_store_static<MV, P>(lbuf + l1off[i], pre1[S][i]);
-        });
-      } else if (interior) {
-#pragma unroll
-        for (int i = 0; i < N1; ++i)
-          if (tid + i * NT < total1) lds_store_pieces<MV>(lbuf + l1off[i], pre1[S][i], piece);
-      } else {
-#pragma unroll
-        for (int i = 0; i < N1; ++i) {
-          const uint32_t idx = tid + i * NT;
-          if (idx >= total1) continue;
-          uint32_t r, cb;
-          mat_item<MV>(a, idx, &r, &cb);
-          __attribute__((aligned(16))) char reg[MV];
-          const bool row_ok = row_base + r < a.mat_size0;
-          const char* gp = mat_c + (r * a.mat_stride0_bytes32 + cb);
-          const uint32_t es = a.elem_bytes;
-          // Whole vector inside the matrix (already loaded), or whole vector
-          // padding: one access.
-          if (row_ok && col_base_bytes + cb + MV <= size1_bytes) {
-            lds_store_pieces<MV>(lbuf + l1off[i], pre1[S][i], piece);
-            continue;
-          }
-          if (!row_ok || col_base_bytes + cb >= size1_bytes) {
-            MatVec padv;
-            uint32_t* pw = reinterpret_cast<uint32_t*>(&padv);
-#pragma unroll
-            for (int w = 0; w < MV / 4; ++w) pw[w] = a.pad32;
-            lds_store_pieces<MV>(lbuf + r * a.lds_pitch + cb, padv, piece);
-            continue;
-          }
-          for (uint32_t bb = 0; bb < MV; bb += es) {
-            const bool ok = row_ok && (col_base_bytes + cb + bb) < size1_bytes;
-            if (es == 4) {
-              *reinterpret_cast<uint32_t*>(reg + bb) =
-                  ok ? *reinterpret_cast<const uint32_t*>(gp + bb) : a.pad32;
-            } else if (es == 2) {
-              *reinterpret_cast<uint16_t*>(reg + bb) =
-                  ok ? *reinterpret_cast<const uint16_t*>(gp + bb) : (uint16_t)a.pad32;
-            } else {
-              reg[bb] = ok ? gp[bb] : (char)a.pad32;
-            }
-          }
-          store_pieces<MV>(lbuf + r * a.lds_pitch + cb, reg, piece);
-        }
-      }
-    } else {
-      // ---- unpack phase 1: tiled runs -> LDS (scatter by granules) ----
-      if (interior && full) {
-#pragma unroll
-        for (int i = 0; i < N2; ++i) scatter_granules<VEC, G>(lbuf, l2off[i], pre2[S][i], rot);
-      } else {
-      bool ok[N2];
-#pragma unroll
-      for (int i = 0; i < N2; ++i) {
-        ok[i] = tid + i * NT < total2;
-        if (!interior) {
-          if (ok[i]) {
-            uint32_t run, t, in_tile, tl0, tl1;
-            tiled_item<VEC>(a, tid + i * NT, &run, &t, &in_tile, &tl0, &tl1);
-            ok[i] = blk0 * a.G0 + tl0 < a.outer0 && blk1 * a.G1 + tl1 < a.outer1;
-          }
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < N2; ++i) {
-        if (ok[i]) scatter_granules<VEC, G>(lbuf, l2off[i], pre2[S][i], rot);
-      }
-      }
-    }
-
-    // This register set's next block, DEPTH turns on.
-    have_pre[S] = false;
-    if (blk + DEPTH * gridDim.x < nblocks) {
-      prefetch(block_at(blk + DEPTH * gridDim.x), slot_c);
-      have_pre[S] = true;
-    }
-    __syncthreads();
-
-    if constexpr (!UNPACK) {
-      // ---- pack phase 2: LDS -> tiled runs ----
-      TileVec reg[N2];
-      if (interior && full) {
-#pragma unroll
-        for (int i = 0; i < N2; ++i) reg[i] = gather_granules<VEC, G>(lbuf, l2off[i], rot);
-#pragma unroll
-        for (int i = 0; i < N2; ++i) store_tiled(const_cast<char*>(tiled_c) + g2off[i], reg[i]);
-        return;
-      }
-#pragma unroll
-      for (int i = 0; i < N2; ++i) {
-        if (tid + i * NT < total2) reg[i] = gather_granules<VEC, G>(lbuf, l2off[i], rot);
-      }
-#pragma unroll
-      for (int i = 0; i < N2; ++i) {
-        if (tid + i * NT < total2) {
-          bool ok = true;
-          if (!interior) {
-            uint32_t run, t, in_tile, tl0, tl1;
-            tiled_item<VEC>(a, tid + i * NT, &run, &t, &in_tile, &tl0, &tl1);
-            ok = blk0 * a.G0 + tl0 < a.outer0 && blk1 * a.G1 + tl1 < a.outer1;
-          }
-          if (ok) store_tiled(const_cast<char*>(tiled_c) + g2off[i], reg[i]);
-        }
-      }
-    } else {
-      // ---- unpack phase 2: LDS rows -> 2-D rows ----
-      if (interior && full) {
-        MatVec reg[N1];
-        with_static_piece<MV>(piece, [&](auto pc) {
-          constexpr int P = decltype(pc)::value;
-#pragma unroll
-          for (int i = 0; i < N1; ++i) reg[i] = lds_load_static<MV, P>(lbuf + l1off[i]);
-        });
-#pragma unroll
-        for (int i = 0; i < N1; ++i) store_mat(const_cast<char*>(mat_c) + g1off[i], reg[i]);
-      } else if (interior) {
-        MatVec reg[N1];
-#pragma unroll
-        for (int i = 0; i < N1; ++i)
-          if (tid + i * NT < total1) reg[i] = lds_load_pieces<MV>(lbuf + l1off[i], piece);
-#pragma unroll
-        for (int i = 0; i < N1; ++i)
-          if (tid + i * NT < total1) store_mat(const_cast<char*>(mat_c) + g1off[i], reg[i]);
-      } else {
-        const uint32_t es = a.elem_bytes;
-        for (uint32_t idx = tid; idx < total1; idx += NT) {
-          uint32_t r, cb;
-          mat_item<MV>(a, idx, &r, &cb);
-          if (row_base + r >= a.mat_size0) continue;
-          char* gp = const_cast<char*>(mat_c) + (r * a.mat_stride0_bytes32 + cb);
-          if (col_base_bytes + cb + MV <= size1_bytes) {  // whole vector inside
-            store_mat(gp, lds_load_pieces<MV>(lbuf + r * a.lds_pitch + cb, piece));
-            continue;
-          }
-          __attribute__((aligned(16))) char reg[MV];
-          load_pieces<MV>(reg, lbuf + r * a.lds_pitch + cb, piece);
-          for (uint32_t bb = 0; bb < MV && col_base_bytes + cb + bb < size1_bytes; bb += es) {
-            if (es == 4) copy_bytes<4>(gp + bb, reg + bb);
-            else if (es == 2) copy_bytes<2>(gp + bb, reg + bb);
-            else gp[bb] = reg[bb];
-          }
-        }
-      }
-    }
-    // No second barrier: the next block uses the other LDS buffer, and its
-    // barrier orders this block's LDS reads before the buffer is reused.
+  uint32_t blk = (gridDim.x & 7) ? blockIdx.x : (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+  if (blk >= nblocks) return;
+  uint32_t buf = 0;  // LDS offset of the buffer whose turn it is
+  // No second barrier per block: the next block uses the other LDS buffer, and
+  // its barrier orders this block's LDS reads before the buffer is reused.
+  auto advance = [&]() __attribute__((always_inline)) {
+    blk += gridDim.x;
+    buf = a.lds_buf_bytes - buf;
   };
-  // Start the pipeline: the first two blocks of this workgroup.
-  if (first_blk < nblocks) {
-    prefetch(block_at(first_blk), std::integral_constant<int, 0>{});
-    have_pre[0] = true;
-    if (DEPTH == 2 && first_blk + gridDim.x < nblocks) {
-      prefetch(block_at(first_blk + gridDim.x), std::integral_constant<int, 1>{});
-      have_pre[1] = true;
+  prefetch(blk);
+  // Interior blocks that are not the last run in a loop of their own whose body
+  // has no branch around a load or a store, and which is entered through a
+  // first copy of the body: the compiler then knows at the loop's head that a
+  // block of stores was issued behind the loads it waits for, and waits for
+  // the loads alone (without the copy, or with the stores in a branch, for the
+  // stores as well).
+  auto steady = [&](const Block& b) { return full && b.interior && blk + gridDim.x < nblocks; };
+  auto steady_body = [&](const Block& b) __attribute__((always_inline)) {
+    phase1_full(lds + buf);
+    prefetch(blk + gridDim.x);
+    __syncthreads();
+    phase2(b, lds + buf, std::true_type{});
+    advance();
+  };
+  while (true) {
+    Block b = block_at(blk);
+    if (steady(b)) {
+      steady_body(b);
+      b = block_at(blk);
+      while (steady(b)) {
+        steady_body(b);
+        b = block_at(blk);
+      }
     }
-  }
-  for (uint32_t blk = first_blk; blk < nblocks; blk += 2 * gridDim.x) {
-    process(blk, std::integral_constant<int, 0>{});
-    if (blk + gridDim.x < nblocks) process(blk + gridDim.x, std::integral_constant<int, 1>{});
+    if (full && (UNPACK || b.interior)) phase1_full(lds + buf);
+    else phase1(b, lds + buf);
+    const bool more = blk + gridDim.x < nblocks;
+    if (more) prefetch(blk + gridDim.x);
+    __syncthreads();
+    if (full && b.interior) phase2(b, lds + buf, std::true_type{});
+    else phase2(b, lds + buf, std::false_type{});
+    if (!more) return;
+    advance();
   }
 }
 
@@ -991,6 +867,7 @@ struct TiledPlan {
   // the walk, and unpack lost 6 % there).
   bool streaming_loads = false;
   uint32_t grid = 0;
+  uint32_t max_workgroups = 512;
   uint32_t lds_bytes = 0;
 };
 
@@ -1026,12 +903,16 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // problems keep the small blocks: they need the parallelism.
   const int64_t total_bytes = v.outer0 * v.outer1 * tile_bytes;
   // Whole tile rows as granules (16 bytes contiguous on both sides, no
-  // transposition) gain from the 64 KB blocks too, from smaller sizes on for
-  // pack than for unpack (f8 28672x8192 pack: 85 -> 65 us; f16 4096x4096
-  // pack: 10.6 -> 10.0 us, slower below that; f32 8192x8192 unpack: 98 -> 74
-  // us, f32 4096x4096 unpack: 19.3 -> 20.0 us).
+  // transposition) gain from the 64 KB blocks too (f8 28672x8192 pack: 85 -> 65
+  // us; f32 8192x8192 unpack: 98 -> 74 us). Their stores are non-temporal, so
+  // what they write has to come from HBM again: a pack whose tiles the
+  // memory-side cache can hand to the next kernel takes the small blocks up to
+  // 72 MB (pack and the unpack that reads it, inputs not in any cache: f16 4096
+  // x 4096 13.0 + 10.6 us against 12.7 + 14.0, f32 4096 x 4096 24.3 + 20.1
+  // against 29.2 + 22.2; f32 4095 x 6001, 98 MB: 45.9 + 31.3 against 38.0 +
+  // 37.1, from where on the pack itself decides).
   const bool big_transposing = G == 4 && total_bytes >= (192ll << 20);
-  const bool big_rows = G == 16 && !to && total_bytes >= ((mat_is_dest ? 192ll : 24ll) << 20);
+  const bool big_rows = G == 16 && !to && total_bytes >= ((mat_is_dest ? 192ll : 72ll) << 20);
   const bool big = allow_big && VEC == 16 && (big_transposing || big_rows);
   const int64_t kMinSpan = big ? 512 : 256;                      // bytes, both sides
   const int64_t kTarget = big ? kStreamBigBlockBytes : kStreamBlockBytes;  // bytes per block, about
@@ -1062,8 +943,11 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   } else {
     // Tiles of one tile row are contiguous on the tiled side, so widening
     // along dim 1 lengthens the segments of both sides; do that up to 1 KB of
-    // matrix row, then add tile rows.
-    while (G0 * G1 * tile_bytes * 2 <= kTarget && G1 * v.tile1 * es < 1024 && G1 < v.outer1) G1 *= 2;
+    // matrix row (4 KB in 64 KB blocks: where rows are not whole cache lines,
+    // fewer lines lie half in the next block; f32 9000 x 9000 in 16x4 tiles,
+    // unpack: 131 us with 1 KB, 126 with 2 KB, 121 with 4 KB; level at 9216 x
+    // 9216), then add tile rows.
+    while (G0 * G1 * tile_bytes * 2 <= kTarget && G1 * v.tile1 * es < (big ? 4096 : 1024) && G1 < v.outer1) G1 *= 2;
     while (G0 * G1 * tile_bytes * 2 <= kTarget) G0 *= 2;
   }
   G0 = std::min<int64_t>(G0, std::max<int64_t>(v.outer0, 1));
@@ -1116,7 +1000,7 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   a.G1 = (uint32_t)G1;
   a.nblk1 = (uint32_t)nblk1;
   a.lds_pitch = (uint32_t)pitch;
-  a.lds_piece = (uint32_t)uk::pow2_divisor(pitch, 16);
+  a.lds_piece = (uint32_t)uk::pow2_divisor(pitch, 16);  // (*_tiled only: the streaming kernels use G)
   a.elem_bytes = (uint32_t)es;
   a.block_rows = (uint32_t)block_rows;
   a.block_row_bytes = (uint32_t)block_row_bytes;
@@ -1139,16 +1023,16 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // Streaming kernels: 32-bit offsets inside one block on both sides, granules
   // of at least 4 bytes, at most 4 granules per vector, block within budget.
   // (and non-negative strides: the 32-bit offsets are unsigned)
-  plan.stream = mat_vec >= 4 && G >= 4 && VEC / G <= 4 && mat_stride0 >= 0 && v.sl0 >= 0 &&
+  plan.stream = block_row_bytes % 4 == 0 && mat_size0 > 0 && mat_size1 * es >= 16 && G >= 4 && VEC / G <= 4 && mat_stride0 >= 0 && v.sl0 >= 0 &&
                 v.sl1 >= 0 &&
                 block_rows * block_row_bytes <= stream_block &&
                 lds_bytes <= (big ? 80 * 1024 : 2 * stream_block) &&
                 block_rows * std::abs(mat_stride0) * es < (1ll << 31) &&
                 (G0 * std::abs(v.sl0) + G1 * std::abs(v.sl1)) * es < (1ll << 31);
   plan.MV = mat_vec >= 16 ? 16 : 4;
-  // The streaming kernels move 16 bytes per lane on the 2-D side from any
-  // 4-byte aligned row start (LDS offsets stay 16-byte aligned: they are
-  // relative to the block's window).
+  // The streaming kernels move 16 bytes per lane on the 2-D side from any row
+  // start (LDS offsets stay 16-byte aligned: they are relative to the block's
+  // window).
   if (plan.stream && block_row_bytes % 16 == 0) plan.MV = 16;
   if (big && !(plan.stream && plan.MV == 16)) {
     return plan_tiled(v, es, mat_ptr, mat_stride0, mat_stride1, mat_size0, mat_size1, tiled_ptr,
@@ -1173,6 +1057,23 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
     a.sl0_bytes32 = (uint32_t)(v.sl0 * es);
     a.sl1_bytes32 = (uint32_t)(v.sl1 * es);
   }
+  // Walk over the blocks: bands of block rows, within a band groups of block
+  // columns row by row. One block row after the other, except for the packs
+  // under TRANSPOSE_OUTER in 64 KB blocks: there the blocks of one block row
+  // write runs that lie a whole column of tiles apart, so the workgroups that
+  // run at the same time take a patch of 32 x 8 blocks, whose runs join up (f32
+  // 12288 x 12289: 263 -> 236 us, 12289 x 12288: 243 -> 235; 16 x 16 and 16 x 32
+  // blocks 237 - 247, and no such gain for unpack, 247 - 254 in all of them).
+  const bool patches = big && to && !mat_is_dest;
+  a.band = patches ? (uint32_t)std::min<int64_t>(32, nblk0) : 1;
+  a.grp = patches ? (uint32_t)std::min<int64_t>(8, nblk1) : (uint32_t)nblk1;
+  // Workgroups of the 16 KB-block kernels: two per compute unit, each with a
+  // block of loads and one of stores in flight (four: f32 9000 x 9000 in 16x4
+  // tiles under TRANSPOSE_OUTER 130 / 135 us against 128 / 132, pack / unpack;
+  // 4096 x 4096 29.7 / 20.7 against 26.7 / 20.8), and one where large problems
+  // scatter short runs over both sides (TRANSPOSE_OUTER: 127 / 124 us; f16 9000
+  // x 9000 pack 75 -> 67, its unpack 56 -> 65).
+  plan.max_workgroups = to && total_bytes >= ((mat_is_dest ? 192ll : 128ll) << 20) ? 256 : 512;
   plan.G = G;
   plan.VEC = VEC;
   plan.grid = (uint32_t)(nblk0 * nblk1);
@@ -1212,7 +1113,7 @@ struct UnpackLauncher {
 
 template <bool UNPACK>
 bool launch_stream(const TiledPlan& plan, hipStream_t stream) {
-  // Persistent grid: up to 4 workgroups per CU, two LDS buffers each.
+  // Persistent grid, two LDS buffers per workgroup.
   const uint32_t nblocks = plan.grid;
   const uint32_t lds = 2 * plan.args.lds_buf_bytes;
   if (plan.big) {
@@ -1226,122 +1127,147 @@ bool launch_stream(const TiledPlan& plan, hipStream_t stream) {
                  stream, plan.args);
       return true;
     };
-    if (plan.G == 4 && plan.streaming_loads) {
-      auto kernel = stream_tiled_kernel<4, 16, 16, UNPACK, kStreamBigBlockBytes, kBigThreads, 1, true>;
-      static hipError_t attr = hipFuncSetAttribute(
-          reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-      return launch_big(kernel, attr);
-    }
-    if (plan.G == 4) {
-      auto kernel = stream_tiled_kernel<4, 16, 16, UNPACK, kStreamBigBlockBytes, kBigThreads, 1>;
-      static hipError_t attr = hipFuncSetAttribute(
-          reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-      return launch_big(kernel, attr);
-    }
-    auto kernel = stream_tiled_kernel<16, 16, 16, UNPACK, kStreamBigBlockBytes, kBigThreads, 1>;
-    static hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    return launch_big(kernel, attr);
+#define UK_BIG(g, ntl)                                                                               \
+  {                                                                                                       \
+    auto kernel = stream_tiled_kernel<g, 16, 16, UNPACK, kStreamBigBlockBytes, kBigThreads, ntl, true>;    \
+    static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),                   \
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
+    return launch_big(kernel, attr);                                                                      \
   }
-  const uint32_t grid = nblocks < 1024 ? nblocks : 1024;
-#define UK_CASE(g, vv, mv)                                                          \
-  if (plan.G == g && plan.VEC == vv && plan.MV == mv) {                              \
-    uk::launch(UNPACK ? 1 : 0, stream_tiled_kernel<g, vv, mv, UNPACK, kStreamBlockBytes>, \
-               dim3(grid), dim3(kThreads), lds, stream, plan.args);                  \
-    return true;                                                                     \
+    if (plan.G == 4 && plan.streaming_loads) UK_BIG(4, true)
+    if (plan.G == 4) UK_BIG(4, false)
+    UK_BIG(16, false)
+#undef UK_BIG
   }
-  UK_CASE(16, 16, 16) UK_CASE(8, 16, 16) UK_CASE(4, 16, 16) UK_CASE(4, 4, 16)
-  UK_CASE(16, 16, 4) UK_CASE(8, 16, 4) UK_CASE(4, 16, 4) UK_CASE(4, 4, 4)
+  const uint32_t grid = nblocks < plan.max_workgroups ? nblocks : plan.max_workgroups;
+#define UK_CASE(g, vv, mv, nts)                                                                             \
+  if (plan.G == g && plan.VEC == vv && plan.MV == mv && (bool)plan.args.streaming_stores == nts) {          \
+    uk::launch(UNPACK ? 1 : 0, stream_tiled_kernel<g, vv, mv, UNPACK, kStreamBlockBytes, kThreads, false, nts>, \
+               dim3(grid), dim3(kThreads), lds, stream, plan.args);                                         \
+    return true;                                                                                            \
+  }
+  UK_CASE(16, 16, 16, false) UK_CASE(8, 16, 16, false) UK_CASE(4, 16, 16, false)
+  UK_CASE(16, 16, 16, true) UK_CASE(8, 16, 16, true) UK_CASE(4, 16, 16, true)
+#undef UK_CASE
+#define UK_CASE(g, vv, mv)                                                                                  \
+  if (plan.G == g && plan.VEC == vv && plan.MV == mv) {                                                     \
+    uk::launch(UNPACK ? 1 : 0, stream_tiled_kernel<g, vv, mv, UNPACK, kStreamBlockBytes, kThreads, false, false>, \
+               dim3(grid), dim3(kThreads), lds, stream, plan.args);                                         \
+    return true;                                                                                            \
+  }
+  UK_CASE(4, 4, 16) UK_CASE(16, 16, 4) UK_CASE(8, 16, 4) UK_CASE(4, 16, 4) UK_CASE(4, 4, 4)
 #undef UK_CASE
   return false;
 }
 
 //===----------------------------------------------------------------------===//
-// Direct pack: untransposed tiles whose rows are whole 16-byte pieces, matrix
-// tiled exactly (no padding). A 16-byte piece of a matrix row is a 16-byte
-// piece of a tile row, so the data needs no regrouping in LDS: every thread
-// moves kDirectPieces pieces from register to register. A workgroup takes 16
-// matrix rows x 1 KiB: a wave reads 256 contiguous bytes of each of 4 rows and
-// writes, per tile, 4 x (tile row bytes) contiguous bytes; the four waves
-// together fill whole tiles when the tile height divides 16. No LDS round
-// trip, no barrier: for problems of a few tens of megabytes, which are bound by
-// the latency of one pass (launch, one load, one store) rather than by HBM.
+// Direct pack: tiles that are not transposed inside and whose rows are whole
+// 8- or 16-byte pieces. Such a piece of a tile row is a piece of a matrix row,
+// so the data needs no regrouping in LDS: every thread moves kDirectPieces
+// pieces from register to register. A workgroup takes 16 rows x 64 pieces: a
+// wave reads 16 neighbouring pieces of each of 4 rows and writes, per tile, 4
+// consecutive tile rows; the four waves together fill whole tiles when the tile
+// height divides 16. No LDS round trip, no barrier: for problems of up to a few
+// tens of megabytes, which are bound by the latency of one pass (launch, one
+// load, one store) rather than by HBM. Rows may start at any element and end
+// anywhere in a tile: every lane loads unconditionally, a piece beyond the end
+// of its row from the row's last bytes (uk::clipped_offset), and shifts and pads
+// in registers (s8 954 x 2499 into 16x16 tiles: 35 -> 4.2 us, bf16 1000 x 777
+// into 16x8: 21 -> 4.2; 4.0 of it are what the shortest kernel measures).
 //===----------------------------------------------------------------------===//
 struct DirectArgs {
   const char* src;
   char* dst;
-  int64_t src_pitch;     // bytes between matrix rows
-  int64_t dst_stride0;   // bytes between rows of tiles
-  uint32_t rows, row_bytes;
-  uint32_t tile_rows, tile_row_bytes, log2_tile_row_bytes;
-  uint32_t col_groups;   // 1 KiB column groups per matrix row
+  int64_t src_pitch;         // bytes between matrix rows
+  int64_t s0, s1;            // tiled side: bytes from one row tile / column tile to the next
+  uint32_t rows, row_bytes;  // the matrix
+  uint32_t padded_rows, padded_row_bytes;  // what its tiles hold
+  uint32_t tile_row_bytes, log2_tile_row_bytes;
+  uint32_t col_groups;       // groups of 64 pieces per row
+  uint32_t pad32;
+  FastDiv div_tile_rows;
 };
 constexpr int kDirectPieces = 4;
 
+template <int PB>
 __global__ __launch_bounds__(kThreads) void pack_direct_kernel(DirectArgs a) {
+  using Piece = typename GBytes<PB>::type;
+  uk::load_arguments_now(a.src, a.dst, a.src_pitch, a.s0, a.s1, a.rows, a.row_bytes, a.padded_rows, a.padded_row_bytes,
+                         a.tile_row_bytes, a.log2_tile_row_bytes, a.col_groups, a.pad32, a.div_tile_rows.mul);
   const uint32_t rg = blockIdx.x / a.col_groups, cg = blockIdx.x - rg * a.col_groups;
-  const uint32_t lane16 = threadIdx.x & 15;            // 16-byte piece within a 256-byte segment
   const uint32_t row = rg * 16 + (threadIdx.x >> 4);
-  if (row >= a.rows) return;
-  const uint32_t o0 = row / a.tile_rows, m0 = row - o0 * a.tile_rows;
-  const char* srow = a.src + (int64_t)row * a.src_pitch;
-  char* drow = a.dst + (int64_t)o0 * a.dst_stride0 + (int64_t)m0 * a.tile_row_bytes;
-  const uint32_t tile_bytes = a.tile_rows * a.tile_row_bytes;
-  v4u v[kDirectPieces];
-  uint32_t col[kDirectPieces];
+  if (row >= a.padded_rows) return;
+  uint32_t o0, m0;
+  a.div_tile_rows.divmod(row, o0, m0);
+  const bool row_ok = row < a.rows;
+  const char* srow = a.src + (int64_t)min(row, a.rows - 1) * a.src_pitch;
+  char* drow = a.dst + (int64_t)o0 * a.s0 + (int64_t)m0 * a.tile_row_bytes;
+  const uint32_t col0 = (cg * 64 + (threadIdx.x & 15)) * PB;
+  Words<PB> v[kDirectPieces];
+  if (a.row_bytes >= PB) {
 #pragma unroll
-  for (int i = 0; i < kDirectPieces; ++i) {
-    col[i] = cg * 1024 + (uint32_t)i * 256 + lane16 * 16;
-    if (col[i] < a.row_bytes) v[i] = gload<16>(srow + col[i]);
+    for (int i = 0; i < kDirectPieces; ++i)
+      v[i] = __builtin_bit_cast(Words<PB>, gload<PB>(srow + uk::clipped_offset<PB>(col0 + i * 16 * PB, a.row_bytes)));
+  } else {
+    const int32_t left = (int32_t)(a.row_bytes - col0);
+#pragma unroll
+    for (int i = 0; i < kDirectPieces; ++i) uk::load_short_row<PB>(v[i].w, srow + col0, i == 0 ? left : 0);
   }
 #pragma unroll
+  for (int i = 0; i < kDirectPieces; ++i)
+    uk::clip_piece<PB>(v[i].w, row_ok ? (int32_t)(a.row_bytes - (col0 + i * 16 * PB)) : 0, a.pad32);
+#pragma unroll
   for (int i = 0; i < kDirectPieces; ++i) {
-    if (col[i] < a.row_bytes) {
-      const uint32_t o1 = col[i] >> a.log2_tile_row_bytes;
-      gstore<16>(drow + (int64_t)o1 * tile_bytes + (col[i] & (a.tile_row_bytes - 1)), v[i]);
+    const uint32_t col = col0 + i * 16 * PB;
+    if (col < a.padded_row_bytes) {
+      const uint32_t o1 = col >> a.log2_tile_row_bytes;
+      *reinterpret_cast<Piece*>(drow + (int64_t)o1 * a.s1 + (col & (a.tile_row_bytes - 1))) =
+          __builtin_bit_cast(Piece, v[i]);
     }
   }
-}
-
-// Launches the direct pack when the call is of that form (see above) and
-// small enough to be latency-bound; false otherwise.
-bool launch_pack_direct(const iree_uk_pack_params_t* p, int es, const char* src, char* dst,
-                        bool transposed, hipStream_t stream) {
-  if (transposed || p->in_stride1 != 1) return false;
-  const int64_t trb = p->out_size3 * es;   // tile row bytes
-  if (trb < 16 || trb > 4096 || (trb & (trb - 1))) return false;
-  if (p->in_size0 != p->out_size0 * p->out_size2 || p->in_size1 != p->out_size1 * p->out_size3) return false;
-  if (p->in_size0 <= 0 || p->in_size1 <= 0) return false;
-  const int64_t row_bytes = p->in_size1 * es, pitch = p->in_stride0 * es;
-  if (pitch < 0 || ((uintptr_t)src | (uintptr_t)dst | (uint64_t)pitch | (uint64_t)(p->out_stride0 * es)) & 15) return false;
-  // Above a few tens of megabytes the streaming kernels (loads two blocks ahead,
-  // larger blocks) are level or ahead (f16 4096 x 4096, 33.5 MB: 11.9 against
-  // 11.6 us); below, one pass of latency is what counts (s8 2048 x 8192 in
-  // 16x32 tiles, 16.8 MB: 8.4 -> 5.7 us).
-  const int64_t total = p->in_size0 * row_bytes;
-  if (total > (24ll << 20) || p->in_size0 >= (1ll << 31) || row_bytes >= (1ll << 31) ||
-      p->out_size2 >= (1 << 20)) {
-    return false;
-  }
-  DirectArgs a;
-  a.src = src; a.dst = dst;
-  a.src_pitch = pitch;
-  a.dst_stride0 = p->out_stride0 * es;
-  a.rows = (uint32_t)p->in_size0; a.row_bytes = (uint32_t)row_bytes;
-  a.tile_rows = (uint32_t)p->out_size2; a.tile_row_bytes = (uint32_t)trb;
-  a.log2_tile_row_bytes = 0;
-  while ((1u << a.log2_tile_row_bytes) < a.tile_row_bytes) ++a.log2_tile_row_bytes;
-  a.col_groups = (uint32_t)((row_bytes + 1023) / 1024);
-  const int64_t grid = ((p->in_size0 + 15) / 16) * a.col_groups;
-  if (grid >= (1ll << 31)) return false;
-  uk::launch(0, pack_direct_kernel, dim3((uint32_t)grid), dim3(kThreads), 0, stream, a);
-  return true;
 }
 
 uint32_t replicate_pad(uint64_t pad, int es) {
   if (es == 1) return (uint32_t)(pad & 0xFF) * 0x01010101u;
   if (es == 2) return (uint32_t)(pad & 0xFFFF) * 0x00010001u;
   return (uint32_t)pad;
+}
+
+// Launches the direct pack when the call is of that form (see above) and
+// small enough to be latency-bound; false otherwise. `v` is the call's view.
+bool launch_pack_direct(const iree_uk_pack_params_t* p, const TiledView& v, int es, const char* src, char* dst,
+                        bool transpose_inner, hipStream_t stream) {
+  if (transpose_inner || p->in_stride1 != 1) return false;
+  const int64_t trb = v.tile1 * es;   // tile row bytes
+  if (trb < 8 || trb > 4096 || (trb & (trb - 1))) return false;
+  if (p->in_size0 <= 0 || p->in_size1 <= 0) return false;
+  const int PB = trb >= 16 ? 16 : 8;
+  const int64_t row_bytes = p->in_size1 * es, pitch = p->in_stride0 * es;
+  const int64_t rows = v.outer0 * v.tile0, padded = v.outer1 * trb;
+  const int64_t s0 = v.sl0 * es, s1 = v.sl1 * es;
+  if (((uintptr_t)dst | (uint64_t)s0 | (uint64_t)s1) & (uint64_t)(PB - 1)) return false;
+  // Above a few tens of megabytes the streaming kernels are level or ahead (f16
+  // 4096 x 4096, 33.5 MB: 13.2 against 13.0 us; f16 4095 x 6001: 24.4 against
+  // 22.6); below, one pass of latency is what counts (s8 2048 x 8192 in 16x32
+  // tiles, 16.8 MB: 8.4 -> 5.7 us).
+  if (rows >= (1ll << 31) || padded >= (1ll << 31) || rows * padded > (24ll << 20) || v.tile0 >= (1 << 20)) return false;
+  DirectArgs a;
+  a.src = src; a.dst = dst;
+  a.src_pitch = pitch;
+  a.s0 = s0; a.s1 = s1;
+  a.rows = (uint32_t)p->in_size0; a.row_bytes = (uint32_t)row_bytes;
+  a.padded_rows = (uint32_t)rows; a.padded_row_bytes = (uint32_t)padded;
+  a.tile_row_bytes = (uint32_t)trb;
+  a.log2_tile_row_bytes = 0;
+  while ((1u << a.log2_tile_row_bytes) < a.tile_row_bytes) ++a.log2_tile_row_bytes;
+  a.col_groups = (uint32_t)uk::ceil_div(padded, 64 * PB);
+  a.pad32 = replicate_pad(p->padding_value, es);
+  a.div_tile_rows = FastDiv((uint32_t)v.tile0);
+  const int64_t grid = uk::ceil_div(rows, 16) * a.col_groups;
+  if (grid >= (1ll << 31)) return false;
+  uk::launch(0, PB == 16 ? pack_direct_kernel<16> : pack_direct_kernel<8>, dim3((uint32_t)grid), dim3(kThreads), 0,
+             stream, a);
+  return true;
 }
 
 int elem_bytes_of(uint32_t flags) {
@@ -1358,8 +1284,8 @@ int elem_bytes_of(uint32_t flags) {
 }  // namespace
 
 // pack_tr.hip: tiles transposed element by element (1-, 2- and 4-byte elements).
-bool iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, const char* src, char* dst,
-                                hipStream_t stream);
+const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, const char* src, char* dst,
+                                       hipStream_t stream);
 
 extern "C" int iree_uk_amd_hip_launch_pack(const iree_uk_pack_params_t* p_in,
                                            void* stream_v, int kernel_mode,
@@ -1389,13 +1315,15 @@ extern "C" int iree_uk_amd_hip_launch_pack(const iree_uk_pack_params_t* p_in,
   // (Any forced mmt4d variant mode keeps pack on the LDS-staged kernels, so that
   // tests and timings can reach both.)
   if (kernel_mode == IREE_UK_AMD_KERNEL_MODE_AUTO &&
-      launch_pack_direct(p, es, src, dst, ti || to, stream)) {
+      launch_pack_direct(p, v, es, src, dst, ti, stream)) {
     *kernel_name = "pack_direct";
     return (int)hipGetLastError();
   }
-  if (kernel_mode == IREE_UK_AMD_KERNEL_MODE_AUTO && iree_uk_amd_launch_pack_tr(p, es, src, dst, stream)) {
-    *kernel_name = "pack_transposing";
-    return (int)hipGetLastError();
+  if (kernel_mode == IREE_UK_AMD_KERNEL_MODE_AUTO) {
+    if (const char* name = iree_uk_amd_launch_pack_tr(p, es, src, dst, stream)) {
+      *kernel_name = name;
+      return (int)hipGetLastError();
+    }
   }
   if (kernel_mode != IREE_UK_AMD_KERNEL_MODE_GENERIC) {
     TiledPlan plan = plan_tiled(v, es, src, p->in_stride0, p->in_stride1,

@@ -44,6 +44,107 @@ struct FastDiv {
   }
 };
 
+// Has the kernel's arguments in scalar registers from here on. Left alone, the
+// compiler loads each argument where it is first needed: a chain of scalar loads,
+// each waited for (the first of every 64 bytes all the way to memory), before a
+// short kernel's first global load.
+template <typename T>
+__device__ __forceinline__ void load_arguments_now(const T& v) {
+  asm volatile("" : : "s"(v));
+}
+template <typename T, typename... Ts>
+__device__ __forceinline__ void load_arguments_now(const T& v, const Ts&... vs) {
+  load_arguments_now(v);
+  load_arguments_now(vs...);
+}
+
+// A piece of N bytes (8 or 16) of a matrix row whose end may fall inside or
+// before the piece. `clipped_offset` is where to load it from: the piece's own
+// offset, or the last N bytes of the row where the piece reaches beyond them
+// (the row must hold at least N bytes), so that every lane issues one
+// unconditional load and the loads of a workgroup stay in flight together.
+// `clip_piece` then moves the bytes of such a piece to where they belong and
+// puts padding behind them; `left` = row bytes - piece offset, <= 0 for a piece
+// that is all padding. (Element by element, the end of a row was a chain of up
+// to sixteen dependent loads in every block of the last column: s8 100 x 97
+// rows took 24 us to pack.)
+template <int N>
+__device__ __forceinline__ uint32_t clipped_offset(uint32_t off, uint32_t row_bytes) {
+  return min(off, row_bytes - N);
+}
+template <int N>
+__device__ __forceinline__ void clip_piece(uint32_t (&w)[N / 4], int32_t left, uint32_t pad32) {
+  static_assert(N == 16 || N == 8 || N == 4, "whole words");
+  if (left >= N) return;
+  const uint64_t pad = ((uint64_t)pad32 << 32) | pad32;
+  if (left <= 0) {
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) w[i] = pad32;
+    return;
+  }
+  const uint32_t keep = 8 * (uint32_t)left, drop = 8 * N - keep;  // bits, both below 8 N
+  if constexpr (N == 4) {
+    const uint32_t mask = (1u << keep) - 1;
+    w[0] = ((w[0] >> drop) & mask) | (pad32 & ~mask);
+  } else if constexpr (N == 8) {
+    const uint64_t x = ((uint64_t)w[1] << 32) | w[0];
+    const uint64_t mask = (1ull << keep) - 1;
+    const uint64_t y = ((x >> drop) & mask) | (pad & ~mask);
+    w[0] = (uint32_t)y; w[1] = (uint32_t)(y >> 32);
+  } else {
+    uint64_t lo = ((uint64_t)w[1] << 32) | w[0], hi = ((uint64_t)w[3] << 32) | w[2];
+    if (drop >= 64) {
+      lo = hi >> (drop - 64);
+      hi = 0;
+    } else {
+      lo = (lo >> drop) | (hi << (64 - drop));  // drop >= 8
+      hi >>= drop;
+    }
+    const uint64_t mlo = keep >= 64 ? ~0ull : (1ull << keep) - 1;
+    const uint64_t mhi = keep <= 64 ? 0ull : (1ull << (keep - 64)) - 1;
+    lo = (lo & mlo) | (pad & ~mlo);
+    hi = (hi & mhi) | (pad & ~mhi);
+    w[0] = (uint32_t)lo; w[1] = (uint32_t)(lo >> 32); w[2] = (uint32_t)hi; w[3] = (uint32_t)(hi >> 32);
+  }
+}
+// The same piece for a row of fewer than N bytes: the `left` bytes at `p`, one by
+// one, to where `clip_piece` expects them. (Rare: kept out of the way as a
+// rolled loop.)
+template <int N>
+__device__ __forceinline__ void load_short_row(uint32_t (&w)[N / 4], const char* p, int32_t left) {
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) w[i] = 0;
+#pragma clang loop unroll(disable)
+  for (int32_t b = 0; b < left; ++b) {
+    const uint32_t x = (uint8_t)p[b];
+#pragma unroll
+    for (int i = 0; i < N / 4; ++i) w[i] = (w[i] >> 8) | ((i + 1 < N / 4 ? w[i + 1] : x) << 24);
+  }
+}
+// Stores the first `n` bytes (0 < n < N) of a piece in at most four accesses.
+template <int N>
+__device__ __forceinline__ void store_head(char* p, const uint32_t (&w)[N / 4], uint32_t n) {
+  typedef uint32_t u32_a1 __attribute__((aligned(1)));
+  typedef uint16_t u16_a1 __attribute__((aligned(1)));
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i)
+    if (n >= 4u * i + 4) *reinterpret_cast<u32_a1*>(p + 4 * i) = w[i];
+  const uint32_t at = n & ~3u;
+  if (n & 3) {
+    uint32_t x = w[0];  // word at / 4
+    if constexpr (N == 8) x = (uint32_t)((((uint64_t)w[1] << 32) | w[0]) >> (8 * at));
+    if constexpr (N == 16) {
+      const uint64_t lo = ((uint64_t)w[1] << 32) | w[0], hi = ((uint64_t)w[3] << 32) | w[2];
+      x = (uint32_t)((at & 8 ? hi : lo) >> (8 * (at & 4)));
+    }
+    if (n & 2) {
+      *reinterpret_cast<u16_a1*>(p + at) = (uint16_t)x;
+      x >>= 16;
+    }
+    if (n & 1) p[at + (n & 2)] = (char)x;
+  }
+}
+
 // Largest power of two <= cap that divides v (v == 0 counts as divisible).
 inline int64_t pow2_divisor(int64_t v, int64_t cap) {
   int64_t p = cap;

@@ -259,6 +259,59 @@ def test_pack_transposing_kernel_declines_what_it_does_not_serve(gpu, oracle):
         assert np.array_equal(got, want), c.label()
 
 
+@pytest.mark.parametrize("tf,t0,t1,flags", [
+    (uk.PACK_TYPE_I8I8, 16, 16, 0), (uk.PACK_TYPE_I8I8, 32, 8, 0), (uk.PACK_TYPE_I8I8, 16, 16, 0x200),
+    (uk.PACK_TYPE_I8I8, 16, 2, 0), (uk.PACK_TYPE_I8I8, 16, 4, 0x200), (uk.PACK_TYPE_I8I8, 16, 16, 0x300),
+    (uk.PACK_TYPE_I8I8, 16, 2, 0x300), (uk.PACK_TYPE_BF16BF16, 16, 8, 0), (uk.PACK_TYPE_BF16BF16, 24, 4, 0),
+    (uk.PACK_TYPE_BF16BF16, 16, 2, 0), (uk.PACK_TYPE_BF16BF16, 16, 8, 0x300), (uk.PACK_TYPE_F32F32, 16, 4, 0),
+    (uk.PACK_TYPE_F32F32, 16, 2, 0)])
+def test_pack_rows_of_any_length_and_alignment(gpu, oracle, tf, t0, t1, flags):
+    """Rows that start at any element and end inside a tile row, a vector of 8
+    or 16 bytes, or before the first one: the direct, the transposing and the
+    streaming kernel on them, whole buffers against the oracle."""
+    lib, torch = gpu
+    es = uk.PACK_TYPE_BYTES[tf]
+    s0, s1 = (t1, t0) if flags & 0x100 else (t0, t1)
+    g = T.Lcg(19)
+    rng = np.random.default_rng(tf + t1)
+    for ci, in1 in enumerate((1, 3, 7, 8, 9, 15, 16, 17, 31, 33, 65, 129, 257, 517, 1031)):
+        in0 = int(rng.integers(1, 70))
+        o0, o1 = -(-in0 // s0) + ci % 2, -(-in1 // s1) + ci % 3
+        os0, os1 = (o1, o0) if flags & 0x200 else (o0, o1)
+        c = T.PackCase(tf | flags, in0, in1, os0, os1, t0, t1, in1 + ci % 4, 1, os1 * t0 * t1, ci % 3,
+                       16 // es * (ci % 2), g.u64())
+        inp, out0 = T.make_pack_buffers(c, rng)
+        want = out0.copy()
+        G.run_pack_case(oracle, c, inp, want)
+        got = T.gpu_pack(lib, torch, c, inp, out0)
+        assert np.array_equal(got, want), (c.label(), lib.last_kernel_name())
+        lib.set_kernel_mode(uk.KERNEL_MODE_MFMA_VARIANT + 1)   # the LDS-staged kernels on the same call
+        try:
+            staged = T.gpu_pack(lib, torch, c, inp, out0)
+        finally:
+            lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+        assert np.array_equal(staged, want), (c.label(), "staged")
+
+
+@pytest.mark.parametrize("tf,t0,t1,flags", [
+    (uk.UNPACK_TYPE_BF16BF16, 16, 16, 0), (uk.UNPACK_TYPE_F16F16, 16, 8, 0x200), (uk.UNPACK_TYPE_F32F32, 16, 16, 0),
+    (uk.UNPACK_TYPE_I32I32, 16, 4, 0)])
+def test_unpack_rows_of_any_length_and_alignment(gpu, oracle, tf, t0, t1, flags):
+    """The same for unpack: what a row ends with is stored in pieces."""
+    lib, torch = gpu
+    rng = np.random.default_rng(tf)
+    for ci, n in enumerate((1, 2, 3, 5, 7, 9, 15, 17, 33, 67, 131, 259, 515, 1033)):
+        m = int(rng.integers(1, 70))
+        o0, o1 = -(-m // t0) + ci % 2, -(-n // t1) + ci % 3
+        s0, s1 = (o1, o0) if flags & 0x200 else (o0, o1)
+        c = T.UnpackCase(tf | flags, s0, s1, t0, t1, m, n, s1 * t0 * t1, n + ci % 4, 1, 0, ci % 3)
+        inp, out0 = T.make_unpack_buffers(c, rng)
+        want = out0.copy()
+        G.run_unpack_case(oracle, c, inp, want)
+        got = T.gpu_unpack(lib, torch, c, inp, out0)
+        assert np.array_equal(got, want), (c.label(), lib.last_kernel_name())
+
+
 SINGLE_LINE_TILES = [
     (uk.PACK_TYPE_F32F32, 16, 1), (uk.PACK_TYPE_F32F32, 1, 16), (uk.PACK_TYPE_I32I32, 8, 1),
     (uk.PACK_TYPE_F16F16, 1, 16), (uk.PACK_TYPE_BF16BF16, 16, 1), (uk.PACK_TYPE_I8I8, 1, 16),
