@@ -79,7 +79,8 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
   a.steps = (int32_t)uk::ceil_div(k_bytes, SH::KS);
   if (a.steps < 1) a.steps = 1;
   a.tail = (k_bytes % SH::KS) != 0;
-  if (PIPE != 0 && PIPE != 4 && (a.tail || kt_count == 0)) return -1;
+  if (PIPE != 0 && PIPE != 4 && ((a.tail && PIPE != 3 && PIPE != 5) || kt_count == 0)) return -1;
+  if (E == Elem::kS16 && a.tail) return -1;           // (K in whole steps only)
   a.accumulate = accumulate;
   // A launch that starts K reads the caller's accumulators; a later one
   // continues from what the previous launch left in the output. Only the
@@ -125,17 +126,23 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
       span_a >= (1ll << 31)) {
     return -1;
   }
-  auto kernel = mmt4d_mfma_kernel<E, RBC, TM, TN, WGM, WGN, NKK, PIPE>;
-  if (SH::kLdsBytes > 64 * 1024) {
-    // Raising the dynamic LDS limit is a per-function setting; do it once.
-    static hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-        (int)SH::kLdsBytes);
-    if (attr != hipSuccess) return (int)attr;
+  auto go = [&](auto tail_c) {
+    auto kernel = mmt4d_mfma_kernel<E, RBC, TM, TN, WGM, WGN, NKK, PIPE, decltype(tail_c)::value>;
+    if (SH::kLdsBytes > 64 * 1024) {
+      // Raising the dynamic LDS limit is a per-function setting; do it once.
+      static hipError_t attr = hipFuncSetAttribute(
+          reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+          (int)SH::kLdsBytes);
+      if (attr != hipSuccess) return (int)attr;
+    }
+    uk::launch(2, kernel, dim3((uint32_t)(grid_m * grid_n)), dim3(WGM * WGN * 64),
+               SH::kLdsBytes, stream, a);
+    return (int)hipGetLastError();
+  };
+  if constexpr (PIPE == 3 || PIPE == 5) {
+    if (a.tail) return go(std::true_type{});
   }
-  uk::launch(2, kernel, dim3((uint32_t)(grid_m * grid_n)), dim3(WGM * WGN * 64),
-             SH::kLdsBytes, stream, a);
-  return (int)hipGetLastError();
+  return go(std::false_type{});
 }
 
 // Workspace of the thin kernel's K split over workgroups: `partial_bytes` of
@@ -586,9 +593,13 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       return 0;
     }
   }
-  // Whole pipeline steps of K go to a software-pipelined variant; what is left
-  // of K (less than one step) to the two-stage variant of the same or a
-  // smaller workgroup shape, as a second, accumulating launch.
+  // The pipelines that need K in whole steps get those; what is left of K (less
+  // than one step) goes to the two-stage variant of the same or a smaller
+  // workgroup shape, as a second, accumulating launch. (Pipelines 3 and 5, which
+  // serve every call that no test or tuning run forces elsewhere, run any K: a
+  // second launch over less than one step cost as much as a small product, and
+  // a pass over the output: s8 300 x 500 x 400 10.6 -> 5.5 us, f16 3000 x 3000 x
+  // 333 40.1 -> 18.7, s8 4095 x 2049 x 2049 53.6 -> 31.2.)
   const int kts_per_step = BIG_KS >> p.lrb;
   // 16-bit outputs are rounded once, after all of K (the reference's
   // SKIP_INTERMEDIATE_ROUNDINGS semantics): a second launch would continue from
@@ -606,21 +617,17 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       // Measured against the register-regrouping kernels at 8192^3: s8 16x16x2
       // 496 -> 382 us, bf16 16x16x2 932 -> 726 us, s8 16x16x8 486 -> 383 us; at
       // 4096^3 s8 16x16x2 76 -> 57 us. (f32 keeps its kernels, as below.)
-      if (kt_main > 0 && (forced == 16 || forced == 17 || (forced == 0 && E != Elem::kF32))) {
+      if (forced == 16 || forced == 17 || (forced == 0 && E != Elem::kF32)) {
         int st = -1;
         if (forced == 17) {
-          st = launch_variant<E, RBC, 8, 4, 1, 8, 1, 5>(p, 0, kt_main, p.accumulate, stream);
+          st = launch_variant<E, RBC, 8, 4, 1, 8, 1, 5>(p, 0, p.K1, p.accumulate, stream);
           if (st == 0) *name = "mmt4d_mfma_128x512_lds_direct";
         }
         if (st < 0) {
-          st = launch_variant<E, RBC, 8, 4, 2, 4, 1, 5>(p, 0, kt_main, p.accumulate, stream);
+          st = launch_variant<E, RBC, 8, 4, 2, 4, 1, 5>(p, 0, p.K1, p.accumulate, stream);
           if (st == 0) *name = "mmt4d_mfma_256x256_lds_direct";
         }
-        if (st == 0) {
-          if (kt_main == p.K1) return 0;
-          return finish_k(launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
-        }
-        if (st > 0) return st;
+        if (st >= 0) return st;
       }
     }
     if constexpr (NARROW) {
@@ -652,9 +659,30 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
         if (st > 0) return st;
       }
     }
+    if constexpr (RBC >= 16) {
+      // Both operands through LDS-direct loads, two wave groups alternating
+      // between memory and compute phases (PIPE 5 of mmt4d_mfma_kernel.h): the
+      // default for the big problems of the 8- and 16-bit types (s8 8192^3
+      // 413 -> 388 us, bf16 8192^3 779 -> 718 us, f16 4096^3 102 -> 98 us, f8
+      // 8192^3 415 -> 390 us against the register-direct-RHS pipeline in its
+      // best shape). f32
+      // keeps that pipeline (matrix-pipe bound there: 925 against 959 us).
+      constexpr bool kDefault = E != Elem::kF32;
+      int st = -1;
+      if (forced == 17) {
+        st = launch_variant<E, RBC, 8, 4, 1, 8, 1, 5>(p, 0, p.K1, p.accumulate, stream);
+        if (st == 0) *name = "mmt4d_mfma_128x512_lds_direct";
+      }
+      if (st < 0 && (forced == 16 || forced == 17 || (forced == 0 && kDefault))) {
+        st = launch_variant<E, RBC, 8, 4, 2, 4, 1, 5>(p, 0, p.K1, p.accumulate, stream);
+        if (st == 0) *name = "mmt4d_mfma_256x256_lds_direct";
+      }
+      if (st >= 0) return st;
+    }
     if (kt_main > 0) {
       int st = -1;
       bool wide = false;
+      const int kt_big = BIG_PIPE == 3 ? p.K1 : kt_main;  // pipeline 3 runs any K
       if constexpr (RBC >= 16 && H == 1 && ElemTraits<E>::Out::kOutBytes == 4) {
         // One persistent workgroup per CU whose pipeline runs across block
         // boundaries. Measured equal to the one-block-per-workgroup launches
@@ -675,29 +703,6 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
         if (st > 0) return st;
       }
       if constexpr (RBC >= 16) {
-        // Both operands through LDS-direct loads, two wave groups alternating
-        // between memory and compute phases (PIPE 5 of mmt4d_mfma_kernel.h): the
-        // default for the big problems of the 8- and 16-bit types (s8 8192^3
-        // 413 -> 388 us, bf16 8192^3 779 -> 718 us, f16 4096^3 102 -> 98 us, f8
-        // 8192^3 415 -> 390 us against the register-direct-RHS pipeline in its
-        // best shape). f32
-        // keeps that pipeline (matrix-pipe bound there: 925 against 959 us).
-        constexpr bool kDefault = E != Elem::kF32;
-        if (forced == 17) {
-          st = launch_variant<E, RBC, 8, 4, 1, 8, 1, 5>(p, 0, kt_main, p.accumulate, stream);
-          if (st == 0) *name = "mmt4d_mfma_128x512_lds_direct";
-        }
-        if (st < 0 && (forced == 16 || forced == 17 || (forced == 0 && kDefault))) {
-          st = launch_variant<E, RBC, 8, 4, 2, 4, 1, 5>(p, 0, kt_main, p.accumulate, stream);
-          if (st == 0) *name = "mmt4d_mfma_256x256_lds_direct";
-        }
-        if (st == 0) {
-          if (kt_main == p.K1) return 0;
-          return finish_k(launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
-        }
-        if (st > 0) return st;
-      }
-      if constexpr (RBC >= 16) {
         // 128 rows x 512 columns, the 8 waves side by side (each 128x64): no two
         // waves load the same RHS fragments and the LDS holds half as much LHS,
         // i.e. fewer bytes moved per MFMA, which is what a power-bound kernel
@@ -707,17 +712,17 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
         const int bpm_w = 128 / p.M0, bpn_w = 512 / p.N0;
         if (forced == 8 || (forced == 0 && bpm_w >= 1 && bpn_w >= 1 && p.M1 % bpm_w == 0 &&
                             p.N1 % bpn_w == 0 && workgroups(p, 128, 512) >= 192)) {
-          st = launch_variant<E, RBC, 8, 4, 1, 8, 1, BIG_PIPE>(p, 0, kt_main, p.accumulate, stream);
+          st = launch_variant<E, RBC, 8, 4, 1, 8, 1, BIG_PIPE>(p, 0, kt_big, p.accumulate, stream);
           wide = st == 0;
         }
       }
       if (st < 0) {
-        st = launch_variant<E, RBC, 8, 4, 2, 4, 1, BIG_PIPE>(p, 0, kt_main, p.accumulate, stream);
+        st = launch_variant<E, RBC, 8, 4, 2, 4, 1, BIG_PIPE>(p, 0, kt_big, p.accumulate, stream);
       }
       if (st == 0) {
         *name = wide ? "mmt4d_mfma_128x512_rhs_direct"
                      : (RBC >= 16 ? "mmt4d_mfma_256x256_rhs_direct" : "mmt4d_mfma_256x256_regroup");
-        if (kt_main == p.K1) return 0;
+        if (kt_big == p.K1) return 0;
         return finish_k(launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
       }
       if (st > 0) return st;
@@ -729,24 +734,14 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     // 256x256 blocks to fill the CUs; moves fewer L1 bytes per MFMA than the
     // 128x128 shape.
     if constexpr (RBC >= 16) {
-      if (kt_main > 0 && (forced == 20 || (forced == 0 && E != Elem::kF32))) {
-        int st = launch_variant<E, RBC, 8, 2, 2, 4, 1, 5>(p, 0, kt_main, p.accumulate, stream);
-        if (st == 0) {
-          *name = "mmt4d_mfma_256x128_lds_direct";
-          if (kt_main == p.K1) return 0;
-          return finish_k(launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
-        }
-        if (st > 0) return st;
+      if (forced == 20 || (forced == 0 && E != Elem::kF32)) {
+        int st = launch_variant<E, RBC, 8, 2, 2, 4, 1, 5>(p, 0, p.K1, p.accumulate, stream);
+        if (st == 0) *name = "mmt4d_mfma_256x128_lds_direct";
+        if (st >= 0) return st;
       }
-      if (kt_main > 0) {
-        int st = launch_variant<E, RBC, 8, 2, 2, 4, 1, 3>(p, 0, kt_main, p.accumulate, stream);
-        if (st == 0) {
-          *name = "mmt4d_mfma_256x128_rhs_direct";
-          if (kt_main == p.K1) return 0;
-          return finish_k(launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
-        }
-        if (st > 0) return st;
-      }
+      int st = launch_variant<E, RBC, 8, 2, 2, 4, 1, 3>(p, 0, p.K1, p.accumulate, stream);
+      if (st == 0) *name = "mmt4d_mfma_256x128_rhs_direct";
+      if (st >= 0) return st;
     }
     choice = 2;
   }
@@ -813,18 +808,14 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     choice = 3;
   }
   if (choice == 2) {
-    if constexpr (H == 1) {
+    {
       // The LDS-direct ping-pong pipeline with 8 waves of 64x32 (measured against
       // the kernels below: s8 2048^3 16x16x2 20.6 -> 14.7 us, 16x16x16 14.8 ->
       // 14.5 us; 3072^3 40.5 -> 36.3 us; bf16 2048^3 23.4 -> 22.6 us).
-      if (kt_main > 0 && (forced == 18 || (forced == 0 && E != Elem::kF32))) {
-        int st = launch_variant<E, RBC, 4, 2, 2, 4, 1, 5>(p, 0, kt_main, p.accumulate, stream);
-        if (st == 0) {
-          *name = "mmt4d_mfma_128x128_lds_direct";
-          if (kt_main == p.K1) return 0;
-          return finish_k(launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
-        }
-        if (st > 0) return st;
+      if (forced == 18 || (forced == 0 && E != Elem::kF32)) {
+        int st = launch_variant<E, RBC, 4, 2, 2, 4, 1, 5>(p, 0, p.K1, p.accumulate, stream);
+        if (st == 0) *name = "mmt4d_mfma_128x128_lds_direct";
+        if (st >= 0) return st;
       }
     }
     if constexpr (NARROW) {
@@ -841,48 +832,29 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       }
     }
     if constexpr (RBC >= 16) {
-      if (kt_main > 0) {
-        int st = launch_variant<E, RBC, 4, 2, 2, 4, 1, 3>(p, 0, kt_main, p.accumulate, stream);
-        if (st == 0) {
-          *name = "mmt4d_mfma_128x128_rhs_direct";
-          if (kt_main == p.K1) return 0;
-          return finish_k(launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
-        }
-        if (st > 0) return st;
-      }
+      int st = launch_variant<E, RBC, 4, 2, 2, 4, 1, 3>(p, 0, p.K1, p.accumulate, stream);
+      if (st == 0) *name = "mmt4d_mfma_128x128_rhs_direct";
+      if (st >= 0) return st;
     }
     int st = launch_variant<E, RBC, 4, 4, 2, 2, NKK2, 0>(p, 0, p.K1, p.accumulate, stream);
     if (st >= 0) { *name = "mmt4d_mfma_128x128"; return st; }
   }
   if constexpr (H == 1) {
     // 64x64 blocks, 8 waves of 32x16, 256 bytes of K per step.
-    const int kts256 = 256 >> p.lrb;
-    int kt_main256 = kts256 > 0 ? (p.K1 / kts256) * kts256 : 0;
-    if (kOneLaunchOnly && kt_main256 != p.K1) kt_main256 = 0;
     // Chosen for narrow tile rows when the 64x64 blocks fill the compute units
     // (s8 1024^3 16x16x2: 7.0 -> 6.4 us; with rows of 16 bytes and more the
     // register-direct kernel below is level or ahead: 5.7 against 5.9 us).
-    const bool small_narrow = forced == 0 && RBC < 16 && E != Elem::kF32 && workgroups(p, 64, 64) >= 192;
-    if (kt_main256 > 0 && (forced == 19 || small_narrow)) {
-      int st = launch_variant<E, RBC, 2, 1, 2, 4, 4, 5>(p, 0, kt_main256, p.accumulate, stream);
-      if (st == 0) {
-        *name = "mmt4d_mfma_64x64_lds_direct";
-        if (kt_main256 == p.K1) return 0;
-        return finish_k(launch_variant<E, RBC, 2, 2, 2, 2, NKK2, 0>(p, kt_main256, p.K1 - kt_main256, true, stream));
-      }
-      if (st > 0) return st;
+    const bool small_default = forced == 0 && RBC < 16 && E != Elem::kF32 && workgroups(p, 64, 64) >= 192;
+    if (forced == 19 || small_default) {
+      int st = launch_variant<E, RBC, 2, 1, 2, 4, 4, 5>(p, 0, p.K1, p.accumulate, stream);
+      if (st == 0) *name = "mmt4d_mfma_64x64_lds_direct";
+      if (st >= 0) return st;
     }
   }
   if constexpr (RBC >= 16) {
-    if (kt_main > 0) {
-      int st = launch_variant<E, RBC, 2, 2, 2, 2, 1, 3>(p, 0, kt_main, p.accumulate, stream);
-      if (st == 0) {
-        *name = "mmt4d_mfma_64x64_rhs_direct";
-        if (kt_main == p.K1) return 0;
-        return finish_k(launch_variant<E, RBC, 2, 2, 2, 2, NKK2, 0>(p, kt_main, p.K1 - kt_main, true, stream));
-      }
-      if (st > 0) return st;
-    }
+    int st = launch_variant<E, RBC, 2, 2, 2, 2, 1, 3>(p, 0, p.K1, p.accumulate, stream);
+    if (st == 0) *name = "mmt4d_mfma_64x64_rhs_direct";
+    if (st >= 0) return st;
   }
   if constexpr (NARROW) {
     if (kt_main > 0 && forced == 15) {

@@ -228,6 +228,32 @@ def test_mmt4d_16bit_outputs_round_once_when_k_has_a_remainder(gpu, oracle, tf, 
     lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
 
 
+@pytest.mark.parametrize("variant", [0, 2, 3, 7, 16, 18, 19, 20])
+@pytest.mark.parametrize("tf,K0", [(uk.MMT4D_TYPE_F16F16F32, 8), (uk.MMT4D_TYPE_BF16BF16F32, 2),
+                                   (uk.MMT4D_TYPE_F32F32F32, 4), (uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32, 32)])
+def test_mmt4d_k_that_ends_inside_a_step_reads_nothing_beyond_it(gpu, oracle, tf, K0, variant):
+    """K a few tiles short of, at and past whole pipeline steps, and NaN in all
+    bytes behind the K-tiles of every panel: a kernel that multiplied them, even
+    by zero, would give NaN. Small integers, so the result is exact."""
+    lib, torch = gpu
+    M0 = N0 = 16
+    es = uk.MMT4D_TYPE_BITS[tf][0] // 8
+    nan = {1: 0x7F, 2: 0xFFFF, 4: 0xFFFFFFFF}[es]
+    lib.set_kernel_mode(uk.KERNEL_MODE_MFMA_VARIANT + variant if variant else uk.KERNEL_MODE_AUTO)
+    for seed, (M, N, K) in enumerate(((9, 11, 1), (17, 5, 3), (5, 18, 17), (16, 16, 32), (9, 9, 37), (7, 9, 131))):
+        gap = 4 * M0 * K0
+        c = T.Mmt4dCase(tf, M, N, K, M0, N0, K0, K * M0 * K0 + gap, K * N0 * K0 + gap, N * M0 * N0, 0, 0, 0)
+        lhs, rhs, out0 = T.make_mmt4d_buffers(c, np.random.default_rng(seed))
+        for buf, panels in ((lhs, M), (rhs, N)):
+            buf.view({1: np.uint8, 2: np.uint16, 4: np.uint32}[es]).reshape(panels, -1)[:, K * M0 * K0:] = nan
+        want = out0.copy()
+        G.run_mmt4d_case(oracle, c, lhs, rhs, want)
+        got = T.gpu_mmt4d(lib, torch, c, lhs, rhs, out0, allow_generic=False)
+        assert np.array_equal(got, want), (c.label(), lib.last_kernel_name())
+        assert lib.last_kernel_name().startswith("mmt4d_mfma"), lib.last_kernel_name()
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+
+
 def test_mmt4d_single_row_tiles_equal_row_major_matmul(gpu):
     """With M0 = N0 = 1 the mmt4d layouts are plain row-major [M][K], [N][K]
     and [M][N]: the call must equal the integer matrix product A . B^T
