@@ -9,7 +9,8 @@
 //     v_mfma_f32_16x16x4_f32: a lane's 16-byte piece of one input pixel (four
 //     ci, straight from global memory) is the operand of four instructions,
 //     one per word, against four filter words of the same four ci (staged
-//     through LDS by the workgroup). Sums are in MFMA order, so results equal the
+//     through LDS by the workgroup, or loaded by each wave in
+//     conv_nchwc_mfma_direct). Sums are in MFMA order, so results equal the
 //     reference's to rounding, and exactly where every partial sum is exact
 //     (the reference's own test data, tools/conv_nchwc_test.c:174-178).
 //   * conv_nchwc_generic, for every other shape: one thread per output
@@ -21,6 +22,7 @@
 
 #include <algorithm>
 #include <type_traits>
+#include <utility>
 
 #include "uk_device_common.h"
 #include "uk_hip_abi.h"
@@ -106,12 +108,19 @@ typedef v4f v4f_a4 __attribute__((aligned(4)));  // dword-aligned wide accesses 
 // With the filter as the first MFMA operand a lane ends up holding output
 // pixel r, channels 4q..4q+3: one 16-byte store. Pixels, panels and channel
 // blocks past the end read the last valid one instead and are not stored; a
-// prefetch past the last step reloads the last step.
+// prefetch past the last step reloads the last step. The launch bound keeps the
+// accumulators in the vector registers the MFMAs name, without a copy to and
+// from the accumulation registers around the loop (3x3, stride 2, 288 -> 96
+// channels at 81x81, batch 5: 217 -> 214 us).
+//
+// Bound by the MFMAs' rate and the workgroups' granularity: 59.2 GFLOP of the
+// batch 16, 256 -> 256 channel layer at 56x56 in 569 us = 104 TFLOP/s, two
+// thirds of the 157 of the matrix cores; 6.25 workgroups per unit run as seven.
 constexpr int kFilterRow = 20;                 // floats per padded ci row in LDS
 constexpr int kFilterTile = 16 * kFilterRow;   // floats per [16][16] tile in LDS
 
 template <int TW, int TO>
-__global__ __launch_bounds__(kThreads) void conv_nchwc_mfma_kernel(ConvArgs a, int64_t px_chunks,
+__global__ __launch_bounds__(kThreads, 2) void conv_nchwc_mfma_kernel(ConvArgs a, int64_t px_chunks,
                                                                    int64_t px_groups,
                                                                    int64_t oc_chunks) {
   static_assert(TO * 64 <= kThreads, "one loader lane per 16 bytes of the step's filter tiles");
@@ -243,6 +252,156 @@ __global__ __launch_bounds__(kThreads) void conv_nchwc_mfma_kernel(ConvArgs a, i
       if (ok[tw][to]) *reinterpret_cast<v4f_a4*>(po[tw][to]) = acc[tw][to];
 }
 
+// The same division of the work without LDS: each wave loads the filter from
+// global memory in the order in which the matrix instructions can take it.
+// Lane (q, r) loads, of the filter rows ci = 4q + w, w = 0..3, TO consecutive
+// floats each (one 4 * TO byte load a row), so that the 16 lanes of a row cover
+// all 16 * TO output channels. MFMA (w, i) multiplies word w of the pixel with
+// float i of row 4q + w: its 16 output rows are the channels i, TO + i, 2 TO + i,
+// ... of the 16 * TO, and the accumulators of i = 0..TO-1 together hold, in each
+// lane, 4 * TO consecutive channels of output pixel r. Sums are the same, in the
+// same order, as with the filter in LDS.
+//
+// Loads run D - 1 steps ahead in D register sets, and no wave waits for another.
+// That is what counts where a compute unit has one workgroup, so one wave per
+// matrix core, and nothing hides a wave's waits: 3x3, batch 16, 256 -> 256
+// channels at 14x14 69 -> 50 us (bound by the 1 wave of MFMAs, 0.58 of their
+// rate), batch 1 at 56x56 75 -> 51 us, batch 4, 272 -> 208, stride 2 at 40x40
+// 115 -> 87 us, batch 8, 512 -> 512 at 28x28 338 -> 297 us. With several
+// workgroups on a unit each wave's own copy of the filter loads costs more than
+// the barriers did (batch 16, 256 -> 256 at 56x56: 569 us with LDS, 611 without).
+template <int... I, typename F>
+__device__ __forceinline__ void for_each_index(std::integer_sequence<int, I...>, F f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+
+template <int TW, int TO, int D>
+__global__ __launch_bounds__(kThreads, 2) void conv_nchwc_mfma_direct_kernel(ConvArgs a, int64_t px_chunks,
+                                                                             int64_t px_groups,
+                                                                             int64_t oc_chunks) {
+  typedef float vTOf __attribute__((ext_vector_type(TO)));
+  typedef vTOf vTOf_a4 __attribute__((aligned(4)));
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  // Consecutive workgroup ids go round-robin to the 8 XCDs, each with its own
+  // L2. Give every XCD a contiguous range of the work instead, so that one L2
+  // sees one image and one filter slice at a time, not a slice of all.
+  const uint32_t nb = gridDim.x, xcd = blockIdx.x & 7u;
+  int64_t t = (int64_t)(xcd * (nb / 8u) + min(xcd, nb % 8u) + (blockIdx.x >> 3));
+  const int64_t pxg = t % px_groups; t /= px_groups;
+  const int64_t occ = t % oc_chunks; t /= oc_chunks;
+  const int64_t n = t % a.N;
+  const int64_t slice = t / a.N;
+  const int64_t ic0 = slice * a.ic_per;
+  const int64_t ic_count = a.ic_slices > 1 ? min(a.ic_per, a.IC - ic0) : a.IC;
+  float* const out_base = a.ic_slices > 1 ? a.partial + slice * a.partial_stride : a.out;
+  const bool accumulate = a.ic_slices > 1 ? false : a.accumulate != 0;
+  const int64_t pxc = pxg * 4 + wave;
+  if (pxc >= px_chunks) return;
+  const int r = lane & 15, q = lane >> 4;
+  const int64_t pixels = a.OH * a.OW;
+
+  // The lane's channels: 4 * TO from channel ko of block occ * TO + 4q * TO / 16.
+  const int64_t oc = occ * TO + q * TO / 4;
+  const int ko = q * 4 * TO % 16;
+  const float* pa[TW];
+  float* po[TW];
+  bool ok[TW];
+#pragma unroll
+  for (int tw = 0; tw < TW; ++tw) {
+    const int64_t px = pxc * (16 * TW) + tw * 16 + r;
+    const int64_t px_in = px < pixels ? px : pixels - 1;
+    const int64_t oh = px_in / a.OW, ow = px_in - oh * a.OW;
+    pa[tw] = a.in + n * a.in_sn + ic0 * a.in_sic + (oh * a.stride_h) * a.in_sh + (ow * a.stride_w) * a.c0 + 4 * q;
+    po[tw] = out_base + n * a.out_sn + oc * a.out_soc + oh * a.out_soh + ow * 16 + ko;
+    ok[tw] = px < pixels && oc < a.OC;
+  }
+  constexpr int kLanesPerBlock = 16 / TO;
+  const int64_t oc_ld = min(occ * TO + r / kLanesPerBlock, a.OC - 1);
+  const float* pf = a.flt + oc_ld * a.f_soc + ic0 * a.f_sic + (4 * q) * 16 + r % kLanesPerBlock * TO;
+
+  // Channel c of the lane's 4 * TO is word c / TO of the accumulator of i = c % TO.
+  v4f acc[TW][TO];
+#pragma unroll
+  for (int tw = 0; tw < TW; ++tw) {
+#pragma unroll
+    for (int to = 0; to < TO; ++to) acc[tw][to] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (accumulate && ok[tw]) {
+#pragma unroll
+      for (int v = 0; v < TO; ++v) {
+        const v4f o = *reinterpret_cast<const v4f_a4*>(po[tw] + 4 * v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[tw][(4 * v + e) % TO][(4 * v + e) / TO] = o[e];
+      }
+    }
+  }
+
+  // Within one (ic_outer, fh) consecutive steps follow each other at 16 input
+  // floats and 256 filter floats.
+  const int64_t taps = a.FW * (a.c0 / 16);
+  const int64_t steps = ic_count * a.FH * taps;
+  if (steps > 0) {
+    const int64_t in_next_fh = a.in_sh - (taps - 1) * 16, f_next_fh = a.f_sfh - (taps - 1) * 256;
+    const int64_t in_next_ic = a.in_sic - (a.FH - 1) * a.in_sh - (taps - 1) * 16;
+    const int64_t f_next_ic = a.f_sic - (a.FH - 1) * a.f_sfh - (taps - 1) * 256;
+    // The step the next prefetch loads: its offsets, how many follow it, and
+    // its distance from the ends of its (ic_outer, fh) and of its ic_outer.
+    int64_t ao = 0, bo = 0, left = steps - 1, tap = taps - 1, fh = a.FH - 1;
+    v4f av[D][TW];
+    vTOf fv[D][4];
+    auto prefetch = [&](auto buf) {
+      constexpr int B = decltype(buf)::value;
+#pragma unroll
+      for (int w = 0; w < 4; ++w) fv[B][w] = *reinterpret_cast<const vTOf_a4*>(pf + bo + w * 16);
+#pragma unroll
+      for (int tw = 0; tw < TW; ++tw) av[B][tw] = *reinterpret_cast<const v4f_a4*>(pa[tw] + ao);
+      const bool last_tap = tap == 0, last_fh = fh == 0, more = left > 0;
+      ao += !more ? 0 : !last_tap ? 16 : !last_fh ? in_next_fh : in_next_ic;
+      bo += !more ? 0 : !last_tap ? 256 : !last_fh ? f_next_fh : f_next_ic;
+      left -= more;
+      fh = !last_tap ? fh : last_fh ? a.FH - 1 : fh - 1;
+      tap = last_tap ? taps - 1 : tap - 1;
+    };
+    auto compute = [&](auto buf) {
+      constexpr int B = decltype(buf)::value;
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int tw = 0; tw < TW; ++tw)
+#pragma unroll
+          for (int to = 0; to < TO; ++to)
+            acc[tw][to] = __builtin_amdgcn_mfma_f32_16x16x4f32(fv[B][w][to], av[B][tw][w],
+                                                               acc[tw][to], 0, 0, 0);
+    };
+    for_each_index(std::make_integer_sequence<int, D - 1>{}, prefetch);
+    auto iteration = [&](auto buf) {
+      constexpr int B = decltype(buf)::value;
+      prefetch(std::integral_constant<int, (B + D - 1) % D>{});
+      // The loads stay ahead of the products that they are a step or more early for.
+      __builtin_amdgcn_sched_barrier(0);
+      compute(buf);
+    };
+    int64_t s = steps;
+    const std::make_integer_sequence<int, D> sets{};
+    for (; s >= D; s -= D) for_each_index(sets, iteration);
+    // The last steps % D are in the first register sets.
+    for_each_index(sets, [&](auto buf) {
+      if (decltype(buf)::value < s) compute(buf);
+    });
+  }
+#pragma unroll
+  for (int tw = 0; tw < TW; ++tw) {
+    if (!ok[tw]) continue;
+#pragma unroll
+    for (int v = 0; v < TO; ++v) {
+      v4f o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = acc[tw][(4 * v + e) % TO][(4 * v + e) / TO];
+      *reinterpret_cast<v4f_a4*>(po[tw] + 4 * v) = o;
+    }
+  }
+}
+
 // out = (ACCUMULATE ? out : 0) + slice 0 + slice 1 + ..., four channels per thread.
 __global__ __launch_bounds__(kThreads) void conv_reduce_slices_kernel(ConvArgs a) {
   const int64_t quads = a.total / 4;   // k0 = 16: four quads per pixel
@@ -263,15 +422,21 @@ __global__ __launch_bounds__(kThreads) void conv_reduce_slices_kernel(ConvArgs a
   }
 }
 
-template <int TW, int TO>
-int launch_mfma(const ConvArgs& a, int64_t N, hipStream_t stream) {
+// D = 0: the filter through LDS, else the direct kernel with D register sets.
+template <int TW, int TO, int D>
+int launch_mfma(const ConvArgs& a, hipStream_t stream) {
   const int64_t px_chunks = uk::ceil_div(a.OH * a.OW, (int64_t)16 * TW);
   const int64_t px_groups = uk::ceil_div(px_chunks, (int64_t)(kThreads / 64));
   const int64_t oc_chunks = uk::ceil_div(a.OC, (int64_t)TO);
-  const int64_t blocks = N * oc_chunks * px_groups * a.ic_slices;
+  const int64_t blocks = a.N * oc_chunks * px_groups * a.ic_slices;
   if (blocks >= (1ll << 31)) return -1;
-  uk::launch(3, conv_nchwc_mfma_kernel<TW, TO>, dim3((uint32_t)blocks), dim3(kThreads), 0, stream,
-             a, px_chunks, px_groups, oc_chunks);
+  if constexpr (D == 0) {
+    uk::launch(3, conv_nchwc_mfma_kernel<TW, TO>, dim3((uint32_t)blocks), dim3(kThreads), 0, stream,
+               a, px_chunks, px_groups, oc_chunks);
+  } else {
+    uk::launch(3, conv_nchwc_mfma_direct_kernel<TW, TO, D>, dim3((uint32_t)blocks), dim3(kThreads), 0, stream,
+               a, px_chunks, px_groups, oc_chunks);
+  }
   if (a.ic_slices > 1) {
     const int64_t rblocks = uk::ceil_div(a.total / 4, (int64_t)kThreads);
     uk::launch(3, conv_reduce_slices_kernel, dim3((uint32_t)std::min<int64_t>(rblocks, 4096)), dim3(kThreads), 0,
@@ -280,19 +445,34 @@ int launch_mfma(const ConvArgs& a, int64_t N, hipStream_t stream) {
   return (int)hipGetLastError();
 }
 
-// Workgroups a launch with TW panels and TO output-channel blocks per wave has.
-int64_t mfma_blocks(const ConvArgs& a, int64_t N, int tw, int to) {
-  const int64_t px_chunks = uk::ceil_div(a.OH * a.OW, (int64_t)16 * tw);
-  return N * uk::ceil_div(a.OC, (int64_t)to) * uk::ceil_div(px_chunks, (int64_t)(kThreads / 64));
-}
+// A kernel and its share of the output: TW panels of pixels and TO
+// output-channel blocks per wave. `cost` is the measured time of one step per
+// panel and block of a wave in 0.1 ns (the four MFMAs alone take 533), from
+// layers of 64 to 512 channels at 14x14 to 112x112, batch 1 to 16.
+struct MfmaTile {
+  int tw, to;
+  enum { kOne, kMore, kAny } rounds;  // of workgroups on the compute units: those that `cost` was measured with
+  int cost;
+  int (*launch)(const ConvArgs&, hipStream_t);
+};
+constexpr MfmaTile kMfmaTiles[] = {
+    {4, 4, MfmaTile::kOne, 645, launch_mfma<4, 4, 2>},
+    {2, 4, MfmaTile::kOne, 710, launch_mfma<2, 4, 2>},
+    {2, 2, MfmaTile::kOne, 870, launch_mfma<2, 2, 4>},
+    {1, 4, MfmaTile::kOne, 905, launch_mfma<1, 4, 4>},
+    {1, 2, MfmaTile::kAny, 1050, launch_mfma<1, 2, 4>},
+    {1, 1, MfmaTile::kAny, 1220, launch_mfma<1, 1, 4>},
+    {4, 4, MfmaTile::kMore, 700, launch_mfma<4, 4, 0>},
+    {2, 4, MfmaTile::kMore, 730, launch_mfma<2, 4, 0>},
+    {1, 4, MfmaTile::kMore, 790, launch_mfma<1, 4, 0>},
+    {2, 2, MfmaTile::kMore, 830, launch_mfma<2, 2, 0>},
+    {2, 1, MfmaTile::kMore, 1000, launch_mfma<2, 1, 0>},
+};
 
-template <int TO>
-int launch_mfma_for_pixels(const ConvArgs& a, int64_t N, hipStream_t stream, bool one_panel) {
-  const int64_t pixels = a.OH * a.OW;
-  // Two panels per wave: four measured no faster (608 against 583 us on a 3x3
-  // 256 -> 256 channel layer at 56x56) and leave fewer, longer work items.
-  if (pixels > 16 && !one_panel) return launch_mfma<2, TO>(a, N, stream);
-  return launch_mfma<1, TO>(a, N, stream);
+// Workgroups a launch of `tile` has, without slices.
+int64_t mfma_blocks(const ConvArgs& a, const MfmaTile& tile) {
+  const int64_t px_chunks = uk::ceil_div(a.OH * a.OW, (int64_t)16 * tile.tw);
+  return a.N * uk::ceil_div(a.OC, (int64_t)tile.to) * uk::ceil_div(px_chunks, (int64_t)(kThreads / 64));
 }
 
 }  // namespace
@@ -334,33 +514,41 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
   }
   if (kernel_mode != IREE_UK_AMD_KERNEL_MODE_GENERIC &&
       iree_uk_amd_hip_conv_nchwc_has_mfma_kernel(p->k0, p->c0, p->flags)) {
-    // Output-channel blocks per wave: four when that pads OC_outer no further
-    // than two would (each input piece then meets four filter tiles: 583 -> 554
-    // us on a 3x3 256 -> 256 channel layer at 56x56), else two, else one.
-    const bool four = a.OC > 2 && uk::ceil_div(a.OC, (int64_t)4) * 4 == uk::ceil_div(a.OC, (int64_t)2) * 2;
-    // A layer with few output pixels (the last stages of an image network at
-    // batch 1: 512 -> 512 channels, 7x7 outputs) leaves most compute units
-    // without a workgroup at those sizes: the wave's share shrinks, first in
-    // output channels, then in pixels, until the workgroups outnumber the units
-    // (8 -> 32 workgroups on that layer: 189 -> 72 us; 256 -> 256 channels at 56x56, batch 1: 97 -> 70 us).
-    int to = four ? 4 : a.OC > 1 ? 2 : 1;
-    int tw = a.OH * a.OW > 16 ? 2 : 1;
+    // The tile whose fullest compute unit is done first: workgroups per unit,
+    // rounded up, times the work of one, times what that costs in this tile.
+    // Large tiles re-read less and cost less per block; small ones waste less
+    // in the last round and at the edges. This puts 256 -> 256 channels at
+    // 56x56, batch 16, on 2x4 through LDS (569 us; 1x4 574, 4x4 611, 2x2 615),
+    // 128 -> 128 on 1x4 (158 us; 2x4 169, 2x2 172).
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     }
-    while (mfma_blocks(a, p->N, tw, to) < cus && (to > 1 || tw > 1)) {
-      if (to > 1) to /= 2;
-      else tw = 1;
+    // Sums of fewer than eight steps (1x1 filters on few channels) are loads
+    // and stores rather than products and want more than one wave on a matrix
+    // core: 64 -> 176 channels, 1x1, 78x78, batch 3 took 13.4 us on 4x4, one
+    // workgroup per unit, and 11.1 on 2x4 through LDS, two per unit.
+    const int64_t steps_per_ic = a.FH * a.FW * (a.c0 / 16);
+    const bool short_sums = a.IC * steps_per_ic < 8;
+    const MfmaTile* tile = nullptr;
+    int64_t least = 0;
+    for (const MfmaTile& t : kMfmaTiles) {
+      const int64_t rounds = uk::ceil_div(mfma_blocks(a, t), (int64_t)cus);
+      if (t.rounds == MfmaTile::kOne && (rounds > 1 || short_sums)) continue;
+      if (t.rounds == MfmaTile::kMore && rounds <= 1) continue;
+      const int64_t cost = rounds * t.tw * t.to * t.cost;
+      if (!tile || cost < least) {
+        tile = &t;
+        least = cost;
+      }
     }
-    // Still fewer workgroups than half the units: IC_outer is split over
+    // Fewer workgroups than half the units: IC_outer is split over
     // several workgroups per output block, whose sums meet in a buffer the
     // library keeps and are added up in slice order by a second kernel (the
-    // same result on every run; 512 -> 512 channels at 7x7, batch 1: 72 -> 17
-    // us). While the stream is being captured into a graph there is no buffer
+    // same result on every run; 512 -> 512 channels at 7x7, batch 1: 14 us,
+    // without slices 72). While the stream is being captured into a graph there is no buffer
     // to be had, and the call runs unsplit.
-    const int64_t blocks0 = mfma_blocks(a, p->N, tw, to);
-    const int64_t steps_per_ic = a.FH * a.FW * (a.c0 / 16);
+    const int64_t blocks0 = mfma_blocks(a, *tile);
     if (blocks0 * 2 <= cus && a.IC >= 2 && a.out_sn >= 0 && a.out_soc >= 0 && a.out_soh >= 0) {
       int64_t slices = std::min<int64_t>(std::min<int64_t>(a.IC, cus / blocks0), 16);
       while (slices > 1 && uk::ceil_div(a.IC, slices) * steps_per_ic < 8) --slices;
@@ -376,9 +564,7 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
         a.partial_stride = span;
       }
     }
-    int st = to == 4   ? launch_mfma_for_pixels<4>(a, p->N, stream, tw == 1)
-             : to == 2 ? launch_mfma_for_pixels<2>(a, p->N, stream, tw == 1)
-                       : launch_mfma_for_pixels<1>(a, p->N, stream, tw == 1);
+    const int st = tile->launch(a, stream);
     if (st >= 0) {
       *kernel_name = "conv_nchwc_mfma";
       return st;
