@@ -536,6 +536,10 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
       const int64_t rounds = uk::ceil_div(mfma_blocks(a, t), (int64_t)cus);
       if (t.rounds == MfmaTile::kOne && (rounds > 1 || short_sums)) continue;
       if (t.rounds == MfmaTile::kMore && rounds <= 1) continue;
+      // Each group of channel blocks reads the input again, from memory where
+      // the layer is a large one: 288 -> 48 channels, 3x3, stride 2, 84x84,
+      // batch 12 (394 MB of input) took 364 us one block at a time, 284 on 2x4.
+      if (t.to == 1 && rounds > 1 && a.OC > 1) continue;
       const int64_t cost = rounds * t.tw * t.to * t.cost;
       if (!tile || cost < least) {
         tile = &t;
