@@ -469,10 +469,14 @@ constexpr MfmaTile kMfmaTiles[] = {
     {2, 1, MfmaTile::kMore, 1000, launch_mfma<2, 1, 0>},
 };
 
-// Workgroups a launch of `tile` has, without slices.
+// Workgroups a launch of `tile` has, without slices. tw and to are powers of
+// two, so that going through the table costs shifts and not divisions: at 5 us
+// a launch the host is what small layers wait for.
 int64_t mfma_blocks(const ConvArgs& a, const MfmaTile& tile) {
-  const int64_t px_chunks = uk::ceil_div(a.OH * a.OW, (int64_t)16 * tile.tw);
-  return a.N * uk::ceil_div(a.OC, (int64_t)tile.to) * uk::ceil_div(px_chunks, (int64_t)(kThreads / 64));
+  const int px_shift = 4 + 2 + __builtin_ctz((unsigned)tile.tw);   // 16 pixels, four waves
+  const int to_shift = __builtin_ctz((unsigned)tile.to);
+  const int64_t px_groups = (a.OH * a.OW + (1ll << px_shift) - 1) >> px_shift;
+  return a.N * ((a.OC + tile.to - 1) >> to_shift) * px_groups;
 }
 
 }  // namespace
