@@ -377,6 +377,10 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
                                        hipStream_t stream) {
   const bool ti = p->flags & IREE_UK_FLAG_PACK_TRANSPOSE_INNER;
   const bool to = p->flags & IREE_UK_FLAG_PACK_TRANSPOSE_OUTER;
+  // A matrix without a row or a column (its tiles are all padding) may come with
+  // no memory at all, and the kernel's loads stand on the last row where there
+  // is nothing to load: the tiled kernel, which predicates them, takes it.
+  if (p->in_size0 <= 0 || p->in_size1 <= 0) return nullptr;
   if (p->in_stride1 != 1 || p->in_stride0 < 0) return nullptr;
   // Element of the transposition and the tile's extents in such elements:
   // t0 along the matrix rows, t1 along its columns.

@@ -312,6 +312,30 @@ def test_unpack_rows_of_any_length_and_alignment(gpu, oracle, tf, t0, t1, flags)
         assert np.array_equal(got, want), (c.label(), lib.last_kernel_name())
 
 
+@pytest.mark.parametrize("in0,in1", [(0, 64), (64, 0), (0, 0), (0, 7)])
+@pytest.mark.parametrize("tf,s2,s3,flags", [
+    (uk.PACK_TYPE_I8I8, 16, 16, 0x100), (uk.PACK_TYPE_I8I8, 16, 2, 0x300), (uk.PACK_TYPE_I8I8, 16, 2, 0),
+    (uk.PACK_TYPE_I8I8, 16, 4, 0x200), (uk.PACK_TYPE_F16F16, 16, 16, 0x300), (uk.PACK_TYPE_BF16BF16, 16, 2, 0),
+    (uk.PACK_TYPE_F32F32, 16, 4, 0x100), (uk.PACK_TYPE_F32F32, 16, 1, 0x200), (uk.PACK_TYPE_F32F32, 16, 16, 0)])
+def test_pack_of_an_empty_matrix_is_all_padding(gpu, oracle, tf, s2, s3, flags, in0, in1):
+    """Rows or columns but no element, and no memory behind them (the source is a
+    null pointer): every tile is padding, and the kernels that load
+    unconditionally stay out of it."""
+    lib, torch = gpu
+    o0, o1 = 65, 66
+    c = T.PackCase(tf | flags, in0, in1, o0, o1, s2, s3, in1, 1, o1 * s2 * s3, 0, 0, 0x1122334455667788)
+    inp, out0 = T.make_pack_buffers(c, np.random.default_rng(in0 + in1))
+    want = out0.copy()
+    G.run_pack_case(oracle, c, inp, want)
+    lib.set_pointer_mode(uk.POINTER_MODE_DEVICE)
+    d_out = T.DeviceBytes(torch, out0)
+    lib.pack(0, 0, c.in_stride0, 1, d_out.ptr, 0, c.out_stride0, c.out_stride1, in0, in1, o0, o1, s2, s3,
+             c.padding_value, c.flags)
+    lib.synchronize()
+    assert np.array_equal(d_out.numpy(), want), (c.label(), lib.last_kernel_name())
+    assert lib.last_kernel_name() in ("pack_tiled", "pack_generic"), lib.last_kernel_name()
+
+
 SINGLE_LINE_TILES = [
     (uk.PACK_TYPE_F32F32, 16, 1), (uk.PACK_TYPE_F32F32, 1, 16), (uk.PACK_TYPE_I32I32, 8, 1),
     (uk.PACK_TYPE_F16F16, 1, 16), (uk.PACK_TYPE_BF16BF16, 16, 1), (uk.PACK_TYPE_I8I8, 1, 16),
