@@ -222,7 +222,7 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
     for (int i = 0; i < N1; ++i) {
       const uint32_t idx = tid + i * kThreads;
       const uint32_t r = idx / VPR, cb = (idx % VPR) * 16;
-      const int32_t left = b.row_base + r < a.rows ? (int32_t)(a.row_bytes - (b.col_base_bytes + cb)) : 0;
+      const int32_t left = b.row_base + r < a.rows ? uk::row_bytes_left(a.row_bytes, b.col_base_bytes + cb) : 0;
       uint32_t w[4] = {pre[i][0], pre[i][1], pre[i][2], pre[i][3]};
       if (a.row_bytes < 16) uk::load_short_row<16>(w, a.src + (int64_t)(b.row_base + r) * a.src_pitch + cb, left);
       uk::clip_piece<16>(w, left, a.pad32);

@@ -748,7 +748,7 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
         uint32_t r, cb;
         mat_item<MV>(a, tid + i * NT, &r, &cb);
         const int32_t left =
-            b.row_base + r < a.mat_size0 ? (int32_t)(size1_bytes - (b.col_base_bytes + cb)) : 0;
+            b.row_base + r < a.mat_size0 ? uk::row_bytes_left(size1_bytes, b.col_base_bytes + cb) : 0;
         Words<MV> w = __builtin_bit_cast(Words<MV>, pre1[i]);
         uk::clip_piece<MV>(w.w, left, a.pad32);
         if (tid + i * NT < total1) lds_store_static<MV, P>(lbuf + l1off[i], __builtin_bit_cast(MatVec, w));
@@ -784,7 +784,7 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
           uint32_t r, cb;
           mat_item<MV>(a, tid + i * NT, &r, &cb);
           if (tid + i * NT >= total1 || b.row_base + r >= a.mat_size0) continue;
-          const int32_t left = (int32_t)(size1_bytes - (b.col_base_bytes + cb));
+          const int32_t left = uk::row_bytes_left(size1_bytes, b.col_base_bytes + cb);
           if (left >= MV) {
             gstore<MV, NTS>(base + g1off[i], reg[i]);
           } else if (left > 0) {

@@ -107,6 +107,12 @@ __device__ __forceinline__ void clip_piece(uint32_t (&w)[N / 4], int32_t left, u
     w[0] = (uint32_t)lo; w[1] = (uint32_t)(lo >> 32); w[2] = (uint32_t)hi; w[3] = (uint32_t)(hi >> 32);
   }
 }
+// What a row of `row_bytes` (below 2^31) still holds from byte `off` on: 0 where
+// it has ended. Tiles may pad a row by any amount, so the difference itself can
+// be -2^31 and less and would come out positive.
+__device__ __forceinline__ int32_t row_bytes_left(uint32_t row_bytes, uint32_t off) {
+  return off < row_bytes ? (int32_t)(row_bytes - off) : 0;
+}
 // The same piece for a row of fewer than N bytes: the `left` bytes at `p`, one by
 // one, to where `clip_piece` expects them. (Rare: kept out of the way as a
 // rolled loop.)
