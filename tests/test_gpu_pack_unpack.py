@@ -345,8 +345,8 @@ def test_pack_and_unpack_of_rows_in_more_than_2_gib_of_padding(gpu):
     tiles = torch.empty(n1 * t1, dtype=torch.int16, device="cuda")
     tiles.fill_(1)
     row = torch.arange(100, 100 + n, dtype=torch.int16, device="cuda")
-    lib.pack(row.data_ptr(), 0, n, 1, tiles.data_ptr(), 0, n1 * t1, t1, 1, n, 1, n1, 1, t1, 0x1234,
-             uk.PACK_TYPE_F16F16)
+    lib.pack(row.data_ptr(), 0, n, 1, tiles.data_ptr(), 0, t1, t1, 1, n, n1, 1, 1, t1, 0x1234,
+             uk.PACK_TYPE_F16F16 | uk.PACK_TRANSPOSE_OUTER)
     lib.synchronize()
     assert lib.last_kernel_name() == "pack_stream"
     assert torch.equal(tiles[:n], row)
@@ -354,7 +354,8 @@ def test_pack_and_unpack_of_rows_in_more_than_2_gib_of_padding(gpu):
     tiles.fill_(7)
     tiles[:n] = row
     out = torch.full((1 << 20,), 3, dtype=torch.int16, device="cuda")
-    lib.unpack(tiles.data_ptr(), 0, n1 * t1, t1, out.data_ptr(), 0, n, 1, 1, n1, 1, t1, 1, n, uk.UNPACK_TYPE_F16F16)
+    lib.unpack(tiles.data_ptr(), 0, t1, t1, out.data_ptr(), 0, n, 1, n1, 1, 1, t1, 1, n,
+               uk.UNPACK_TYPE_F16F16 | uk.UNPACK_TRANSPOSE_OUTER)
     lib.synchronize()
     assert lib.last_kernel_name() == "unpack_stream"
     assert torch.equal(out[:n], row)
