@@ -427,6 +427,7 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
   // 32-bit offsets inside a block, 32-bit sizes.
   if (pitch * kBlockRows >= (1ll << 31) || tiles0 * s0 + tiles1 * s1 >= (1ll << 31)) return nullptr;
   if (p->in_size0 >= (1ll << 31) || size1 * eb >= (1ll << 31) || outer0 >= (1ll << 24) || outer1 >= (1ll << 24)) return nullptr;
+  if (outer1 * t1 * eb > (1ll << 32) - (1 << 17)) return nullptr;  // (padded row, counted in 32 bits)
   const int64_t nblk0 = uk::ceil_div(outer0, tiles0), nblk1 = uk::ceil_div(outer1, tiles1);
   if (nblk0 * nblk1 >= (1ll << 31) || nblk0 * nblk1 == 0) return nullptr;
 

@@ -884,6 +884,10 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   if (tile_bytes == 0 || tile_bytes > 16384) return plan;
   if (v.outer0 >= (1ll << 24) || v.outer1 >= (1ll << 24)) return plan;
   if (mat_size0 >= (1ll << 31) || mat_size1 * es >= (1ll << 31)) return plan;
+  // Rows, and bytes along a row, are counted in 32 bits to the end of the last
+  // block, and tiles may pad the matrix by any amount.
+  const int64_t kMostPadded = (1ll << 32) - (1 << 17);
+  if (v.outer0 * v.tile0 > kMostPadded || v.outer1 * v.tile1 * es > kMostPadded) return plan;
   // Tiled-side vector width: alignment of base, outer stride and tile size.
   const int64_t tiled_align = std::min(
       {uk::pow2_divisor((int64_t)(uintptr_t)tiled_ptr, 16),

@@ -336,19 +336,21 @@ def test_pack_of_an_empty_matrix_is_all_padding(gpu, oracle, tf, s2, s3, flags, 
     assert lib.last_kernel_name() in ("pack_tiled", "pack_generic"), lib.last_kernel_name()
 
 
-def test_pack_and_unpack_of_rows_in_more_than_2_gib_of_padding(gpu):
-    """One row of 16 elements in tiles that pad it to just over 2^31 bytes: what a
-    piece of a tile lies beyond the row's end is a distance of more than 31 bits.
-    pack pads all of it, unpack stores the 16 elements and nothing else."""
+@pytest.mark.parametrize("n1,kernel", [((1 << 19) + 40, "stream"), ((1 << 20) + 40, "generic")])
+def test_pack_and_unpack_of_rows_in_gigabytes_of_padding(gpu, n1, kernel):
+    """One row of 16 elements in tiles that pad it to just over 2^31 and 2^32
+    bytes: what a piece of a tile lies beyond the row's end is a distance of more
+    than 31 bits, and its position a number of more than 32. pack pads all of it,
+    unpack stores the 16 elements and nothing else."""
     lib, torch = gpu
-    n1, t1, n = (1 << 19) + 40, 2048, 16
+    t1, n = 2048, 16
     tiles = torch.empty(n1 * t1, dtype=torch.int16, device="cuda")
     tiles.fill_(1)
     row = torch.arange(100, 100 + n, dtype=torch.int16, device="cuda")
     lib.pack(row.data_ptr(), 0, n, 1, tiles.data_ptr(), 0, t1, t1, 1, n, n1, 1, 1, t1, 0x1234,
              uk.PACK_TYPE_F16F16 | uk.PACK_TRANSPOSE_OUTER)
     lib.synchronize()
-    assert lib.last_kernel_name() == "pack_stream"
+    assert lib.last_kernel_name() == "pack_" + kernel
     assert torch.equal(tiles[:n], row)
     assert bool((tiles[n:] == 0x1234).all())
     tiles.fill_(7)
@@ -357,7 +359,7 @@ def test_pack_and_unpack_of_rows_in_more_than_2_gib_of_padding(gpu):
     lib.unpack(tiles.data_ptr(), 0, t1, t1, out.data_ptr(), 0, n, 1, n1, 1, 1, t1, 1, n,
                uk.UNPACK_TYPE_F16F16 | uk.UNPACK_TRANSPOSE_OUTER)
     lib.synchronize()
-    assert lib.last_kernel_name() == "unpack_stream"
+    assert lib.last_kernel_name() == "unpack_" + kernel
     assert torch.equal(out[:n], row)
     assert bool((out[n:] == 3).all())
 
