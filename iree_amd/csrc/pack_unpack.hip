@@ -169,13 +169,26 @@ template <int N> struct Bytes;
 template <> struct Bytes<1> { using type = uint8_t; };
 template <> struct Bytes<2> { using type = uint16_t; };
 template <> struct Bytes<4> { using type = uint32_t; };
-template <> struct Bytes<8> { using type = uint2; };
-template <> struct Bytes<16> { using type = uint4; };
+template <> struct Bytes<8> { typedef uint32_t type __attribute__((ext_vector_type(2))); };
+template <> struct Bytes<16> { typedef uint32_t type __attribute__((ext_vector_type(4))); };
 
 template <int N>
 __device__ __forceinline__ void copy_bytes(void* dst, const void* src) {
   using T = typename Bytes<N>::type;
   *reinterpret_cast<T*>(dst) = *reinterpret_cast<const T*>(src);
+}
+// The same where `src` / `dst` is global memory at any address (see gload).
+template <int N>
+__device__ __forceinline__ void copy_from_global(void* dst, const char* src) {
+  typedef typename Bytes<N>::type T;
+  typedef T T1 __attribute__((aligned(1)));
+  *reinterpret_cast<T*>(dst) = *reinterpret_cast<const T1*>(src);
+}
+template <int N>
+__device__ __forceinline__ void copy_to_global(char* dst, const void* src) {
+  typedef typename Bytes<N>::type T;
+  typedef T T1 __attribute__((aligned(1)));
+  *reinterpret_cast<T1*>(dst) = *reinterpret_cast<const T*>(src);
 }
 
 // Copies n = VEC bytes between a register buffer and memory using accesses of
@@ -287,10 +300,10 @@ __global__ __launch_bounds__(kThreads) void pack_tiled_kernel(TiledArgs a) {
       const char* gp = a.src + (int64_t)grow * a.mat_stride0_bytes + cb;
       if (row_ok && cb + mv <= size1_bytes) {
         switch (mv) {
-          case 16: copy_bytes<16>(reg, gp); break;
-          case 8: copy_bytes<8>(reg, gp); break;
-          case 4: copy_bytes<4>(reg, gp); break;
-          case 2: copy_bytes<2>(reg, gp); break;
+          case 16: copy_from_global<16>(reg, gp); break;
+          case 8: copy_from_global<8>(reg, gp); break;
+          case 4: copy_from_global<4>(reg, gp); break;
+          case 2: copy_from_global<2>(reg, gp); break;
           default: reg[0] = gp[0]; break;
         }
       } else {
@@ -406,10 +419,10 @@ __global__ __launch_bounds__(kThreads) void unpack_tiled_kernel(TiledArgs a) {
       char* gp = a.dst + (int64_t)grow * a.mat_stride0_bytes + cb;
       if (cb + mv <= size1_bytes) {
         switch (mv) {
-          case 16: copy_bytes<16>(gp, reg); break;
-          case 8: copy_bytes<8>(gp, reg); break;
-          case 4: copy_bytes<4>(gp, reg); break;
-          case 2: copy_bytes<2>(gp, reg); break;
+          case 16: copy_to_global<16>(gp, reg); break;
+          case 8: copy_to_global<8>(gp, reg); break;
+          case 4: copy_to_global<4>(gp, reg); break;
+          case 2: copy_to_global<2>(gp, reg); break;
           default: gp[0] = reg[0]; break;
         }
       } else {
@@ -917,7 +930,17 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // 37.1, from where on the pack itself decides).
   const bool big_transposing = G == 4 && total_bytes >= (192ll << 20);
   const bool big_rows = G == 16 && !to && total_bytes >= ((mat_is_dest ? 192ll : 72ll) << 20);
-  const bool big = allow_big && VEC == 16 && (big_transposing || big_rows);
+  // Narrow matrices, whose rows end within the first hundred bytes: every block
+  // of the streaming kernels is an edge block of theirs, and the tiled kernels,
+  // which have no edge path apart, are ahead by up to three times (16-byte rows of
+  // f32, unpack 912329 x 4 from 16x4 14.7 us against 34; pack 2215721 x 14 bf16 into
+  // 32x8 86 against 122; f16 1303882 x 13 unpack, 12x12 under TRANSPOSE_OUTER, 117
+  // against 285). From 96 padded bytes on they are level or behind (pack f32
+  // 427710 x 21 into 24x4: 40 against 39), under TRANSPOSE_OUTER beyond 128 (pack
+  // f32 2103812 x 5 into 16x32, 128 bytes: 245 against 652).
+  const int64_t padded_row_bytes = v.outer1 * v.tile1 * es;
+  const bool narrow = to ? padded_row_bytes <= 128 : padded_row_bytes < 96;
+  const bool big = allow_big && !narrow && VEC == 16 && (big_transposing || big_rows);
   const int64_t kMinSpan = big ? 512 : 256;                      // bytes, both sides
   const int64_t kTarget = big ? kStreamBigBlockBytes : kStreamBlockBytes;  // bytes per block, about
   const int64_t stream_block = kTarget;
@@ -1026,7 +1049,8 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   a.lds_buf_bytes = (uint32_t)((lds_bytes + 255) / 256 * 256);
   // Streaming kernels: 32-bit offsets inside one block on both sides, granules
   // of at least 4 bytes, at most 4 granules per vector, block within budget.
-  // (and non-negative strides: the 32-bit offsets are unsigned)
+  // (and non-negative strides: the 32-bit offsets are unsigned; rows of at least
+  // 16 bytes, which pack's loads need and below which unpack is level)
   plan.stream = block_row_bytes % 4 == 0 && mat_size0 > 0 && mat_size1 * es >= 16 && G >= 4 && VEC / G <= 4 && mat_stride0 >= 0 && v.sl0 >= 0 &&
                 v.sl1 >= 0 &&
                 block_rows * block_row_bytes <= stream_block &&
@@ -1054,13 +1078,18 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // (f32 8192x8192 unpack under TRANSPOSE_OUTER: 106 -> 77 us). Below that
   // size the plain stores are as fast or faster.
   a.streaming_stores = total_bytes >= (192ll << 20) && uk::pow2_divisor(mat_stride0 * es, 16) >= 16;
-  if (plan.stream) {
+  // (The tiled kernels too move such vectors where rows are not whole words
+  // apart, for an element at a time is what they would be left with: s8 31405 x
+  // 85, 12x12 under TRANSPOSE_OUTER, 12.1 -> 8.4 us. With whole words their own choice
+  // is level or ahead.)
+  if (plan.stream && !(narrow && mat_vec >= 4)) {
     a.mat_vec = (uint32_t)plan.MV;
     a.div_row_vecs = FastDiv((uint32_t)(block_row_bytes / plan.MV));
     a.mat_stride0_bytes32 = (uint32_t)(mat_stride0 * es);
     a.sl0_bytes32 = (uint32_t)(v.sl0 * es);
     a.sl1_bytes32 = (uint32_t)(v.sl1 * es);
   }
+  if (narrow) plan.stream = false;
   // Walk over the blocks: bands of block rows, within a band groups of block
   // columns row by row. One block row after the other, except for the packs
   // under TRANSPOSE_OUTER in 64 KB blocks: there the blocks of one block row

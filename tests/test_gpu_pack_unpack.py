@@ -364,6 +364,46 @@ def test_pack_and_unpack_of_rows_in_gigabytes_of_padding(gpu, n1, kernel):
     assert bool((out[n:] == 3).all())
 
 
+@pytest.mark.parametrize("tf,t0,t1,flags", [
+    (uk.PACK_TYPE_F32F32, 16, 4, 0), (uk.PACK_TYPE_F32F32, 8, 8, 0x200), (uk.PACK_TYPE_F32F32, 16, 1, 0x300),
+    (uk.PACK_TYPE_BF16BF16, 12, 12, 0), (uk.PACK_TYPE_BF16BF16, 16, 8, 0x200), (uk.PACK_TYPE_I8I8, 12, 12, 0x200),
+    (uk.PACK_TYPE_I8I8, 16, 16, 0)])
+def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
+    """Rows whose tiles end below 96 bytes (128 under TRANSPOSE_OUTER), and the
+    first ones beyond, from all row alignments: which kernel, and its bytes."""
+    lib, torch = gpu
+    es = uk.PACK_TYPE_BYTES[tf]
+    rng = np.random.default_rng(t0 * 100 + t1)
+    tile_row = t1 * es
+    for ci, cols in enumerate(sorted({c for b in (16, 33, 64, 80, 95, 96, 97, 112, 128, 129, 144) for c in
+                                      (b // es, b // es + 1)})):
+        rows = int(rng.integers(100, 300))
+        padded = -(-cols // t1) * tile_row
+        narrow = padded <= 128 if flags & 0x200 else padded < 96
+        o0, o1 = -(-rows // t0), -(-cols // t1)
+        so0, so1 = (o1, o0) if flags & 0x200 else (o0, o1)
+        s2, s3 = (t1, t0) if flags & 0x100 else (t0, t1)
+        want_kernel = "tiled" if narrow or cols * es < 16 else "stream"
+        c = T.PackCase(tf | flags, rows, cols, so0, so1, s2, s3, cols + ci % 2, 1, so1 * s2 * s3, 0, 0, 0x0102030405060708)
+        inp, out0 = T.make_pack_buffers(c, rng)
+        want = out0.copy()
+        G.run_pack_case(oracle, c, inp, want)
+        lib.set_kernel_mode(uk.KERNEL_MODE_MFMA_VARIANT + 1)   # past the direct and the transposing kernel
+        got = T.gpu_pack(lib, torch, c, inp, out0)
+        assert np.array_equal(got, want), c.label()
+        assert lib.last_kernel_name() == "pack_" + want_kernel, (c.label(), lib.last_kernel_name())
+        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+        if es == 1:
+            continue
+        u = T.UnpackCase(tf | flags, so0, so1, s2, s3, rows, cols, so1 * s2 * s3, cols + ci % 2, 1, 0, 0)
+        inp, out0 = T.make_unpack_buffers(u, rng)
+        want = out0.copy()
+        G.run_unpack_case(oracle, u, inp, want)
+        got = T.gpu_unpack(lib, torch, u, inp, out0)
+        assert np.array_equal(got, want), u.label()
+        assert lib.last_kernel_name() == "unpack_" + want_kernel, (u.label(), lib.last_kernel_name())
+
+
 SINGLE_LINE_TILES = [
     (uk.PACK_TYPE_F32F32, 16, 1), (uk.PACK_TYPE_F32F32, 1, 16), (uk.PACK_TYPE_I32I32, 8, 1),
     (uk.PACK_TYPE_F16F16, 1, 16), (uk.PACK_TYPE_BF16BF16, 16, 1), (uk.PACK_TYPE_I8I8, 1, 16),
