@@ -224,8 +224,8 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
       const uint32_t r = idx / VPR, cb = (idx % VPR) * 16;
       const int32_t left = b.row_base + r < a.rows ? uk::row_bytes_left(a.row_bytes, b.col_base_bytes + cb) : 0;
       uint32_t w[4] = {pre[i][0], pre[i][1], pre[i][2], pre[i][3]};
-      if (a.row_bytes < 16) uk::load_short_row<16>(w, a.src + (int64_t)(b.row_base + r) * a.src_pitch + cb, left);
-      uk::clip_piece<16>(w, left, a.pad32);
+      if (a.row_bytes < 16) uk::load_short_row<16>(w, a.src + (int64_t)(b.row_base + r) * a.src_pitch + cb, left, a.pad32);
+      else uk::clip_piece<16>(w, left, a.pad32);
       *reinterpret_cast<v4u*>(lbuf + l1off[i]) = v4u{w[0], w[1], w[2], w[3]};
     }
   };

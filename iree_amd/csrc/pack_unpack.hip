@@ -1241,14 +1241,14 @@ __global__ __launch_bounds__(kThreads) void pack_direct_kernel(DirectArgs a) {
 #pragma unroll
     for (int i = 0; i < kDirectPieces; ++i)
       v[i] = __builtin_bit_cast(Words<PB>, gload<PB>(srow + uk::clipped_offset<PB>(col0 + i * 16 * PB, a.row_bytes)));
+#pragma unroll
+    for (int i = 0; i < kDirectPieces; ++i)
+      uk::clip_piece<PB>(v[i].w, row_ok ? (int32_t)(a.row_bytes - (col0 + i * 16 * PB)) : 0, a.pad32);
   } else {
-    const int32_t left = (int32_t)(a.row_bytes - col0);
+    const int32_t left = row_ok ? (int32_t)(a.row_bytes - col0) : 0;
 #pragma unroll
-    for (int i = 0; i < kDirectPieces; ++i) uk::load_short_row<PB>(v[i].w, srow + col0, i == 0 ? left : 0);
+    for (int i = 0; i < kDirectPieces; ++i) uk::load_short_row<PB>(v[i].w, srow + col0, i == 0 ? left : 0, a.pad32);
   }
-#pragma unroll
-  for (int i = 0; i < kDirectPieces; ++i)
-    uk::clip_piece<PB>(v[i].w, row_ok ? (int32_t)(a.row_bytes - (col0 + i * 16 * PB)) : 0, a.pad32);
 #pragma unroll
   for (int i = 0; i < kDirectPieces; ++i) {
     const uint32_t col = col0 + i * 16 * PB;
