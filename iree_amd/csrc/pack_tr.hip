@@ -430,6 +430,18 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
   if (outer1 * t1 * eb > (1ll << 32) - (1 << 17)) return nullptr;  // (padded row, counted in 32 bits)
   const int64_t nblk0 = uk::ceil_div(outer0, tiles0), nblk1 = uk::ceil_div(outer1, tiles1);
   if (nblk0 * nblk1 >= (1ll << 31) || nblk0 * nblk1 == 0) return nullptr;
+  // Narrow matrices: a block's lanes stand for 512 bytes of every row, and rows of
+  // a few bytes leave nearly all of them idle. Beyond a round of blocks (half a
+  // round where rows are under 16 bytes and loaded in parts) the tiled kernel is
+  // ahead, whose blocks follow the matrix's shape: bf16 353322 x 5 into 16x1 11.3 us
+  // there and 42 here, f32 565676 x 8 into 16x1 16 and 47, s8 114948 x 10 into 32x8
+  // transposed 6.9 and 16; at 580 blocks of short rows 4.3 and 4.9, at 490 level.
+  // Rows that are whole words, which the tiled kernel loads as such, are better off
+  // there up to 64 bytes, others up to 32: f32 90303 x 8 into 16x4 7.7 and 9.9; s8
+  // 111358 x 18 into 8x8 transposed 9.9 and 14.9, but 114248 x 49 into 16x1 22 and 14.
+  const int64_t row_bytes = p->in_size1 * es;
+  const bool whole_words = (((uintptr_t)src | (uint64_t)pitch) & 3) == 0;
+  if (nblk0 * nblk1 > (row_bytes < 16 ? 512 : 1024) && row_bytes <= (whole_words ? 64 : 32)) return nullptr;
 
   // Rows that are not whole words apart, or that end inside a tile row.
   const bool ragged = (((uintptr_t)src | (uint64_t)pitch) & 3) || (!ti && p->in_size1 % p->out_size3 != 0);

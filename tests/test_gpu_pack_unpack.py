@@ -404,6 +404,34 @@ def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
         assert lib.last_kernel_name() == "unpack_" + want_kernel, (u.label(), lib.last_kernel_name())
 
 
+@pytest.mark.parametrize("tf,s2,s3,flags", [
+    (uk.PACK_TYPE_BF16BF16, 16, 2, 0), (uk.PACK_TYPE_F32F32, 4, 16, 0x100), (uk.PACK_TYPE_I8I8, 8, 16, 0x300)])
+def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3, flags):
+    """Rows up to 64 bytes (32 where they are not whole words) once the blocks of 32
+    rows are more than 1024, more than 512 for rows under 16 bytes: the
+    transposing kernel's blocks are 512 bytes wide."""
+    lib, torch = gpu
+    es = uk.PACK_TYPE_BYTES[tf]
+    t0, t1 = (s3, s2) if flags & 0x100 else (s2, s3)
+    rng = np.random.default_rng(s2)
+    for rows in (100, 32 * 512, 32 * 512 + 1, 32 * 1024, 32 * 1024 + 1):
+        for cols in (15 // es, 16 // es, 32 // es, 32 // es + 1, 64 // es, 64 // es + 4):
+            row_bytes = cols * es
+            words = row_bytes % 4 == 0
+            few = rows <= (32 * 512 if row_bytes < 16 else 32 * 1024)
+            transposing = few or row_bytes > (64 if words else 32)
+            o0, o1 = -(-rows // t0), -(-cols // t1)
+            so0, so1 = (o1, o0) if flags & 0x200 else (o0, o1)
+            c = T.PackCase(tf | flags, rows, cols, so0, so1, s2, s3, cols, 1, so1 * s2 * s3, 0, 0, 0x0102030405060708)
+            inp, out0 = T.make_pack_buffers(c, rng)
+            want = out0.copy()
+            G.run_pack_case(oracle, c, inp, want)
+            got = T.gpu_pack(lib, torch, c, inp, out0)
+            assert np.array_equal(got, want), c.label()
+            assert lib.last_kernel_name().startswith("pack_transposing") == transposing, (
+                c.label(), lib.last_kernel_name())
+
+
 SINGLE_LINE_TILES = [
     (uk.PACK_TYPE_F32F32, 16, 1), (uk.PACK_TYPE_F32F32, 1, 16), (uk.PACK_TYPE_I32I32, 8, 1),
     (uk.PACK_TYPE_F16F16, 1, 16), (uk.PACK_TYPE_BF16BF16, 16, 1), (uk.PACK_TYPE_I8I8, 1, 16),
