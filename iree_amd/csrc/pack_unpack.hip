@@ -1284,6 +1284,19 @@ bool launch_pack_direct(const iree_uk_pack_params_t* p, const TiledView& v, int 
   // 22.6); below, one pass of latency is what counts (s8 2048 x 8192 in 16x32
   // tiles, 16.8 MB: 8.4 -> 5.7 us).
   if (rows >= (1ll << 31) || padded >= (1ll << 31) || rows * padded > (24ll << 20) || v.tile0 >= (1 << 20)) return false;
+  const int64_t col_groups = uk::ceil_div(padded, 64 * PB);
+  const int64_t grid = uk::ceil_div(rows, 16) * col_groups;
+  if (grid >= (1ll << 31)) return false;
+  // Narrow matrices: with up to three pieces to a row most lanes have none, and
+  // from some 4000 workgroups on that is what the launch takes (bf16 635273 x 9
+  // into 16x16: 55 us here, 26 on the tiled kernel; s8 78306 x 17 into 16x32 10.1
+  // and 6.1; f32 67637 x 7 into 1x16, 4228 workgroups, 5.4 and 5.3). Under
+  // TRANSPOSE_OUTER, where the tiled kernel's stores are short too, only rows of
+  // whole 8-byte pieces gain there (f32 437187 x 2 into 16x2: 19 and 12), not
+  // longer pieces or rows of less than one (f32 634628 x 5 into 8x4: 39 and 53,
+  // bf16 408183 x 4 into 16x16: 20 and 34).
+  const bool to = p->flags & IREE_UK_FLAG_PACK_TRANSPOSE_OUTER;
+  if (grid > 4096 && padded <= 3 * PB && (!to || (PB == 8 && row_bytes >= 8))) return false;
   DirectArgs a;
   a.src = src; a.dst = dst;
   a.src_pitch = pitch;
@@ -1293,11 +1306,9 @@ bool launch_pack_direct(const iree_uk_pack_params_t* p, const TiledView& v, int 
   a.tile_row_bytes = (uint32_t)trb;
   a.log2_tile_row_bytes = 0;
   while ((1u << a.log2_tile_row_bytes) < a.tile_row_bytes) ++a.log2_tile_row_bytes;
-  a.col_groups = (uint32_t)uk::ceil_div(padded, 64 * PB);
+  a.col_groups = (uint32_t)col_groups;
   a.pad32 = replicate_pad(p->padding_value, es);
   a.div_tile_rows = FastDiv((uint32_t)v.tile0);
-  const int64_t grid = uk::ceil_div(rows, 16) * a.col_groups;
-  if (grid >= (1ll << 31)) return false;
   uk::launch(0, PB == 16 ? pack_direct_kernel<16> : pack_direct_kernel<8>, dim3((uint32_t)grid), dim3(kThreads), 0,
              stream, a);
   return true;

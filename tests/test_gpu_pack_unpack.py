@@ -432,6 +432,29 @@ def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3
                 c.label(), lib.last_kernel_name())
 
 
+@pytest.mark.parametrize("tf,t0,t1,flags,cols,narrow", [
+    (uk.PACK_TYPE_BF16BF16, 16, 16, 0, 9, True), (uk.PACK_TYPE_F32F32, 16, 4, 0, 12, True),
+    (uk.PACK_TYPE_F32F32, 16, 4, 0, 13, False), (uk.PACK_TYPE_I8I8, 16, 16, 0, 3, True),
+    (uk.PACK_TYPE_F32F32, 16, 2, 0x200, 2, True), (uk.PACK_TYPE_F32F32, 16, 2, 0x200, 1, False),
+    (uk.PACK_TYPE_BF16BF16, 16, 16, 0x200, 4, False), (uk.PACK_TYPE_F32F32, 8, 4, 0x200, 5, False)])
+def test_narrow_matrices_leave_the_direct_kernel(gpu, oracle, tf, t0, t1, flags, cols, narrow):
+    """Up to three pieces of 8 or 16 bytes to a row, beyond 4096 workgroups of 16
+    rows; under TRANSPOSE_OUTER rows of whole 8-byte pieces only."""
+    lib, torch = gpu
+    for rows in (300, 16 * 4096, 16 * 4096 + 1):
+        o0, o1 = -(-rows // t0), -(-cols // t1)
+        so0, so1 = (o1, o0) if flags & 0x200 else (o0, o1)
+        c = T.PackCase(tf | flags, rows, cols, so0, so1, t0, t1, cols, 1, so1 * t0 * t1, 0, 0, 0x0102030405060708)
+        inp, out0 = T.make_pack_buffers(c, np.random.default_rng(cols))
+        want = out0.copy()
+        G.run_pack_case(oracle, c, inp, want)
+        got = T.gpu_pack(lib, torch, c, inp, out0)
+        assert np.array_equal(got, want), c.label()
+        assert (lib.last_kernel_name() == "pack_tiled") == (narrow and rows > 16 * 4096), (
+            c.label(), lib.last_kernel_name())
+        assert lib.last_kernel_name() in ("pack_direct", "pack_tiled")
+
+
 SINGLE_LINE_TILES = [
     (uk.PACK_TYPE_F32F32, 16, 1), (uk.PACK_TYPE_F32F32, 1, 16), (uk.PACK_TYPE_I32I32, 8, 1),
     (uk.PACK_TYPE_F16F16, 1, 16), (uk.PACK_TYPE_BF16BF16, 16, 1), (uk.PACK_TYPE_I8I8, 1, 16),
