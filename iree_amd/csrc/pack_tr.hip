@@ -35,7 +35,7 @@
 
 namespace {
 
-// A block is 32 rows x 512 bytes of the matrix: 16 KB, 256 threads, four
+// A block is 32 rows x 512 bytes of the matrix: 16 KB, 256 threads, two or four
 // workgroups per CU. Measured on operands of 128 to 600 MB that no earlier
 // launch had left in the memory-side cache: 64 x 256 is 3 to 8 % slower
 // (row segments of 256 bytes), 64 x 512 with 512 threads in between, 64 x 1024
@@ -439,9 +439,14 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
   // Rows that are whole words, which the tiled kernel loads as such, are better off
   // there up to 64 bytes, others up to 32: f32 90303 x 8 into 16x4 7.7 and 9.9; s8
   // 111358 x 18 into 8x8 transposed 9.9 and 14.9, but 114248 x 49 into 16x1 22 and 14.
+  // Not so under TRANSPOSE_OUTER in tiles that take 32 bytes and more of such a row, of
+  // which the tiled kernel then writes one at a time: bf16 150976 x 8 into 16x32 20.6
+  // there and 16.0 here, f32 899711 x 3 into 8x8 101 and 87; tiles of 16 bytes, f32
+  // 587196 x 2 into 8x4, 37 and 48.
   const int64_t row_bytes = p->in_size1 * es;
   const bool whole_words = (((uintptr_t)src | (uint64_t)pitch) & 3) == 0;
-  if (nblk0 * nblk1 > (row_bytes < 16 ? 512 : 1024) && row_bytes <= (whole_words ? 64 : 32)) return nullptr;
+  const bool wide_tiles = to && whole_words && t1 * eb >= 32;
+  if (!wide_tiles && nblk0 * nblk1 > (row_bytes < 16 ? 512 : 1024) && row_bytes <= (whole_words ? 64 : 32)) return nullptr;
 
   // Rows that are not whole words apart, or that end inside a tile row.
   const bool ragged = (((uintptr_t)src | (uint64_t)pitch) & 3) || (!ti && p->in_size1 % p->out_size3 != 0);
@@ -476,8 +481,11 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
   const size_t lds = 2 * (size_t)a.lds_buf_bytes;
   // Two workgroups per compute unit, four where that leaves them two blocks or
   // less each (f16 4096 x 4096: 13.7 against 14.2 us, f32 4096 x 4096 24.5
-  // against 23.6, s8 9000 x 9000 27.4 against 27.1).
-  const uint32_t grid = std::min<uint32_t>(nblocks, nblocks <= 2048 ? 1024 : 512);
+  // against 23.6, s8 9000 x 9000 27.4 against 27.1) and where rows are at most half a
+  // block, so that all blocks are edge blocks (s8 459581 x 48 into 16x8 transposed
+  // 28 against 38, f32 722497 x 23 into 8x8 57 against 77; s8 82466 x 318 into 8x4
+  // 18.6 against 16.0).
+  const uint32_t grid = std::min<uint32_t>(nblocks, nblocks <= 2048 || row_bytes <= kBlockRowBytes / 2 ? 1024 : 512);
   // Non-temporal stores from 72 MB of tiles on. They make the pack itself the
   // faster one from some 10 MB on (f16 4096 x 4096: 13.3 against 14.2 us), but
   // what they write has to come from HBM again, and up to that size the next

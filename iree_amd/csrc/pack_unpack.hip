@@ -939,7 +939,12 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // 427710 x 21 into 24x4: 40 against 39), under TRANSPOSE_OUTER beyond 128 (pack
   // f32 2103812 x 5 into 16x32, 128 bytes: 245 against 652).
   const int64_t padded_row_bytes = v.outer1 * v.tile1 * es;
-  const bool narrow = to ? padded_row_bytes <= 128 : padded_row_bytes < 96;
+  // Rows of single bytes that are not whole words go over only below that, where
+  // the streaming kernels have 8- or 16-byte vectors for them (s8 421410 x 70 into
+  // 1x16, 80 bytes: 51 against 30; 2264133 x 34 into 16x16, 48 bytes: 160 against
+  // 189; 283972 x 47 into 24x4 under TRANSPOSE_OUTER, 48 bytes: 49 against 23).
+  const bool byte_rows = es == 1 && (((uintptr_t)mat_ptr | (uint64_t)mat_stride0) & 3) && padded_row_bytes % 8 == 0;
+  const bool narrow = padded_row_bytes <= (byte_rows ? (to ? 47 : 48) : to ? 128 : 95);
   const bool big = allow_big && !narrow && VEC == 16 && (big_transposing || big_rows);
   const int64_t kMinSpan = big ? 512 : 256;                      // bytes, both sides
   const int64_t kTarget = big ? kStreamBigBlockBytes : kStreamBlockBytes;  // bytes per block, about
@@ -1049,9 +1054,9 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   a.lds_buf_bytes = (uint32_t)((lds_bytes + 255) / 256 * 256);
   // Streaming kernels: 32-bit offsets inside one block on both sides, granules
   // of at least 4 bytes, at most 4 granules per vector, block within budget.
-  // (and non-negative strides: the 32-bit offsets are unsigned; rows of at least
-  // 16 bytes, which pack's loads need and below which unpack is level)
-  plan.stream = block_row_bytes % 4 == 0 && mat_size0 > 0 && mat_size1 * es >= 16 && G >= 4 && VEC / G <= 4 && mat_stride0 >= 0 && v.sl0 >= 0 &&
+  // (and non-negative strides: the 32-bit offsets are unsigned; pack's loads need
+  // rows of at least 16 bytes)
+  plan.stream = block_row_bytes % 4 == 0 && mat_size0 > 0 && (mat_is_dest || mat_size1 * es >= 16) && G >= 4 && VEC / G <= 4 && mat_stride0 >= 0 && v.sl0 >= 0 &&
                 v.sl1 >= 0 &&
                 block_rows * block_row_bytes <= stream_block &&
                 lds_bytes <= (big ? 80 * 1024 : 2 * stream_block) &&
@@ -1079,10 +1084,11 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // size the plain stores are as fast or faster.
   a.streaming_stores = total_bytes >= (192ll << 20) && uk::pow2_divisor(mat_stride0 * es, 16) >= 16;
   // (The tiled kernels too move such vectors where rows are not whole words
-  // apart, for an element at a time is what they would be left with: s8 31405 x
-  // 85, 12x12 under TRANSPOSE_OUTER, 12.1 -> 8.4 us. With whole words their own choice
-  // is level or ahead.)
-  if (plan.stream && !(narrow && mat_vec >= 4)) {
+  // apart, for an element at a time is what they would be left with: s8 1303882 x
+  // 27, 12x12 under TRANSPOSE_OUTER, 153 -> 100 us, bf16 2264133 x 17 unpacked from
+  // 16x16 127 -> 76. Not 16-byte ones under TRANSPOSE_OUTER, bf16 615217 x 11 into
+  // 16x8 42 -> 65, and with whole words their own choice is level or ahead.)
+  if (plan.stream && !(narrow && (mat_vec >= 4 || (to && plan.MV == 16)))) {
     a.mat_vec = (uint32_t)plan.MV;
     a.div_row_vecs = FastDiv((uint32_t)(block_row_bytes / plan.MV));
     a.mat_stride0_bytes32 = (uint32_t)(mat_stride0 * es);
@@ -1107,6 +1113,17 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // scatter short runs over both sides (TRANSPOSE_OUTER: 127 / 124 us; f16 9000
   // x 9000 pack 75 -> 67, its unpack 56 -> 65).
   plan.max_workgroups = to && total_bytes >= ((mat_is_dest ? 192ll : 128ll) << 20) ? 256 : 512;
+  // Four where one round of them is all there is to an unpack into long rows (f16
+  // 256 x 20480 from 1x16, 640 blocks: 7.0 us against 8.9 with two of which one in
+  // four takes a second block; f32 9728 x 320 from 16x4, short rows: 11.1 and
+  // 10.4), and where blocks span whole rows under TRANSPOSE_OUTER, all of them edge
+  // blocks, and granules are 16 bytes (f32 513513 x 32 into 12x12: 97 and 123; f32
+  // 228560 x 75 from 12x12: 48 and 59; but f16 197299 x 240 from 16x2, 4-byte ones, 49
+  // and 44).
+  if ((mat_is_dest && padded_row_bytes >= 16384 && nblk0 * nblk1 <= 1024) ||
+      (to && G == 16 && padded_row_bytes < 640)) {
+    plan.max_workgroups = 1024;
+  }
   plan.G = G;
   plan.VEC = VEC;
   plan.grid = (uint32_t)(nblk0 * nblk1);
@@ -1291,12 +1308,17 @@ bool launch_pack_direct(const iree_uk_pack_params_t* p, const TiledView& v, int 
   // from some 4000 workgroups on that is what the launch takes (bf16 635273 x 9
   // into 16x16: 55 us here, 26 on the tiled kernel; s8 78306 x 17 into 16x32 10.1
   // and 6.1; f32 67637 x 7 into 1x16, 4228 workgroups, 5.4 and 5.3). Under
-  // TRANSPOSE_OUTER, where the tiled kernel's stores are short too, only rows of
-  // whole 8-byte pieces gain there (f32 437187 x 2 into 16x2: 19 and 12), not
-  // longer pieces or rows of less than one (f32 634628 x 5 into 8x4: 39 and 53,
-  // bf16 408183 x 4 into 16x16: 20 and 34).
+  // TRANSPOSE_OUTER, where the tiled kernel's stores are short too, only 8-byte
+  // pieces gain there (f32 437187 x 2 into 16x2: 19 and 12, bf16 1492886 x 3 into
+  // 8x4 54 and 46) and rows of two longer ones that are not whole words (bf16
+  // 615217 x 11 into 16x8: 55 and 42; 404813 x 21, three, 39 and 44), but f32 634628 x 5 into 8x4: 39 and 53, bf16 408183 x
+  // 4 into 16x16, less than a piece: 20 and 34.
   const bool to = p->flags & IREE_UK_FLAG_PACK_TRANSPOSE_OUTER;
-  if (grid > 4096 && padded <= 3 * PB && (!to || (PB == 8 && row_bytes >= 8))) return false;
+  const bool whole_words = (((uintptr_t)src | (uint64_t)pitch) & 3) == 0;
+  if (grid > 4096 && padded <= 3 * PB &&
+      (!to || PB == 8 || (row_bytes >= PB && padded <= 2 * PB && !whole_words))) {
+    return false;
+  }
   DirectArgs a;
   a.src = src; a.dst = dst;
   a.src_pitch = pitch;

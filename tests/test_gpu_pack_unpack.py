@@ -369,8 +369,9 @@ def test_pack_and_unpack_of_rows_in_gigabytes_of_padding(gpu, n1, kernel):
     (uk.PACK_TYPE_BF16BF16, 12, 12, 0), (uk.PACK_TYPE_BF16BF16, 16, 8, 0x200), (uk.PACK_TYPE_I8I8, 12, 12, 0x200),
     (uk.PACK_TYPE_I8I8, 16, 16, 0)])
 def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
-    """Rows whose tiles end below 96 bytes (128 under TRANSPOSE_OUTER), and the
-    first ones beyond, from all row alignments: which kernel, and its bytes."""
+    """Rows whose tiles end below 96 bytes (up to 128 under TRANSPOSE_OUTER, up to 48
+    where they are single bytes and not whole words), and the first ones beyond:
+    which kernel, and its bytes."""
     lib, torch = gpu
     es = uk.PACK_TYPE_BYTES[tf]
     rng = np.random.default_rng(t0 * 100 + t1)
@@ -379,37 +380,42 @@ def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
                                       (b // es, b // es + 1)})):
         rows = int(rng.integers(100, 300))
         padded = -(-cols // t1) * tile_row
-        narrow = padded <= 128 if flags & 0x200 else padded < 96
+        pitch = cols + ci % 2
+        byte_rows = es == 1 and pitch % 4 != 0 and padded % 8 == 0
+        narrow = padded <= ((47 if flags & 0x200 else 48) if byte_rows else 128 if flags & 0x200 else 95)
         o0, o1 = -(-rows // t0), -(-cols // t1)
         so0, so1 = (o1, o0) if flags & 0x200 else (o0, o1)
         s2, s3 = (t1, t0) if flags & 0x100 else (t0, t1)
-        want_kernel = "tiled" if narrow or cols * es < 16 else "stream"
-        c = T.PackCase(tf | flags, rows, cols, so0, so1, s2, s3, cols + ci % 2, 1, so1 * s2 * s3, 0, 0, 0x0102030405060708)
+        c = T.PackCase(tf | flags, rows, cols, so0, so1, s2, s3, pitch, 1, so1 * s2 * s3, 0, 0, 0x0102030405060708)
         inp, out0 = T.make_pack_buffers(c, rng)
         want = out0.copy()
         G.run_pack_case(oracle, c, inp, want)
         lib.set_kernel_mode(uk.KERNEL_MODE_MFMA_VARIANT + 1)   # past the direct and the transposing kernel
         got = T.gpu_pack(lib, torch, c, inp, out0)
         assert np.array_equal(got, want), c.label()
-        assert lib.last_kernel_name() == "pack_" + want_kernel, (c.label(), lib.last_kernel_name())
+        want_kernel = "pack_tiled" if narrow or cols * es < 16 else "pack_stream"
+        assert lib.last_kernel_name() == want_kernel, (c.label(), lib.last_kernel_name())
         lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
         if es == 1:
             continue
-        u = T.UnpackCase(tf | flags, so0, so1, s2, s3, rows, cols, so1 * s2 * s3, cols + ci % 2, 1, 0, 0)
+        u = T.UnpackCase(tf | flags, so0, so1, s2, s3, rows, cols, so1 * s2 * s3, pitch, 1, 0, 0)
         inp, out0 = T.make_unpack_buffers(u, rng)
         want = out0.copy()
         G.run_unpack_case(oracle, u, inp, want)
         got = T.gpu_unpack(lib, torch, u, inp, out0)
         assert np.array_equal(got, want), u.label()
-        assert lib.last_kernel_name() == "unpack_" + want_kernel, (u.label(), lib.last_kernel_name())
+        want_kernel = "unpack_tiled" if narrow else "unpack_stream"
+        assert lib.last_kernel_name() == want_kernel, (u.label(), lib.last_kernel_name())
 
 
 @pytest.mark.parametrize("tf,s2,s3,flags", [
-    (uk.PACK_TYPE_BF16BF16, 16, 2, 0), (uk.PACK_TYPE_F32F32, 4, 16, 0x100), (uk.PACK_TYPE_I8I8, 8, 16, 0x300)])
+    (uk.PACK_TYPE_BF16BF16, 16, 2, 0), (uk.PACK_TYPE_F32F32, 4, 16, 0x100), (uk.PACK_TYPE_I8I8, 8, 16, 0x300),
+    (uk.PACK_TYPE_BF16BF16, 16, 16, 0x300)])
 def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3, flags):
     """Rows up to 64 bytes (32 where they are not whole words) once the blocks of 32
     rows are more than 1024, more than 512 for rows under 16 bytes: the
-    transposing kernel's blocks are 512 bytes wide."""
+    transposing kernel's blocks are 512 bytes wide. Not tiles of 32 bytes along
+    rows of whole words under TRANSPOSE_OUTER."""
     lib, torch = gpu
     es = uk.PACK_TYPE_BYTES[tf]
     t0, t1 = (s3, s2) if flags & 0x100 else (s2, s3)
@@ -419,7 +425,8 @@ def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3
             row_bytes = cols * es
             words = row_bytes % 4 == 0
             few = rows <= (32 * 512 if row_bytes < 16 else 32 * 1024)
-            transposing = few or row_bytes > (64 if words else 32)
+            wide_tiles = flags & 0x200 and words and t1 * es >= 32
+            transposing = few or wide_tiles or row_bytes > (64 if words else 32)
             o0, o1 = -(-rows // t0), -(-cols // t1)
             so0, so1 = (o1, o0) if flags & 0x200 else (o0, o1)
             c = T.PackCase(tf | flags, rows, cols, so0, so1, s2, s3, cols, 1, so1 * s2 * s3, 0, 0, 0x0102030405060708)
@@ -435,11 +442,13 @@ def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3
 @pytest.mark.parametrize("tf,t0,t1,flags,cols,narrow", [
     (uk.PACK_TYPE_BF16BF16, 16, 16, 0, 9, True), (uk.PACK_TYPE_F32F32, 16, 4, 0, 12, True),
     (uk.PACK_TYPE_F32F32, 16, 4, 0, 13, False), (uk.PACK_TYPE_I8I8, 16, 16, 0, 3, True),
-    (uk.PACK_TYPE_F32F32, 16, 2, 0x200, 2, True), (uk.PACK_TYPE_F32F32, 16, 2, 0x200, 1, False),
-    (uk.PACK_TYPE_BF16BF16, 16, 16, 0x200, 4, False), (uk.PACK_TYPE_F32F32, 8, 4, 0x200, 5, False)])
+    (uk.PACK_TYPE_F32F32, 16, 2, 0x200, 2, True), (uk.PACK_TYPE_BF16BF16, 16, 8, 0x200, 11, True),
+    (uk.PACK_TYPE_BF16BF16, 16, 8, 0x200, 17, False), (uk.PACK_TYPE_BF16BF16, 16, 16, 0x200, 4, False),
+    (uk.PACK_TYPE_F32F32, 8, 4, 0x200, 5, False)])
 def test_narrow_matrices_leave_the_direct_kernel(gpu, oracle, tf, t0, t1, flags, cols, narrow):
     """Up to three pieces of 8 or 16 bytes to a row, beyond 4096 workgroups of 16
-    rows; under TRANSPOSE_OUTER rows of whole 8-byte pieces only."""
+    rows; under TRANSPOSE_OUTER pieces of 8 bytes, and up to two longer ones of
+    rows that are not whole words."""
     lib, torch = gpu
     for rows in (300, 16 * 4096, 16 * 4096 + 1):
         o0, o1 = -(-rows // t0), -(-cols // t1)
