@@ -84,8 +84,8 @@ __device__ __forceinline__ v2u read_tr(uint32_t lds_addr) {
 // bytes of each of IL neighbouring rows, read as they lie and interleaved in
 // registers (v_perm_b32); neighbouring lanes take neighbouring columns, which
 // are neighbours in the tile.
-// NTS: the stores are non-temporal.
-template <int EB, int V, int IL, bool NTS>
+// S: how the tiles are stored.
+template <int EB, int V, int IL, uk::Store S>
 __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kernel(TrArgs a) {
   static_assert(IL == 0 || (V == 16 && (IL * EB == 2 || IL * EB == 4)), "interleaved rows of 2 or 4 bytes");
   static_assert(EB != 4 || (V == 16 && IL == 0), "4-byte elements: four rows per 16-byte vector");
@@ -208,10 +208,6 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
 #pragma unroll
     for (int i = 0; i < N1; ++i) pre[i] = *reinterpret_cast<const v4u_a1*>(base + off[i]);
   };
-  auto store = [&](char* p, auto v) __attribute__((always_inline)) {
-    if constexpr (NTS) __builtin_nontemporal_store(v, reinterpret_cast<decltype(v)*>(p));
-    else *reinterpret_cast<decltype(v)*>(p) = v;
-  };
   // ---- matrix rows -> LDS ----
   auto phase1_inside = [&](char* lbuf) __attribute__((always_inline)) {
 #pragma unroll
@@ -262,7 +258,7 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
 #pragma unroll
       for (int i = 0; i < N2; ++i) {
         if (!kInside && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
-        store(b.dst + g2off[i], out[i]);
+        uk::store_as<S>(b.dst, g2off[i], out[i]);
       }
       return;
     }
@@ -278,7 +274,7 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
 #pragma unroll
       for (int i = 0; i < N2; ++i) {
         if (!kInside && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
-        store(b.dst + g2off[i], out[i]);
+        uk::store_as<S>(b.dst, g2off[i], out[i]);
       }
       return;
     }
@@ -301,12 +297,11 @@ __global__ __launch_bounds__(kBlockRows * kBlockRowBytes / 64) void pack_tr_kern
 #pragma unroll
     for (int i = 0; i < N2; ++i) {
       if (!kInside && !(b.blk0 * tiles0 + tl0[i] < a.outer0 && b.blk1 * tiles1 + tl1[i] < a.outer1)) continue;
-      char* gp = b.dst + g2off[i];
       if constexpr (V == 16) {
         const v4u val = v4u{got[i][0][0], got[i][0][1], got[i][1][0], got[i][1][1]};
-        store(gp, val);
+        uk::store_as<S>(b.dst, g2off[i], val);
       } else {
-        store(gp, got[i][0]);
+        uk::store_as<S>(b.dst, g2off[i], got[i][0]);
       }
     }
   };
@@ -486,18 +481,29 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
   // 28 against 38, f32 722497 x 23 into 8x8 57 against 77; s8 82466 x 318 into 8x4
   // 18.6 against 16.0).
   const uint32_t grid = std::min<uint32_t>(nblocks, nblocks <= 2048 || row_bytes <= kBlockRowBytes / 2 ? 1024 : 512);
-  // Non-temporal stores from 72 MB of tiles on. They make the pack itself the
-  // faster one from some 10 MB on (f16 4096 x 4096: 13.3 against 14.2 us), but
-  // what they write has to come from HBM again, and up to that size the next
-  // kernel finds it in the memory-side cache otherwise (the unpack that follows:
-  // 21.3 against 16.4 us; f32 4096 x 4096, 67 MB: 29.4 + 23.8 against 23.6 +
-  // 21.7; f16 6000 x 8192, 98 MB: 37.5 + 51.5 against 39.8 + 58).
-  const bool nts = outer0 * outer1 * tile_bytes >= (72ll << 20);
+  // Non-temporal stores from 72 MB of tiles on. Below, what they write would have to
+  // come from HBM again where the next kernel finds it in the memory-side cache
+  // otherwise (f32 4096 x 4096, 67 MB, and the unpack that follows: 29.4 + 23.8 us
+  // against 23.6 + 21.7; f16 6000 x 8192, 98 MB: 37.5 + 51.5 against 39.8 + 58).
+  // From 16 MB on the stores go through the L2s into that cache: plain ones leave
+  // the L2s full of tiles that are written back when the kernel ends (f16 320 x
+  // 33472 into 16x16, 21 MB: 13.8 us plain, 11.9 non-temporal, 12.3 through; with
+  // the mmt4d that reads the tiles, 16 to 72 MB, 0.95 of the time with
+  // non-temporal ones, plain ones 0.98). Not where TRANSPOSE_OUTER makes runs of
+  // less than 256 bytes of a block's tiles, parts of lines that the L2s had better
+  // join (s8 2857 x 8251 into 16x1: 16.7 plain, 35 non-temporal, 25.9 through).
+  const int64_t total = outer0 * outer1 * tile_bytes;
+  const bool long_runs = !to || kBlockRows * t1 * eb >= 256;
+  const uk::Store how = total >= (72ll << 20)                ? uk::Store::kNonTemporal
+                        : total >= (16ll << 20) && long_runs ? uk::Store::kThrough
+                                                             : uk::Store::kPlain;
   const dim3 block(kBlockRows * kBlockRowBytes / 64);
   auto go = [&](auto eb_c, auto v_c, auto il_c) {
     constexpr int EB = decltype(eb_c)::value, VV = decltype(v_c)::value, IL = decltype(il_c)::value;
-    if (nts) uk::launch(0, pack_tr_kernel<EB, VV, IL, true>, dim3(grid), block, lds, stream, a);
-    else uk::launch(0, pack_tr_kernel<EB, VV, IL, false>, dim3(grid), block, lds, stream, a);
+    auto kernel = how == uk::Store::kNonTemporal ? pack_tr_kernel<EB, VV, IL, uk::Store::kNonTemporal>
+                  : how == uk::Store::kThrough   ? pack_tr_kernel<EB, VV, IL, uk::Store::kThrough>
+                                                 : pack_tr_kernel<EB, VV, IL, uk::Store::kPlain>;
+    uk::launch(0, kernel, dim3(grid), block, lds, stream, a);
   };
   using std::integral_constant;
   typedef integral_constant<int, 0> I0; typedef integral_constant<int, 1> I1; typedef integral_constant<int, 2> I2;

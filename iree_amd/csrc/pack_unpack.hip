@@ -162,7 +162,6 @@ struct TiledArgs {
   uint32_t mat_stride0_bytes32;     // == mat_stride0_bytes when it fits
   uint32_t sl0_bytes32, sl1_bytes32;
   uint32_t band, grp;               // walk: bands of block rows, groups of block columns
-  uint32_t streaming_stores;        // 16 KB-block streaming kernels: non-temporal stores
 };
 
 template <int N> struct Bytes;
@@ -599,13 +598,14 @@ __device__ __forceinline__ void scatter_granules(char* lbuf, const uint32_t (&of
         __builtin_bit_cast(typename GBytes<G>::type, y);
   }
 }
-// NTL / NTS: the loads / stores are non-temporal.
-template <int G, int VEC, int MV, bool UNPACK, int BLK, int NT, bool NTL, bool NTS>
+// NTL: the loads are non-temporal. S: how the destination is stored.
+template <int G, int VEC, int MV, bool UNPACK, int BLK, int NT, bool NTL, uk::Store S>
 __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   constexpr int N1 = BLK / MV / NT;   // 2-D side items per thread
   constexpr int N2 = BLK / VEC / NT;  // tiled side items per thread
   constexpr int NG = VEC / G;                             // granules per tiled vector
+  constexpr bool NTS = S == uk::Store::kNonTemporal;
   constexpr int P = G < MV ? G : MV;                      // LDS access width on a row (rows are G-aligned)
   using MatVec = typename GBytes<MV>::type;
   using TileVec = typename GBytes<VEC>::type;
@@ -783,7 +783,10 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
       for (int i = 0; i < N2; ++i) reg[i] = gather_granules<VEC, G>(lbuf, l2off[i], rot);
 #pragma unroll
       for (int i = 0; i < N2; ++i)
-        if (kInside || tile_exists(b, i)) gstore<VEC, NTS>(base + g2off[i], reg[i]);
+        if (kInside || tile_exists(b, i)) {
+          if constexpr (S == uk::Store::kThrough) uk::store_as<S>(base, g2off[i], reg[i]);
+          else gstore<VEC, NTS>(base + g2off[i], reg[i]);
+        }
     } else {
       char* base = a.dst + (int64_t)b.row_base * a.mat_stride0_bytes + b.col_base_bytes;
       MatVec reg[N1];
@@ -881,6 +884,7 @@ struct TiledPlan {
   bool streaming_loads = false;
   uint32_t grid = 0;
   uint32_t max_workgroups = 512;
+  uk::Store store = uk::Store::kPlain;  // of the 16 KB-block streaming kernels with 16-byte vectors
   uint32_t lds_bytes = 0;
 };
 
@@ -1079,10 +1083,16 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
     plan.streaming_loads = !mat_is_dest || ((uintptr_t)tiled_ptr | run_bytes | run_pitch) % 128 == 0;
   }
   // Outputs beyond the memory-side cache are not worth allocating there: the
-  // interior blocks of the 16 KB-block kernels store them non-temporally too
+  // 16 KB-block kernels store them non-temporally too
   // (f32 8192x8192 unpack under TRANSPOSE_OUTER: 106 -> 77 us). Below that
   // size the plain stores are as fast or faster.
-  a.streaming_stores = total_bytes >= (192ll << 20) && uk::pow2_divisor(mat_stride0 * es, 16) >= 16;
+  // An untransposed pack's go through the L2s into that cache from 24 MB on:
+  // plain ones leave the L2s full of tiles that are written back when the kernel
+  // ends (25 to 72 MB of f32, bf16 and s8: 0.94 of the time with plain stores, and
+  // 0.98 with the mmt4d that reads the tiles counted in).
+  plan.store = total_bytes >= (192ll << 20) && uk::pow2_divisor(mat_stride0 * es, 16) >= 16 ? uk::Store::kNonTemporal
+               : !mat_is_dest && !to && total_bytes >= (24ll << 20)                     ? uk::Store::kThrough
+                                                                                        : uk::Store::kPlain;
   // (The tiled kernels too move such vectors where rows are not whole words
   // apart, for an element at a time is what they would be left with: s8 1303882 x
   // 27, 12x12 under TRANSPOSE_OUTER, 153 -> 100 us, bf16 2264133 x 17 unpacked from
@@ -1179,7 +1189,7 @@ bool launch_stream(const TiledPlan& plan, hipStream_t stream) {
     };
 #define UK_BIG(g, ntl)                                                                               \
   {                                                                                                       \
-    auto kernel = stream_tiled_kernel<g, 16, 16, UNPACK, kStreamBigBlockBytes, kBigThreads, ntl, true>;    \
+    auto kernel = stream_tiled_kernel<g, 16, 16, UNPACK, kStreamBigBlockBytes, kBigThreads, ntl, uk::Store::kNonTemporal>; \
     static hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),                   \
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); \
     return launch_big(kernel, attr);                                                                      \
@@ -1190,23 +1200,26 @@ bool launch_stream(const TiledPlan& plan, hipStream_t stream) {
 #undef UK_BIG
   }
   const uint32_t grid = nblocks < plan.max_workgroups ? nblocks : plan.max_workgroups;
-#define UK_CASE(g, vv, mv, nts)                                                                             \
-  if (plan.G == g && plan.VEC == vv && plan.MV == mv && (bool)plan.args.streaming_stores == nts) {          \
-    uk::launch(UNPACK ? 1 : 0, stream_tiled_kernel<g, vv, mv, UNPACK, kStreamBlockBytes, kThreads, false, nts>, \
-               dim3(grid), dim3(kThreads), lds, stream, plan.args);                                         \
-    return true;                                                                                            \
+  auto go = [&](auto kernel) {
+    uk::launch(UNPACK ? 1 : 0, kernel, dim3(grid), dim3(kThreads), lds, stream, plan.args);
+    return true;
+  };
+#define UK_KERNEL(g, vv, mv, s) stream_tiled_kernel<g, vv, mv, UNPACK, kStreamBlockBytes, kThreads, false, uk::Store::s>
+#define UK_CASE(g)                                                                                   \
+  if (plan.G == g && plan.VEC == 16 && plan.MV == 16) {                                              \
+    if (plan.store == uk::Store::kNonTemporal) return go(UK_KERNEL(g, 16, 16, kNonTemporal));        \
+    if constexpr (!UNPACK) {                                                                         \
+      if (plan.store == uk::Store::kThrough) return go(UK_KERNEL(g, 16, 16, kThrough));              \
+    }                                                                                                \
+    return go(UK_KERNEL(g, 16, 16, kPlain));                                                         \
   }
-  UK_CASE(16, 16, 16, false) UK_CASE(8, 16, 16, false) UK_CASE(4, 16, 16, false)
-  UK_CASE(16, 16, 16, true) UK_CASE(8, 16, 16, true) UK_CASE(4, 16, 16, true)
+  UK_CASE(16) UK_CASE(8) UK_CASE(4)
 #undef UK_CASE
-#define UK_CASE(g, vv, mv)                                                                                  \
-  if (plan.G == g && plan.VEC == vv && plan.MV == mv) {                                                     \
-    uk::launch(UNPACK ? 1 : 0, stream_tiled_kernel<g, vv, mv, UNPACK, kStreamBlockBytes, kThreads, false, false>, \
-               dim3(grid), dim3(kThreads), lds, stream, plan.args);                                         \
-    return true;                                                                                            \
-  }
-  UK_CASE(4, 4, 16) UK_CASE(16, 16, 4) UK_CASE(8, 16, 4) UK_CASE(4, 16, 4) UK_CASE(4, 4, 4)
+#define UK_CASE(g, vv, mv) \
+  if (plan.G == g && plan.VEC == vv && plan.MV == mv) return go(UK_KERNEL(g, vv, mv, kPlain));
+  UK_CASE(4, 4, 16) UK_CASE(8, 16, 4) UK_CASE(4, 16, 4) UK_CASE(4, 4, 4)
 #undef UK_CASE
+#undef UK_KERNEL
   return false;
 }
 

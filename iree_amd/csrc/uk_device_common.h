@@ -163,6 +163,28 @@ __device__ __forceinline__ void store_head(char* p, const uint32_t (&w)[N / 4], 
   }
 }
 
+// How a kernel stores what the next kernel reads.
+enum class Store {
+  kPlain,        // stays in the L2s, which are written back when the kernel ends
+  kThrough,      // through the L2s into the memory-side cache as it is stored
+  kNonTemporal,  // to HBM, past that cache too
+};
+// Stores `v`, 8 or 16 bytes, at `base` + `off`; `base` is the same in all lanes
+// and `off` below 2^31.
+template <Store S, typename V>
+__device__ __forceinline__ void store_as(char* base, uint32_t off, V v) {
+  if constexpr (S == Store::kThrough) {
+    // (the cache policy operand's bit 4 is SC1: device scope, written through)
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(base, 0, -1, 0x00027000);
+    if constexpr (sizeof(V) == 16) __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off, 0, 16);
+    else __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, off, 0, 16);
+  } else if constexpr (S == Store::kNonTemporal) {
+    __builtin_nontemporal_store(v, reinterpret_cast<V*>(base + off));
+  } else {
+    *reinterpret_cast<V*>(base + off) = v;
+  }
+}
+
 // Largest power of two <= cap that divides v (v == 0 counts as divisible).
 inline int64_t pow2_divisor(int64_t v, int64_t cap) {
   int64_t p = cap;

@@ -464,6 +464,31 @@ def test_narrow_matrices_leave_the_direct_kernel(gpu, oracle, tf, t0, t1, flags,
         assert lib.last_kernel_name() in ("pack_direct", "pack_tiled")
 
 
+@pytest.mark.parametrize("tf,t0,t1,flags,rows,cols", [
+    (uk.PACK_TYPE_F16F16, 16, 16, 0x300, 1031, 8261), (uk.PACK_TYPE_I8I8, 16, 8, 0x100, 2050, 8301),
+    (uk.PACK_TYPE_F32F32, 16, 4, 0x300, 2056, 2052), (uk.PACK_TYPE_I8I8, 16, 2, 0, 2050, 8302),
+    (uk.PACK_TYPE_I8I8, 16, 1, 0x200, 2050, 8302), (uk.PACK_TYPE_F32F32, 16, 4, 0, 2500, 2622),
+    (uk.PACK_TYPE_BF16BF16, 24, 4, 0, 3001, 4300), (uk.PACK_TYPE_I8I8, 16, 16, 0, 4001, 6300)])
+def test_pack_of_tiles_that_are_stored_through(gpu, tf, t0, t1, flags, rows, cols):
+    """Tiles of 16 MB and more on the transposing kernel (runs of less than 256
+    bytes under TRANSPOSE_OUTER are stored as before), of 24 MB and more on the
+    streaming one, ragged on both sides; against pad + reshape + transpose."""
+    lib, torch = gpu
+    es = uk.PACK_TYPE_BYTES[tf]
+    rng = np.random.default_rng(cols)
+    x = rng.integers(0, 1 << 8 * es, (rows, cols), dtype={1: np.uint8, 2: np.uint16, 4: np.uint32}[es])
+    ti, to = bool(flags & 0x100), bool(flags & 0x200)
+    s2, s3 = (t1, t0) if ti else (t0, t1)
+    want = T.numpy_pack(x, t0, t1, ti, to, 0x5A & 0xFF)
+    so0, so1 = want.shape[:2]
+    assert want.nbytes >= 16 << 20
+    d_in, d_out = T.DeviceBytes(torch, x), T.DeviceBytes(torch, np.zeros(want.nbytes, np.uint8))
+    lib.pack(d_in.ptr, 0, cols, 1, d_out.ptr, 0, so1 * s2 * s3, s2 * s3, rows, cols, so0, so1, s2, s3, 0x5A, tf | flags)
+    lib.synchronize()
+    assert lib.last_kernel_name().startswith(("pack_transposing", "pack_stream")), lib.last_kernel_name()
+    assert np.array_equal(d_out.numpy(), np.ascontiguousarray(want).view(np.uint8).reshape(-1))
+
+
 SINGLE_LINE_TILES = [
     (uk.PACK_TYPE_F32F32, 16, 1), (uk.PACK_TYPE_F32F32, 1, 16), (uk.PACK_TYPE_I32I32, 8, 1),
     (uk.PACK_TYPE_F16F16, 1, 16), (uk.PACK_TYPE_BF16BF16, 16, 1), (uk.PACK_TYPE_I8I8, 1, 16),
