@@ -50,8 +50,9 @@
 //      bytes >= 16, eight waves).
 // Pipelines 1 and 2 need K in whole steps; the launcher gives a K remainder to a
 // second, accumulating launch of a PIPE 0 variant. Pipelines 3 and 5 run any K
-// (TAIL): 3 adds the last, partial step when the others are done, in 5 the lanes
-// whose K-tile lies beyond K load from a piece of zeros.
+// in the shapes that have an instance for it (TAIL): 3 adds the last, partial
+// step when the others are done, in 5 the lanes whose K-tile lies beyond K load
+// from a piece of zeros.
 #ifndef IREE_UK_AMD_MMT4D_MFMA_KERNEL_H_
 #define IREE_UK_AMD_MMT4D_MFMA_KERNEL_H_
 

@@ -43,6 +43,23 @@ struct Problem {
   bool accumulate;
 };
 
+// Whether a shape has an instance for a K that ends inside a step (TAIL of the
+// kernel): those that a call can reach by its sizes. Shapes that only a forced
+// variant reaches decline such a K and leave it to the next one in line: with
+// instances of theirs the library was half as large again. The 16-bit integers
+// take K in whole steps only.
+template <Elem E, int RBC, int TM, int TN, int WGM, int WGN, int PIPE>
+constexpr bool has_tail_instance() {
+  constexpr bool k64x64 = TM * WGM == 4 && TN * WGN == 4;
+  if (E == Elem::kS16) return false;
+  if (PIPE == 3) return E == Elem::kF32 || k64x64;
+  if (PIPE == 5) {
+    if (k64x64) return RBC < 16 && ElemTraits<E>::Out::kOutBytes == 4 && E != Elem::kF32;
+    return E != Elem::kF32 && WGN != 8;  // (WGN == 8: 128x512)
+  }
+  return false;
+}
+
 // Launches one kernel variant over K-tiles [kt_begin, kt_begin + kt_count).
 // Returns a HIP status, or -1 if the variant cannot serve the shape.
 template <Elem E, int RBC, int TM, int TN, int WGM, int WGN, int NKK, int PIPE>
@@ -79,8 +96,8 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
   a.steps = (int32_t)uk::ceil_div(k_bytes, SH::KS);
   if (a.steps < 1) a.steps = 1;
   a.tail = (k_bytes % SH::KS) != 0;
-  if (PIPE != 0 && PIPE != 4 && ((a.tail && PIPE != 3 && PIPE != 5) || kt_count == 0)) return -1;
-  if (E == Elem::kS16 && a.tail) return -1;           // (K in whole steps only)
+  constexpr bool kTail = has_tail_instance<E, RBC, TM, TN, WGM, WGN, PIPE>();
+  if (PIPE != 0 && PIPE != 4 && ((a.tail && !kTail) || kt_count == 0)) return -1;
   a.accumulate = accumulate;
   // A launch that starts K reads the caller's accumulators; a later one
   // continues from what the previous launch left in the output. Only the
@@ -139,7 +156,7 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
                SH::kLdsBytes, stream, a);
     return (int)hipGetLastError();
   };
-  if constexpr (PIPE == 3 || PIPE == 5) {
+  if constexpr (kTail) {
     if (a.tail) return go(std::true_type{});
   }
   return go(std::false_type{});
@@ -436,11 +453,12 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 }
 
 // Variant choice for row-bytes class RBC:
-//   big   256x256 workgroup tile, 8 waves of 128x64, software-pipelined
-//         (register-direct RHS when RB >= 16): needs K in whole steps, the
-//         remainder of K (if any) is a second, accumulating launch;
-//   mid   128x128, 4 waves, any K;
-//   small 64x64, 4 waves, any K: for problems with too few 128x128 blocks to
+//   big   256x256 workgroup tile, 8 waves of 128x64, software-pipelined, both
+//         operands through LDS-direct loads, any K; f32: RHS straight to
+//         registers, any K, or with rows under 16 bytes both operands regrouped
+//         in registers, where a remainder of K is a second, accumulating launch;
+//   mid   128x128, 8 waves (f32 rows under 16 bytes: 4), any K;
+//   small 64x64, 4 or 8 waves, any K: for problems with too few 128x128 blocks to
 //         occupy the 256 CUs;
 // `forced` (1 big, 2 mid, 3 small, 4 thin, 5 thin on the transposed problem,
 // 6 the 64x64 K-split kernel, 7 the 256x128 shape, 8 the 128x512 shape,
@@ -595,11 +613,11 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   }
   // The pipelines that need K in whole steps get those; what is left of K (less
   // than one step) goes to the two-stage variant of the same or a smaller
-  // workgroup shape, as a second, accumulating launch. (Pipelines 3 and 5, which
-  // serve every call that no test or tuning run forces elsewhere, run any K: a
-  // second launch over less than one step cost as much as a small product, and
-  // a pass over the output: s8 300 x 500 x 400 10.6 -> 5.5 us, f16 3000 x 3000 x
-  // 333 40.1 -> 18.7, s8 4095 x 2049 x 2049 53.6 -> 31.2.)
+  // workgroup shape, as a second, accumulating launch: large f32 products in tile
+  // rows under 16 bytes, and forced variants. (All others run any K, see
+  // has_tail_instance: a second launch over less than one step cost as much as a
+  // small product, and a pass over the output: s8 300 x 500 x 400 10.6 -> 5.5 us,
+  // f16 3000 x 3000 x 333 40.1 -> 18.7, s8 4095 x 2049 x 2049 53.6 -> 31.2.)
   const int kts_per_step = BIG_KS >> p.lrb;
   // 16-bit outputs are rounded once, after all of K (the reference's
   // SKIP_INTERMEDIATE_ROUNDINGS semantics): a second launch would continue from
@@ -682,7 +700,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if (kt_main > 0) {
       int st = -1;
       bool wide = false;
-      const int kt_big = BIG_PIPE == 3 ? p.K1 : kt_main;  // pipeline 3 runs any K
+      const int kt_big = E == Elem::kF32 && BIG_PIPE == 3 ? p.K1 : kt_main;  // (runs any K)
       if constexpr (RBC >= 16 && H == 1 && ElemTraits<E>::Out::kOutBytes == 4) {
         // One persistent workgroup per CU whose pipeline runs across block
         // boundaries. Measured equal to the one-block-per-workgroup launches
@@ -808,15 +826,13 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     choice = 3;
   }
   if (choice == 2) {
-    {
-      // The LDS-direct ping-pong pipeline with 8 waves of 64x32 (measured against
-      // the kernels below: s8 2048^3 16x16x2 20.6 -> 14.7 us, 16x16x16 14.8 ->
-      // 14.5 us; 3072^3 40.5 -> 36.3 us; bf16 2048^3 23.4 -> 22.6 us).
-      if (forced == 18 || (forced == 0 && E != Elem::kF32)) {
-        int st = launch_variant<E, RBC, 4, 2, 2, 4, 1, 5>(p, 0, p.K1, p.accumulate, stream);
-        if (st == 0) *name = "mmt4d_mfma_128x128_lds_direct";
-        if (st >= 0) return st;
-      }
+    // The LDS-direct ping-pong pipeline with 8 waves of 64x32 (measured against
+    // the kernels below: s8 2048^3 16x16x2 20.6 -> 14.7 us, 16x16x16 14.8 ->
+    // 14.5 us; 3072^3 40.5 -> 36.3 us; bf16 2048^3 23.4 -> 22.6 us).
+    if (forced == 18 || (forced == 0 && E != Elem::kF32)) {
+      int st = launch_variant<E, RBC, 4, 2, 2, 4, 1, 5>(p, 0, p.K1, p.accumulate, stream);
+      if (st == 0) *name = "mmt4d_mfma_128x128_lds_direct";
+      if (st >= 0) return st;
     }
     if constexpr (NARROW) {
       // (Not chosen by size: measured level with or behind the 128x128 kernel

@@ -105,16 +105,16 @@ def _variant_applies(n, variant):
     """Forced shapes that a tile cannot take hand the call on to the choice by
     size, i.e. repeat variant 0: the deep 64x64 pipeline (11) exists for tile
     rows under 16 bytes, the narrow-row kernels (12 .. 15) for rows of 2 or 4
-    bytes with N0 = 16, the LDS-direct pipeline (16 .. 20): its small shapes (18,
-    19) not for the 8-bit floats, its 256x128 shape (20) for rows of 16 bytes and more."""
+    bytes with N0 = 16, the LDS-direct pipeline (16 .. 20) for all but: its 64x64
+    shape (19) not for the 8-bit floats, its 256x128 shape (20) for rows of 16 bytes and more."""
     tf, M0, N0, K0 = MFMA_TILES[n]
     row_bytes = K0 * uk.MMT4D_TYPE_BITS[tf][0] // 8
     if variant == 11:
         return row_bytes < 16
     if variant in (12, 13, 14, 15):
         return row_bytes in (2, 4) and N0 == 16
-    if variant in (18, 19):
-        # the LDS-direct pipeline in its small shapes: one 16-byte piece per lane operand (not the 8-bit floats)
+    if variant == 19:
+        # one 16-byte piece per lane operand (not the 8-bit floats)
         return tf != uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32
     if variant == 20:
         return row_bytes >= 16
@@ -228,9 +228,36 @@ def test_mmt4d_16bit_outputs_round_once_when_k_has_a_remainder(gpu, oracle, tf, 
     lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
 
 
-@pytest.mark.parametrize("variant", [0, 2, 3, 7, 16, 18, 19, 20])
-@pytest.mark.parametrize("tf,K0", [(uk.MMT4D_TYPE_F16F16F32, 8), (uk.MMT4D_TYPE_BF16BF16F32, 2),
-                                   (uk.MMT4D_TYPE_F32F32F32, 4), (uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32, 32)])
+def _kernel_of_forced_variant(tf, K0, K, variant):
+    """The kernel that a forced variant comes to in 16 x 16 x K0 tiles: pipelines
+    that run any K, and those that leave a K that ends inside a step (64 bytes, 128
+    for the 8-bit floats) to the next shape in line or, from one whole step on, its
+    remainder to a second launch. (The 8-bit floats have no 128x512 LDS-direct
+    shape, whose stages would be more than a unit's LDS, and no 64x64 one.)"""
+    row_bytes = K0 * uk.MMT4D_TYPE_BITS[tf][0] // 8
+    f32, f8 = tf == uk.MMT4D_TYPE_F32F32F32, tf == uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32
+    step = 128 if f8 else 64
+    k_bytes = K * row_bytes
+    tail, wide = k_bytes % step != 0, row_bytes >= 16
+    mid = "128x128_rhs_direct" if wide and (f32 or not tail) else "128x128"
+    big = ("256x256_rhs_direct" if wide else "256x256_regroup") if k_bytes >= step else mid
+    if variant in (1, 8) or (variant in (16, 17) and f32 and tail):
+        return big.replace("256x256_rhs", "128x512_rhs") if variant == 8 else big
+    if variant == 2 or (variant == 18 and f32 and tail):
+        return mid
+    if variant == 3 or (variant == 19 and (f8 or (wide or f32) and k_bytes % 256 != 0)):
+        return "64x64_rhs_direct" if wide else "64x64"
+    if variant == 7 or (variant == 20 and (not wide or f32 and tail)):
+        return "256x128_rhs_direct" if wide and (f32 or not tail) else mid
+    shape = {16: "256x256", 17: "256x256" if tail or f8 else "128x512", 18: "128x128", 19: "64x64", 20: "256x128"}[variant]
+    return shape + "_lds_direct"
+
+
+@pytest.mark.parametrize("variant", [0, 1, 2, 3, 7, 8, 16, 17, 18, 19, 20])
+@pytest.mark.parametrize("tf,K0", [(uk.MMT4D_TYPE_F16F16F32, 8), (uk.MMT4D_TYPE_F16F16F32, 1),
+                                   (uk.MMT4D_TYPE_BF16BF16F32, 2), (uk.MMT4D_TYPE_BF16BF16F32, 4),
+                                   (uk.MMT4D_TYPE_F32F32F32, 4), (uk.MMT4D_TYPE_F32F32F32, 1),
+                                   (uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32, 32)])
 def test_mmt4d_k_that_ends_inside_a_step_reads_nothing_beyond_it(gpu, oracle, tf, K0, variant):
     """K a few tiles short of, at and past whole pipeline steps, and NaN in all
     bytes behind the K-tiles of every panel: a kernel that multiplied them, even
@@ -251,6 +278,8 @@ def test_mmt4d_k_that_ends_inside_a_step_reads_nothing_beyond_it(gpu, oracle, tf
         got = T.gpu_mmt4d(lib, torch, c, lhs, rhs, out0, allow_generic=False)
         assert np.array_equal(got, want), (c.label(), lib.last_kernel_name())
         assert lib.last_kernel_name().startswith("mmt4d_mfma"), lib.last_kernel_name()
+        if variant:
+            assert lib.last_kernel_name() == "mmt4d_mfma_" + _kernel_of_forced_variant(tf, K0, K, variant), c.label()
     lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
 
 
