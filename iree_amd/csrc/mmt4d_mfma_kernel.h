@@ -88,6 +88,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 enum class Elem { kS8, kF16, kBF16, kF8, kF32, kF16F16, kBF16BF16, kS8S4, kS16 };
 
 typedef uint16_t v4u16 __attribute__((ext_vector_type(4)));
+typedef uint32_t v2u32 __attribute__((ext_vector_type(2)));
 
 // Output access for 4-byte outputs: the accumulator quad as it is.
 template <typename Acc, typename T>
@@ -120,17 +121,20 @@ struct Out16 {
     *reinterpret_cast<v4u16*>(p) = v4u16{uk::f32_to_small16<EB>(v[0]), uk::f32_to_small16<EB>(v[1]),
                                          uk::f32_to_small16<EB>(v[2]), uk::f32_to_small16<EB>(v[3])};
   }
-  static __device__ __forceinline__ void store4_nt(char* p, v4f v) {
-    const v4u16 h = v4u16{uk::f32_to_small16<EB>(v[0]), uk::f32_to_small16<EB>(v[1]),
-                          uk::f32_to_small16<EB>(v[2]), uk::f32_to_small16<EB>(v[3])};
-    typedef uint32_t v2u32 __attribute__((ext_vector_type(2)));
-    asm volatile("global_store_dwordx2 %0, %1, off nt" : : "v"(p), "v"(__builtin_bit_cast(v2u32, h)) : "memory");
-  }
   static __device__ __forceinline__ float load1(const char* p) {
     return uk::small16_to_f32<EB>(*reinterpret_cast<const uint16_t*>(p));
   }
   static __device__ __forceinline__ void store1(char* p, float v) {
     *reinterpret_cast<uint16_t*>(p) = uk::f32_to_small16<EB>(v);
+  }
+  // Four elements as they lie in memory, in two words.
+  static __device__ __forceinline__ v4f from_bits(v2u32 b) {
+    return v4f{uk::small16_to_f32<EB>((uint16_t)b[0]), uk::small16_to_f32<EB>((uint16_t)(b[0] >> 16)),
+               uk::small16_to_f32<EB>((uint16_t)b[1]), uk::small16_to_f32<EB>((uint16_t)(b[1] >> 16))};
+  }
+  static __device__ __forceinline__ v2u32 to_bits(v4f v) {
+    return v2u32{uk::f32_to_small16<EB>(v[0]) | (uint32_t)uk::f32_to_small16<EB>(v[1]) << 16,
+                 uk::f32_to_small16<EB>(v[2]) | (uint32_t)uk::f32_to_small16<EB>(v[3]) << 16};
   }
 };
 
@@ -574,10 +578,32 @@ void mmt4d_mfma_kernel(Args a) {
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = Acc{0, 0, 0, 0};
+  // 16-bit outputs are converted apart from the loads and stores: with the
+  // conversions in the bodies of for_each_output the 256x256 and 128x512 shapes
+  // were too long for the compiler to unroll, and their accumulators, indexed by
+  // a running number, lived in scratch memory all through the K loop (bf16 4616 x
+  // 4207 x 560: 513 us).
   if (a.accumulate) {
-    for_each_output(a.acc, a.acc_stride, a.acc_sm0, a.acc_spn,
-                    [&](int tm, int tn, char* p) { acc[tm][tn] = Out::load4(p); },
-                    [&](int tm, int tn, int e, char* p) { acc[tm][tn][e] = Out::load1(p); });
+    if constexpr (OB == 2) {
+      v2u32 bits[TM][TN];
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) bits[tm][tn] = v2u32{0, 0};
+      for_each_output(a.acc, a.acc_stride, a.acc_sm0, a.acc_spn,
+                      [&](int tm, int tn, char* p) { bits[tm][tn] = *reinterpret_cast<const v2u32*>(p); },
+                      [&](int tm, int tn, int e, char* p) {
+                        bits[tm][tn][e / 2] |= (uint32_t)*reinterpret_cast<const uint16_t*>(p) << e % 2 * 16;
+                      });
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = Out::from_bits(bits[tm][tn]);
+    } else {
+      for_each_output(a.acc, a.acc_stride, a.acc_sm0, a.acc_spn,
+                      [&](int tm, int tn, char* p) { acc[tm][tn] = Out::load4(p); },
+                      [&](int tm, int tn, int e, char* p) { acc[tm][tn][e] = Out::load1(p); });
+    }
   }
 
   // ---- pipeline -----------------------------------------------------------
@@ -1622,12 +1648,32 @@ void mmt4d_mfma_kernel(Args a) {
   // 8192^3, 268 MB: 387-397 -> 377-385 us in the same process); smaller ones
   // are not: whoever reads them next finds them in that cache (the f16 chain's
   // step takes 3 us longer with non-temporal stores here, all of it in unpack).
-  for_each_output(a.out, a.out_stride, a.out_sm0, a.out_spn,
-                  [&](int tm, int tn, char* p) {
-                    if (a.nt_out) Out::store4_nt(p, acc[tm][tn]);
-                    else Out::store4(p, acc[tm][tn]);
-                  },
-                  [&](int tm, int tn, int e, char* p) { Out::store1(p, acc[tm][tn][e]); });
+  if constexpr (OB == 2) {
+    v2u32 bits[TM][TN];
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) bits[tm][tn] = Out::to_bits(acc[tm][tn]);
+    for_each_output(a.out, a.out_stride, a.out_sm0, a.out_spn,
+                    [&](int tm, int tn, char* p) {
+                      // (the non-temporal one as assembly: see Out32)
+                      if (a.nt_out) {
+                        asm volatile("global_store_dwordx2 %0, %1, off nt" : : "v"(p), "v"(bits[tm][tn]) : "memory");
+                      } else {
+                        *reinterpret_cast<v2u32*>(p) = bits[tm][tn];
+                      }
+                    },
+                    [&](int tm, int tn, int e, char* p) {
+                      *reinterpret_cast<uint16_t*>(p) = (uint16_t)(bits[tm][tn][e / 2] >> e % 2 * 16);
+                    });
+  } else {
+    for_each_output(a.out, a.out_stride, a.out_sm0, a.out_spn,
+                    [&](int tm, int tn, char* p) {
+                      if (a.nt_out) Out::store4_nt(p, acc[tm][tn]);
+                      else Out::store4(p, acc[tm][tn]);
+                    },
+                    [&](int tm, int tn, int e, char* p) { Out::store1(p, acc[tm][tn][e]); });
+  }
 }
 
 template <Elem E, int TM, int TN, int WGM, int WGN, int NKK, int PIPE>
