@@ -527,6 +527,10 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   } else {
     choice = 3;
   }
+  // K of less than one step fills no pipeline, and the smaller blocks, several to
+  // a unit, overlap their prologues and stores (s8 16x16x2 7070 x 2547 x 16: 21.9
+  // us in 256x256 blocks, 17.5 in 128x128).
+  if (forced == 0 && (choice == 1 || choice == 7) && ((int64_t)p.K1 << p.lrb) < BIG_KS) choice = 2;
   if (choice == 1 && forced == 0) {
     // Tile quantization: a last row or column of 256x256 workgroups that is
     // mostly padding can cost a whole extra round on the 256 CUs. Compare, in
@@ -859,8 +863,16 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     // 64x64 blocks, 8 waves of 32x16, 256 bytes of K per step.
     // Chosen for narrow tile rows when the 64x64 blocks fill the compute units
     // (s8 1024^3 16x16x2: 7.0 -> 6.4 us; with rows of 16 bytes and more the
-    // register-direct kernel below is level or ahead: 5.7 against 5.9 us).
-    const bool small_default = forced == 0 && RBC < 16 && E != Elem::kF32 && workgroups(p, 64, 64) >= 192;
+    // register-direct kernel below is level or ahead: 5.7 against 5.9 us) and K
+    // is a whole step at least. Its stages take the LDS of a compute unit, the deep
+    // kernel below runs two and more workgroups on one and wins where there is no
+    // pipeline to fill (s8 16x16x2 5000 x 200 x 124 5.0 against 8.7 us, 1400 x 1700
+    // x 124 8.2 against 12.5), and with 16-bit outputs, which would need the
+    // instance for a K that ends inside a step, at any such K (bf16 16x16x2 1400 x
+    // 1700 x 508: 16.1 against 20.9 us).
+    const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
+    const bool small_default = forced == 0 && RBC < 16 && E != Elem::kF32 && workgroups(p, 64, 64) >= 192 &&
+                               k_bytes >= 256 && (!kOneLaunchOnly || k_bytes % 256 == 0);
     if (forced == 19 || small_default) {
       int st = launch_variant<E, RBC, 2, 1, 2, 4, 4, 5>(p, 0, p.K1, p.accumulate, stream);
       if (st == 0) *name = "mmt4d_mfma_64x64_lds_direct";

@@ -283,6 +283,31 @@ def test_mmt4d_k_that_ends_inside_a_step_reads_nothing_beyond_it(gpu, oracle, tf
     lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
 
 
+@pytest.mark.parametrize("flags,K0,M,N,K,kernel", [
+    (uk.MMT4D_TYPE_S8S8S32, 2, 313, 13, 62, "64x64_deep"), (uk.MMT4D_TYPE_S8S8S32, 2, 313, 13, 127, "64x64_deep"),
+    (uk.MMT4D_TYPE_S8S8S32, 2, 313, 13, 128, "64x64_lds_direct"),
+    (uk.MMT4D_TYPE_S8S8S32, 2, 313, 13, 129, "64x64_lds_direct"),
+    (uk.MMT4D_TYPE_BF16BF16BF16 | uk.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS, 2, 88, 107, 127, "64x64_deep"),
+    (uk.MMT4D_TYPE_BF16BF16BF16 | uk.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS, 2, 88, 107, 128, "64x64_lds_direct"),
+    (uk.MMT4D_TYPE_S8S8S32, 16, 208, 256, 3, "128x128_lds_direct"),
+    (uk.MMT4D_TYPE_S8S8S32, 16, 208, 256, 4, "256x256_lds_direct"),
+    (uk.MMT4D_TYPE_F16F16F32, 8, 256, 100, 3, "128x128_lds_direct"),
+    (uk.MMT4D_TYPE_F16F16F32, 8, 256, 100, 4, "256x128_lds_direct")])
+def test_mmt4d_short_k_stays_on_the_kernels_without_a_long_pipeline(gpu, oracle, flags, K0, M, N, K, kernel):
+    """The shapes whose stages take a compute unit's LDS serve K from one of their
+    steps on (64 bytes, 256 in 64x64 blocks), in 64x64 blocks with 16-bit outputs
+    whole steps only."""
+    lib, torch = gpu
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    c = T.Mmt4dCase(flags, M, N, K, 16, 16, K0, K * 16 * K0, K * 16 * K0, N * 256, 0, 0, 0)
+    lhs, rhs, out0 = T.make_mmt4d_buffers(c, np.random.default_rng(K))
+    want = out0.copy()
+    G.run_mmt4d_case(oracle, c, lhs, rhs, want)
+    got = T.gpu_mmt4d(lib, torch, c, lhs, rhs, out0, allow_generic=False)
+    assert np.array_equal(got, want), lib.last_kernel_name()
+    assert lib.last_kernel_name() == "mmt4d_mfma_" + kernel
+
+
 def test_mmt4d_single_row_tiles_equal_row_major_matmul(gpu):
     """With M0 = N0 = 1 the mmt4d layouts are plain row-major [M][K], [N][K]
     and [M][N]: the call must equal the integer matrix product A . B^T
