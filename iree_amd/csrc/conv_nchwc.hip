@@ -454,19 +454,20 @@ struct MfmaTile {
   enum { kOne, kMore, kAny } rounds;  // of workgroups on the compute units: those that `cost` was measured with
   int cost;
   int (*launch)(const ConvArgs&, hipStream_t);
+  const char* name;
 };
 constexpr MfmaTile kMfmaTiles[] = {
-    {4, 4, MfmaTile::kOne, 645, launch_mfma<4, 4, 2>},
-    {2, 4, MfmaTile::kOne, 710, launch_mfma<2, 4, 2>},
-    {2, 2, MfmaTile::kOne, 870, launch_mfma<2, 2, 4>},
-    {1, 4, MfmaTile::kOne, 905, launch_mfma<1, 4, 4>},
-    {1, 2, MfmaTile::kAny, 1050, launch_mfma<1, 2, 4>},
-    {1, 1, MfmaTile::kAny, 1220, launch_mfma<1, 1, 4>},
-    {4, 4, MfmaTile::kMore, 700, launch_mfma<4, 4, 0>},
-    {2, 4, MfmaTile::kMore, 730, launch_mfma<2, 4, 0>},
-    {1, 4, MfmaTile::kMore, 790, launch_mfma<1, 4, 0>},
-    {2, 2, MfmaTile::kMore, 830, launch_mfma<2, 2, 0>},
-    {2, 1, MfmaTile::kMore, 1000, launch_mfma<2, 1, 0>},
+    {4, 4, MfmaTile::kOne, 645, launch_mfma<4, 4, 2>, "conv_nchwc_mfma_direct_4x4"},
+    {2, 4, MfmaTile::kOne, 710, launch_mfma<2, 4, 2>, "conv_nchwc_mfma_direct_2x4"},
+    {2, 2, MfmaTile::kOne, 870, launch_mfma<2, 2, 4>, "conv_nchwc_mfma_direct_2x2"},
+    {1, 4, MfmaTile::kOne, 905, launch_mfma<1, 4, 4>, "conv_nchwc_mfma_direct_1x4"},
+    {1, 2, MfmaTile::kAny, 1050, launch_mfma<1, 2, 4>, "conv_nchwc_mfma_direct_1x2"},
+    {1, 1, MfmaTile::kAny, 1220, launch_mfma<1, 1, 4>, "conv_nchwc_mfma_direct_1x1"},
+    {4, 4, MfmaTile::kMore, 700, launch_mfma<4, 4, 0>, "conv_nchwc_mfma_lds_4x4"},
+    {2, 4, MfmaTile::kMore, 730, launch_mfma<2, 4, 0>, "conv_nchwc_mfma_lds_2x4"},
+    {1, 4, MfmaTile::kMore, 790, launch_mfma<1, 4, 0>, "conv_nchwc_mfma_lds_1x4"},
+    {2, 2, MfmaTile::kMore, 830, launch_mfma<2, 2, 0>, "conv_nchwc_mfma_lds_2x2"},
+    {2, 1, MfmaTile::kMore, 1000, launch_mfma<2, 1, 0>, "conv_nchwc_mfma_lds_2x1"},
 };
 
 // Workgroups a launch of `tile` has, without slices. tw and to are powers of
@@ -574,7 +575,7 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
     }
     const int st = tile->launch(a, stream);
     if (st >= 0) {
-      *kernel_name = "conv_nchwc_mfma";
+      *kernel_name = tile->name;
       return st;
     }
   }

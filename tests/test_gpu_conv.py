@@ -67,7 +67,7 @@ def test_conv_reference_test_grid(gpu, oracle, host, exact, mode):
             early = (c.N == 0 or c.OC_outer == 0 or c.OH == 0 or c.OW == 0 or
                      ((c.IC_outer == 0 or c.FH == 0 or c.FW == 0) and c.flags & C.CONV_ACCUMULATE))
             if not early:
-                assert lib.last_kernel_name() == ("conv_nchwc_mfma" if mfma else "conv_nchwc_generic")
+                assert lib.last_kernel_name().startswith("conv_nchwc_mfma_" if mfma else "conv_nchwc_generic")
     finally:
         lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
 
@@ -84,7 +84,7 @@ def test_conv_mfma_wide_shapes(gpu, oracle, exact):
     for ci, c in enumerate(C.cases(seed=33, tiles=[(16, 16), (16, 32), (16, 48)],
                                    shapes=C.WIDE_SHAPES)):
         _check(lib, torch, oracle, c, 500 + ci, False, exact, True)
-        assert lib.last_kernel_name() == "conv_nchwc_mfma"
+        assert lib.last_kernel_name().startswith("conv_nchwc_mfma_")
         n += 1
     assert n == 24
 
@@ -135,34 +135,34 @@ def test_conv_few_pixels_many_channels_splits_the_input_channels(gpu, oracle, ex
         # a few hundred) differ by a few 1e-4; the exact-data run pins the
         # indexing bit for bit.
         _check(lib, torch, oracle, c, 40 + ci, host=False, exact=exact, mfma=True, atol=2e-3)
-        assert lib.last_kernel_name() == "conv_nchwc_mfma"
+        assert lib.last_kernel_name().startswith("conv_nchwc_mfma_")
         assert lib.workspace_bytes() > 0
 
 
-# One shape (N, OC_outer, OH, OW, IC_outer, FH, FW, strides, c0) for each tile
-# the MFMA launch chooses from on a device of 256 compute units, with ragged
-# pixels and channel blocks; the steps of a sum leave every remainder of the
-# direct kernel's register sets.
+# One shape (N, OC_outer, OH, OW, IC_outer, FH, FW, strides, c0) for each kernel
+# and tile the MFMA launch chooses from on a device of 256 compute units, with
+# ragged pixels and channel blocks; the steps of a sum leave every remainder of
+# the direct kernel's register sets.
 TILE_SHAPES = [
-    (16, 7, 40, 39, 3, 1, 1, 1, 1, 48),   # 4x4 direct, 9 steps
-    (3, 7, 57, 55, 4, 2, 1, 1, 1, 16),    # 2x4 direct, 8 steps
-    (1, 15, 56, 55, 3, 1, 3, 2, 1, 16),   # 2x2 direct, 9 steps
-    (65, 9, 7, 7, 5, 1, 2, 1, 1, 16),     # 1x4 direct, 10 steps
-    (65, 5, 1, 1, 7, 1, 1, 1, 2, 16),     # 1x2 direct, 7 steps
-    (3, 3, 5, 3, 1, 1, 1, 1, 1, 16),      # 1x1 direct, 1 step
-    (16, 31, 31, 33, 1, 1, 1, 1, 1, 16),  # 4x4 through LDS
-    (300, 7, 13, 17, 1, 1, 2, 1, 1, 16),  # 2x4 through LDS
-    (65, 31, 1, 1, 3, 1, 1, 1, 1, 16),    # 1x4 through LDS
-    (300, 2, 13, 17, 1, 3, 1, 1, 2, 16),   # 2x2 through LDS
-    (300, 1, 13, 17, 2, 1, 1, 2, 2, 16),   # 2x1 through LDS
+    ((16, 7, 40, 39, 3, 1, 1, 1, 1, 48), "direct_4x4"),  # 9 steps
+    ((3, 7, 57, 55, 4, 2, 1, 1, 1, 16), "direct_2x4"),  # 8 steps
+    ((1, 15, 56, 55, 3, 1, 3, 2, 1, 16), "direct_2x2"),  # 9 steps
+    ((65, 9, 7, 7, 5, 1, 2, 1, 1, 16), "direct_1x4"),  # 10 steps
+    ((65, 5, 1, 1, 7, 1, 1, 1, 2, 16), "direct_1x2"),  # 7 steps
+    ((3, 3, 5, 3, 1, 1, 1, 1, 1, 16), "direct_1x1"),  # 1 step
+    ((16, 31, 31, 33, 1, 1, 1, 1, 1, 16), "lds_4x4"),
+    ((300, 7, 13, 17, 1, 1, 2, 1, 1, 16), "lds_2x4"),
+    ((65, 31, 1, 1, 3, 1, 1, 1, 1, 16), "lds_1x4"),
+    ((300, 2, 13, 17, 1, 3, 1, 1, 2, 16), "lds_2x2"),
+    ((300, 1, 13, 17, 2, 1, 1, 2, 2, 16), "lds_2x1"),
 ]
 
 
-@pytest.mark.parametrize("shape", TILE_SHAPES, ids=lambda s: "x".join(map(str, s)))
-def test_conv_mfma_tiles(gpu, oracle, shape):
+@pytest.mark.parametrize("shape,tile", TILE_SHAPES, ids=lambda s: s if isinstance(s, str) else "x".join(map(str, s)))
+def test_conv_mfma_tiles(gpu, oracle, shape, tile):
     lib, torch = gpu
     lib.set_pointer_mode(uk.POINTER_MODE_AUTO)
     lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
     for ci, c in enumerate(C.cases(seed=51, tiles=[(16, shape[9])], shapes=[shape[:9]])):
         _check(lib, torch, oracle, c, 900 + ci, host=False, exact=True, mfma=True)
-        assert lib.last_kernel_name() == "conv_nchwc_mfma"
+        assert lib.last_kernel_name() == "conv_nchwc_mfma_" + tile
