@@ -449,25 +449,30 @@ int launch_mfma(const ConvArgs& a, hipStream_t stream) {
 // output-channel blocks per wave. `cost` is the measured time of one step per
 // panel and block of a wave in 0.1 ns (the four MFMAs alone take 533), from
 // layers of 64 to 512 channels at 14x14 to 112x112, batch 1 to 16.
+// `short_cost`, on the same scale, is for sums of fewer than eight steps (1x1
+// filters on few channels), which are loads and stores rather than products and
+// want several small waves on a matrix core; 0: not taken for them (16 -> 224
+// channels, 1x1, 107x107, batch 7: 23.8 us on 4x4 through LDS, 18.4 on 2x2; 64
+// -> 64, stride 2, 62x62, batch 5: 8.6 on 1x2 direct, 7.3 on 1x4 through LDS).
 struct MfmaTile {
   int tw, to;
   enum { kOne, kMore, kAny } rounds;  // of workgroups on the compute units: those that `cost` was measured with
-  int cost;
+  int cost, short_cost;
   int (*launch)(const ConvArgs&, hipStream_t);
   const char* name;
 };
 constexpr MfmaTile kMfmaTiles[] = {
-    {4, 4, MfmaTile::kOne, 645, launch_mfma<4, 4, 2>, "conv_nchwc_mfma_direct_4x4"},
-    {2, 4, MfmaTile::kOne, 710, launch_mfma<2, 4, 2>, "conv_nchwc_mfma_direct_2x4"},
-    {2, 2, MfmaTile::kOne, 870, launch_mfma<2, 2, 4>, "conv_nchwc_mfma_direct_2x2"},
-    {1, 4, MfmaTile::kOne, 905, launch_mfma<1, 4, 4>, "conv_nchwc_mfma_direct_1x4"},
-    {1, 2, MfmaTile::kAny, 1050, launch_mfma<1, 2, 4>, "conv_nchwc_mfma_direct_1x2"},
-    {1, 1, MfmaTile::kAny, 1220, launch_mfma<1, 1, 4>, "conv_nchwc_mfma_direct_1x1"},
-    {4, 4, MfmaTile::kMore, 700, launch_mfma<4, 4, 0>, "conv_nchwc_mfma_lds_4x4"},
-    {2, 4, MfmaTile::kMore, 730, launch_mfma<2, 4, 0>, "conv_nchwc_mfma_lds_2x4"},
-    {1, 4, MfmaTile::kMore, 790, launch_mfma<1, 4, 0>, "conv_nchwc_mfma_lds_1x4"},
-    {2, 2, MfmaTile::kMore, 830, launch_mfma<2, 2, 0>, "conv_nchwc_mfma_lds_2x2"},
-    {2, 1, MfmaTile::kMore, 1000, launch_mfma<2, 1, 0>, "conv_nchwc_mfma_lds_2x1"},
+    {4, 4, MfmaTile::kOne, 645, 0, launch_mfma<4, 4, 2>, "conv_nchwc_mfma_direct_4x4"},
+    {2, 4, MfmaTile::kOne, 710, 0, launch_mfma<2, 4, 2>, "conv_nchwc_mfma_direct_2x4"},
+    {2, 2, MfmaTile::kOne, 870, 0, launch_mfma<2, 2, 4>, "conv_nchwc_mfma_direct_2x2"},
+    {1, 4, MfmaTile::kOne, 905, 0, launch_mfma<1, 4, 4>, "conv_nchwc_mfma_direct_1x4"},
+    {1, 2, MfmaTile::kAny, 1050, 1370, launch_mfma<1, 2, 4>, "conv_nchwc_mfma_direct_1x2"},
+    {1, 1, MfmaTile::kAny, 1220, 1220, launch_mfma<1, 1, 4>, "conv_nchwc_mfma_direct_1x1"},
+    {4, 4, MfmaTile::kMore, 700, 0, launch_mfma<4, 4, 0>, "conv_nchwc_mfma_lds_4x4"},
+    {2, 4, MfmaTile::kMore, 730, 800, launch_mfma<2, 4, 0>, "conv_nchwc_mfma_lds_2x4"},
+    {1, 4, MfmaTile::kMore, 790, 750, launch_mfma<1, 4, 0>, "conv_nchwc_mfma_lds_1x4"},
+    {2, 2, MfmaTile::kMore, 830, 830, launch_mfma<2, 2, 0>, "conv_nchwc_mfma_lds_2x2"},
+    {2, 1, MfmaTile::kMore, 1000, 1000, launch_mfma<2, 1, 0>, "conv_nchwc_mfma_lds_2x1"},
 };
 
 // Workgroups a launch of `tile` has, without slices. tw and to are powers of
@@ -529,23 +534,21 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
     if (hipGetDevice(&dev) == hipSuccess) {
       (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     }
-    // Sums of fewer than eight steps (1x1 filters on few channels) are loads
-    // and stores rather than products and want more than one wave on a matrix
-    // core: 64 -> 176 channels, 1x1, 78x78, batch 3 took 13.4 us on 4x4, one
-    // workgroup per unit, and 11.1 on 2x4 through LDS, two per unit.
     const int64_t steps_per_ic = a.FH * a.FW * (a.c0 / 16);
     const bool short_sums = a.IC * steps_per_ic < 8;
     const MfmaTile* tile = nullptr;
     int64_t least = 0;
     for (const MfmaTile& t : kMfmaTiles) {
+      const int step_cost = short_sums ? t.short_cost : t.cost;
+      if (step_cost == 0) continue;
       const int64_t rounds = uk::ceil_div(mfma_blocks(a, t), (int64_t)cus);
-      if (t.rounds == MfmaTile::kOne && (rounds > 1 || short_sums)) continue;
+      if (t.rounds == MfmaTile::kOne && rounds > 1) continue;
       if (t.rounds == MfmaTile::kMore && rounds <= 1) continue;
       // Each group of channel blocks reads the input again, from memory where
       // the layer is a large one: 288 -> 48 channels, 3x3, stride 2, 84x84,
       // batch 12 (394 MB of input) took 364 us one block at a time, 284 on 2x4.
       if (t.to == 1 && rounds > 1 && a.OC > 1) continue;
-      const int64_t cost = rounds * t.tw * t.to * t.cost;
+      const int64_t cost = rounds * t.tw * t.to * step_cost;
       if (!tile || cost < least) {
         tile = &t;
         least = cost;

@@ -150,8 +150,10 @@ TILE_SHAPES = [
     ((65, 9, 7, 7, 5, 1, 2, 1, 1, 16), "direct_1x4"),  # 10 steps
     ((65, 5, 1, 1, 7, 1, 1, 1, 2, 16), "direct_1x2"),  # 7 steps
     ((3, 3, 5, 3, 1, 1, 1, 1, 1, 16), "direct_1x1"),  # 1 step
-    ((16, 31, 31, 33, 1, 1, 1, 1, 1, 16), "lds_4x4"),
-    ((300, 7, 13, 17, 1, 1, 2, 1, 1, 16), "lds_2x4"),
+    ((65, 25, 35, 6, 4, 1, 1, 1, 1, 32), "lds_4x4"),  # 8 steps
+    ((130, 11, 17, 4, 3, 1, 3, 1, 1, 16), "lds_2x4"),  # 9 steps
+    ((16, 31, 31, 33, 1, 1, 1, 1, 1, 16), "lds_1x4"),  # 1 step: sums of fewer than eight choose by costs of their own
+    ((300, 7, 13, 17, 1, 1, 2, 1, 1, 16), "lds_1x4"),  # 2 steps
     ((65, 31, 1, 1, 3, 1, 1, 1, 1, 16), "lds_1x4"),
     ((300, 2, 13, 17, 1, 3, 1, 1, 2, 16), "lds_2x2"),
     ((300, 1, 13, 17, 2, 1, 1, 2, 2, 16), "lds_2x1"),
