@@ -667,10 +667,14 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
   const bool full = total1 == (uint32_t)N1 * NT && total2 == (uint32_t)N2 * NT;
 
   // Block coordinates and whether the whole block lies inside the matrix and
-  // the tile grid ("interior").
+  // the tile grid. unpack looks at each where it matters: of a matrix whose tiles
+  // pad every row all blocks reach beyond the matrix, which its stores have to
+  // see, and nearly none beyond the tiles that it loads (f32 473301 x 37 from 16x8
+  // under TRANSPOSE_OUTER 79 -> 58 us, 1440079 x 12 from 12x64 122 -> 109). pack was
+  // the slower one with the two apart (the same matrices 83 -> 90 and 136 -> 151).
   struct Block {
     uint32_t blk0, blk1, row_base, col_base_bytes;
-    uint32_t interior;
+    uint32_t mat_inside, tiles_inside;
   };
   auto block_at = [&](uint32_t blk) {
     Block b;
@@ -683,9 +687,9 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
     b.blk1 = g * a.grp + (rem2 - rr * w);
     b.row_base = b.blk0 * a.block_rows;
     b.col_base_bytes = b.blk1 * a.block_row_bytes;
-    b.interior = (b.row_base + a.block_rows <= a.mat_size0) &
-                 (b.col_base_bytes + a.block_row_bytes <= size1_bytes) &
-                 ((b.blk0 + 1) * a.G0 <= a.outer0) & ((b.blk1 + 1) * a.G1 <= a.outer1);
+    b.mat_inside = (b.row_base + a.block_rows <= a.mat_size0) & (b.col_base_bytes + a.block_row_bytes <= size1_bytes);
+    b.tiles_inside = ((b.blk0 + 1) * a.G0 <= a.outer0) & ((b.blk1 + 1) * a.G1 <= a.outer1);
+    if (!UNPACK) b.mat_inside = b.tiles_inside = b.mat_inside & b.tiles_inside;
     return b;
   };
   auto tiled_base = [&](const Block& b) {
@@ -718,7 +722,7 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
       uint32_t off[N1];
 #pragma unroll
       for (int i = 0; i < N1; ++i) off[i] = g1off[i];
-      if (!b.interior) {
+      if (!b.mat_inside) {
 #pragma unroll
         for (int i = 0; i < N1; ++i) {
           uint32_t r, cb;
@@ -734,7 +738,7 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
       uint32_t off[N2];
 #pragma unroll
       for (int i = 0; i < N2; ++i) off[i] = g2off[i];
-      if (!b.interior) {
+      if (!b.tiles_inside) {
 #pragma unroll
         for (int i = 0; i < N2; ++i)
           if (!tile_exists(b, i)) off[i] = 0;
@@ -775,7 +779,7 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
   };
   // Phase 2: LDS -> destination.
   auto phase2 = [&](const Block& b, const char* lbuf, auto inside_c) __attribute__((always_inline)) {
-    constexpr bool kInside = decltype(inside_c)::value;  // interior block, all items
+    constexpr bool kInside = decltype(inside_c)::value;  // of the destination, all items
     if constexpr (!UNPACK) {
       char* base = a.dst + tiled_base(b);
       TileVec reg[N2];
@@ -832,7 +836,7 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
   // block of stores was issued behind the loads it waits for, and waits for
   // the loads alone (without the copy, or with the stores in a branch, for the
   // stores as well).
-  auto steady = [&](const Block& b) { return full && b.interior && blk + gridDim.x < nblocks; };
+  auto steady = [&](const Block& b) { return full && b.mat_inside && b.tiles_inside && blk + gridDim.x < nblocks; };
   auto steady_body = [&](const Block& b) __attribute__((always_inline)) {
     phase1_full(lds + buf);
     prefetch(blk + gridDim.x);
@@ -850,12 +854,12 @@ __global__ __launch_bounds__(NT) void stream_tiled_kernel(TiledArgs a) {
         b = block_at(blk);
       }
     }
-    if (full && (UNPACK || b.interior)) phase1_full(lds + buf);
+    if (full && (UNPACK || b.mat_inside)) phase1_full(lds + buf);
     else phase1(b, lds + buf);
     const bool more = blk + gridDim.x < nblocks;
     if (more) prefetch(blk + gridDim.x);
     __syncthreads();
-    if (full && b.interior) phase2(b, lds + buf, std::true_type{});
+    if (full && (UNPACK ? b.mat_inside : b.tiles_inside)) phase2(b, lds + buf, std::true_type{});
     else phase2(b, lds + buf, std::false_type{});
     if (!more) return;
     advance();
