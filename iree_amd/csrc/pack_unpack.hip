@@ -945,14 +945,22 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // 32x8 86 against 122; f16 1303882 x 13 unpack, 12x12 under TRANSPOSE_OUTER, 117
   // against 285). From 96 padded bytes on they are level or behind (pack f32
   // 427710 x 21 into 24x4: 40 against 39), under TRANSPOSE_OUTER beyond 128 (pack
-  // f32 2103812 x 5 into 16x32, 128 bytes: 245 against 652).
+  // f32 2103812 x 5 into 16x32, 128 bytes: 245 against 652); there beyond 192 where
+  // granules are 16 bytes (f32 262144 x 42 into 12x12, 192 bytes: 42 against 64, from
+  // it 28 and 44; but 8x2 tiles, 160 bytes, 34 and 26, and 16x8, 256 bytes, 34 and
+  // 29) or the tile is transposed, and then beyond 320 from tile rows of 16 bytes on
+  // (363366 x 12 into 12x64, 256 bytes: 52 against 101; 16x8 from 320 bytes 30 and 33).
   const int64_t padded_row_bytes = v.outer1 * v.tile1 * es;
   // Rows of single bytes that are not whole words go over only below that, where
   // the streaming kernels have 8- or 16-byte vectors for them (s8 421410 x 70 into
   // 1x16, 80 bytes: 51 against 30; 2264133 x 34 into 16x16, 48 bytes: 160 against
   // 189; 283972 x 47 into 24x4 under TRANSPOSE_OUTER, 48 bytes: 49 against 23).
   const bool byte_rows = es == 1 && (((uintptr_t)mat_ptr | (uint64_t)mat_stride0) & 3) && padded_row_bytes % 8 == 0;
-  const bool narrow = padded_row_bytes <= (byte_rows ? (to ? 47 : 48) : to ? 128 : 95);
+  const int64_t narrow_bytes = byte_rows ? (to ? 47 : 48)
+                               : to && ti ? (v.tile1 * es >= 16 ? 320 : 192)
+                               : to       ? (G == 16 ? 192 : 128)
+                                          : 95;
+  const bool narrow = padded_row_bytes <= narrow_bytes;
   const bool big = allow_big && !narrow && VEC == 16 && (big_transposing || big_rows);
   const int64_t kMinSpan = big ? 512 : 256;                      // bytes, both sides
   const int64_t kTarget = big ? kStreamBigBlockBytes : kStreamBlockBytes;  // bytes per block, about
@@ -1131,11 +1139,11 @@ TiledPlan plan_tiled(const TiledView& v, int es, const char* mat_ptr,
   // 256 x 20480 from 1x16, 640 blocks: 7.0 us against 8.9 with two of which one in
   // four takes a second block; f32 9728 x 320 from 16x4, short rows: 11.1 and
   // 10.4), and where blocks span whole rows under TRANSPOSE_OUTER, all of them edge
-  // blocks, and granules are 16 bytes (f32 513513 x 32 into 12x12: 97 and 123; f32
-  // 228560 x 75 from 12x12: 48 and 59; but f16 197299 x 240 from 16x2, 4-byte ones, 49
+  // blocks, and granules are 8 or 16 bytes (f32 228560 x 75 from 12x12: 48 and 59, f32
+  // 534553 x 40 into 32x2 40 and 46; but f16 197299 x 240 from 16x2, 4-byte ones, 49
   // and 44).
   if ((mat_is_dest && padded_row_bytes >= 16384 && nblk0 * nblk1 <= 1024) ||
-      (to && G == 16 && padded_row_bytes < 640)) {
+      (to && G >= 8 && padded_row_bytes < 640)) {
     plan.max_workgroups = 1024;
   }
   plan.G = G;

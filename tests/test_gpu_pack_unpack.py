@@ -367,22 +367,32 @@ def test_pack_and_unpack_of_rows_in_gigabytes_of_padding(gpu, n1, kernel):
 @pytest.mark.parametrize("tf,t0,t1,flags", [
     (uk.PACK_TYPE_F32F32, 16, 4, 0), (uk.PACK_TYPE_F32F32, 8, 8, 0x200), (uk.PACK_TYPE_F32F32, 16, 1, 0x300),
     (uk.PACK_TYPE_BF16BF16, 12, 12, 0), (uk.PACK_TYPE_BF16BF16, 16, 8, 0x200), (uk.PACK_TYPE_I8I8, 12, 12, 0x200),
-    (uk.PACK_TYPE_I8I8, 16, 16, 0)])
+    (uk.PACK_TYPE_I8I8, 16, 16, 0), (uk.PACK_TYPE_F32F32, 16, 32, 0), (uk.PACK_TYPE_F32F32, 8, 2, 0x200),
+    (uk.PACK_TYPE_F32F32, 8, 2, 0x300), (uk.PACK_TYPE_F32F32, 16, 8, 0x300)])
 def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
-    """Rows whose tiles end below 96 bytes (up to 128 under TRANSPOSE_OUTER, up to 48
-    where they are single bytes and not whole words), and the first ones beyond:
-    which kernel, and its bytes."""
+    """Rows whose tiles end below 96 bytes (up to 128 under TRANSPOSE_OUTER, there
+    up to 192 in tile rows of whole 16-byte granules, 192 or 320 in transposed
+    tiles; up to 48 where they are single bytes and not whole words), and the first
+    ones beyond: which kernel, and its bytes."""
     lib, torch = gpu
     es = uk.PACK_TYPE_BYTES[tf]
     rng = np.random.default_rng(t0 * 100 + t1)
     tile_row = t1 * es
-    for ci, cols in enumerate(sorted({c for b in (16, 33, 64, 80, 95, 96, 97, 112, 128, 129, 144) for c in
+    for ci, cols in enumerate(sorted({c for b in (16, 33, 64, 80, 95, 96, 97, 112, 128, 129, 144, 192, 320) for c in
                                       (b // es, b // es + 1)})):
         rows = int(rng.integers(100, 300))
         padded = -(-cols // t1) * tile_row
         pitch = cols + ci % 2
         byte_rows = es == 1 and pitch % 4 != 0 and padded % 8 == 0
-        narrow = padded <= ((47 if flags & 0x200 else 48) if byte_rows else 128 if flags & 0x200 else 95)
+        if byte_rows:
+            limit = 47 if flags & 0x200 else 48
+        elif flags & 0x300 == 0x300 and t1 > 1:
+            limit = 320 if tile_row >= 16 else 192
+        elif flags & 0x200:
+            limit = 192 if tile_row % 16 == 0 else 128
+        else:
+            limit = 95
+        narrow = padded <= limit
         o0, o1 = -(-rows // t0), -(-cols // t1)
         so0, so1 = (o1, o0) if flags & 0x200 else (o0, o1)
         s2, s3 = (t1, t0) if flags & 0x100 else (t0, t1)
@@ -412,8 +422,7 @@ def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
     (uk.PACK_TYPE_BF16BF16, 16, 2, 0), (uk.PACK_TYPE_F32F32, 4, 16, 0x100), (uk.PACK_TYPE_I8I8, 8, 16, 0x300),
     (uk.PACK_TYPE_BF16BF16, 16, 16, 0x300)])
 def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3, flags):
-    """Rows up to 64 bytes (32 where they are not whole words) once the blocks of 32
-    rows are more than 1024, more than 512 for rows under 16 bytes: the
+    """Rows up to 64 bytes (32 where they are not whole words) once the blocks of 32 rows are more than 1024, more than 512 for rows under 16 bytes: the
     transposing kernel's blocks are 512 bytes wide. Not tiles of 32 bytes along
     rows of whole words under TRANSPOSE_OUTER."""
     lib, torch = gpu
@@ -421,7 +430,7 @@ def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3
     t0, t1 = (s3, s2) if flags & 0x100 else (s2, s3)
     rng = np.random.default_rng(s2)
     for rows in (100, 32 * 512, 32 * 512 + 1, 32 * 1024, 32 * 1024 + 1):
-        for cols in (15 // es, 16 // es, 32 // es, 32 // es + 1, 64 // es, 64 // es + 4):
+        for cols in (15 // es, 16 // es, 32 // es, 32 // es + 1, 50 // es, 54 // es, 64 // es, 64 // es + 4):
             row_bytes = cols * es
             words = row_bytes % 4 == 0
             few = rows <= (32 * 512 if row_bytes < 16 else 32 * 1024)
