@@ -434,14 +434,20 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
   // Rows that are whole words, which the tiled kernel loads as such, are better off
   // there up to 64 bytes, others up to 32: f32 90303 x 8 into 16x4 7.7 and 9.9; s8
   // 111358 x 18 into 8x8 transposed 9.9 and 14.9, but 114248 x 49 into 16x1 22 and 14.
+  // Whole half words in tiles that are not transposed up to 50: s8 120000 x 42 into 16x2
+  // 10.0 and 12.5, x 62 12.8 and 12.7.
   // Not so under TRANSPOSE_OUTER in tiles that take 32 bytes and more of such a row, of
   // which the tiled kernel then writes one at a time: bf16 150976 x 8 into 16x32 20.6
   // there and 16.0 here, f32 899711 x 3 into 8x8 101 and 87; tiles of 16 bytes, f32
   // 587196 x 2 into 8x4, 37 and 48.
   const int64_t row_bytes = p->in_size1 * es;
   const bool whole_words = (((uintptr_t)src | (uint64_t)pitch) & 3) == 0;
+  const bool half_words = !ti && (((uintptr_t)src | (uint64_t)pitch) & 1) == 0;
   const bool wide_tiles = to && whole_words && t1 * eb >= 32;
-  if (!wide_tiles && nblk0 * nblk1 > (row_bytes < 16 ? 512 : 1024) && row_bytes <= (whole_words ? 64 : 32)) return nullptr;
+  if (!wide_tiles && nblk0 * nblk1 > (row_bytes < 16 ? 512 : 1024) &&
+      row_bytes <= (whole_words ? 64 : half_words ? 50 : 32)) {
+    return nullptr;
+  }
 
   // Rows that are not whole words apart, or that end inside a tile row.
   const bool ragged = (((uintptr_t)src | (uint64_t)pitch) & 3) || (!ti && p->in_size1 % p->out_size3 != 0);
@@ -485,17 +491,18 @@ const char* iree_uk_amd_launch_pack_tr(const iree_uk_pack_params_t* p, int es, c
   // come from HBM again where the next kernel finds it in the memory-side cache
   // otherwise (f32 4096 x 4096, 67 MB, and the unpack that follows: 29.4 + 23.8 us
   // against 23.6 + 21.7; f16 6000 x 8192, 98 MB: 37.5 + 51.5 against 39.8 + 58).
-  // From 16 MB on the stores go through the L2s into that cache: plain ones leave
+  // From 12 MB on the stores go through the L2s into that cache: plain ones leave
   // the L2s full of tiles that are written back when the kernel ends (f16 320 x
-  // 33472 into 16x16, 21 MB: 13.8 us plain, 11.9 non-temporal, 12.3 through; with
-  // the mmt4d that reads the tiles, 16 to 72 MB, 0.95 of the time with
-  // non-temporal ones, plain ones 0.98). Not where TRANSPOSE_OUTER makes runs of
+  // 33472 into 16x16, 21 MB: 13.8 us plain, 11.9 non-temporal, 12.3 through, s8 3500
+  // x 4096 into 16x2, 14 MB: 5.8, 4.7, 5.0; with the mmt4d that reads the tiles, 16
+  // to 72 MB, 0.95 of the time with non-temporal ones, plain ones 0.98, 12 to 16 MB
+  // 0.90 and 0.99; below, plain ones are level). Not where TRANSPOSE_OUTER makes runs of
   // less than 256 bytes of a block's tiles, parts of lines that the L2s had better
   // join (s8 2857 x 8251 into 16x1: 16.7 plain, 35 non-temporal, 25.9 through).
   const int64_t total = outer0 * outer1 * tile_bytes;
   const bool long_runs = !to || kBlockRows * t1 * eb >= 256;
   const uk::Store how = total >= (72ll << 20)                ? uk::Store::kNonTemporal
-                        : total >= (16ll << 20) && long_runs ? uk::Store::kThrough
+                        : total >= (12ll << 20) && long_runs ? uk::Store::kThrough
                                                              : uk::Store::kPlain;
   const dim3 block(kBlockRows * kBlockRowBytes / 64);
   auto go = [&](auto eb_c, auto v_c, auto il_c) {

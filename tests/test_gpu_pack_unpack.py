@@ -422,7 +422,8 @@ def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
     (uk.PACK_TYPE_BF16BF16, 16, 2, 0), (uk.PACK_TYPE_F32F32, 4, 16, 0x100), (uk.PACK_TYPE_I8I8, 8, 16, 0x300),
     (uk.PACK_TYPE_BF16BF16, 16, 16, 0x300)])
 def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3, flags):
-    """Rows up to 64 bytes (32 where they are not whole words) once the blocks of 32 rows are more than 1024, more than 512 for rows under 16 bytes: the
+    """Rows up to 64 bytes (32 where they are not whole words, 50 of half words in
+    tiles that are not transposed) once the blocks of 32 rows are more than 1024, more than 512 for rows under 16 bytes: the
     transposing kernel's blocks are 512 bytes wide. Not tiles of 32 bytes along
     rows of whole words under TRANSPOSE_OUTER."""
     lib, torch = gpu
@@ -435,7 +436,8 @@ def test_narrow_matrices_stay_off_the_transposing_kernel(gpu, oracle, tf, s2, s3
             words = row_bytes % 4 == 0
             few = rows <= (32 * 512 if row_bytes < 16 else 32 * 1024)
             wide_tiles = flags & 0x200 and words and t1 * es >= 32
-            transposing = few or wide_tiles or row_bytes > (64 if words else 32)
+            half_words = not flags & 0x100 and row_bytes % 2 == 0
+            transposing = few or wide_tiles or row_bytes > (64 if words else 50 if half_words else 32)
             o0, o1 = -(-rows // t0), -(-cols // t1)
             so0, so1 = (o1, o0) if flags & 0x200 else (o0, o1)
             c = T.PackCase(tf | flags, rows, cols, so0, so1, s2, s3, cols, 1, so1 * s2 * s3, 0, 0, 0x0102030405060708)
@@ -479,7 +481,7 @@ def test_narrow_matrices_leave_the_direct_kernel(gpu, oracle, tf, t0, t1, flags,
     (uk.PACK_TYPE_I8I8, 16, 1, 0x200, 2050, 8302), (uk.PACK_TYPE_F32F32, 16, 4, 0, 2500, 2622),
     (uk.PACK_TYPE_BF16BF16, 24, 4, 0, 3001, 4300), (uk.PACK_TYPE_I8I8, 16, 16, 0, 4001, 6300)])
 def test_pack_of_tiles_that_are_stored_through(gpu, tf, t0, t1, flags, rows, cols):
-    """Tiles of 16 MB and more on the transposing kernel (runs of less than 256
+    """Tiles of 12 MB and more on the transposing kernel (runs of less than 256
     bytes under TRANSPOSE_OUTER are stored as before), of 24 MB and more on the
     streaming one, ragged on both sides; against pad + reshape + transpose."""
     lib, torch = gpu
