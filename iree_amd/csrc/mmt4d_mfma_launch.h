@@ -396,11 +396,14 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
       (int64_t)(TN * 16 / p.N0 + 2) * p.rhs_stride + k_bytes * p.N0 / (S4 ? 2 : 1);
   if (span_m >= (1ll << 31) || span_n >= (1ll << 31)) return -1;
   // Still too few output blocks for the chip, and a long K: split K over
-  // workgroups as well, aiming at one workgroup per compute unit, each wave
-  // keeping at least four steps. The split costs a few microseconds at the end
-  // of the launch (the slices meet through device-scope accesses, three
-  // dependent round trips to where the XCDs meet), so it has to at least halve
-  // the streaming time to pay.
+  // workgroups as well, aiming at one workgroup per compute unit. The split costs
+  // 1.5 to 2.5 us at the end of the launch (the slices meet through device-scope
+  // accesses, three dependent round trips to where the XCDs meet), so a slice
+  // keeps at least as many operand bytes as a workgroup streams in several times
+  // that: 192 KB (16 rows, weights not cached: s8 1024 x 16384, 512 KB a block, 10.6
+  // -> 9.3 us in two slices; s8 1024 x 4096, 128 KB, 4.7 against 6.2; f16 64 rows
+  // 1024 x 4096, 640 KB, 13.8 -> 11.1 in three). With so few blocks that most units
+  // would idle, 64 KB. In any case 16 steps.
   int64_t kslices = 1;
   if (allow_k_slices) {
     const int64_t blocks = grid_m * grid_n;
@@ -408,9 +411,11 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
     if (k_slices_override() > 0) {
       kslices = k_slices_override();
     } else if (cus > 0 && 2 * blocks <= cus) {
-      kslices = std::min<int64_t>(max_k_slices, cus / blocks);
+      const int64_t share = k_bytes * 16 * (TM + TN) - (S4 ? k_bytes * 8 * TN : 0);
+      const int64_t least = TM * TN >= 16 || 8 * blocks <= cus ? 65536 : 196608;
+      kslices = std::min<int64_t>(std::min<int64_t>(max_k_slices, cus / blocks), share / least);
     }
-    kslices = std::max<int64_t>(1, std::min<int64_t>(kslices, a.steps / (4 * KSPLIT)));
+    kslices = std::max<int64_t>(1, std::min<int64_t>(kslices, a.steps / 16));
     if (blocks * kslices >= (1ll << 31)) kslices = 1;
   }
   if (kslices > 1) {
@@ -437,6 +442,36 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D>,
              dim3((uint32_t)(grid_m * grid_n * kslices)), dim3(KSPLIT * 64), 0, stream, a);
   return (int)hipGetLastError();
+}
+
+// The thin kernel with TM 16-row blocks against `wide_cols` columns (rows of the
+// right-hand side; N-thin problems come transposed). The launch streams the
+// weights, so what counts is how evenly they lie on the compute units and how
+// many loads a unit has in flight:
+//   * one 16-column block a workgroup, its K over eight waves, up to one block a
+//     unit, and for up to 16 rows wherever the most loaded unit gets fewer columns
+//     that way. us in 1x1 blocks of eight waves against 1x1 / 1x2 of four, weights
+//     not cached: s4 4 x 4096 x 16384 11.1 / 15.5 / 15.1; s8 8-byte rows 16 x 2048 x
+//     4096 6.5 / 6.8 / 8.4; f16 4 x 4096 x 4096 9.0 / 9.8 / 11.0; f8 4 x 10240 x 4096
+//     10.6 / 10.8 / 11.8;
+//   * else 32 columns a workgroup over four waves: s8 4 x 6144 x 16384 20.8 against
+//     21.2, 32 x 14336 x 4096 15 % and 64 x 14336 x 4096 20 to 40 % ahead (a second
+//     column block shares the rows' loads).
+// With 16 and fewer rows four steps are in flight in a wave, with more two (their
+// registers: 2x1 and 4x1 blocks of eight waves 1 to 5 % ahead of four steps).
+template <Elem E, int RBC, int TM>
+int launch_thin_rows(const Problem& p, bool swapped, int64_t wide_cols, hipStream_t stream) {
+  constexpr int H = ElemTraits<E>::kHalves;
+  const int64_t rows = swapped ? std::min<int64_t>((int64_t)p.N1 * p.N0, p.out_cols)
+                               : std::min<int64_t>((int64_t)p.M1 * p.M0, p.out_rows);
+  const int64_t row_blocks = std::max<int64_t>(1, uk::ceil_div(rows, (int64_t)(TM * 16)));
+  const int64_t cus = std::max(compute_units(), 1);
+  const int64_t blocks16 = row_blocks * uk::ceil_div(wide_cols, (int64_t)16);
+  const int64_t blocks32 = row_blocks * uk::ceil_div(wide_cols, (int64_t)32);
+  const bool narrow = blocks16 <= cus ||
+                      (TM == 1 && uk::ceil_div(blocks16, cus) < 2 * uk::ceil_div(blocks32, cus));
+  if (narrow) return launch_thin<E, RBC, TM, 1, 8, TM == 1 && H == 1 ? 4 : 2>(p, swapped, stream, true);
+  return launch_thin<E, RBC, TM, 2, 4, TM == 4 ? 3 : 4>(p, swapped, stream, true);
 }
 
 // Status of the second, accumulating launch over the remainder of K. The
@@ -784,25 +819,13 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     choice = 3;
   }
   // The thin kernel for a problem with `thin_rows` rows on its thin side and
-  // `wide_cols` columns on the other (M-thin as it is, N-thin transposed):
-  // 32 columns per workgroup, or 16 when 32 would leave compute units without
-  // a workgroup (a decode step against a weight matrix of few rows, e.g.
-  // 16 x 4096 x 14336 s8: 16.1 -> 12.8 us); what K split over workgroups adds
-  // on top is decided in launch_thin.
+  // `wide_cols` columns on the other (M-thin as it is, N-thin transposed).
   // (A generic lambda: its body is only instantiated for the row widths that call it.)
   auto thin_launch = [&](auto swapped_c, int64_t thin_rows, int64_t wide_cols) {
     const bool swapped = swapped_c;
-    const bool narrow = uk::ceil_div(wide_cols, (int64_t)32) < compute_units();
-    if (thin_rows <= 16) {
-      return narrow ? launch_thin<E, RBC, 1, 1, 4, 4>(p, swapped, stream, true)
-                    : launch_thin<E, RBC, 1, 2, 4, 4>(p, swapped, stream, true);
-    }
-    if (thin_rows <= 32) {
-      return narrow ? launch_thin<E, RBC, 2, 1, 4, 4>(p, swapped, stream, true)
-                    : launch_thin<E, RBC, 2, 2, 4, 4>(p, swapped, stream, true);
-    }
-    return narrow ? launch_thin<E, RBC, 4, 1, 4, 4>(p, swapped, stream, true)
-                  : launch_thin<E, RBC, 4, 2, 4, 3>(p, swapped, stream, true);
+    if (thin_rows <= 16) return launch_thin_rows<E, RBC, 1>(p, swapped, wide_cols, stream);
+    if (thin_rows <= 32) return launch_thin_rows<E, RBC, 2>(p, swapped, wide_cols, stream);
+    return launch_thin_rows<E, RBC, 4>(p, swapped, wide_cols, stream);
   };
   if (choice == 5) {
     // N-thin (a few columns against many rows, e.g. the last column strip of

@@ -88,18 +88,19 @@ void mmt4d_thin_kernel(Args a) {
   const uint32_t sstep_a = kts_per_step * kt_m, sstep_b = kts_per_step * kt_n;
 
   // Byte offset of the lane's piece(s) of block row `x` (a row of 16 rows of
-  // the M or N dimension) at K step 0; 0 for rows outside the problem, whose
-  // (valid) bytes only reach accumulators that are never stored.
+  // the M or N dimension) at K step 0; 0 for rows outside the problem or the
+  // result (tile padding), whose (valid) bytes only reach accumulators that are
+  // never stored: those lanes share the cache lines of the first row.
   // Offsets are 32-bit and relative to the first panel the workgroup touches.
   const int pa0 = bm * TM * 16 / a.M0, pb0 = bn * TN * 16 / a.N0;
   const char* base_a = a.lhs + (int64_t)pa0 * a.lhs_stride;
   const char* base_b = a.rhs + (int64_t)pb0 * a.rhs_stride;
-  auto operand_offsets = [&](uint32_t (&off)[HALVES][PIECES], int x, int X0, int X1, int p0,
+  auto operand_offsets = [&](uint32_t (&off)[HALVES][PIECES], int x, int X0, int X1, int rows, int p0,
                              int64_t stride, uint32_t kt_bytes, int lrb, uint32_t piece_bytes) {
     const uint32_t row = (uint32_t)x * 16 + r;
     const uint32_t pabs = row / (uint32_t)X0;
     const uint32_t x0 = row - pabs * X0;
-    const bool ok = (int)pabs < X1;
+    const bool ok = (int)pabs < X1 && (int)row < rows;
     const uint32_t pl = pabs - (uint32_t)p0;
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) {
@@ -120,10 +121,10 @@ void mmt4d_thin_kernel(Args a) {
   uint32_t offa[TM][HALVES][PIECES], offb[TN][HALVES][PIECES];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
-    operand_offsets(offa[tm], bm * TM + tm, a.M0, a.M1, pa0, a.lhs_stride, kt_m, lrb, 16);
+    operand_offsets(offa[tm], bm * TM + tm, a.M0, a.M1, a.out_rows, pa0, a.lhs_stride, kt_m, lrb, 16);
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn)
-    operand_offsets(offb[tn], bn * TN + tn, a.N0, a.N1, pb0, a.rhs_stride, kt_n, lrb_b,
+    operand_offsets(offb[tn], bn * TN + tn, a.N0, a.N1, a.out_cols, pb0, a.rhs_stride, kt_n, lrb_b,
                     S4 ? 8 : 16);
 
   auto load_operand = [&](const char* base, const uint32_t (&off)[PIECES], uint32_t adv) {

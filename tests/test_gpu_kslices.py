@@ -200,3 +200,35 @@ def test_few_blocks_and_a_long_k_split_k_over_workgroups(gpu, oracle, tf, K0):
         assert lib.last_kernel_name() == "mmt4d_mfma_64x64_ksplit", lib.last_kernel_name()
         assert lib.last_k_slices() > 1
         assert np.array_equal(got, want), c.label()
+
+
+@pytest.mark.parametrize("tile", [(uk.MMT4D_TYPE_S8S8S32, 32, 16, 8), (uk.MMT4D_TYPE_S8S8S32, 16, 16, 16),
+                                  (uk.MMT4D_TYPE_F16F16F32, 16, 16, 8), (uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32, 16, 16, 32),
+                                  (uk.MMT4D_TYPE_S8S4S32, 16, 16, 16)])
+def test_thin_blocks_by_columns_rows_and_steps(gpu, oracle, tile):
+    """The thin kernel where its choice of blocks changes (one 16-column block a
+    compute unit, one more, two and a half) and with fewer K steps than waves,
+    as many and one more; only some rows of the tile exist in the result, the
+    others hold whatever the tile holds. Exact on the reference tests' values."""
+    lib, torch = gpu
+    tf, M0, N0, K0 = tile
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    lib.set_k_slices(0)
+    lb, _, ob = uk.MMT4D_TYPE_BITS[tf]
+    step = (128 if tf == uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32 else 64) * 8 // lb
+    assert ob == 32
+    for ci, (rows, N1, steps) in enumerate(((1, 256, 9), (15, 257, 1), (3, 640, 7), (17, 256, 8), (33, 257, 3),
+                                            (16, 3, 33), (2, 1, 8))):
+        M1, K1 = -(-rows // M0), steps * step // K0
+        c = T.Mmt4dCase(tf | 0x200, M1, N1, K1, M0, N0, K0, K1 * M0 * K0, K1 * N0 * K0, N1 * M0 * N0, 0, 0, 0)
+        lhs, rhs, tiled = T.make_mmt4d_buffers(c, np.random.default_rng(70 + ci))
+        G.run_mmt4d_case(oracle, c, lhs, rhs, tiled)
+        cols = N1 * N0 - ci % 5
+        want = tiled.view(np.int32).reshape(M1, N1, M0, N0).transpose(0, 2, 1, 3).reshape(M1 * M0, -1)[:rows, :cols]
+        d_lhs, d_rhs = T.DeviceBytes(torch, lhs), T.DeviceBytes(torch, rhs)
+        out = torch.full((rows, cols), -7, device="cuda", dtype=torch.int32)
+        lib.mmt4d_unpack(d_lhs.ptr, 0, c.lhs_stride0, d_rhs.ptr, 0, c.rhs_stride0, out.data_ptr(), 0, cols, rows, cols,
+                         M1, N1, K1, M0, N0, K0, c.flags)
+        lib.synchronize()
+        assert lib.last_kernel_name().startswith("mmt4d_mfma_thin"), lib.last_kernel_name()
+        assert np.array_equal(out.cpu().numpy(), want), (tile, rows, N1, steps)
