@@ -327,7 +327,9 @@ int launch_narrow(const Problem& p, int kt_count, hipStream_t stream) {
 // status, or -1 if it cannot serve the shape.
 // `swapped`: the caller's problem is N-thin and is computed as its transpose
 // (out^T = rhs * lhs^T): the kernel's rows are the caller's columns.
-template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D>
+// A K that ends inside a step is served where TAIL_OK says that there is an
+// instance for it.
+template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool TAIL_OK = false>
 int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool allow_k_slices = false,
                 int max_k_slices = 8) {
   constexpr int OBYTES = ElemTraits<E>::Out::kOutBytes;
@@ -348,9 +350,10 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   constexpr int KS = 64 * ElemTraits<E>::kHalves;
   constexpr int OB = OBYTES;
   constexpr bool S4 = E == Elem::kS8S4;  // rb, lrb describe the LHS; RHS rows are half as wide
-  if (p.rb > KS || p.rb < (S4 ? 16 : 8)) return -1;
+  if (p.rb > KS || p.rb < (S4 ? 16 : std::min(RBC, 8))) return -1;
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
-  if (k_bytes == 0 || k_bytes % KS) return -1;
+  const bool tail = k_bytes % KS != 0;
+  if (k_bytes == 0 || (tail && !TAIL_OK)) return -1;
   // 4-bit RHS: the accumulators hold 16 * sum; |sum| <= K * 128 * 8 must stay
   // below 2^27 for that to be exact.
   if (S4 && k_bytes >= 131072) return -1;
@@ -374,7 +377,7 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   }
   a.grid_m = (int32_t)grid_m;
   a.grid_n = (int32_t)grid_n;
-  a.steps = (int32_t)(k_bytes / KS);
+  a.steps = (int32_t)uk::ceil_div(k_bytes, (int64_t)KS);
   a.accumulate = p.accumulate;
   a.acc = p.acc; a.acc_stride = p.acc_stride;
   a.acc_sm0 = (uint32_t)(swapped ? OBYTES : p.acc_sm0);
@@ -432,15 +435,20 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
       kslices = 1;
     }
   }
+  const dim3 grid((uint32_t)(grid_m * grid_n * kslices)), block(KSPLIT * 64);
+  if constexpr (TAIL_OK) {
+    // (Not a shape of calls that stream weights: no non-temporal instance.)
+    if (tail) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, true>, grid, block, 0, stream, a);
+    else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D>, grid, block, 0, stream, a);
+    return (int)hipGetLastError();
+  }
   // Weights that the caller has declared streamed, when they are too large for
   // the L2s anyway: loaded non-temporally.
   if (streamed_weights() && (int64_t)p.N1 * p.N0 * k_bytes / (S4 ? 2 : 1) >= (16ll << 20)) {
-    uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, true>,
-               dim3((uint32_t)(grid_m * grid_n * kslices)), dim3(KSPLIT * 64), 0, stream, a);
+    uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, true>, grid, block, 0, stream, a);
     return (int)hipGetLastError();
   }
-  uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D>,
-             dim3((uint32_t)(grid_m * grid_n * kslices)), dim3(KSPLIT * 64), 0, stream, a);
+  uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D>, grid, block, 0, stream, a);
   return (int)hipGetLastError();
 }
 
@@ -474,6 +482,21 @@ int launch_thin_rows(const Problem& p, bool swapped, int64_t wide_cols, hipStrea
   return launch_thin<E, RBC, TM, 2, 4, TM == 4 ? 3 : 4>(p, swapped, stream, true);
 }
 
+// The thin kernel for `thin_rows` rows: the fewest 16-row blocks a workgroup that still
+// leave at most one workgroup a compute unit, as long as the weights that several row
+// blocks then read are no more than what the L2s hold (us, f16 64 x 2048 x 8 KB in one
+// 64-row block / two of 32: 10.9 / 7.5; s8 64 x 300 x 4 KB in one / four of 16: 8.3 / 4.1).
+template <Elem E, int RBC>
+int launch_thin_any(const Problem& p, bool swapped, int64_t thin_rows, int64_t wide_cols, hipStream_t stream) {
+  const int64_t cus = compute_units(), cols16 = uk::ceil_div(wide_cols, (int64_t)16);
+  const bool cached = wide_cols * ((int64_t)p.K1 << p.lrb) <= (16ll << 20);
+  if (thin_rows <= 16 || (cached && uk::ceil_div(thin_rows, (int64_t)16) * cols16 <= cus))
+    return launch_thin_rows<E, RBC, 1>(p, swapped, wide_cols, stream);
+  if (thin_rows <= 32 || (cached && uk::ceil_div(thin_rows, (int64_t)32) * cols16 <= cus))
+    return launch_thin_rows<E, RBC, 2>(p, swapped, wide_cols, stream);
+  return launch_thin_rows<E, RBC, 4>(p, swapped, wide_cols, stream);
+}
+
 // Status of the second, accumulating launch over the remainder of K. The
 // first launch has already written the output: "not served" (negative) must
 // not reach the dispatcher, which would recompute the whole problem on the
@@ -485,6 +508,59 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
   const int bpm = BM / p.M0, bpn = BN / p.N0;
   if (bpm < 1 || bpn < 1) return 0;
   return uk::ceil_div(p.M1, bpm) * uk::ceil_div(p.N1, bpn);
+}
+
+// Problems whose 64x64 blocks leave compute units idle or take a last round that is
+// nearly empty: the barrier-free kernel in 16x16 or 32x32 blocks, several waves of a
+// block sharing K, so that the chain of K steps a wave walks through is short and many
+// more loads are in flight than one workgroup a unit keeps. `b64` / `b128`: which
+// kernel it would be otherwise. Any K, any tile rows. Returns a HIP status, or -1 where
+// those kernels are the better ones. us before / in these blocks, same buffers:
+//   one 16x16 block a unit or fewer, from 256 bytes of K (rows under 16 bytes: 64):
+//     f16 220 x 215, K 512 B 4.5 / 4.2, 2 KB 6.8 / 4.2, 7.6 KB 14.9 / 5.4; s8 16x16x2
+//     128 x 512, 100 B 4.4 / 3.8, 1 KB 6.5 / 4.0; f32 16x16x1 220 x 215, 3 KB 22.1 /
+//     5.9 (there up to three blocks a unit: 374 x 391, 1 KB 11.1 / 5.5);
+//   two 32x32 blocks a unit or fewer, from 1 KB (f32: 256 B): s8 500 x 500, 3.8 KB
+//     9.6 / 6.5; f16 512 x 1024, 1 KB 5.5 / 5.3, 7.6 KB 15.7 / 13.6; bf16 16x16x2 500 x
+//     500, 1 KB 6.8 / 5.3 (rows of 2 bytes load an element at a time: one block a unit,
+//     s8 16x16x2 500 x 500, 3.8 KB 13.9 / 10.6, 512 x 1024 14.1 / 13.7);
+//   f32, whose MFMAs are slow enough to hide the loads of 32x32 blocks, wherever these
+//     are fewer than 7/2 (64x64) or 14 (128x128) for each block slot of the other
+//     kernel's rounds: 16x16x1 515 x 1027, 3 KB 22.6 / 17.5, 1500 x 1500 54.3 / 46.2, 3000
+//     x 3000 166 / 153, 8 KB 405 / 322; 16x16x4 1000 x 1500, 3 KB 28.5 / 25.3; but 2000 x
+//     1000, two full rounds of 64x64, 37.3 / 39.5, 4096 x 2048 110 / 137.
+template <Elem E, int RBC>
+int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, hipStream_t stream,
+                        const char** name) {
+  constexpr bool F32 = E == Elem::kF32;
+  const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
+  const int64_t cus = compute_units();
+  const int64_t b16 = uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16);
+  const int64_t b32 = uk::ceil_div(rows, (int64_t)32) * uk::ceil_div(cols, (int64_t)32);
+  int st = -1;
+  if (b16 <= cus && k_bytes >= (RBC < 16 ? 64 : 256)) {
+    st = launch_thin<E, RBC, 1, 1, F32 ? 4 : 8, F32 ? 4 : 2, true>(p, false, stream);
+    if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
+    return st;
+  }
+  if constexpr (F32) {
+    if (k_bytes < (b128 || (RBC >= 16 && b32 > 2 * cus) ? 1024 : 256)) return -1;
+    if (b16 <= 3 * cus) {
+      st = launch_thin<E, RBC, 1, 1, 4, 4, true>(p, false, stream);
+      if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
+      return st;
+    }
+    const int64_t slots = uk::ceil_div(b128 ? workgroups(p, 128, 128) : workgroups(p, 64, 64), cus) * cus;
+    if (2 * b32 > (b128 ? 28 : 7) * slots) return -1;
+    // From four blocks a unit on two waves a block are enough.
+    st = b32 >= 4 * cus ? launch_thin<E, RBC, 2, 2, 2, 2, true>(p, false, stream)
+                        : launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
+  } else {
+    if (b32 > (RBC == 2 ? 1 : 2) * cus || k_bytes < 1024) return -1;
+    st = launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
+  }
+  if (st >= 0) *name = "mmt4d_mfma_32x32_ksplit";
+  return st;
 }
 
 // Variant choice for row-bytes class RBC:
@@ -555,9 +631,10 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     choice = 7;
   } else if (workgroups(p, 128, 128) >= 192) {
     choice = 2;
-  } else if (RBC >= 8 && ((int64_t)p.K1 << p.lrb) >= 8192) {
-    // Measured: with 8 KiB of K per row and more, the 64x64 blocks' operands
-    // outgrow the L2 and the K-split kernel's deeper queue of loads wins.
+  } else if (RBC >= 8 && ((int64_t)p.K1 << p.lrb) >= 6144) {
+    // Measured: with 6 KiB of K per row and more, the 64x64 blocks' operands
+    // outgrow the L2 and the K-split kernel's deeper queue of loads wins (f16 1000
+    // x 1000, 7.6 KB: 21.8 -> 17.1 us).
     choice = 6;
   } else {
     choice = 3;
@@ -802,6 +879,13 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     }
     choice = 2;
   }
+  // (With 24 KB of K and more the 64x64 blocks below split K over workgroups.)
+  const bool long_k = ((int64_t)p.K1 << p.lrb) >= 24576;
+  if (forced == 0 && (choice == 3 || (choice == 6 && (!long_k || E == Elem::kF32)) || (RBC < 8 && choice == 4) ||
+                      (choice == 2 && E == Elem::kF32))) {
+    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, stream, name);
+    if (st >= 0) return st;
+  }
   if (choice == 6) {
     // Few 64x64 blocks and a long K: the barrier-free kernel with a 64x64
     // block per workgroup, whose four waves split K.
@@ -812,8 +896,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       // 128 x 128 x 65536, four blocks: 177 -> 52 us; 256 x 256 x 32768: 80 ->
       // 35; 512 x 512 x 16384: 44 -> 27; with 8 KB of K per row, 384 x 384 x
       // 4096, it loses: 16 -> 20 us).
-      const bool long_k = ((int64_t)p.K1 << p.lrb) >= 24576;
-      int st = launch_thin<E, RBC, 4, 4, 4, 2>(p, false, stream, long_k, 32);
+      int st = launch_thin<E, RBC, 4, 4, 4, 2, true>(p, false, stream, long_k, 32);
       if (st >= 0) { *name = "mmt4d_mfma_64x64_ksplit"; return st; }
     }
     choice = 3;
@@ -823,9 +906,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   // (A generic lambda: its body is only instantiated for the row widths that call it.)
   auto thin_launch = [&](auto swapped_c, int64_t thin_rows, int64_t wide_cols) {
     const bool swapped = swapped_c;
-    if (thin_rows <= 16) return launch_thin_rows<E, RBC, 1>(p, swapped, wide_cols, stream);
-    if (thin_rows <= 32) return launch_thin_rows<E, RBC, 2>(p, swapped, wide_cols, stream);
-    return launch_thin_rows<E, RBC, 4>(p, swapped, wide_cols, stream);
+    return launch_thin_any<E, RBC>(p, swapped, thin_rows, wide_cols, stream);
   };
   if (choice == 5) {
     // N-thin (a few columns against many rows, e.g. the last column strip of
@@ -833,6 +914,9 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if constexpr (RBC >= 8) {
       int st = thin_launch(std::true_type{}, cols_n, rows_m);
       if (st >= 0) { *name = "mmt4d_mfma_thin_transposed"; return st; }
+      // (K ends inside a step)
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, stream, name);
+      if (st >= 0) return st;
     }
     choice = 3;
   }
@@ -840,6 +924,8 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if constexpr (RBC >= 8) {
       int st = thin_launch(std::false_type{}, rows_m, cols_n);
       if (st >= 0) { *name = "mmt4d_mfma_thin"; return st; }
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, stream, name);
+      if (st >= 0) return st;
     }
     // With 2-byte rows a 16-byte piece spans 8 rows and 32 rows do not fill a
     // loader block; that combination takes the 64x64 variant.

@@ -112,9 +112,8 @@ int launch_s8s4(const Problem& p, hipStream_t stream, const char** name) {
   }
   if (p.rb < 16) return -1;  // the thin kernel unpacks 16 nibbles per lane: tile rows of 16 and more
   const int64_t cols_n = std::min<int64_t>((int64_t)p.N1 * p.N0, p.out_cols);
-  const int st = rows_m <= 16   ? launch_thin_rows<Elem::kS8S4, 16, 1>(p, false, cols_n, stream)
-                 : rows_m <= 32 ? launch_thin_rows<Elem::kS8S4, 16, 2>(p, false, cols_n, stream)
-                                : launch_thin_rows<Elem::kS8S4, 16, 4>(p, false, cols_n, stream);
+  const int st = rows_m <= 64 ? launch_thin_any<Elem::kS8S4, 16>(p, false, rows_m, cols_n, stream)
+                              : launch_thin_rows<Elem::kS8S4, 16, 4>(p, false, cols_n, stream);
   if (st >= 0) *name = "mmt4d_mfma_thin_s8s4";
   return st;
 }

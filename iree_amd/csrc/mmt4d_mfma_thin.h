@@ -27,7 +27,9 @@
 // scales of a dequantizing store are applied column scale first. Row widths of 16
 // bytes and more load one 16-byte piece per operand; 8-byte rows load the two
 // 8-byte halves from two K-tiles (chunk g of a step holds K-tiles g and
-// g + 4). K must be a whole number of steps.
+// g + 4), 4- and 2-byte rows likewise from four and eight. A K that
+// ends inside a step (TAIL): the pieces beyond it are read from the operand's
+// first row instead and are zero for the MFMA.
 //
 // s8 x s4 -> s32 (Elem::kS8S4) runs here too. A lane loads 8 RHS bytes (16
 // nibbles, the same 16 K elements as its 16 LHS bytes) and turns them into two
@@ -47,12 +49,30 @@ namespace uk_mfma {
 
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef v2i v2i_g __attribute__((aligned(1)));  // as v4i_g: read from global memory at any address
+typedef int int_g __attribute__((aligned(1)));
+
+// 16, 8 and 4 bytes from any address, non-temporally if NT.
+template <bool NT>
+__device__ __forceinline__ v4i load16(const char* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const v4i_g*>(p));
+  else return *reinterpret_cast<const v4i_g*>(p);
+}
+template <bool NT>
+__device__ __forceinline__ v2i load8(const char* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const v2i_g*>(p));
+  else return *reinterpret_cast<const v2i_g*>(p);
+}
+template <bool NT>
+__device__ __forceinline__ int load4(const char* p) {
+  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const int_g*>(p));
+  else return *reinterpret_cast<const int_g*>(p);
+}
 
 // STREAMED: the wide operand (the kernel's RHS: weights) is loaded
 // non-temporally. For callers that say their weights come from HBM every time
 // (iree_uk_amd_set_streamed_weights): a layer's weights then pass through the
 // caches without displacing what is used again.
-template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false>
+template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false, bool TAIL = false>
 __global__ __launch_bounds__(KSPLIT * 64)
 void mmt4d_thin_kernel(Args a) {
   using TT = ElemTraits<E>;
@@ -62,10 +82,10 @@ void mmt4d_thin_kernel(Args a) {
   constexpr int HALVES = TT::kHalves;
   constexpr int NCH = 4 * HALVES;             // 16-byte chunks per row per step
   constexpr int KS = NCH * 16;                // bytes of K per row per step
-  constexpr int PIECES = RBC >= 16 ? 1 : 2;   // loads per 16-byte operand
+  constexpr int PIECES = RBC >= 16 ? 1 : 16 / RBC;   // loads per 16-byte operand
   constexpr bool S4 = E == Elem::kS8S4;       // 4-bit RHS: half the bytes per row
-  static_assert(RBC >= 8, "rows narrower than 8 bytes take the LDS kernels");
-  static_assert(!S4 || RBC >= 16, "4-bit RHS: LHS rows of at least 16 bytes");
+  static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
+  static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
 
   __shared__ v4i partial[KSPLIT > 1 ? KSPLIT - 1 : 1][TM * TN][64];
 
@@ -112,7 +132,7 @@ void mmt4d_thin_kernel(Args a) {
           const uint32_t kb = g * piece_bytes;
           o = (kb >> lrb) * kt_bytes + (x0 << lrb) + (kb & ((1u << lrb) - 1));
         } else {
-          o = (g + (uint32_t)t * NCH) * kt_bytes + x0 * 8;
+          o = (g + (uint32_t)t * NCH) * kt_bytes + x0 * RBC;
         }
         off[h][t] = ok ? pl * (uint32_t)stride + o : 0u;
       }
@@ -127,24 +147,31 @@ void mmt4d_thin_kernel(Args a) {
     operand_offsets(offb[tn], bn * TN + tn, a.N0, a.N1, a.out_cols, pb0, a.rhs_stride, kt_n, lrb_b,
                     S4 ? 8 : 16);
 
-  auto load_operand = [&](const char* base, const uint32_t (&off)[PIECES], uint32_t adv) {
+  // Whether piece t of chunk (h, q) of K step s lies inside K.
+  auto in_k = [&](uint32_t s, int h, int t) {
     if constexpr (RBC >= 16) {
-      return *reinterpret_cast<const v4i_g*>(base + (off[0] + adv));
+      return s * KS + ((uint32_t)h * 4 + q) * 16 < (uint32_t)a.K1 << lrb;
     } else {
-      const v2i lo = *reinterpret_cast<const v2i_g*>(base + (off[0] + adv));
-      const v2i hi = *reinterpret_cast<const v2i_g*>(base + (off[1] + adv));
-      return v4i{lo[0], lo[1], hi[0], hi[1]};
+      return s * kts_per_step + (uint32_t)h * 4 + q + (uint32_t)t * NCH < (uint32_t)a.K1;
     }
   };
-  auto load_wide_operand = [&](const char* base, const uint32_t (&off)[PIECES], uint32_t adv) {
-    if constexpr (!STREAMED) {
-      return load_operand(base, off, adv);
-    } else if constexpr (RBC >= 16) {
-      return __builtin_nontemporal_load(reinterpret_cast<const v4i_g*>(base + (off[0] + adv)));
-    } else {
-      const v2i lo = __builtin_nontemporal_load(reinterpret_cast<const v2i_g*>(base + (off[0] + adv)));
-      const v2i hi = __builtin_nontemporal_load(reinterpret_cast<const v2i_g*>(base + (off[1] + adv)));
+  auto load_operand = [&](auto nontemporal, const char* base, const uint32_t (&off)[PIECES], uint32_t adv,
+                          uint32_t s, int h) {
+    auto at = [&](int t) { return base + (!TAIL || in_k(s, h, t) ? off[t] + adv : 0u); };
+    constexpr bool NT = decltype(nontemporal)::value;
+    if constexpr (RBC >= 16) {
+      return load16<NT>(at(0));
+    } else if constexpr (RBC == 8) {
+      const v2i lo = load8<NT>(at(0)), hi = load8<NT>(at(1));
       return v4i{lo[0], lo[1], hi[0], hi[1]};
+    } else if constexpr (RBC == 4) {
+      return v4i{load4<NT>(at(0)), load4<NT>(at(1)), load4<NT>(at(2)), load4<NT>(at(3))};
+    } else {
+      typedef short short8 __attribute__((ext_vector_type(8)));
+      short8 v;
+#pragma unroll
+      for (int t = 0; t < 8; ++t) v[t] = *reinterpret_cast<const short*>(at(t));
+      return __builtin_bit_cast(v4i, v);
     }
   };
   using BFrag = typename std::conditional<S4, v2i, v4i>::type;
@@ -158,17 +185,16 @@ void mmt4d_thin_kernel(Args a) {
 #pragma unroll
       for (int h = 0; h < HALVES; ++h) {
         if constexpr (S4) {
-          const v2i_g* pb = reinterpret_cast<const v2i_g*>(base_b + (offb[tn][h][0] + s * sstep_b));
-          if constexpr (STREAMED) fb[d][tn][h] = __builtin_nontemporal_load(pb);
-          else fb[d][tn][h] = *pb;
+          fb[d][tn][h] = load8<STREAMED>(base_b + (offb[tn][h][0] + s * sstep_b));
         } else {
-          fb[d][tn][h] = load_wide_operand(base_b, offb[tn][h], s * sstep_b);
+          fb[d][tn][h] = load_operand(std::bool_constant<STREAMED>{}, base_b, offb[tn][h], s * sstep_b, s, h);
         }
       }
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-      for (int h = 0; h < HALVES; ++h) fa[d][tm][h] = load_operand(base_a, offa[tm][h], s * sstep_a);
+      for (int h = 0; h < HALVES; ++h)
+        fa[d][tm][h] = load_operand(std::false_type{}, base_a, offa[tm][h], s * sstep_a, s, h);
   };
 
   // ---- output addressing (see for_each_output in mmt4d_mfma_kernel.h) ------
@@ -266,7 +292,30 @@ void mmt4d_thin_kernel(Args a) {
       }
     }
   }
-  auto compute = [&](int d) {
+  auto compute = [&](int d, int i) {
+    if constexpr (TAIL) {
+      // The step K ends in: nothing beyond it reaches the sums (a zero in both
+      // operands: what was read instead may be an infinity).
+      const uint32_t s = step_begin + (uint32_t)(wave + i * KSPLIT);
+      if (s == (uint32_t)a.steps - 1) {
+        auto cut = [&](v4i& f, int h) {
+#pragma unroll
+          for (int t = 0; t < PIECES; ++t) {
+            const bool in = in_k(s, h, t);
+#pragma unroll
+            for (int w = 0; w < 4 / PIECES; ++w) f[t * (4 / PIECES) + w] = in ? f[t * (4 / PIECES) + w] : 0;
+            if constexpr (PIECES == 8) f[t / 2] = in ? f[t / 2] : f[t / 2] & (t & 1 ? 0xFFFF : (int)0xFFFF0000);
+          }
+        };
+#pragma unroll
+        for (int h = 0; h < HALVES; ++h) {
+#pragma unroll
+          for (int tm = 0; tm < TM; ++tm) cut(fa[d][tm][h], h);
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn) cut(fb[d][tn][h], h);
+        }
+      }
+    }
     if constexpr (S4) {
       // LHS: even K bytes, then odd K bytes; RHS: low nibbles, then high ones.
       v4i ea[TM], eb[TN];
@@ -301,7 +350,7 @@ void mmt4d_thin_kernel(Args a) {
   for (; i + 2 * D <= my_steps; i += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      compute(d);
+      compute(d, i + d);
       load_step(d, i + d + D);
     }
   }
@@ -309,13 +358,13 @@ void mmt4d_thin_kernel(Args a) {
 #pragma unroll
   for (int d = 0; d < D; ++d) {
     if (i + d < my_steps) {
-      compute(d);
+      compute(d, i + d);
       if (i + d + D < my_steps) load_step(d, i + d + D);
     }
   }
 #pragma unroll
   for (int d = 0; d < D; ++d)
-    if (i + D + d < my_steps) compute(d);
+    if (i + D + d < my_steps) compute(d, i + D + d);
 
   // ---- meet the partial sums ---------------------------------------------------
   if constexpr (KSPLIT > 1) {
