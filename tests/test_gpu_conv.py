@@ -168,3 +168,89 @@ def test_conv_mfma_tiles(gpu, oracle, shape, tile):
     for ci, c in enumerate(C.cases(seed=51, tiles=[(16, shape[9])], shapes=[shape[:9]])):
         _check(lib, torch, oracle, c, 900 + ci, host=False, exact=True, mfma=True)
         assert lib.last_kernel_name() == "conv_nchwc_mfma_" + tile
+
+
+# The same for sums of more than ten steps: tiles of a wave, and tiles whose steps four
+# waves, or those of two and four workgroups, divide unevenly.
+LONG_SHAPES = [
+    ((40, 9, 3, 22, 2, 3, 1, 1, 1, 32), "direct_1x4"),  # 12 steps
+    ((40, 1, 15, 27, 3, 2, 2, 1, 1, 16), "direct_2x2"),
+    ((40, 3, 29, 14, 2, 3, 1, 1, 1, 32), "direct_2x4"),
+    ((1, 1, 1, 2, 5, 3, 1, 1, 1, 16), "split_1x1"),  # 15 steps
+    ((5, 13, 1, 1, 5, 7, 7, 1, 1, 16), "split_1x1"),  # 245 steps, two workgroups a tile
+    ((3, 1, 1, 1, 5, 5, 5, 2, 1, 16), "split_1x1"),  # 125 steps, four
+    ((40, 9, 1, 1, 2, 3, 3, 1, 2, 16), "split_1x4"),
+    ((16, 18, 1, 1, 3, 5, 5, 1, 1, 32), "split_1x4"),  # 150 steps, two
+    ((40, 1, 8, 13, 2, 1, 3, 1, 1, 32), "split_2x2"),
+]
+
+
+@pytest.mark.parametrize("shape,tile", LONG_SHAPES, ids=lambda s: s if isinstance(s, str) else "x".join(map(str, s)))
+def test_conv_long_sums(gpu, oracle, shape, tile):
+    lib, torch = gpu
+    lib.set_pointer_mode(uk.POINTER_MODE_AUTO)
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    for ci, c in enumerate(C.cases(seed=57, tiles=[(16, shape[9])], shapes=[shape[:9]])):
+        for run in range(2):   # the second call finds the counters of the first one's workgroups
+            _check(lib, torch, oracle, c, 960 + ci + 10 * run, host=False, exact=True, mfma=True)
+            assert lib.last_kernel_name() == "conv_nchwc_mfma_" + tile
+
+
+@pytest.mark.parametrize("flip", ["h", "ic", "oc", "fh"])
+@pytest.mark.parametrize("dims", [(2, 3, 9, 11, 3, 2, 2), (40, 5, 7, 9, 2, 3, 3)])   # a split and a direct kernel
+def test_conv_negative_strides(gpu, flip, dims):
+    """A dimension stored back to front and walked with a negative stride: the
+    result of the layer on the buffer the right way round, bit for bit."""
+    lib, torch = gpu
+    lib.set_pointer_mode(uk.POINTER_MODE_AUTO)
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    N, OC, OH, OW, IC, FH, FW = dims
+    H, W = OH + FH - 1, OW + FW - 1
+    g = torch.Generator(device="cuda"); g.manual_seed(9)
+    x = torch.randn((N, IC, H, W * 16), generator=g, device="cuda")
+    f = torch.randn((OC, IC, FH, FW * 256), generator=g, device="cuda")
+    results = []
+    for turned in (False, True):
+        xs, fs = [IC * H * W * 16, H * W * 16, W * 16], [IC * FH * FW * 256, FH * FW * 256, FW * 256]
+        xb, fb, x_off, f_off = x, f, 0, 0
+        if turned and flip in ("h", "ic"):
+            d = 2 if flip == "h" else 1
+            xb = x.flip(d).contiguous()
+            x_off, xs[d] = (x.shape[d] - 1) * xs[d], -xs[d]
+        if turned and flip in ("oc", "fh"):
+            d = 2 if flip == "fh" else 0
+            fb = f.flip(d).contiguous()
+            f_off, fs[d] = (f.shape[d] - 1) * fs[d], -fs[d]
+        y = torch.zeros((N, OC, OH, OW * 16), device="cuda")
+        lib.conv_nchwc(xb.data_ptr(), x_off, *xs, fb.data_ptr(), f_off, *fs, y.data_ptr(), 0, OC * OH * OW * 16,
+                       OH * OW * 16, OW * 16, N, OC, OH, OW, IC, FH, FW, 16, 16, 1, 1, C.CONV_TYPE_F32F32F32)
+        lib.synchronize()
+        assert lib.last_kernel_name().startswith("conv_nchwc_mfma_")
+        results.append(y)
+    assert bool(results[0].any()) and torch.equal(results[0], results[1])
+
+
+def test_conv_image_beyond_32_bit_offsets(gpu):
+    """Planes of input channels 2 GiB apart: more than the direct kernel's 32-bit
+    offsets reach, the LDS kernel serves the call."""
+    lib, torch = gpu
+    lib.set_pointer_mode(uk.POINTER_MODE_AUTO)
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    OC, OH, OW, IC, F = 3, 6, 10, 2, 3
+    H, W, plane = OH + F - 1, OW + F - 1, 1 << 29
+    g = torch.Generator(device="cuda"); g.manual_seed(11)
+    x = torch.randint(-3, 4, (IC, H * W * 16), generator=g, device="cuda").float()
+    f = torch.randint(-3, 4, (OC * IC * F * F * 256,), generator=g, device="cuda").float()
+    far = torch.empty(plane + H * W * 16, device="cuda")
+    far[:H * W * 16], far[plane:] = x[0], x[1]
+    results, names = [], []
+    for buf, sic in ((x, H * W * 16), (far, plane)):
+        y = torch.zeros(OC * OH * OW * 16, device="cuda")
+        lib.conv_nchwc(buf.data_ptr(), 0, IC * sic, sic, W * 16, f.data_ptr(), 0, IC * F * F * 256, F * F * 256, F * 256,
+                       y.data_ptr(), 0, OC * OH * OW * 16, OH * OW * 16, OW * 16, 1, OC, OH, OW, IC, F, F, 16, 16, 1, 1,
+                       C.CONV_TYPE_F32F32F32)
+        lib.synchronize()
+        results.append(y)
+        names.append(lib.last_kernel_name())
+    assert "lds" not in names[0] and "lds" in names[1], names
+    assert bool(results[0].any()) and torch.equal(results[0], results[1])
