@@ -40,10 +40,10 @@
 //      and want as many bytes in flight per workgroup as registers allow.
 //   5  both operands brought into LDS by LDS-direct global loads
 //      (global_load_lds, 16 bytes per lane: one instruction moves one 1 KiB
-//      fragment and touches no register), kStages5 stages deep; the eight
+//      fragment and touches no register), stages5() stages deep; the eight
 //      waves form two groups of four (one wave of each group per SIMD) that
 //      alternate, half a step apart, between a memory phase (fragment reads,
-//      issue of the loads kStages5 - 1 steps ahead) and a compute phase (all MFMAs of
+//      issue of the loads stages5() - 1 steps ahead) and a compute phase (all MFMAs of
 //      the step back to back), with a workgroup barrier between phases: while
 //      one wave of a SIMD feeds the matrix pipe, the other one's memory
 //      instructions issue beside it instead of in between its MFMAs (row
@@ -232,15 +232,18 @@ __device__ __forceinline__ void wait_vmem_in_flight() {
 }
 // Waits for the wave's LDS reads (and scalar loads), not for vector memory.
 __device__ __forceinline__ void wait_lds_reads() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-// LDS stages of PIPE 5.
-constexpr int kStages5 = 4;
+// LDS stages of PIPE 5: twice as many where K is in slices, whose blocks have a compute
+// unit to themselves and weights that come from HBM (us, in 4 / 8 stages: f8 512 x 4096 x
+// 8192 in two slices 37.0 / 31.8, bf16 100 x 14336 x 4096 37.6 / 36.3).
+template <bool SLICED>
+constexpr int stages5() { return SLICED ? 8 : 4; }
 // Half-step slots of PIPE 5's ring for lane operands of two 16-byte pieces. The
 // 16-bit integers finish a step in half the time of the 8-bit floats (same
 // instruction count, instructions half as long), so the same distance in time
 // between a load's issue and its use takes a ring twice as deep, where it fits.
-template <Elem E, int BM, int BN>
+template <Elem E, int BM, int BN, bool SLICED = false>
 constexpr int ring_slots() {
-  return (E == Elem::kS16 && 9 * (BM + BN) * 64 <= 160 * 1024) ? 9 : 5;
+  return ((E == Elem::kS16 || SLICED) && 9 * (BM + BN) * 64 <= 160 * 1024) ? 9 : 5;
 }
 // f(integral_constant<int, I>) for I = BEGIN .. END - 1.
 template <int BEGIN, int END, typename F>
@@ -299,7 +302,9 @@ struct Args {
   uint32_t col_scale_first;
   // mmt4d_mfma_persistent.h only: log2 of M0 and N0 (powers of two there).
   int32_t lm0, ln0;
-  // mmt4d_mfma_thin.h only: K split over `kslices` workgroups per output block
+  // K split over `kslices` workgroups per output block in SLICED instances of
+  // mmt4d_mfma_kernel.h (slice i stores its sums M1 row panels after slice i - 1's)
+  // and in mmt4d_mfma_thin.h, where the rest of this comment holds
   // (1 = none). Workgroup b works on block b / kslices, K slice b % kslices;
   // the slices' partial accumulators meet in `ws_partials` (kslices x 16 bytes
   // per lane and accumulator block, per output block) and the workgroup that
@@ -347,13 +352,19 @@ __device__ __forceinline__ void regroup(const v4i* in, v4i* out) {
 // Workgroup -> output block. Consecutive workgroup ids go round-robin to the
 // 8 XCDs, each with its own L2; give every XCD a contiguous share of the
 // blocks and walk that share in bands of `band` block rows so that the
-// workgroups resident on one XCD at a time reuse each other's panels.
+// workgroups resident on one XCD at a time reuse each other's panels. With K in
+// `slices`, the blocks of one slice follow those of the one before.
 __device__ __forceinline__ void block_of_workgroup(uint32_t wg, const Args& a,
-                                                   int* bm, int* bn) {
-  const uint32_t total = (uint32_t)a.grid_m * (uint32_t)a.grid_n;
+                                                   int* bm, int* bn, uint32_t slices = 1,
+                                                   uint32_t* slice = nullptr) {
+  const uint32_t blocks = (uint32_t)a.grid_m * (uint32_t)a.grid_n, total = blocks * slices;
   const uint32_t per_xcd = (total + 7) / 8;
   uint32_t id = (wg & 7) * per_xcd + (wg >> 3);
   if (id >= total || (total & 7)) id = wg;  // uneven split: plain order
+  if (slice) {
+    *slice = id / blocks;
+    id -= *slice * blocks;
+  }
   const uint32_t band_blocks = a.band * (uint32_t)a.grid_n;
   const uint32_t b = id / band_blocks;
   const uint32_t in_band = id - b * band_blocks;
@@ -368,8 +379,10 @@ __device__ __forceinline__ void block_of_workgroup(uint32_t wg, const Args& a,
 // RBC: 16 = row bytes >= 16 (direct), 8/4/2 = regrouping loaders. TAIL (PIPE 3
 // and 5): K ends inside the last step. An instance of its own, because a test of
 // it beside every load costs the others (f16 2000 x 3000 x 1024: 17.3 -> 21.0
-// us, 4096 x 2048 x 2048 34.6 -> 37.1).
-template <Elem E, int RBC, int TM, int TN, int WGM, int WGN, int NKK, int PIPE, bool TAIL = false>
+// us, 4096 x 2048 x 2048 34.6 -> 37.1). SLICED (K in whole steps): each workgroup
+// computes one of a.kslices parts of K of its block.
+template <Elem E, int RBC, int TM, int TN, int WGM, int WGN, int NKK, int PIPE, bool TAIL = false,
+          bool SLICED = false>
 __global__ __launch_bounds__(WGM* WGN * 64)
 void mmt4d_mfma_kernel(Args a) {
   using TT = ElemTraits<E>;
@@ -405,11 +418,24 @@ void mmt4d_mfma_kernel(Args a) {
   const int wm = wave / WGN;
   const int wn = wave - wm * WGN;
   int wg_m, wg_n;
-  block_of_workgroup(blockIdx.x, a, &wg_m, &wg_n);
-  const int pm0 = wg_m * a.bpm;  // first LHS panel of this workgroup
-  const int pn0 = wg_n * a.bpn;
   const int lrb = a.lrb;
   const int kts_per_step = KS >> lrb;
+  if constexpr (SLICED) {
+    static_assert(!TAIL, "K in whole steps");
+    uint32_t slice;
+    block_of_workgroup(blockIdx.x, a, &wg_m, &wg_n, a.kslices, &slice);
+    const uint32_t steps = (uint32_t)a.steps, s0 = (uint32_t)((uint64_t)slice * steps / a.kslices);
+    const int64_t kt = (int64_t)s0 * kts_per_step;
+    a.steps = (int32_t)((uint64_t)(slice + 1) * steps / a.kslices) - (int32_t)s0;
+    a.K1 = a.steps * kts_per_step;
+    a.lhs += kt * a.M0 << lrb;
+    a.rhs += kt * a.N0 << lrb;
+    a.out += (int64_t)slice * a.M1 * a.out_stride;
+  } else {
+    block_of_workgroup(blockIdx.x, a, &wg_m, &wg_n);
+  }
+  const int pm0 = wg_m * a.bpm;  // first LHS panel of this workgroup
+  const int pn0 = wg_n * a.bpn;
   const uint32_t q = lane >> 4, r = lane & 15;
 
   // ---- loader set-up: per-unit constants --------------------------------
@@ -506,6 +532,16 @@ void mmt4d_mfma_kernel(Args a) {
   // contiguously). `vec_out` is 0 when that does not hold or the output is not
   // 16-byte aligned; elements then move one by one.
   Acc acc[TM][TN];
+  // Slices of a float product sum even and odd steps apart: two slices then add no
+  // more terms one after the other than four waves that share K do.
+  constexpr bool TWO_SUMS = SLICED && !std::is_same<Acc, v4i>::value;
+  Acc acc_odd[TWO_SUMS ? TM : 1][TWO_SUMS ? TN : 1];
+  if constexpr (TWO_SUMS) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) acc_odd[tm][tn] = Acc{0, 0, 0, 0};
+  }
   // Output element (row, col) of the workgroup's block, with pl = row / M0,
   // m0 = row % M0, pc = col / N0, n0 = col % N0, lives at
   //   out + (pm0 + pl) * out_stride + m0 * out_sm0 + (pn0 + pc) * out_spn + n0 * elem,
@@ -678,11 +714,15 @@ void mmt4d_mfma_kernel(Args a) {
   // pairs: s8 8192^3 374.8 / 378.9 / 376.4 -> 371.7 / 371.7 / 375.2 us,
   // 16x16x2 382.0 / 382.5 / 384.5 -> 378.5 / 379.4 / 382.2, f16 4096^3 91.2 /
   // 91.3 / 91.3 -> 90.8 / 90.7 / 90.6, bf16 8192^3 unchanged.
-  auto mfmas_by_columns = [&](const v4i (&fa)[TM][HALVES], const v4i (&fb)[TN][HALVES]) {
+  // `odd`: whether the step has an odd number (as a constant).
+  auto mfmas_by_columns = [&](const v4i (&fa)[TM][HALVES], const v4i (&fb)[TN][HALVES], auto odd) {
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) acc[tm][tn] = TT::mfma(fb[tn], fa[tm], acc[tm][tn]);
+      for (int tm = 0; tm < TM; ++tm) {
+        if constexpr (TWO_SUMS && decltype(odd)::value) acc_odd[tm][tn] = TT::mfma(fb[tn], fa[tm], acc_odd[tm][tn]);
+        else acc[tm][tn] = TT::mfma(fb[tn], fa[tm], acc[tm][tn]);
+      }
   };
   const int last = a.steps - 1;
   const bool has_tail = a.tail != 0;
@@ -1135,7 +1175,7 @@ void mmt4d_mfma_kernel(Args a) {
     // step, i.e. two 64-byte halves) do not leave room for four stages of whole
     // steps: their LDS is a ring of half-step slots instead (HALVES == 2
     // below).
-    constexpr int NS = kStages5;
+    constexpr int NS = stages5<SLICED>();
     constexpr int IW = HALVES == 2 ? 4 : NW;          // waves that share one issue of loads
     constexpr int DCH = HALVES == 2 ? 1 : NCHB;       // 64-byte chunks of K per issue
     constexpr int DB = (BM + BN) / 16 * DCH;          // 1 KiB blocks per issue
@@ -1253,7 +1293,7 @@ void mmt4d_mfma_kernel(Args a) {
       // of its compute phase (D - 2 issues), group 1 at the end of its memory
       // phase (D - 1 issues).
       static_assert(NKK == 1, "one MFMA K-group per step");
-      constexpr int RING = ring_slots<E, BM, BN>();
+      constexpr int RING = ring_slots<E, BM, BN, SLICED>();
       constexpr int D = (RING - 1) / 2;
       constexpr uint32_t SLOT = (BM + BN) * 64;
       constexpr uint32_t IMG_B = BM * 64;
@@ -1463,7 +1503,7 @@ void mmt4d_mfma_kernel(Args a) {
       };
       // `first`: the slot of the step's first half, 2 s % RING, as a compile-time
       // constant or (TAIL) a running number.
-      auto step_body = [&](int s, auto first) __attribute__((always_inline)) {
+      auto step_body = [&](int s, auto first, auto odd) __attribute__((always_inline)) {
         auto slot_at = [&](int ahead) { return (uint32_t)(((int)first + ahead) % RING) * SLOT; };
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
@@ -1484,7 +1524,7 @@ void mmt4d_mfma_kernel(Args a) {
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(3);
-        mfmas_by_columns(fa, fb);
+        mfmas_by_columns(fa, fb, odd);
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
         if (group == 0) wait_vmem_in_flight<DU*(D - 2)>();   // the second half of step s + 1 has landed
@@ -1493,7 +1533,8 @@ void mmt4d_mfma_kernel(Args a) {
       };
       auto step = [&](int s, auto phase_c) __attribute__((always_inline)) {
         if constexpr (S16) step_body16(s, phase_c);
-        else step_body(s, std::integral_constant<int, 2 * decltype(phase_c)::value % RING>{});
+        else step_body(s, std::integral_constant<int, 2 * decltype(phase_c)::value % RING>{},
+                       std::bool_constant<decltype(phase_c)::value % 2 != 0>{});
       };
       if constexpr (TAIL && !S16) {
         // Rolled: the test of every load against the end of K, in every copy of
@@ -1501,7 +1542,7 @@ void mmt4d_mfma_kernel(Args a) {
         // 4096 x 4001: 256 us against 55, which is also what K = 4096 takes unrolled).
         int first = 0;
         for (int s = 0; s < a.steps; ++s) {
-          step_body(s, first);
+          step_body(s, first, std::false_type{});
           first = first + 2 >= RING ? first + 2 - RING : first + 2;
         }
       } else {
@@ -1556,7 +1597,7 @@ void mmt4d_mfma_kernel(Args a) {
       v4i fa[NKK][TM][HALVES], fb[NKK][TN][HALVES];
       // `stage`: s % NS, as a compile-time constant or (TAIL, the last steps) a
       // running number.
-      auto step_body = [&](int s, auto stage, bool may_end = true) {
+      auto step_body = [&](int s, auto stage, auto odd, bool may_end = true) {
         const uint32_t st = (uint32_t)(int)stage * STAGE, st_load = (uint32_t)(((int)stage + NS - 1) % NS) * STAGE;
 #pragma unroll
         for (int kk = 0; kk < NKK; ++kk) {
@@ -1575,28 +1616,30 @@ void mmt4d_mfma_kernel(Args a) {
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_setprio(3);
 #pragma unroll
-        for (int kk = 0; kk < NKK; ++kk) mfmas_by_columns(fa[kk], fb[kk]);
+        for (int kk = 0; kk < NKK; ++kk) mfmas_by_columns(fa[kk], fb[kk], odd);
         __builtin_amdgcn_s_setprio(0);
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
       };
-      static_assert(NS == 4, "the loop below is unrolled by the stage count");
+      auto step = [&](int s, auto p, bool may_end) {
+        step_body(s, p, std::bool_constant<decltype(p)::value % 2 != 0>{}, may_end);
+      };
       int s = 0;
       if constexpr (TAIL) {
         // Unrolled as long as the loads stay before the last step, then rolled
         // with the test of every load against the end of K (rolled all the way:
         // f16 4095 x 2049 x 2049 51.2 -> 58.8 us; tested in every copy: spilled
         // registers in 256x256 blocks).
-        for (; s + 3 + NS - 1 < last; s += 4)
-          static_for<0, 4>([&](auto p) { step_body(s + decltype(p)::value, p, false); });
-        for (; s < a.steps; ++s) step_body(s, s & (NS - 1));
+        for (; s + 2 * NS - 2 < last; s += NS)
+          static_for<0, NS>([&](auto p) { step(s + decltype(p)::value, p, false); });
+        for (; s < a.steps; ++s) step_body(s, s & (NS - 1), std::false_type{});
       } else {
-        for (; s + 4 <= a.steps; s += 4)
-          static_for<0, 4>([&](auto p) { step_body(s + decltype(p)::value, p); });
-        if (s < a.steps) step_body(s, std::integral_constant<int, 0>{});
-        if (s + 1 < a.steps) step_body(s + 1, std::integral_constant<int, 1>{});
-        if (s + 2 < a.steps) step_body(s + 2, std::integral_constant<int, 2>{});
+        for (; s + NS <= a.steps; s += NS)
+          static_for<0, NS>([&](auto p) { step(s + decltype(p)::value, p, true); });
+        static_for<0, NS - 1>([&](auto p) {
+          if (s + decltype(p)::value < a.steps) step(s + decltype(p)::value, p, true);
+        });
       }
     }
     // (the 16-bit integers have done both already, before their exchange through LDS)
@@ -1604,6 +1647,12 @@ void mmt4d_mfma_kernel(Args a) {
     // No LDS-direct load may still be on its way when the workgroup ends (its
     // LDS goes to the next workgroup on the CU).
     wait_vmem_in_flight<0>();
+  }
+  if constexpr (TWO_SUMS) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) acc[tm][tn] += acc_odd[tm][tn];
   }
   // ---- epilogue -----------------------------------------------------------
   if constexpr (OB == 4) {
@@ -1676,7 +1725,7 @@ void mmt4d_mfma_kernel(Args a) {
   }
 }
 
-template <Elem E, int TM, int TN, int WGM, int WGN, int NKK, int PIPE>
+template <Elem E, int TM, int TN, int WGM, int WGN, int NKK, int PIPE, bool SLICED = false>
 struct Shape {
   static constexpr int NCH = NKK * ElemTraits<E>::kHalves * 4;
   static constexpr int KS = NCH * 16;
@@ -1684,8 +1733,8 @@ struct Shape {
   static constexpr int BN = WGN * TN * 16;
   static constexpr size_t kLdsBytes =
       (PIPE == 5 && ElemTraits<E>::kHalves == 2)
-          ? ring_slots<E, BM, BN>() * (size_t)(BM + BN) * 64   // a ring of half-step slots
-          : (PIPE == 5 ? kStages5 : PIPE == 0 || PIPE == 4 ? 2 : 3) *
+          ? ring_slots<E, BM, BN, SLICED>() * (size_t)(BM + BN) * 64   // a ring of half-step slots
+          : (PIPE == 5 ? stages5<SLICED>() : PIPE == 0 || PIPE == 4 ? 2 : 3) *
                 (size_t)(PIPE == 2 || PIPE == 3 ? BM : BM + BN) * KS;
 };
 

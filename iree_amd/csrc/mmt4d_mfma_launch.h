@@ -8,10 +8,12 @@
 
 #include <algorithm>
 #include <climits>
+#include <cmath>
 
 #include "mmt4d_mfma_kernel.h"
 #include "mmt4d_mfma_narrow.h"
 #include "mmt4d_mfma_persistent.h"
+#include "mmt4d_mfma_sum.h"
 #include "mmt4d_mfma_thin.h"
 #include "uk_device_common.h"
 #include "uk_hip_abi.h"
@@ -61,11 +63,12 @@ constexpr bool has_tail_instance() {
 }
 
 // Launches one kernel variant over K-tiles [kt_begin, kt_begin + kt_count).
-// Returns a HIP status, or -1 if the variant cannot serve the shape.
-template <Elem E, int RBC, int TM, int TN, int WGM, int WGN, int NKK, int PIPE>
+// Returns a HIP status, or -1 if the variant cannot serve the shape. SLICED: all
+// of K in `kslices` parts, each into a result of its own (see the kernel).
+template <Elem E, int RBC, int TM, int TN, int WGM, int WGN, int NKK, int PIPE, bool SLICED = false>
 int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate,
-                   hipStream_t stream) {
-  using SH = Shape<E, TM, TN, WGM, WGN, NKK, PIPE>;
+                   hipStream_t stream, int kslices = 1) {
+  using SH = Shape<E, TM, TN, WGM, WGN, NKK, PIPE, SLICED>;
   constexpr int R = RBC >= 16 ? 1 : 16 / RBC;
   if (SH::kLdsBytes > 160 * 1024) return -1;          // more LDS than a compute unit has
   if (p.rb > SH::KS) return -1;                       // a tile row must fit one step
@@ -89,14 +92,15 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
   a.bpm = SH::BM / p.M0;
   a.bpn = SH::BN / p.N0;
   const int64_t grid_m = uk::ceil_div(p.M1, a.bpm), grid_n = uk::ceil_div(p.N1, a.bpn);
-  if (grid_m * grid_n >= (1ll << 31)) return -1;
+  if (grid_m * grid_n * kslices >= (1ll << 31)) return -1;
   a.grid_m = (int32_t)grid_m;
   a.grid_n = (int32_t)grid_n;
+  a.kslices = (uint32_t)kslices;
   const int64_t k_bytes = (int64_t)kt_count << p.lrb;
   a.steps = (int32_t)uk::ceil_div(k_bytes, SH::KS);
   if (a.steps < 1) a.steps = 1;
   a.tail = (k_bytes % SH::KS) != 0;
-  constexpr bool kTail = has_tail_instance<E, RBC, TM, TN, WGM, WGN, PIPE>();
+  constexpr bool kTail = !SLICED && has_tail_instance<E, RBC, TM, TN, WGM, WGN, PIPE>();
   if (PIPE != 0 && PIPE != 4 && ((a.tail && !kTail) || kt_count == 0)) return -1;
   a.accumulate = accumulate;
   // A launch that starts K reads the caller's accumulators; a later one
@@ -145,7 +149,7 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
     return -1;
   }
   auto go = [&](auto tail_c) {
-    auto kernel = mmt4d_mfma_kernel<E, RBC, TM, TN, WGM, WGN, NKK, PIPE, decltype(tail_c)::value>;
+    auto kernel = mmt4d_mfma_kernel<E, RBC, TM, TN, WGM, WGN, NKK, PIPE, decltype(tail_c)::value, SLICED>;
     if (SH::kLdsBytes > 64 * 1024) {
       // Raising the dynamic LDS limit is a per-function setting; do it once.
       static hipError_t attr = hipFuncSetAttribute(
@@ -153,7 +157,7 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
           (int)SH::kLdsBytes);
       if (attr != hipSuccess) return (int)attr;
     }
-    uk::launch(2, kernel, dim3((uint32_t)(grid_m * grid_n)), dim3(WGM * WGN * 64),
+    uk::launch(2, kernel, dim3((uint32_t)(grid_m * grid_n * kslices)), dim3(WGM * WGN * 64),
                SH::kLdsBytes, stream, a);
     return (int)hipGetLastError();
   };
@@ -504,6 +508,65 @@ int launch_thin_any(const Problem& p, bool swapped, int64_t thin_rows, int64_t w
 // scalar kernel on top of it.
 inline int finish_k(int st) { return st < 0 ? (int)hipErrorUnknown : st; }
 
+// Few 128x128 blocks and a long K: K in slices of the LDS-direct pipeline, each
+// slice's sums as a row-major matrix in the K split's workspace, and a second launch
+// that adds them up (mmt4d_mfma_sum.h). Returns a HIP status, or -1 where K is no
+// whole number of steps, `slices` are too many for it, or there is no workspace (a
+// stream under capture, iree_uk_amd_mmt4d_no_alloc with a large result).
+template <Elem E, int RBC>
+int launch_slices(const Problem& p, int slices, hipStream_t stream) {
+  // 16-bit results: the sums of the slices are 32-bit floats like those of a block.
+  constexpr Elem P = E == Elem::kF16F16 ? Elem::kF16 : E == Elem::kBF16BF16 ? Elem::kBF16 : E;
+  using Out = typename ElemTraits<E>::Out;
+  constexpr int KS = 64 * ElemTraits<E>::kHalves;
+  const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
+  if (p.out_rows <= 0 || p.out_cols <= 0) return 0;
+  if (k_bytes % KS || slices < 2 || k_bytes / KS < 16 * slices) return -1;
+  const int64_t rows = (int64_t)p.M1 * p.M0, cols = (int64_t)p.N1 * p.N0;
+  if (p.out_sm0 >= (1ll << 32) || p.out_spn >= (1ll << 32) || p.acc_sm0 >= (1ll << 32) ||
+      p.acc_spn >= (1ll << 32) || rows * cols * slices >= (1ll << 26)) {
+    return -1;
+  }
+  KSplitWorkspace ws{};
+  const int got = acquire_ksplit_workspace((size_t)(slices * rows * cols) * 4, 1, stream, &ws);
+  if (got != 0) return got > 1 ? got : -1;
+  Problem q = p;
+  q.out = ws.partials;
+  q.out_stride = p.M0 * cols * 4;
+  q.out_sm0 = cols * 4;
+  q.out_spn = p.N0 * 4;
+  q.acc = q.out; q.acc_stride = q.out_stride; q.acc_sm0 = q.out_sm0; q.acc_spn = q.out_spn;
+  q.accumulate = q.dequant = false;
+  int st = launch_variant<P, RBC, 4, 2, 2, 4, 1, 5, true>(q, 0, q.K1, false, stream, slices);
+  if (st != 0) return st;
+  note_k_slices(slices);
+  SumArgs s{};
+  s.partials = ws.partials;
+  s.slice_bytes = rows * cols * 4;
+  s.pitch = cols * 4;
+  s.slices = slices;
+  s.rows = (int32_t)std::min(rows, p.out_rows);
+  s.cols = (int32_t)std::min(cols, p.out_cols);
+  s.M0 = p.M0; s.N0 = p.N0;
+  s.out = p.out; s.out_stride = p.out_stride;
+  s.out_sm0 = (uint32_t)p.out_sm0; s.out_spn = (uint32_t)p.out_spn;
+  s.acc = p.accumulate ? p.acc : nullptr; s.acc_stride = p.acc_stride;
+  s.acc_sm0 = (uint32_t)p.acc_sm0; s.acc_spn = (uint32_t)p.acc_spn;
+  s.dequant = p.dequant; s.row_scale = p.row_scale; s.col_scale = p.col_scale;
+  constexpr int OB = Out::kOutBytes;
+  auto vector_ok = [&](const char* base, int64_t stride, int64_t sm0, int64_t spn) {
+    const bool contiguous4 = p.N0 % 4 == 0 || spn == (int64_t)p.N0 * OB;
+    const bool aligned4 = OB == 4 || (((uintptr_t)base | (uint64_t)stride | (uint64_t)sm0 |
+                                       (uint64_t)spn) % 8) == 0;
+    return contiguous4 && aligned4;
+  };
+  s.vec = vector_ok(p.out, p.out_stride, p.out_sm0, p.out_spn) &&
+          (!p.accumulate || vector_ok(p.acc, p.acc_stride, p.acc_sm0, p.acc_spn));
+  const dim3 grid((uint32_t)uk::ceil_div(s.cols, 4 * kSumThreads), (uint32_t)s.rows);
+  uk::launch(2, mmt4d_sum_slices_kernel<typename ElemTraits<E>::Acc, Out>, grid, dim3(kSumThreads), 0, stream, s);
+  return finish_k((int)hipGetLastError());
+}
+
 // Number of workgroups a BM x BN blocking gives for the problem.
 inline int64_t workgroups(const Problem& p, int BM, int BN) {
   const int bpm = BM / p.M0, bpn = BN / p.N0;
@@ -564,6 +627,42 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
   return st;
 }
 
+// K slices for launch_slices, one workgroup a compute unit or fewer; 0 where the blocks
+// that a problem of few 128x128 blocks and 6 KB of K and more has otherwise take less.
+// A 64x64 block loads 128 rows of K for 64x64 sums, at 2 us a KB whatever the type: each
+// unit's L1 and L2 traffic bounds these calls. A 128x128 block needs half as much for
+// each sum, but then the slices' sums pass through memory (a write and a read of 4 bytes
+// each) and a second launch. The constants are fitted to 30 calls with weights from HBM,
+// and lie on the side of the blocks in place where the two are close. us before / in
+// slices (how many):
+//   bf16 -> bf16 200 x 4096 x 14336 59.9 / 45.1 (4), 128 x 4096 x 14336 50.3 / 34.1 (8),
+//     300 x 4096 x 8192 52.6 / 43.1 (2), 100 x 14336 x 4096 43.6 / 36.3 (2)
+//   f16 512 x 2048 x 16384 61.9 / 49.5 (4), 256 x 8192 x 8192 66.5 / 52.7 (2), 512 x 512 x
+//     16384 29.2 / 22.3 (16), 70 x 16384 x 4096 45.0 / 36.2 (2)
+//   s8 256 x 2048 x 16384 30.8 / 22.6 (8), 512 x 4096 x 8192 33.9 / 31.1 (2), 8-byte rows 200
+//     x 4096 x 14336 41.2 / 29.9 (4); f8 512 x 4096 x 8192 41.5 / 31.8 (2)
+//   but f16 640 x 3072 x 3072 24.8 / 26.6 (2), f8 128 x 8192 x 8192 26.8 / 28.9 (4), f16 256 x
+//     1024 x 4096 9.5 / 15.4 (8)
+template <int RBC>
+int slices_that_pay(const Problem& p, int64_t rows, int64_t cols, bool long_k) {
+  const int64_t cus = compute_units();
+  const int64_t k_bytes = (int64_t)p.K1 << p.lrb, b128 = workgroups(p, 128, 128);
+  const int64_t b64 = workgroups(p, 64, 64);
+  const int64_t b32 = uk::ceil_div(rows, (int64_t)32) * uk::ceil_div(cols, (int64_t)32);
+  const int64_t b16 = uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16);
+  // (With fewer than 32 64x64 blocks K is in more parts there than it would be here.)
+  if (cus < 1 || b128 < 1 || b64 < 32 || b16 <= cus) return 0;
+  const int64_t slices = std::min<int64_t>(std::min<int64_t>(cus / b128, 16), k_bytes / 2048);
+  if (slices < 2) return 0;
+  const double kb = (double)k_bytes / 1024;
+  const double here = 5 + 4.3 * kb / (double)slices + 2.4e-6 * (double)(slices * rows * cols);
+  const double units = (double)b64 / (double)cus;
+  double blocks = 2 + (RBC == 8 ? 2.8 : 2.05) * kb * std::max(1.0, std::min(std::ceil(units), units + 0.3));
+  if (!long_k && b32 <= 2 * cus) blocks = 2 + 0.9 * kb * (double)uk::ceil_div(b32, cus);
+  else if (long_k && 2 * b64 <= cus) blocks = 15 + 2.05 * kb / (double)(cus / b64);
+  return here < blocks ? (int)slices : 0;
+}
+
 // Variant choice for row-bytes class RBC:
 //   big   256x256 workgroup tile, 8 waves of 128x64, software-pipelined, both
 //         operands through LDS-direct loads, any K; f32: RHS straight to
@@ -578,7 +677,8 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
 // shape with 256-byte steps three steps ahead (tile rows under 16 bytes),
 // 12 .. 15 the narrow-row kernel (tile rows of 2 or 4 bytes, N0 = 16) in the
 // 256x256 / 128x512 / 128x128 / 64x64 shape, 16 / 17 / 18 / 19 the LDS-direct
-// ping-pong pipeline in the 256x256 / 128x512 / 128x128 / 64x64 shape;
+// ping-pong pipeline in the 256x256 / 128x512 / 128x128 / 64x64 shape, 21 the K
+// slices of launch_slices, as many as iree_uk_amd_set_k_slices says;
 // 0 = choose) overrides the
 // size heuristic for tests and tuning.
 //   thin  M-thin (decode-shaped) problems, up to 64 rows, which are bound by
@@ -619,6 +719,8 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     // shape (9) or in the square one (10); the plain square shape where the
     // requested one cannot serve.
     choice = 1;
+  } else if (forced == 21) {
+    choice = 6;  // K in slices over 128x128 blocks, where they serve
   } else if (forced >= 1 && forced <= 7) {
     choice = forced;
   } else if (rows_m <= (RBC >= 8 ? 64 : 32) && workgroups(p, 32, 64) >= 1) {
@@ -882,6 +984,13 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   }
   // (With 24 KB of K and more the 64x64 blocks below split K over workgroups.)
   const bool long_k = ((int64_t)p.K1 << p.lrb) >= 24576;
+  if constexpr (RBC >= 8 && E != Elem::kF32) {
+    if (choice == 6 && (forced == 21 || (forced == 0 && k_slices_override() == 0))) {
+      const int slices = forced == 21 ? k_slices_override() : slices_that_pay<RBC>(p, rows_m, cols_n, long_k);
+      const int st = launch_slices<E, RBC>(p, slices, stream);
+      if (st >= 0) { *name = "mmt4d_mfma_128x128_kslices"; return st; }
+    }
+  }
   if (forced == 0 && (choice == 3 || (choice == 6 && (!long_k || E == Elem::kF32)) || (RBC < 8 && choice == 4) ||
                       (choice == 2 && E == Elem::kF32))) {
     const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, stream, name);
