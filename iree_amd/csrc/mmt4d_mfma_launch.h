@@ -536,6 +536,10 @@ int launch_slices(const Problem& p, int slices, hipStream_t stream) {
   q.out_sm0 = cols * 4;
   q.out_spn = p.N0 * 4;
   q.acc = q.out; q.acc_stride = q.out_stride; q.acc_sm0 = q.out_sm0; q.acc_spn = q.out_spn;
+  // What exists of the partial sums are this problem's own rows and columns: of a part of
+  // a larger problem the result may have more, and a row here has no room for them.
+  q.out_rows = std::min(p.out_rows, rows);
+  q.out_cols = std::min(p.out_cols, cols);
   q.accumulate = q.dequant = false;
   int st = launch_variant<P, RBC, 4, 2, 2, 4, 1, 5, true>(q, 0, q.K1, false, stream, slices);
   if (st != 0) return st;
