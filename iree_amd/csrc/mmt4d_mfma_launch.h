@@ -800,9 +800,16 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       }
     }
     if (split_m || split_n) {
+      // Each part has the rows and columns of its own panels and no more: kernels
+      // store groups of four columns whole where as many exist, and a part may end
+      // inside a group (tiles of 7, 9 or 10 columns).
+      const int64_t own_rows = std::min(p.out_rows, (int64_t)main_m * p.M0);
+      const int64_t own_cols = std::min(p.out_cols, (int64_t)main_n * p.N0);
       Problem q = p;
       q.M1 = main_m;
       q.N1 = main_n;
+      q.out_rows = own_rows;
+      q.out_cols = own_cols;
       int st = launch_class<E, RBC>(q, 0, stream, name);
       if (st != 0) return st;
       const char* strip_name = nullptr;
@@ -826,6 +833,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
         q.acc = p.acc + (int64_t)main_m * p.acc_stride;
         if (p.row_scale) q.row_scale = p.row_scale + (int64_t)main_m * p.M0;
         q.out_rows = p.out_rows - (int64_t)main_m * p.M0;
+        q.out_cols = own_cols;
         q.M1 = p.M1 - main_m;
         q.N1 = main_n;
         st = launch_class<E, RBC>(q, 0, stream, &strip_name);

@@ -42,3 +42,11 @@ def _check(gpu, dtype, m1, k1, accumulate):
 def test_a_row_strip_with_k_in_slices_keeps_to_its_columns(gpu, dtype):
     """80 rows against a K of 14 KB: the strip's sums meet in rows of its own width."""
     assert _check(gpu, dtype, 277, 448 * (2 if dtype == "s8" else 1), False) == 7
+
+
+@pytest.mark.parametrize("dtype", list(TYPES))
+@pytest.mark.parametrize("m1", [273, 277])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_a_row_strip_keeps_to_its_columns(gpu, dtype, m1, accumulate):
+    """16 and 80 rows, a short K: the strip runs last, beside the finished column strip."""
+    assert _check(gpu, dtype, m1, 5, accumulate) == 1
