@@ -84,6 +84,13 @@ void mmt4d_thin_kernel(Args a) {
   constexpr int KS = NCH * 16;                // bytes of K per row per step
   constexpr int PIECES = RBC >= 16 ? 1 : 16 / RBC;   // loads per 16-byte operand
   constexpr bool S4 = E == Elem::kS8S4;       // 4-bit RHS: half the bytes per row
+  // Sums of floats whose K eight waves share are in several chains, steps i, i +
+  // CHAINS, .. of a wave apart: as many parts of K and more, each a shorter chain of
+  // roundings, as four waves in up to eight workgroups add up. Error against 64 bits of
+  // 32 x 512 results in one chain / here / in those workgroups, 1e-7: f16, K = 4096 1.56 /
+  // 1.03 / 1.03; f32, K = 2048 2.94 / 1.60 / 1.59. (The matrix instructions of 8-bit
+  // floats round to 1.5e-5 by themselves, however K is divided.)
+  constexpr int CHAINS = KSPLIT < 8 || HALVES == 2 || std::is_same<Acc, v4i>::value ? 1 : TM == 1 ? 4 : 2;
   static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
   static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
 
@@ -234,11 +241,14 @@ void mmt4d_thin_kernel(Args a) {
     }
   };
 
-  Acc acc[TM][TN];
+  Acc chains[CHAINS][TM][TN];
+  Acc (&acc)[TM][TN] = chains[0];
 #pragma unroll
-  for (int tm = 0; tm < TM; ++tm)
+  for (int c = 0; c < CHAINS; ++c)
 #pragma unroll
-    for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = Acc{0, 0, 0, 0};
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) chains[c][tm][tn] = Acc{0, 0, 0, 0};
 
   // ---- K loop ---------------------------------------------------------------
   const int my_steps = wg_steps > wave ? (wg_steps - wave + KSPLIT - 1) / KSPLIT : 0;
@@ -292,7 +302,8 @@ void mmt4d_thin_kernel(Args a) {
       }
     }
   }
-  auto compute = [&](int d, int i) {
+  // The products of step i, whose operands are in registers d, onto chain c.
+  auto compute = [&](int d, int c, int i) {
     if constexpr (TAIL) {
       // The step K ends in: nothing beyond it reaches the sums (a zero in both
       // operands: what was read instead may be an infinity).
@@ -341,30 +352,39 @@ void mmt4d_thin_kernel(Args a) {
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = TT::mfma(fb[d][tn], fa[d][tm], acc[tm][tn]);
+        for (int tn = 0; tn < TN; ++tn)
+          chains[c][tm][tn] = TT::mfma(fb[d][tn], fa[d][tm], chains[c][tm][tn]);
     }
   };
+  constexpr int U = D > CHAINS ? D : CHAINS;   // steps unrolled: whole rounds of both
+  static_assert(U % D == 0 && U % CHAINS == 0, "");
   int i = 0;
   // Steady state: every step computed is followed by the load of the step D
   // further on, which exists.
-  for (; i + 2 * D <= my_steps; i += D) {
+  for (; i + U + D <= my_steps; i += U) {
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      compute(d, i + d);
-      load_step(d, i + d + D);
+    for (int u = 0; u < U; ++u) {
+      compute(u % D, u % CHAINS, i + u);
+      load_step(u % D, i + u + D);
     }
   }
-  // Fewer than 2 D steps left: the same with bounds.
+  // Fewer than U + D steps left: the same with bounds.
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    if (i + d < my_steps) {
-      compute(d, i + d);
-      if (i + d + D < my_steps) load_step(d, i + d + D);
+  for (int u = 0; u < U; ++u) {
+    if (i + u < my_steps) {
+      compute(u % D, u % CHAINS, i + u);
+      if (i + u + D < my_steps) load_step(u % D, i + u + D);
     }
   }
 #pragma unroll
-  for (int d = 0; d < D; ++d)
-    if (i + D + d < my_steps) compute(d, i + D + d);
+  for (int u = U; u < U + D; ++u)
+    if (i + u < my_steps) compute(u % D, u % CHAINS, i + u);
+#pragma unroll
+  for (int c = 1; c < CHAINS; ++c)
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) acc[tm][tn] += chains[c][tm][tn];
 
   // ---- meet the partial sums ---------------------------------------------------
   if constexpr (KSPLIT > 1) {

@@ -1,0 +1,63 @@
+"""Rounding errors of decode calls with few columns: no larger than with K in the parts
+that four waves in up to eight workgroups would sum, each part a chain of roundings,
+the waves' sums and then the workgroups' added in order. The same chains on the CPU
+give the bound. A matrix instruction rounds after `unit` products (f32: every one;
+16-bit floats, whose products it sums in groups first: fitted to calls whose parts are
+known, 0.2 to 4 % off). Eight parts where there were 12 to 32 had 1.2 to 1.85 times the
+error; the bound leaves 8 %."""
+import pytest
+
+from iree_amd import ukernel as uk
+
+pytestmark = pytest.mark.gpu
+
+TYPES = {"f16": (uk.MMT4D_TYPE_F16F16F32, "float16", 2, 8), "bf16": (uk.MMT4D_TYPE_BF16BF16F32, "bfloat16", 2, 8),
+         "f32": (uk.MMT4D_TYPE_F32F32F32, "float32", 4, 1)}
+
+
+def _error(got, want):
+    return float(((got.double() - want) ** 2).sum() / (want ** 2).sum()) ** 0.5
+
+
+def _chains(torch, a, b, unit, step, waves, groups):
+    parts = waves * groups
+    sums = torch.zeros(parts, a.shape[0], b.shape[0])
+    for s in range(a.shape[1] // step):
+        for k in range(s * step, (s + 1) * step, unit):
+            p = a[:, k:k + unit] @ b[:, k:k + unit].T
+            sums[s % parts] = (sums[s % parts].double() + p).float()
+    out = torch.zeros(a.shape[0], b.shape[0])
+    for group in sums.view(groups, waves, *out.shape):
+        part = group[0].clone()
+        for w in group[1:]:
+            part += w
+        out += part
+    return out
+
+
+@pytest.mark.parametrize("dtype,rows,cols,k,groups", [
+    ("f16", 32, 512, 4096, 8), ("f16", 4, 1024, 2048, 4), ("f16", 64, 1200, 2048, 3), ("bf16", 24, 320, 4096, 8),
+    ("f32", 16, 640, 2048, 6), ("f32", 64, 512, 2048, 8)])
+@pytest.mark.parametrize("swapped", [False, True])
+def test_error_of_few_columns(gpu, dtype, rows, cols, k, groups, swapped):
+    lib, torch = gpu
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the parts are for 256 compute units")
+    flags, t, elem, unit = TYPES[dtype]
+    k0 = 16 // elem
+    gen = torch.Generator(); gen.manual_seed(k + cols)
+    a, b = (torch.randn(r, k, generator=gen).to(getattr(torch, t)) for r in (rows, cols))
+    lhs, rhs = (torch.nn.functional.pad(x.float(), (0, 0, 0, -x.shape[0] % 16)).view(-1, 16, k // k0, k0)
+                .permute(0, 2, 1, 3).contiguous().to(x.dtype).cuda() for x in ((b, a) if swapped else (a, b)))
+    m, n = (cols, rows) if swapped else (rows, cols)
+    out = torch.zeros(m, n, device="cuda")
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    lib.mmt4d_unpack(lhs.data_ptr(), 0, 16 * k, rhs.data_ptr(), 0, 16 * k, out.data_ptr(), 0, n, m, n, -(-m // 16),
+                     -(-n // 16), k // k0, 16, 16, k0, flags)
+    lib.synchronize()
+    assert lib.last_kernel_name().startswith("mmt4d_mfma_thin"), lib.last_kernel_name()
+    got = out.cpu().T if swapped else out.cpu()
+    a, b = a.double(), b.double()
+    want = a @ b.T
+    bound = 1.08 * _error(_chains(torch, a, b, unit, 64 // elem, 4, groups), want)
+    assert _error(got, want) <= bound, (_error(got, want), bound)
