@@ -647,7 +647,11 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
 //     x 4096 x 14336 41.2 / 29.9 (4); f8 512 x 4096 x 8192 41.5 / 31.8 (2)
 //   but f16 640 x 3072 x 3072 24.8 / 26.6 (2), f8 128 x 8192 x 8192 26.8 / 28.9 (4), f16 256 x
 //     1024 x 4096 9.5 / 15.4 (8)
-template <int RBC>
+// A slice has 2 KB of K at least, with 24 KB of K and more 1.5 KB, where 32 64x64 blocks
+// have K in 32 parts: 16 slices of two sums each are as many (f16 128 x 1024 x 12288, 26.3
+// us and an error of 1.45e-7 there, 20.1 and 1.58e-7 in 12 slices, 18.9 and 1.43e-7 in 16;
+// 8-bit floats, whose matrix instructions round to 1.5e-5, stay at 16 steps and 2 KB).
+template <Elem E, int RBC>
 int slices_that_pay(const Problem& p, int64_t rows, int64_t cols, bool long_k) {
   const int64_t cus = compute_units();
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb, b128 = workgroups(p, 128, 128);
@@ -656,7 +660,8 @@ int slices_that_pay(const Problem& p, int64_t rows, int64_t cols, bool long_k) {
   const int64_t b16 = uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16);
   // (With fewer than 32 64x64 blocks K is in more parts there than it would be here.)
   if (cus < 1 || b128 < 1 || b64 < 32 || b16 <= cus) return 0;
-  const int64_t slices = std::min<int64_t>(std::min<int64_t>(cus / b128, 16), k_bytes / 2048);
+  const int64_t least_k = long_k && ElemTraits<E>::kHalves == 1 ? 1536 : 2048;
+  const int64_t slices = std::min<int64_t>(std::min<int64_t>(cus / b128, 16), k_bytes / least_k);
   if (slices < 2) return 0;
   const double kb = (double)k_bytes / 1024;
   const double here = 5 + 4.3 * kb / (double)slices + 2.4e-6 * (double)(slices * rows * cols);
@@ -998,7 +1003,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   const bool long_k = ((int64_t)p.K1 << p.lrb) >= 24576;
   if constexpr (RBC >= 8 && E != Elem::kF32) {
     if (choice == 6 && (forced == 21 || (forced == 0 && k_slices_override() == 0))) {
-      const int slices = forced == 21 ? k_slices_override() : slices_that_pay<RBC>(p, rows_m, cols_n, long_k);
+      const int slices = forced == 21 ? k_slices_override() : slices_that_pay<E, RBC>(p, rows_m, cols_n, long_k);
       const int st = launch_slices<E, RBC>(p, slices, stream);
       if (st >= 0) { *name = "mmt4d_mfma_128x128_kslices"; return st; }
     }

@@ -148,3 +148,31 @@ def test_no_workspace_runs_without_slices(gpu):
     finally:
         lib.set_stream(None)
         lib.set_pointer_mode(uk.POINTER_MODE_AUTO)
+
+
+@pytest.mark.parametrize("dtype,m,n,k", [("f16", 128, 1024, 12288), ("bf16", 384, 384, 12288), ("bf16", 512, 256, 13312),
+                                         ("f16", 65, 1024, 14336), ("f16", 128, 1024, 16384)])
+def test_errors_are_not_above_those_of_the_blocks_in_place(gpu, dtype, m, n, k):
+    """Against 64 bits, beside the 64x64 blocks with K over four waves and seven or eight
+    workgroups. Fewer parts of K or one chain of 16 slices had 1.03 to 1.14 times their
+    error, the slices taken now have 0.95 to 1.00; two estimates from 130000 results
+    differ by half a percent."""
+    lib, torch = gpu
+    flags, tin, _, _ = TYPES[dtype]
+    gen = torch.Generator(); gen.manual_seed(k)
+    a, b = (torch.randn(-(-r // 16), k // 8, 16, 8, generator=gen).to(getattr(torch, tin)).cuda() for r in (m, n))
+    want = (a.double().permute(0, 2, 1, 3).reshape(-1, k) @ b.double().permute(0, 2, 1, 3).reshape(-1, k).T)[:m]
+    errors = []
+    try:
+        for mode in (uk.KERNEL_MODE_AUTO, uk.KERNEL_MODE_MFMA_VARIANT + 6):
+            lib.set_kernel_mode(mode)
+            out = torch.zeros(m, n, device="cuda")
+            torch.cuda.synchronize()
+            lib.mmt4d_unpack(a.data_ptr(), 0, k * 16, b.data_ptr(), 0, k * 16, out.data_ptr(), 0, n, m, n, a.shape[0],
+                             b.shape[0], k // 8, 16, 16, 8, flags)
+            assert lib.last_kernel_name() == ("mmt4d_mfma_64x64_ksplit" if errors else KSLICES)
+            lib.synchronize()
+            errors.append(float(((out.double() - want) ** 2).sum() / (want ** 2).sum()) ** 0.5)
+    finally:
+        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    assert errors[0] <= 1.02 * errors[1], errors
