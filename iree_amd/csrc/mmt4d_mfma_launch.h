@@ -603,6 +603,7 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
   constexpr bool F32 = E == Elem::kF32;
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
   const int64_t cus = compute_units();
+  if (cus < 1) return -1;   // the device query failed, as the launch will
   const int64_t b16 = uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16);
   const int64_t b32 = uk::ceil_div(rows, (int64_t)32) * uk::ceil_div(cols, (int64_t)32);
   int st = -1;
