@@ -297,6 +297,29 @@ __device__ __forceinline__ auto load_floats(__amdgpu_buffer_rsrc_t from, uint32_
   }
 }
 
+// Where the loads of a sum come from: `base` + a lane's bytes + the step's bytes, 32-bit
+// ones through a buffer resource or (WIDE: images and filters that span more) 64-bit ones.
+template <bool WIDE>
+struct LoadFrom {
+  using Bytes = uint32_t;   // a step back is an addition that wraps
+  __amdgpu_buffer_rsrc_t rsrc;
+  __device__ explicit LoadFrom(const float* base) : rsrc(buffer_at(base)) {}
+  template <int TO>
+  __device__ __forceinline__ auto load(Bytes lane, Bytes step) const { return load_floats<TO>(rsrc, lane, step); }
+};
+template <>
+struct LoadFrom<true> {
+  using Bytes = int64_t;
+  const char* base;
+  __device__ explicit LoadFrom(const float* b) : base((const char*)b) {}
+  template <int TO>
+  __device__ __forceinline__ auto load(Bytes lane, Bytes step) const {
+    typedef float vTOf __attribute__((ext_vector_type(TO)));
+    typedef vTOf vTOf_a4 __attribute__((aligned(4)));
+    return (vTOf)*reinterpret_cast<const vTOf_a4*>(base + lane + step);
+  }
+};
+
 // One of two values that are both there: a select, where ?: would choose between two
 // places to load from.
 template <typename T>
@@ -356,7 +379,7 @@ __device__ __forceinline__ void conv_store(const ConvArgs& a, int32_t pxc, int32
 // (the split kernel's parts of a sum are fewer than the slices of input channels that it
 // took the place of: 3x3, 256 -> 32 channels at 10x10, batch 8, relative error 4.3e-7 with
 // one chain, 2.2e-7 with four), and MFMAs that do not wait for each other in small tiles.
-template <int TW, int TO, int D, int CHAINS>
+template <int TW, int TO, int D, int CHAINS, bool WIDE = false>
 __device__ __forceinline__ void conv_add_steps(const ConvArgs& a, int32_t pxc, int32_t occ, int32_t n, int32_t begin,
                                                int32_t steps, v4f (&sum)[TW][TO]) {
   typedef float vTOf __attribute__((ext_vector_type(TO)));
@@ -371,37 +394,37 @@ __device__ __forceinline__ void conv_add_steps(const ConvArgs& a, int32_t pxc, i
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, q = lane >> 4;
   const int32_t last_px = (int32_t)(a.OH * a.OW) - 1, OW = (int32_t)a.OW;
-  uint32_t pa[TW];   // bytes
+  using Bytes = typename LoadFrom<WIDE>::Bytes;
+  Bytes pa[TW];
 #pragma unroll
   for (int tw = 0; tw < TW; ++tw) {
     const int32_t px = min((pxc * TW + tw) * 16 + r, last_px);
     const int32_t oh = px / OW, ow = px - oh * OW;
-    pa[tw] = (uint32_t)(((int64_t)oh * a.stride_h * a.in_sh + (int64_t)ow * a.stride_w * a.c0 + 4 * q -
+    pa[tw] = (Bytes)(((int64_t)oh * a.stride_h * a.in_sh + (int64_t)ow * a.stride_w * a.c0 + 4 * q -
                          a.in_low_px) * 4);
   }
   constexpr int kLanesPerBlock = 16 / TO;
   const int32_t oc_ld = min(r / kLanesPerBlock, (int32_t)a.OC - 1 - occ * TO);
-  const uint32_t pf = (uint32_t)((oc_ld * a.f_soc + (4 * q) * 16 + r % kLanesPerBlock * TO - a.f_low_oc) * 4);
+  const Bytes pf = (Bytes)((oc_ld * a.f_soc + (4 * q) * 16 + r % kLanesPerBlock * TO - a.f_low_oc) * 4);
 
   // Within one (ic_outer, fh) consecutive steps follow each other at 16 input
   // floats and 256 filter floats.
   const int32_t IC = (int32_t)a.IC, FH = (int32_t)a.FH, taps = (int32_t)(a.FW * (a.c0 / 16));
-  // In bytes; a step back is an addition that wraps.
-  const uint32_t in_next_fh = (uint32_t)((a.in_sh - (taps - 1) * 16) * 4);
-  const uint32_t f_next_fh = (uint32_t)((a.f_sfh - (taps - 1) * 256) * 4);
-  const uint32_t in_next_ic = (uint32_t)((a.in_sic - (FH - 1) * a.in_sh - (taps - 1) * 16) * 4);
-  const uint32_t f_next_ic = (uint32_t)((a.f_sic - (FH - 1) * a.f_sfh - (taps - 1) * 256) * 4);
+  const Bytes in_next_fh = (Bytes)((a.in_sh - (taps - 1) * 16) * 4);
+  const Bytes f_next_fh = (Bytes)((a.f_sfh - (taps - 1) * 256) * 4);
+  const Bytes in_next_ic = (Bytes)((a.in_sic - (FH - 1) * a.in_sh - (taps - 1) * 16) * 4);
+  const Bytes f_next_ic = (Bytes)((a.f_sic - (FH - 1) * a.f_sfh - (taps - 1) * 256) * 4);
   // From the last step of all back to the first, for the prefetches past the end.
-  const uint32_t in_again = (uint32_t)(-((IC - 1) * a.in_sic + (FH - 1) * a.in_sh + (taps - 1) * 16) * 4);
-  const uint32_t f_again = (uint32_t)(-((IC - 1) * a.f_sic + (FH - 1) * a.f_sfh + (taps - 1) * 256) * 4);
-  const __amdgpu_buffer_rsrc_t in = buffer_at(a.in + n * a.in_sn + a.in_low_px + a.in_low_step);
-  const __amdgpu_buffer_rsrc_t flt = buffer_at(a.flt + occ * TO * a.f_soc + a.f_low_oc + a.f_low_step);
+  const Bytes in_again = (Bytes)(-((IC - 1) * a.in_sic + (FH - 1) * a.in_sh + (taps - 1) * 16) * 4);
+  const Bytes f_again = (Bytes)(-((IC - 1) * a.f_sic + (FH - 1) * a.f_sfh + (taps - 1) * 256) * 4);
+  const LoadFrom<WIDE> in(a.in + n * a.in_sn + a.in_low_px + a.in_low_step);
+  const LoadFrom<WIDE> flt(a.flt + occ * TO * a.f_soc + a.f_low_oc + a.f_low_step);
   // The step the next prefetch loads: its offsets and its distance from the ends of
   // its (ic_outer, fh), its ic_outer and the sum.
   const int32_t row0 = begin / taps, tap0 = begin - row0 * taps;
   const int32_t ic0 = row0 / FH, fh0 = row0 - ic0 * FH;
-  uint32_t ao = (uint32_t)((ic0 * a.in_sic + fh0 * a.in_sh + tap0 * 16 - a.in_low_step) * 4);
-  uint32_t bo = (uint32_t)((ic0 * a.f_sic + fh0 * a.f_sfh + tap0 * 256 - a.f_low_step) * 4);
+  Bytes ao = (Bytes)((ic0 * a.in_sic + fh0 * a.in_sh + tap0 * 16 - a.in_low_step) * 4);
+  Bytes bo = (Bytes)((ic0 * a.f_sic + fh0 * a.f_sfh + tap0 * 256 - a.f_low_step) * 4);
   int32_t tap = taps - 1 - tap0, fh = FH - 1 - fh0, ic = IC - 1 - ic0;
   constexpr int kProducts = 4 * TW * TO, kLoads = TW + 4;
   v4f av[D][TW];
@@ -409,15 +432,15 @@ __device__ __forceinline__ void conv_add_steps(const ConvArgs& a, int32_t pxc, i
   auto prefetch = [&](auto buf) {
     constexpr int B = decltype(buf)::value;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) fv[B][w] = load_floats<TO>(flt, pf + w * 64, bo);
+    for (int w = 0; w < 4; ++w) fv[B][w] = flt.template load<TO>(pf + w * 64, bo);
 #pragma unroll
-    for (int tw = 0; tw < TW; ++tw) av[B][tw] = load_floats<4>(in, pa[tw], ao);
+    for (int tw = 0; tw < TW; ++tw) av[B][tw] = in.template load<4>(pa[tw], ao);
     if constexpr (kProducts >= 16) {
       // All scalar selects: there are MFMAs enough to hide them, which a branch
       // between them would keep apart.
       const bool next_tap = tap != 0, next_fh = fh != 0, next_ic = ic != 0;
-      ao += pick(next_tap, 64u, pick(next_fh, in_next_fh, pick(next_ic, in_next_ic, in_again)));
-      bo += pick(next_tap, 1024u, pick(next_fh, f_next_fh, pick(next_ic, f_next_ic, f_again)));
+      ao += pick(next_tap, (Bytes)64, pick(next_fh, in_next_fh, pick(next_ic, in_next_ic, in_again)));
+      bo += pick(next_tap, (Bytes)1024, pick(next_fh, f_next_fh, pick(next_ic, f_next_ic, f_again)));
       ic = pick(next_tap | next_fh, ic, pick(next_ic, ic - 1, IC - 1));
       fh = pick(next_tap, fh, pick(next_fh, fh - 1, FH - 1));
       tap = pick(next_tap, tap - 1, taps - 1);
@@ -482,11 +505,11 @@ __device__ __forceinline__ void conv_add_steps(const ConvArgs& a, int32_t pxc, i
     }
 }
 
-template <int TW, int TO, int D>
+template <int TW, int TO, int D, bool WIDE>
 __device__ __forceinline__ void conv_wave_tile(const ConvArgs& a, int32_t pxc, int32_t occ, int32_t n) {
   v4f acc[TW][TO];
   conv_begin<TW, TO>(a, pxc, occ, n, acc);
-  conv_add_steps<TW, TO, D, TW * TO == 1 ? 4 : 1>(a, pxc, occ, n, 0, a.steps, acc);
+  conv_add_steps<TW, TO, D, TW * TO == 1 ? 4 : 1, WIDE>(a, pxc, occ, n, 0, a.steps, acc);
   conv_store<TW, TO>(a, pxc, occ, n, acc);
 }
 
@@ -499,14 +522,14 @@ __device__ __forceinline__ uint32_t xcd_contiguous(uint32_t id, uint32_t count) 
 }
 
 // A workgroup of four waves owns (n, TO channel blocks, 4 x TW panels).
-template <int TW, int TO, int D>
+template <int TW, int TO, int D, bool WIDE = false>
 __global__ __launch_bounds__(kThreads, 1) void conv_nchwc_mfma_direct_kernel(ConvArgs a, uint32_t px_chunks,
                                                                              uint32_t px_groups, uint32_t oc_chunks) {
   uint32_t t = xcd_contiguous(blockIdx.x, gridDim.x);
   const uint32_t pxg = t % px_groups; t /= px_groups;
   const uint32_t pxc = pxg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (pxc >= px_chunks) return;
-  conv_wave_tile<TW, TO, D>(a, (int32_t)pxc, (int32_t)(t % oc_chunks), (int32_t)(t / oc_chunks));
+  conv_wave_tile<TW, TO, D, WIDE>(a, (int32_t)pxc, (int32_t)(t % oc_chunks), (int32_t)(t / oc_chunks));
 }
 
 // Layers with too few tiles for the chip: the four waves of a workgroup own one tile and
@@ -517,7 +540,7 @@ __global__ __launch_bounds__(kThreads, 1) void conv_nchwc_mfma_direct_kernel(Con
 // acknowledged, and the one that is last adds the slices up in order and stores the
 // result; see mmt4d_thin_kernel for why no fence is needed. Results are the same on
 // every run.
-template <int TW, int TO, int D>
+template <int TW, int TO, int D, bool WIDE = false>
 __global__ __launch_bounds__(kThreads) void conv_nchwc_mfma_split_kernel(ConvArgs a, uint32_t px_chunks,
                                                                          uint32_t oc_chunks) {
   __shared__ v4f partial[kWaves - 1][TW * TO][64];
@@ -537,7 +560,7 @@ __global__ __launch_bounds__(kThreads) void conv_nchwc_mfma_split_kernel(ConvArg
 #pragma unroll
     for (int to = 0; to < TO; ++to) acc[tw][to] = v4f{0.f, 0.f, 0.f, 0.f};
   if (share == 0) conv_begin<TW, TO>(a, pxc, occ, n, acc);
-  conv_add_steps<TW, TO, D, TW * TO == 1 ? 4 : 2>(a, pxc, occ, n, (int32_t)begin, (int32_t)(end - begin), acc);
+  conv_add_steps<TW, TO, D, TW * TO == 1 ? 4 : 2, WIDE>(a, pxc, occ, n, (int32_t)begin, (int32_t)(end - begin), acc);
   if (wave > 0) {
 #pragma unroll
     for (int tw = 0; tw < TW; ++tw)
@@ -593,7 +616,7 @@ __global__ __launch_bounds__(kThreads) void conv_nchwc_mfma_split_kernel(ConvArg
 }
 
 // D = 0: the filter through LDS, else the direct kernel with D register sets.
-template <int TW, int TO, int D>
+template <int TW, int TO, int D, bool WIDE = false>
 int launch_mfma(const ConvArgs& a, hipStream_t stream) {
   const int64_t px_chunks = uk::ceil_div(a.OH * a.OW, (int64_t)16 * TW);
   const int64_t px_groups = uk::ceil_div(px_chunks, (int64_t)(kThreads / 64));
@@ -604,7 +627,7 @@ int launch_mfma(const ConvArgs& a, hipStream_t stream) {
     uk::launch(3, conv_nchwc_mfma_lds_kernel<TW, TO>, dim3((uint32_t)blocks), dim3(kThreads), 0, stream,
                a, px_chunks, px_groups, oc_chunks);
   } else {
-    uk::launch(3, conv_nchwc_mfma_direct_kernel<TW, TO, D>, dim3((uint32_t)blocks), dim3(kThreads), 0, stream, a,
+    uk::launch(3, conv_nchwc_mfma_direct_kernel<TW, TO, D, WIDE>, dim3((uint32_t)blocks), dim3(kThreads), 0, stream, a,
                (uint32_t)px_chunks, (uint32_t)px_groups, (uint32_t)oc_chunks);
   }
   return (int)hipGetLastError();
@@ -612,7 +635,7 @@ int launch_mfma(const ConvArgs& a, hipStream_t stream) {
 
 // The split kernel with up to `slices` workgroups a tile (fewer when no workspace is to
 // be had: calls under capture).
-template <int TW, int TO, int D>
+template <int TW, int TO, int D, bool WIDE = false>
 int launch_split(ConvArgs a, int32_t slices, hipStream_t stream) {
   const int64_t px_chunks = uk::ceil_div(a.OH * a.OW, (int64_t)16 * TW);
   const int64_t oc_chunks = uk::ceil_div(a.OC, (int64_t)TO);
@@ -629,7 +652,7 @@ int launch_split(ConvArgs a, int32_t slices, hipStream_t stream) {
       a.counters = ws.counters;
     }
   }
-  uk::launch(3, conv_nchwc_mfma_split_kernel<TW, TO, D>, dim3((uint32_t)(tiles * a.slices)), dim3(kThreads), 0,
+  uk::launch(3, conv_nchwc_mfma_split_kernel<TW, TO, D, WIDE>, dim3((uint32_t)(tiles * a.slices)), dim3(kThreads), 0,
              stream, a, (uint32_t)px_chunks, (uint32_t)oc_chunks);
   return (int)hipGetLastError();
 }
@@ -688,16 +711,31 @@ constexpr LongTile kLongTiles[] = {
     {1, 1, 1170, 4200, nullptr, launch_split<1, 1, 8>, "conv_nchwc_mfma_split_1x1"},
 };
 constexpr int64_t kSlicesMeet = 27000;
+// The same for layers beyond 32-bit offsets, with 64-bit ones, from five steps a wave of
+// the split kernel on. The direct kernel then runs its MFMAs at 0.7 of the rate where a
+// matrix core has several waves: one round of it. us through LDS / here, planes of input
+// channels 64 MB and more apart: 3x3, 512 -> 512 at 7x7 91.6 / 13.1, 256 -> 256 at 14x14
+// 47.0 / 10.7, 128 -> 128 at 56x56 25.5 / 15.3, 256 -> 256 at 28x28, batch 4 62.1 / 45.5,
+// batch 8 98.4 / 79.7.
+constexpr LongTile kWideTiles[] = {
+    {2, 2, 870, 3000, launch_mfma<2, 2, 4, true>, nullptr, "conv_nchwc_mfma_direct_wide_2x2"},
+    {2, 4, 710, 3000, launch_mfma<2, 4, 3, true>, nullptr, "conv_nchwc_mfma_direct_wide_2x4"},
+    {1, 4, 1050, 4200, nullptr, launch_split<1, 4, 4, true>, "conv_nchwc_mfma_split_wide_1x4"},
+};
 
-// For sums of `a.steps` > 10 steps. Returns a HIP status, or -1 when not served.
-int launch_long(const ConvArgs& a, int64_t cus, hipStream_t stream, const char** name) {
+// For sums of `a.steps` > 10 steps: the tile and slices of `tiles` that are estimated to
+// be done first, if that is before `least`; the direct kernel in up to `most_direct`
+// workgroups. Returns a HIP status, or -1 when not served.
+template <size_t TILES>
+int launch_long(const ConvArgs& a, const LongTile (&tiles)[TILES], int64_t most_direct, int64_t least, int64_t cus,
+                hipStream_t stream, const char** name) {
   const int64_t pixels = a.OH * a.OW, steps = a.steps;
   const LongTile* best = nullptr;
   int best_slices = 1;
-  int64_t least = INT64_MAX;
-  for (const LongTile& t : kLongTiles) {
+  for (const LongTile& t : tiles) {
     const int64_t px = 16 * t.tw * (t.direct ? kWaves : 1);
     const int64_t groups = a.N * uk::ceil_div(pixels, px) * uk::ceil_div(a.OC, (int64_t)t.to);
+    if (t.direct && groups > most_direct) continue;
     for (int slices = 1; slices <= (t.direct ? 1 : 4); slices *= 2) {
       // (16 MB of partial sums at most.)
       if (slices > 1 && groups * slices * t.tw * t.to > 16384) break;
@@ -711,6 +749,7 @@ int launch_long(const ConvArgs& a, int64_t cus, hipStream_t stream, const char**
       }
     }
   }
+  if (!best) return -1;
   *name = best->name;
   return best->direct ? best->direct(a, stream) : best->split(a, best_slices, stream);
 }
@@ -770,8 +809,9 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
     }
     const int64_t steps_per_ic = a.FH * a.FW * (a.c0 / 16);
     const int64_t steps = a.IC * steps_per_ic;
-    // The direct kernel addresses an image and the filters of a few channel blocks
-    // with 32 bits; what is larger takes the LDS kernel.
+    // The direct and the split kernel address an image and the filters of a few channel
+    // blocks with 32 bits; what is larger takes the LDS kernel, or the split kernel with
+    // 64-bit addresses.
     const int64_t in_ext[] = {(a.OH - 1) * a.stride_h * a.in_sh, (a.OW - 1) * a.stride_w * a.c0,
                               (a.IC - 1) * a.in_sic, (a.FH - 1) * a.in_sh};
     const int64_t f_ext[] = {3 * a.f_soc, (a.IC - 1) * a.f_sic, (a.FH - 1) * a.f_sfh};
@@ -782,11 +822,11 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
     int64_t in_span = a.FW * a.c0, f_span = a.FW * a.c0 * 16;   // floats
     for (int64_t e : in_ext) in_span += std::abs(e);
     for (int64_t e : f_ext) f_span += std::abs(e);
-    const bool direct = in_span < (1ll << 29) && f_span < (1ll << 29) && a.OH * a.OW < (1ll << 30) &&
-                        steps < (1ll << 20);
+    const bool indexed = a.OH * a.OW < (1ll << 30) && steps < (1ll << 20);
+    const bool direct = indexed && in_span < (1ll << 29) && f_span < (1ll << 29);
     a.steps = (int32_t)std::min<int64_t>(steps, INT32_MAX);
     if (direct && steps > 10) {
-      const int st = launch_long(a, cus, stream, kernel_name);
+      const int st = launch_long(a, kLongTiles, INT64_MAX, INT64_MAX, cus, stream, kernel_name);
       if (st >= 0) return st;
     }
     // The tile whose fullest compute unit is done first: workgroups per unit,
@@ -811,6 +851,12 @@ extern "C" int iree_uk_amd_hip_launch_conv_nchwc(const iree_uk_conv_nchwc_params
         tile = &t;
         least = cost;
       }
+    }
+    if (!direct && indexed && steps >= 20) {
+      // (The LDS tiles' costs are those of several rounds.)
+      const bool one_round = mfma_blocks(a, *tile) <= cus;
+      const int st = launch_long(a, kWideTiles, cus, one_round ? least * steps * 5 / 4 : least * steps, cus, stream, kernel_name);
+      if (st >= 0) return st;
     }
     const int st = tile->launch(a, stream);
     if (st >= 0) {

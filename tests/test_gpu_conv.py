@@ -254,3 +254,43 @@ def test_conv_image_beyond_32_bit_offsets(gpu):
         names.append(lib.last_kernel_name())
     assert "lds" not in names[0] and "lds" in names[1], names
     assert bool(results[0].any()) and torch.equal(results[0], results[1])
+
+
+@pytest.mark.parametrize("dims,kernel", [((1, 3, 6, 10, 3), "split_wide_1x4"),       # 27 steps
+                                         ((2, 33, 7, 7, 7), "split_wide_1x4"),       # 147 steps, workgroups meet
+                                         ((1, 5, 60, 59, 3), "split_wide_1x4"),      # several rounds
+                                         ((4, 16, 28, 28, 3), "direct_wide_2x2"),
+                                         ((8, 15, 28, 27, 3), "direct_wide_2x4")])
+@pytest.mark.parametrize("back", [False, True])
+def test_conv_far_planes_and_few_tiles(gpu, dims, kernel, back):
+    """The same with sums long enough for the split and the direct kernel with 64-bit
+    addresses, the planes in order and back to front; ACCUMULATE. Equal to the layer with
+    its planes side by side."""
+    lib, torch = gpu
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the tiles are chosen for 256 compute units")
+    lib.set_pointer_mode(uk.POINTER_MODE_AUTO)
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    N, OC, OH, OW, F = dims
+    IC, H, W, plane = 3, OH + F - 1, OW + F - 1, 1 << 28
+    size = H * W * 16
+    g = torch.Generator(device="cuda"); g.manual_seed(12)
+    x = torch.randint(-3, 4, (IC, N * size), generator=g, device="cuda").float()
+    f = torch.randint(-3, 4, (OC * IC * F * F * 256,), generator=g, device="cuda").float()
+    y0 = torch.randint(-9, 9, (N * OC * OH * OW * 16,), generator=g, device="cuda").float()
+    far = torch.empty((IC - 1) * plane + N * size, device="cuda")
+    for i in range(IC):
+        at = (IC - 1 - i if back else i) * plane
+        far[at:at + N * size] = x[i]
+    results, names = [], []
+    for buf, off, sic in ((x, 0, N * size), (far, (IC - 1) * plane if back else 0, -plane if back else plane)):
+        for run in range(2):   # the second call finds the counters of the first one's workgroups
+            y = y0.clone()
+            lib.conv_nchwc(buf.data_ptr(), off, size, sic, W * 16, f.data_ptr(), 0, IC * F * F * 256, F * F * 256, F * 256,
+                           y.data_ptr(), 0, OC * OH * OW * 16, OH * OW * 16, OW * 16, N, OC, OH, OW, IC, F, F, 16, 16, 1, 1,
+                           C.CONV_TYPE_F32F32F32 | C.CONV_ACCUMULATE)
+            lib.synchronize()
+            results.append(y)
+            names.append(lib.last_kernel_name())
+    assert "wide" not in names[0] and names[2] == "conv_nchwc_mfma_" + kernel, names
+    assert all(torch.equal(results[0], r) for r in results[1:])
