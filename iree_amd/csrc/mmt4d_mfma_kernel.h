@@ -559,13 +559,14 @@ void mmt4d_mfma_kernel(Args a) {
     const int row_origin = pm0 * a.M0, col_origin = pn0 * a.N0;
     if (a.vec_out) {
       uint32_t col_off[TN];
-      int col_n[TN];  // how many of the 4 columns exist
+      int col_n[TN];  // how many of the 4 columns exist and are this workgroup's
+      const int cols = min(a.out_cols - col_origin, a.bpn * a.N0);
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) {
         const int col = (wn * TN + tn) * 16 + 4 * (int)oq;
         const int pl = col / a.N0, n0 = col - pl * a.N0;
         const bool ok = pl < a.bpn && pn0 + pl < a.N1;
-        const int left = a.out_cols - (col_origin + col);
+        const int left = cols - col;
         col_n[tn] = ok ? (left >= 4 ? 4 : (left > 0 ? left : 0)) : 0;
         col_off[tn] = (uint32_t)pl * s_pn + (uint32_t)n0 * OB;
       }
