@@ -411,8 +411,9 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   // keeps at least as many operand bytes as a workgroup streams in several times
   // that: 192 KB (16 rows, weights not cached: s8 1024 x 16384, 512 KB a block, 10.6
   // -> 9.3 us in two slices; s8 1024 x 4096, 128 KB, 4.7 against 6.2; f16 64 rows
-  // 1024 x 4096, 640 KB, 13.8 -> 11.1 in three). With so few blocks that most units
-  // would idle, 64 KB. In any case 16 steps.
+  // 1024 x 4096, 640 KB, 13.8 -> 11.1 in three); 128 KB with 8-byte rows, two loads an
+  // operand (s8 1024 x 14336 8.8 us in two slices, 8.2 in three). With so few blocks that
+  // most units would idle, 64 KB. In any case 16 steps.
   int64_t kslices = 1;
   if (allow_k_slices) {
     const int64_t blocks = grid_m * grid_n;
@@ -421,7 +422,7 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
       kslices = k_slices_override();
     } else if (cus > 0 && 2 * blocks <= cus) {
       const int64_t share = k_bytes * 16 * (TM + TN) - (S4 ? k_bytes * 8 * TN : 0);
-      const int64_t least = TM * TN >= 16 || 8 * blocks <= cus ? 65536 : 196608;
+      const int64_t least = TM * TN >= 16 || 8 * blocks <= cus ? 65536 : RBC == 8 ? 131072 : 196608;
       kslices = std::min<int64_t>(std::min<int64_t>(max_k_slices, cus / blocks), share / least);
     }
     kslices = std::max<int64_t>(1, std::min<int64_t>(kslices, a.steps / 16));
@@ -471,6 +472,11 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
 //     not cached: s4 4 x 4096 x 16384 11.1 / 15.5 / 15.1; s8 8-byte rows 16 x 2048 x
 //     4096 6.5 / 6.8 / 8.4; f16 4 x 4096 x 4096 9.0 / 9.8 / 11.0; f8 4 x 10240 x 4096
 //     10.6 / 10.8 / 11.8;
+//   * 16 columns over four waves where there are more such blocks than units and K is
+//     short, eight steps and less a wave: these are stores and launches of waves (f32 16
+//     x 6144 x 1024 6.7, 7.8 in 32 columns; s8 32 x 7168 x 1536 4.9 / 5.6; s8 8-byte rows
+//     16 x 10240 x 512 4.2, 5.6 in eight waves). The K up to which they are ahead was
+//     measured for each number of rows and row width on 4352 to 20480 columns;
 //   * else 32 columns a workgroup over four waves: s8 4 x 6144 x 16384 20.8 against
 //     21.2, 32 x 14336 x 4096 15 % and 64 x 14336 x 4096 20 to 40 % ahead (a second
 //     column block shares the rows' loads).
@@ -485,6 +491,15 @@ int launch_thin_rows(const Problem& p, bool swapped, int64_t wide_cols, hipStrea
   const int64_t cus = std::max(compute_units(), 1);
   const int64_t blocks16 = row_blocks * uk::ceil_div(wide_cols, (int64_t)16);
   const int64_t blocks32 = row_blocks * uk::ceil_div(wide_cols, (int64_t)32);
+  constexpr bool kInteger = std::is_same<typename ElemTraits<E>::Acc, v4i>::value;
+  constexpr int64_t kShort = E == Elem::kF32 || TM == 1 ? 4096
+                             : TM == 2                  ? (RBC == 8 ? 1024 : 2560)
+                             : H == 2                   ? 0
+                                                        : (RBC == 8 ? 512 : 1536);
+  // (Where eight waves would take a float's K in 32 parts, they do.)
+  const int64_t short_k = blocks32 < cus ? kShort : TM == 1 && kInteger ? 1024 : 0;
+  if (blocks16 > cus && ((int64_t)p.K1 << p.lrb) <= short_k)
+    return launch_thin<E, RBC, TM, 1, 4, 4>(p, swapped, stream, true);
   const bool narrow = blocks16 <= cus ||
                       (TM == 1 && uk::ceil_div(blocks16, cus) < 2 * uk::ceil_div(blocks32, cus));
   if (narrow) return launch_thin<E, RBC, TM, 1, 8, TM == 1 && H == 1 ? 4 : 2>(p, swapped, stream, true);
