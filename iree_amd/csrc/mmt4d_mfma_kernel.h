@@ -232,6 +232,15 @@ __device__ __forceinline__ void wait_vmem_in_flight() {
 }
 // Waits for the wave's LDS reads (and scalar loads), not for vector memory.
 __device__ __forceinline__ void wait_lds_reads() { __builtin_amdgcn_s_waitcnt(0xC07F); }
+// Twelve issue slots: as many as have to lie between a matrix instruction and one that
+// reads its result in another pipe (8 after a product of 8- and 16-bit elements, 10 of
+// f32, 12 of 8-bit floats), where control flow comes between the two. The compiler
+// inserts what it finds missing, but looks along one of several paths only.
+__device__ __forceinline__ void settle_products() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_nop 11");
+  __builtin_amdgcn_sched_barrier(0);
+}
 // LDS stages of PIPE 5: twice as many where K is in slices, whose blocks have a compute
 // unit to themselves and weights that come from HBM (us, in 4 / 8 stages: f8 512 x 4096 x
 // 8192 in two slices 37.0 / 31.8, bf16 100 x 14336 x 4096 37.6 / 36.3).
@@ -1649,6 +1658,7 @@ void mmt4d_mfma_kernel(Args a) {
     // LDS goes to the next workgroup on the CU).
     wait_vmem_in_flight<0>();
   }
+  settle_products();
   if constexpr (TWO_SUMS) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)

@@ -368,17 +368,26 @@ void mmt4d_thin_kernel(Args a) {
       load_step(u % D, i + u + D);
     }
   }
+  // The products of the last steps: a chain's sum is read, to be added up or copied, soon
+  // after them, and the compiler counts the instructions that have to lie in between
+  // along the longer of two paths through `if (compute) { if (load) }` (too few on the
+  // shorter one: sums without their last product). So they lie behind the product itself.
+  auto compute_last = [&](int d, int c, int i) {
+    compute(d, c, i);
+    if constexpr (CHAINS > 1) settle_products();
+  };
   // Fewer than U + D steps left: the same with bounds.
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (i + u < my_steps) {
-      compute(u % D, u % CHAINS, i + u);
+      compute_last(u % D, u % CHAINS, i + u);
       if (i + u + D < my_steps) load_step(u % D, i + u + D);
     }
   }
 #pragma unroll
   for (int u = U; u < U + D; ++u)
-    if (i + u < my_steps) compute(u % D, u % CHAINS, i + u);
+    if (i + u < my_steps) compute_last(u % D, u % CHAINS, i + u);
+  settle_products();
 #pragma unroll
   for (int c = 1; c < CHAINS; ++c)
 #pragma unroll

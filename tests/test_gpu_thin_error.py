@@ -61,3 +61,31 @@ def test_error_of_few_columns(gpu, dtype, rows, cols, k, groups, swapped):
     want = a @ b.T
     bound = 1.08 * _error(_chains(torch, a, b, unit, 64 // elem, 4, groups), want)
     assert _error(got, want) <= bound, (_error(got, want), bound)
+
+
+@pytest.mark.parametrize("flags,t,tout,k0", [
+    (uk.MMT4D_TYPE_F16F16F32, "float16", "float32", 8), (uk.MMT4D_TYPE_F32F32F32, "float32", "float32", 4),
+    (uk.MMT4D_TYPE_F32F32F32, "float32", "float32", 2),
+    (uk.MMT4D_TYPE_F16F16F16 | uk.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS, "float16", "float16", 8),
+    (uk.MMT4D_TYPE_BF16BF16BF16 | uk.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS, "bfloat16", "bfloat16", 4)])
+@pytest.mark.parametrize("rows", [16, 48])
+def test_the_last_products_of_every_chain_count(gpu, flags, t, tout, k0, rows):
+    """Every number of steps a wave's chains end with, on small integers: equal to the
+    product. (The matrix instructions' results were read a few cycles early where control
+    flow lay in between.)"""
+    lib, torch = gpu
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    cols, t, tout = (512 if rows == 16 else 4000), getattr(torch, t), getattr(torch, tout)
+    step = 64 // t.itemsize
+    gen = torch.Generator(device="cuda"); gen.manual_seed(rows)
+    a, b = (torch.randint(-2, 3, (r, 104 * step), generator=gen, device="cuda") for r in (rows, cols))
+    for steps in range(9, 105):
+        k = steps * step
+        lhs, rhs = (x[:, :k].view(-1, 16, k // k0, k0).permute(0, 2, 1, 3).contiguous().to(t) for x in (a, b))
+        out = torch.zeros(rows, cols, device="cuda", dtype=tout)
+        torch.cuda.synchronize()
+        lib.mmt4d_unpack(lhs.data_ptr(), 0, 16 * k, rhs.data_ptr(), 0, 16 * k, out.data_ptr(), 0, cols, rows, cols,
+                         rows // 16, cols // 16, k // k0, 16, 16, k0, flags)
+        lib.synchronize()
+        want = (a[:, :k].float() @ b[:, :k].float().T).to(tout)
+        assert torch.equal(out, want), (steps, lib.last_kernel_name())
