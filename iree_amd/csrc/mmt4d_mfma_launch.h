@@ -600,9 +600,10 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 // Problems whose 64x64 blocks leave compute units idle or take a last round that is
 // nearly empty: the barrier-free kernel in 16x16 or 32x32 blocks, several waves of a
 // block sharing K, so that the chain of K steps a wave walks through is short and many
-// more loads are in flight than one workgroup a unit keeps. `b64` / `b128`: which
-// kernel it would be otherwise. Any K, any tile rows. Returns a HIP status, or -1 where
-// those kernels are the better ones. us before / in these blocks, same buffers:
+// more loads are in flight than one workgroup a unit keeps. `b128`, `ksplit64`: whether
+// it would be the 128x128 kernels or the 64x64 K split otherwise (else 64x64). Any K, any
+// tile rows. Returns a HIP status, or -1 where those kernels are the better ones. us
+// before / in these blocks, same buffers:
 //   one 16x16 block a unit or fewer, from 256 bytes of K (rows under 16 bytes: 64):
 //     f16 220 x 215, K 512 B 4.5 / 4.2, 2 KB 6.8 / 4.2, 7.6 KB 14.9 / 5.4; s8 16x16x2
 //     128 x 512, 100 B 4.4 / 3.8, 1 KB 6.5 / 4.0; f32 16x16x1 220 x 215, 3 KB 22.1 /
@@ -610,14 +611,15 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 //   two 32x32 blocks a unit or fewer, from 1 KB (f32: 256 B): s8 500 x 500, 3.8 KB
 //     9.6 / 6.5; f16 512 x 1024, 1 KB 5.5 / 5.3, 7.6 KB 15.7 / 13.6; bf16 16x16x2 500 x
 //     500, 1 KB 6.8 / 5.3 (rows of 2 bytes load an element at a time: one block a unit,
-//     s8 16x16x2 500 x 500, 3.8 KB 13.9 / 10.6, 512 x 1024 14.1 / 13.7);
-//   f32, whose MFMAs are slow enough to hide the loads of 32x32 blocks, wherever these
-//     are fewer than 7/2 (64x64) or 14 (128x128) for each block slot of the other
-//     kernel's rounds: 16x16x1 515 x 1027, 3 KB 22.6 / 17.5, 1500 x 1500 54.3 / 46.2, 3000
-//     x 3000 166 / 153, 8 KB 405 / 322; 16x16x4 1000 x 1500, 3 KB 28.5 / 25.3; but 2000 x
-//     1000, two full rounds of 64x64, 37.3 / 39.5, 4096 x 2048 110 / 137.
+//     s8 16x16x2 500 x 500, 3.8 KB 13.9 / 10.6, 512 x 1024 14.1 / 13.7); 8-bit floats up to
+//     7/4 blocks a unit (139 x 3012, 4 KB, 1.86 blocks 9.2 / 12.3);
+//   f32, whose MFMAs are slow enough to hide the loads of 32x32 blocks, by costs fitted to
+//     483 products of 100 to 6000 rows and columns, 256 B to 28 KB of K: 16x16x1 515 x 1027,
+//     3 KB 22.6 / 17.5, 1500 x 1500 54.3 / 46.2, 3000 x 3000, 8 KB 405 / 322; 16x16x4 1000 x
+//     1500, 3 KB 28.5 / 25.3; but 893 x 4064, 13.5 KB 203 / 245. With more than 1 KB of K also
+//     where they are estimated up to 5 % behind: their sums are in twice the parts and more.
 template <Elem E, int RBC>
-int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, hipStream_t stream,
+int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, bool ksplit64, hipStream_t stream,
                         const char** name) {
   constexpr bool F32 = E == Elem::kF32;
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
@@ -638,13 +640,26 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
       if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
       return st;
     }
-    const int64_t slots = uk::ceil_div(b128 ? workgroups(p, 128, 128) : workgroups(p, 64, 64), cus) * cus;
-    if (2 * b32 > (b128 ? 28 : 7) * slots) return -1;
-    // From four blocks a unit on two waves a block are enough.
-    st = b32 >= 4 * cus ? launch_thin<E, RBC, 2, 2, 2, 2, true>(p, false, stream)
-                        : launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
+    // us, by the KB of K and the blocks a unit: of these blocks in four waves, in two (which
+    // are enough from four blocks a unit on, but not as precise as the 64x64 K split), and
+    // of the kernel that it would be otherwise.
+    const double kb = (double)k_bytes / 1024, u = (double)b32 / (double)cus;
+    const double r64 = (double)uk::ceil_div(workgroups(p, 64, 64), cus);
+    const double r128 = (double)uk::ceil_div(workgroups(p, 128, 128), cus);
+    const double four = 3.3 + 0.6 * u + kb * (0.6 + 1.1 * u);
+    const double two = b32 >= 4 * cus && !ksplit64 ? 3.5 + 0.4 * u + kb * (2 + 0.97 * u) : four;
+    const double other = b128            ? (RBC < 16 ? 3 + 5 * r128 + kb * (5.5 + 13 * r128)
+                                                     : 3.5 + 2.5 * r128 + kb * (1.1 + 13.6 * r128))
+                         : ksplit64      ? 3.5 + 3 * r64 + kb * (0.3 + 3.6 * r64)
+                         : RBC >= 16     ? 3 + 0.8 * r64 + kb * (0.5 + 3.7 * r64)
+                         : k_bytes <= 8192 ? 3 + 0.8 * r64 + kb * (0.8 + 4.6 * r64)
+                                         : 3.2 + kb * (2.2 + 3.6 * r64);
+    if (std::min(four, two) > (ksplit64 ? 0.95 : k_bytes <= 1024 ? 1.02 : 1.05) * other) return -1;
+    st = two < four ? launch_thin<E, RBC, 2, 2, 2, 2, true>(p, false, stream)
+                    : launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
   } else {
-    if (b32 > (RBC == 2 ? 1 : 2) * cus || k_bytes < 1024) return -1;
+    // (8-bit floats, two loads an operand: 7/4 blocks a unit. Rows of 2 bytes: one.)
+    if (4 * b32 > (RBC == 2 ? 4 : ElemTraits<E>::kHalves == 2 ? 7 : 8) * cus || k_bytes < 1024) return -1;
     st = launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
   }
   if (st >= 0) *name = "mmt4d_mfma_32x32_ksplit";
@@ -1030,7 +1045,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   }
   if (forced == 0 && (choice == 3 || (choice == 6 && (!long_k || E == Elem::kF32)) || (RBC < 8 && choice == 4) ||
                       (choice == 2 && E == Elem::kF32))) {
-    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, stream, name);
+    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, stream, name);
     if (st >= 0) return st;
   }
   if (choice == 6) {
@@ -1062,7 +1077,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       int st = thin_launch(std::true_type{}, cols_n, rows_m);
       if (st >= 0) { *name = "mmt4d_mfma_thin_transposed"; return st; }
       // (K ends inside a step)
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, stream, name);
       if (st >= 0) return st;
     }
     choice = 3;
@@ -1071,7 +1086,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if constexpr (RBC >= 8) {
       int st = thin_launch(std::false_type{}, rows_m, cols_n);
       if (st >= 0) { *name = "mmt4d_mfma_thin"; return st; }
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, stream, name);
       if (st >= 0) return st;
     }
     // With 2-byte rows a 16-byte piece spans 8 rows and 32 rows do not fill a
