@@ -335,7 +335,7 @@ int launch_narrow(const Problem& p, int kt_count, hipStream_t stream) {
 // (out^T = rhs * lhs^T): the kernel's rows are the caller's columns.
 // A K that ends inside a step is served where TAIL_OK says that there is an
 // instance for it.
-template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool TAIL_OK = false>
+template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool TAIL_OK = false, int CH = 0>
 int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool allow_k_slices = false,
                 int max_k_slices = 8) {
   constexpr int OBYTES = ElemTraits<E>::Out::kOutBytes;
@@ -448,8 +448,8 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
     // by several row blocks here, which then wait for HBM one after the other (64x64
     // blocks, ordinary / non-temporal us: f16 200 x 8192 x 4096 34.6 / 44.5, s8 80 x 8192 x
     // 8192 21.4 / 25.0, 128 x 4096 x 14336 34.9 / 35.6; at best f8 192 x 4096 x 8192 21.6 / 21.1).
-    if (tail) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, true>, grid, block, 0, stream, a);
-    else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D>, grid, block, 0, stream, a);
+    if (tail) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, true, CH>, grid, block, 0, stream, a);
+    else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, CH>, grid, block, 0, stream, a);
     return (int)hipGetLastError();
   }
   // Weights that the caller has declared streamed, when they are too large for
@@ -602,7 +602,10 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 // block sharing K, so that the chain of K steps a wave walks through is short and many
 // more loads are in flight than one workgroup a unit keeps. `b128`, `ksplit64`: whether
 // it would be the 128x128 kernels or the 64x64 K split otherwise (else 64x64). Any K, any
-// tile rows. Returns a HIP status, or -1 where those kernels are the better ones. us
+// tile rows. Returns a HIP status, or -1 where those kernels are the better ones. `parts`
+// (f32): that K split would have K in workgroups too, up to 128 parts; up to three 16x16
+// blocks a unit then have it in four or eight waves of sixteen chains, and as small an error
+// (128 x 128 x 6144 41 us, 1.77e-7 / 11.3, 1.56e-7; 128 x 1024 x 6144 31.8 / 22.5). us
 // before / in these blocks, same buffers:
 //   one 16x16 block a unit or fewer, from 256 bytes of K (rows under 16 bytes: 64):
 //     f16 220 x 215, K 512 B 4.5 / 4.2, 2 KB 6.8 / 4.2, 7.6 KB 14.9 / 5.4; s8 16x16x2
@@ -619,8 +622,8 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 //     1500, 3 KB 28.5 / 25.3; but 893 x 4064, 13.5 KB 203 / 245. With more than 1 KB of K also
 //     where they are estimated up to 5 % behind: their sums are in twice the parts and more.
 template <Elem E, int RBC>
-int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, bool ksplit64, hipStream_t stream,
-                        const char** name) {
+int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, bool ksplit64, bool parts,
+                        hipStream_t stream, const char** name) {
   constexpr bool F32 = E == Elem::kF32;
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
   const int64_t cus = compute_units();
@@ -628,6 +631,15 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
   const int64_t b16 = uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16);
   const int64_t b32 = uk::ceil_div(rows, (int64_t)32) * uk::ceil_div(cols, (int64_t)32);
   int st = -1;
+  if constexpr (F32) {
+    if (parts) {
+      if (b16 > 3 * cus) return -1;
+      st = b16 <= cus ? launch_thin<E, RBC, 1, 1, 8, 4, true, 16>(p, false, stream)
+                      : launch_thin<E, RBC, 1, 1, 4, 4, true, 16>(p, false, stream);
+      if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
+      return st;
+    }
+  }
   if (b16 <= cus && k_bytes >= (RBC < 16 ? 64 : 256)) {
     st = launch_thin<E, RBC, 1, 1, F32 ? 4 : 8, F32 ? 4 : 2, true>(p, false, stream);
     if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
@@ -1043,9 +1055,11 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       if (st >= 0) { *name = "mmt4d_mfma_128x128_kslices"; return st; }
     }
   }
-  if (forced == 0 && (choice == 3 || (choice == 6 && (!long_k || E == Elem::kF32)) || (RBC < 8 && choice == 4) ||
+  const bool splits_k = long_k && (E != Elem::kF32 || 2 * workgroups(p, 64, 64) <= compute_units());
+  if (forced == 0 && (choice == 3 || (choice == 6 && (!splits_k || E == Elem::kF32)) || (RBC < 8 && choice == 4) ||
                       (choice == 2 && E == Elem::kF32))) {
-    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, stream, name);
+    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, choice == 6 && splits_k, stream,
+                                              name);
     if (st >= 0) return st;
   }
   if (choice == 6) {
@@ -1077,7 +1091,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       int st = thin_launch(std::true_type{}, cols_n, rows_m);
       if (st >= 0) { *name = "mmt4d_mfma_thin_transposed"; return st; }
       // (K ends inside a step)
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, stream, name);
       if (st >= 0) return st;
     }
     choice = 3;
@@ -1086,7 +1100,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if constexpr (RBC >= 8) {
       int st = thin_launch(std::false_type{}, rows_m, cols_n);
       if (st >= 0) { *name = "mmt4d_mfma_thin"; return st; }
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, stream, name);
       if (st >= 0) return st;
     }
     // With 2-byte rows a 16-byte piece spans 8 rows and 32 rows do not fill a

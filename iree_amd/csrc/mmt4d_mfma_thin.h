@@ -68,11 +68,24 @@ __device__ __forceinline__ int load4(const char* p) {
   else return *reinterpret_cast<const int_g*>(p);
 }
 
+// Sums of floats whose K eight waves share are in several chains, steps i, i + chains, ..
+// of a wave apart: as many parts of K and more, each a shorter chain of roundings, as four
+// waves in up to eight workgroups add up. Error against 64 bits of 32 x 512 results in one
+// chain / here / in those workgroups, 1e-7: f16, K = 4096 1.56 / 1.03 / 1.03; f32, K = 2048
+// 2.94 / 1.60 / 1.59. (The matrix instructions of 8-bit floats round to 1.5e-5 by
+// themselves, however K is divided.)
+template <Elem E, int TM, int KSPLIT>
+constexpr int thin_chains() {
+  using TT = ElemTraits<E>;
+  return KSPLIT < 8 || TT::kHalves == 2 || std::is_same<typename TT::Acc, v4i>::value ? 1 : TM == 1 ? 4 : 2;
+}
+
 // STREAMED: the wide operand (the kernel's RHS: weights) is loaded
 // non-temporally. For callers that say their weights come from HBM every time
 // (iree_uk_amd_set_streamed_weights): a layer's weights then pass through the
 // caches without displacing what is used again.
-template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false, bool TAIL = false>
+// CH: chains of a wave's sums (0: thin_chains).
+template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false, bool TAIL = false, int CH = 0>
 __global__ __launch_bounds__(KSPLIT * 64)
 void mmt4d_thin_kernel(Args a) {
   using TT = ElemTraits<E>;
@@ -84,13 +97,7 @@ void mmt4d_thin_kernel(Args a) {
   constexpr int KS = NCH * 16;                // bytes of K per row per step
   constexpr int PIECES = RBC >= 16 ? 1 : 16 / RBC;   // loads per 16-byte operand
   constexpr bool S4 = E == Elem::kS8S4;       // 4-bit RHS: half the bytes per row
-  // Sums of floats whose K eight waves share are in several chains, steps i, i +
-  // CHAINS, .. of a wave apart: as many parts of K and more, each a shorter chain of
-  // roundings, as four waves in up to eight workgroups add up. Error against 64 bits of
-  // 32 x 512 results in one chain / here / in those workgroups, 1e-7: f16, K = 4096 1.56 /
-  // 1.03 / 1.03; f32, K = 2048 2.94 / 1.60 / 1.59. (The matrix instructions of 8-bit
-  // floats round to 1.5e-5 by themselves, however K is divided.)
-  constexpr int CHAINS = KSPLIT < 8 || HALVES == 2 || std::is_same<Acc, v4i>::value ? 1 : TM == 1 ? 4 : 2;
+  constexpr int CHAINS = CH > 0 ? CH : thin_chains<E, TM, KSPLIT>();
   static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
   static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
 
