@@ -50,6 +50,7 @@ namespace uk_mfma {
 typedef int v2i __attribute__((ext_vector_type(2)));
 typedef v2i v2i_g __attribute__((aligned(1)));  // as v4i_g: read from global memory at any address
 typedef int int_g __attribute__((aligned(1)));
+typedef short short_g __attribute__((aligned(1)));
 
 // 16, 8 and 4 bytes from any address, non-temporally if NT.
 template <bool NT>
@@ -184,7 +185,7 @@ void mmt4d_thin_kernel(Args a) {
       typedef short short8 __attribute__((ext_vector_type(8)));
       short8 v;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) v[t] = *reinterpret_cast<const short*>(at(t));
+      for (int t = 0; t < 8; ++t) v[t] = *reinterpret_cast<const short_g*>(at(t));
       return __builtin_bit_cast(v4i, v);
     }
   };

@@ -148,3 +148,21 @@ def test_f32_errors_are_not_above_those_of_the_k_split(gpu, m, n, k):
     finally:
         lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
     assert errors[0] <= errors[1], errors
+
+
+@pytest.mark.parametrize("k0", [2, 4, 16])
+def test_operands_at_odd_addresses(gpu, k0):
+    lib, torch = gpu
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    m, n, k = 128, 208, 1040
+    gen = torch.Generator(device="cuda"); gen.manual_seed(k0)
+    a, b = (torch.randint(-128, 128, (r, k), generator=gen, device="cuda") for r in (m, n))
+    lhs, rhs = (torch.nn.functional.pad(x.view(-1, 16, k // k0, k0).permute(0, 2, 1, 3).reshape(-1).to(torch.int8), (3, 0))
+                for x in (a, b))
+    out = torch.zeros(m, n, device="cuda", dtype=torch.int32)
+    torch.cuda.synchronize()
+    lib.mmt4d_unpack(lhs.data_ptr(), 3, 16 * k, rhs.data_ptr(), 3, 16 * k, out.data_ptr(), 0, n, m, n, m // 16, n // 16,
+                     k // k0, 16, 16, k0, uk.MMT4D_TYPE_S8S8S32)
+    lib.synchronize()
+    assert "16x16_ksplit" in lib.last_kernel_name()
+    assert torch.equal(out, (a.double() @ b.double().T).int())
