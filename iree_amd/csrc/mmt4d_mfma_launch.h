@@ -134,6 +134,7 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
   };
   a.vec_out = vector_ok(p.out, p.out_stride, p.out_sm0, p.out_spn) &&
               (!accumulate || vector_ok(a.acc, a.acc_stride, a.acc_sm0, a.acc_spn));
+  if (a.vec_out && a.bpn * p.N0 % 4 != 0) a.vec_out = 2;
   // The launch that finishes K stores non-temporally when the output is
   // larger than the memory-side cache can hand to its reader.
   a.nt_out = kt_begin + kt_count == p.K1 &&
