@@ -762,6 +762,13 @@ void mmt4d_mfma_kernel(Args a) {
       __syncthreads();
     }
   } else if constexpr (PIPE == 4) {
+    // Where this instance's loop, 1.5 KB of products, lies in the instruction cache's lines
+    // decides over a quarter of its time, and moves with any change before it: f32 16x16x1
+    // 3582 x 3328 x 1792 375 us 20 bytes behind a multiple of 256, 452 to 458 at 0, 32, 64 and 96.
+    if constexpr (E == Elem::kF32 && RBC == 4 && TM == 4 && TN == 4) {
+      asm volatile(".p2align 8");
+      asm volatile(".fill 5, 4, 0xBF800000");   // s_nop 0
+    }
     // Two LDS stages as in PIPE 0, three register sets: iteration s issues the
     // global loads of step s+3 into the set that step s occupied, computes
     // step s from LDS and stores step s+1 (loaded two iterations ago) for the
