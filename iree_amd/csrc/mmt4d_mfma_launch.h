@@ -601,10 +601,10 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 // Problems whose 64x64 blocks leave compute units idle or take a last round that is
 // nearly empty: the barrier-free kernel in 16x16 or 32x32 blocks, several waves of a
 // block sharing K, so that the chain of K steps a wave walks through is short and many
-// more loads are in flight than one workgroup a unit keeps. `b128`, `ksplit64`: whether
-// it would be the 128x128 kernels or the 64x64 K split otherwise (else 64x64). Any K, any
-// tile rows. Returns a HIP status, or -1 where those kernels are the better ones. `parts`
-// (f32): that K split would have K in workgroups too, up to 128 parts; up to three 16x16
+// more loads are in flight than one workgroup a unit keeps. `b128`, `ksplit64`, `b32x64`:
+// whether it would be the 128x128 kernels, the 64x64 K split (or what takes its place) or
+// 32x64 blocks through LDS otherwise (else 64x64). Any K, any tile rows. Returns a HIP
+// status, or -1 where those kernels are the better ones. `parts` (f32): that K split would have K in workgroups too, up to 128 parts; up to three 16x16
 // blocks a unit then have it in four or eight waves of sixteen chains, and as small an error
 // (128 x 128 x 6144 41 us, 1.77e-7 / 11.3, 1.56e-7; 128 x 1024 x 6144 31.8 / 22.5). us
 // before / in these blocks, same buffers:
@@ -616,15 +616,16 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 //     9.6 / 6.5; f16 512 x 1024, 1 KB 5.5 / 5.3, 7.6 KB 15.7 / 13.6; bf16 16x16x2 500 x
 //     500, 1 KB 6.8 / 5.3 (rows of 2 bytes load an element at a time: one block a unit,
 //     s8 16x16x2 500 x 500, 3.8 KB 13.9 / 10.6, 512 x 1024 14.1 / 13.7); 8-bit floats up to
-//     7/4 blocks a unit (139 x 3012, 4 KB, 1.86 blocks 9.2 / 12.3);
+//     7/4 blocks a unit (139 x 3012, 4 KB, 1.86 blocks 9.2 / 12.3), 5/4 from 6 KB on (212 x
+//     1280, 7.1 KB, 1.1 blocks 13.9 / 11.1; 235 x 1631, 11.9 KB, 1.6 blocks 22.2 / 29.0);
 //   f32, whose MFMAs are slow enough to hide the loads of 32x32 blocks, by costs fitted to
-//     483 products of 100 to 6000 rows and columns, 256 B to 28 KB of K: 16x16x1 515 x 1027,
-//     3 KB 22.6 / 17.5, 1500 x 1500 54.3 / 46.2, 3000 x 3000, 8 KB 405 / 322; 16x16x4 1000 x
-//     1500, 3 KB 28.5 / 25.3; but 893 x 4064, 13.5 KB 203 / 245. With more than 1 KB of K also
-//     where they are estimated up to 5 % behind: their sums are in twice the parts and more.
+//     1500 products of 64 to 4096 rows and columns, 256 B to 32 KB of K (3 to 10 % off in the
+//     mean; the choice is 1.8 % behind the fastest in the geometric mean, 21 calls are more
+//     than 4 % behind the kernel otherwise): 16x16x1 515 x 1027, 3 KB 22.6 / 17.5, 1500 x 1500
+//     54.3 / 46.2, 3000 x 3000, 8 KB 405 / 322; 16x16x4 1000 x 1500, 3 KB 28.5 / 25.3; but 893 x 4064, 13.5 KB 203 / 245, 16x16x1 1879 x 1045, 1.7 KB 25.0 / 28.0.
 template <Elem E, int RBC>
 int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, bool ksplit64, bool parts,
-                        hipStream_t stream, const char** name) {
+                        bool b32x64, hipStream_t stream, const char** name) {
   constexpr bool F32 = E == Elem::kF32;
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
   const int64_t cus = compute_units();
@@ -653,26 +654,31 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
       if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
       return st;
     }
-    // us, by the KB of K and the blocks a unit: of these blocks in four waves, in two (which
-    // are enough from four blocks a unit on, but not as precise as the 64x64 K split), and
-    // of the kernel that it would be otherwise.
-    const double kb = (double)k_bytes / 1024, u = (double)b32 / (double)cus;
+    // us, by the KB of K and the rounds of blocks: of these blocks in four waves, in two (not
+    // as precise as the 64x64 K split, and not in its place), and of the kernel that it would
+    // be otherwise.
+    const double kb = (double)k_bytes / 1024, r32 = (double)uk::ceil_div(b32, cus);
     const double r64 = (double)uk::ceil_div(workgroups(p, 64, 64), cus);
     const double r128 = (double)uk::ceil_div(workgroups(p, 128, 128), cus);
-    const double four = 3.3 + 0.6 * u + kb * (0.6 + 1.1 * u);
-    const double two = b32 >= 4 * cus && !ksplit64 ? 3.5 + 0.4 * u + kb * (2 + 0.97 * u) : four;
-    const double other = b128            ? (RBC < 16 ? 3 + 5 * r128 + kb * (5.5 + 13 * r128)
-                                                     : 3.5 + 2.5 * r128 + kb * (1.1 + 13.6 * r128))
-                         : ksplit64      ? 3.5 + 3 * r64 + kb * (0.3 + 3.6 * r64)
-                         : RBC >= 16     ? 3 + 0.8 * r64 + kb * (0.5 + 3.7 * r64)
-                         : k_bytes <= 8192 ? 3 + 0.8 * r64 + kb * (0.8 + 4.6 * r64)
-                                         : 3.2 + kb * (2.2 + 3.6 * r64);
-    if (std::min(four, two) > (ksplit64 ? 0.95 : k_bytes <= 1024 ? 1.02 : 1.05) * other) return -1;
+    const double four = RBC >= 16 ? 3.6 + 0.5 * r32 + kb * (0.13 + 1.09 * r32)
+                                  : 3.3 + 0.7 * r32 + kb * (0.37 + 1.28 * r32);
+    const double two = ksplit64    ? four
+                       : RBC >= 16 ? 3.75 + 0.33 * r32 + kb * (1.56 + 0.99 * r32)
+                                   : 3.5 + 0.43 * r32 + kb * (2.6 + 1.13 * r32);
+    const double other = b128              ? (RBC < 16 ? 5 + 3.6 * r128 + kb * (4 + 14.7 * r128)
+                                                       : 3 + 3.4 * r128 + kb * (2.4 + 13.65 * r128))
+                         : ksplit64        ? 6.7 + 1.1 * r64 + kb * 4 * r64
+                         : RBC >= 16       ? 3.4 + 0.7 * r64 + kb * (0.63 + 3.9 * r64)
+                         : k_bytes <= 8192 ? 2.9 + 1.9 * r64 + kb * (1.2 + 4.56 * r64)
+                                           : 4.3 + kb * (2 + 3.95 * r64);
+    if (b32x64 ? 2 * b32 > 7 * (int64_t)r64 * cus : std::min(four, two) > 1.02 * other) return -1;
     st = two < four ? launch_thin<E, RBC, 2, 2, 2, 2, true>(p, false, stream)
                     : launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
   } else {
-    // (8-bit floats, two loads an operand: 7/4 blocks a unit. Rows of 2 bytes: one.)
-    if (4 * b32 > (RBC == 2 ? 4 : ElemTraits<E>::kHalves == 2 ? 7 : 8) * cus || k_bytes < 1024) return -1;
+    // (8-bit floats, two loads an operand: 7/4 blocks a unit, 5/4 with 6 KB of K and more,
+    // but in the place of 32x64 blocks. Rows of 2 bytes: one.)
+    const int64_t most4 = RBC == 2 ? 4 : ElemTraits<E>::kHalves == 2 && !b32x64 ? (ksplit64 ? 5 : 7) : 8;
+    if (4 * b32 > most4 * cus || k_bytes < 1024) return -1;
     st = launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
   }
   if (st >= 0) *name = "mmt4d_mfma_32x32_ksplit";
@@ -1059,8 +1065,8 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   const bool splits_k = long_k && (E != Elem::kF32 || 2 * workgroups(p, 64, 64) <= compute_units());
   if (forced == 0 && (choice == 3 || (choice == 6 && (!splits_k || E == Elem::kF32)) || (RBC < 8 && choice == 4) ||
                       (choice == 2 && E == Elem::kF32))) {
-    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, choice == 6 && splits_k, stream,
-                                              name);
+    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, choice == 6 && splits_k,
+                                               choice == 4 && RBC != 2, stream, name);
     if (st >= 0) return st;
   }
   if (choice == 6) {
@@ -1092,7 +1098,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       int st = thin_launch(std::true_type{}, cols_n, rows_m);
       if (st >= 0) { *name = "mmt4d_mfma_thin_transposed"; return st; }
       // (K ends inside a step)
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, true, stream, name);
       if (st >= 0) return st;
     }
     choice = 3;
@@ -1101,7 +1107,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if constexpr (RBC >= 8) {
       int st = thin_launch(std::false_type{}, rows_m, cols_n);
       if (st >= 0) { *name = "mmt4d_mfma_thin"; return st; }
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, false, stream, name);
       if (st >= 0) return st;
     }
     // With 2-byte rows a 16-byte piece spans 8 rows and 32 rows do not fill a

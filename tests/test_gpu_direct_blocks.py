@@ -1,4 +1,5 @@
-"""K slices whose workgroups do not divide evenly over the XCDs."""
+"""Which blocks f32 products of few rounds take, and K slices whose workgroups do not divide
+evenly over the XCDs."""
 import pytest
 
 from iree_amd import ukernel as uk
@@ -6,6 +7,8 @@ from iree_amd import ukernel as uk
 pytestmark = pytest.mark.gpu
 
 F16 = (uk.MMT4D_TYPE_F16F16F32, "float16", "float32")
+
+F32 = (uk.MMT4D_TYPE_F32F32F32, "float32", "float32")
 
 
 def _tiles(torch, x, m0, k0):
@@ -29,6 +32,21 @@ def _run(lib, torch, kind, a, b, m0, n0, k0):
 def _small(torch, rows, k, seed):
     gen = torch.Generator(device="cuda"); gen.manual_seed(seed)
     return torch.randint(-2, 3, (rows, k), generator=gen, device="cuda")
+
+
+@pytest.mark.parametrize("kind,tile,m,n,k,name", [
+    (F32, (16, 16, 4), 41, 12664, 855, "32x32_ksplit"),            # else 32x64 blocks
+    (F32, (16, 16, 1), 1879, 1045, 431, "64x64_deep")])
+def test_which_blocks(gpu, kind, tile, m, n, k, name):
+    lib, torch = gpu
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the rules count 256 compute units")
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    a, b = _small(torch, m, k, 1), _small(torch, n, k, 2)
+    out = _run(lib, torch, kind, a, b, *tile)
+    assert lib.last_kernel_name() == "mmt4d_mfma_" + name
+    want = (a.float() @ b.float().T).to(out.dtype)   # whole numbers below 2^24: exact
+    assert torch.equal(out, want)
 
 
 @pytest.mark.parametrize("m,n,slices", [(292, 768, 14), (292, 768, 13), (140, 200, 3), (130, 640, 5), (100, 128, 7)])
