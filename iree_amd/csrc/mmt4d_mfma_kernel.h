@@ -545,6 +545,19 @@ void mmt4d_mfma_kernel(Args a) {
   // contiguously). `vec_out` is 0 when that does not hold or the output is not
   // 16-byte aligned; elements then move one by one.
   Acc acc[TM][TN];
+  // 64x64 blocks of floats with K of 96 steps and more sum it in four parts, one after
+  // the other: as many, and as short chains of roundings, as four waves that share K
+  // (launch_class takes one kernel or the other by their times). Error against 64 bits,
+  // f16 2576 x 400 x 3280: one sum 3.6e-7, here 1.8e-7, those waves 1.9e-7; 1.5 % of the time.
+  constexpr bool IN_PARTS = PIPE == 3 && BM == 64 && BN == 64 && HALVES == 1 && E != Elem::kF32 &&
+                            !std::is_same<Acc, v4i>::value;
+  Acc parts[IN_PARTS ? TM : 1][IN_PARTS ? TN : 1];
+  if constexpr (IN_PARTS) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) parts[tm][tn] = Acc{0, 0, 0, 0};
+  }
   // Slices of a float product sum even and odd steps apart: two slices then add no
   // more terms one after the other than four waves that share K do.
   constexpr bool TWO_SUMS = SLICED && !std::is_same<Acc, v4i>::value;
@@ -580,6 +593,9 @@ void mmt4d_mfma_kernel(Args a) {
         const bool ok = pl < a.bpn && pn0 + pl < a.N1;
         const int left = a.out_cols - (col_origin + col);
         col_n[tn] = ok ? (left >= 4 ? 4 : (left > 0 ? left : 0)) : 0;
+        // (Tested for here: with the end of all columns taken as the nearer of the two, stores
+        // of a short K waited, f8 2792 x 7472 x 132 25.9 -> 27.7 us.)
+        if (a.vec_out == 2) col_n[tn] = min(col_n[tn], a.bpn * a.N0 - col);
         col_off[tn] = (uint32_t)pl * s_pn + (uint32_t)n0 * OB;
       }
 #pragma unroll
@@ -596,9 +612,6 @@ void mmt4d_mfma_kernel(Args a) {
             // the matrix ends inside this group of four columns
 #pragma unroll
             for (int e = 0; e < 3; ++e)
-        // (Tested for here: with the end of all columns taken as the nearer of the two, stores
-        // of a short K waited, f8 2792 x 7472 x 132 25.9 -> 27.7 us.)
-        if (a.vec_out == 2) col_n[tn] = min(col_n[tn], a.bpn * a.N0 - col);
               if (e < col_n[tn]) f1(tm, tn, e, out_base + (row_off + col_off[tn] + e * OB));
           }
         }
@@ -749,6 +762,13 @@ void mmt4d_mfma_kernel(Args a) {
     load_global(regs, 0, has_tail && last == 0);
     store_lds(regs, 0);
     __syncthreads();
+    // Where this instance's loop, 1.5 KB of products, lies in the instruction cache's lines
+    // decides over a quarter of its time, and moves with any change before it: f32 16x16x1
+    // 3582 x 3328 x 1792 375 us 20 bytes behind a multiple of 256, 452 to 458 at 0, 32, 64 and 96.
+    if constexpr (E == Elem::kF32 && RBC == 4 && TM == 4 && TN == 4) {
+      asm volatile(".p2align 8");
+      asm volatile(".fill 5, 4, 0xBF800000");   // s_nop 0
+    }
     for (int s = 0; s < a.steps; ++s) {
       const uint32_t cur = (s & 1) * STAGE;
       if (s < last) {
@@ -765,13 +785,6 @@ void mmt4d_mfma_kernel(Args a) {
       __syncthreads();
     }
   } else if constexpr (PIPE == 4) {
-    // Where this instance's loop, 1.5 KB of products, lies in the instruction cache's lines
-    // decides over a quarter of its time, and moves with any change before it: f32 16x16x1
-    // 3582 x 3328 x 1792 375 us 20 bytes behind a multiple of 256, 452 to 458 at 0, 32, 64 and 96.
-    if constexpr (E == Elem::kF32 && RBC == 4 && TM == 4 && TN == 4) {
-      asm volatile(".p2align 8");
-      asm volatile(".fill 5, 4, 0xBF800000");   // s_nop 0
-    }
     // Two LDS stages as in PIPE 0, three register sets: iteration s issues the
     // global loads of step s+3 into the set that step s occupied, computes
     // step s from LDS and stores step s+1 (loaded two iterations ago) for the
@@ -1119,7 +1132,23 @@ void mmt4d_mfma_kernel(Args a) {
         __syncthreads();
       };
       int s = 0;
+      // A part ends after a whole number of rounds of the phases.
+      const int part = IN_PARTS && steps >= 96 ? steps / 12 * 3 : INT_MAX;
+      int end = part;
       for (; s + 2 < steps; s += 3) {
+        if constexpr (IN_PARTS) {
+          if (s == end) {
+            end += part;
+            settle_products();
+#pragma unroll
+            for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+              for (int tn = 0; tn < TN; ++tn) {
+                parts[tm][tn] += acc[tm][tn];
+                acc[tm][tn] = Acc{0, 0, 0, 0};
+              }
+          }
+        }
         iteration(s, std::integral_constant<int, 0>{});
         iteration(s + 1, std::integral_constant<int, 1>{});
         iteration(s + 2, std::integral_constant<int, 2>{});
@@ -1672,6 +1701,12 @@ void mmt4d_mfma_kernel(Args a) {
     wait_vmem_in_flight<0>();
   }
   settle_products();
+  if constexpr (IN_PARTS) {
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn) acc[tm][tn] += parts[tm][tn];
+  }
   if constexpr (TWO_SUMS) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)

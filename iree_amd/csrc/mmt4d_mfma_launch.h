@@ -726,6 +726,26 @@ int slices_that_pay(const Problem& p, int64_t rows, int64_t cols, bool long_k) {
   return here < blocks ? (int)slices : 0;
 }
 
+// Whether 64x64 blocks with less than 8 KB of K, or with a K that ends inside a step, are
+// faster in the kernels that stage through LDS than with K over the waves of a block,
+// whose operands pass through the L1s twice as often: from about one block a unit on, 16-bit
+// results earlier, 8-bit floats always (their two loads an operand bound the K split). us
+// in them / K over the waves: f16 2159 x 786 x 3602 25.1 / 35.7, 3124 x 410 x 8936 55.9 / 82.2;
+// bf16 -> bf16 2308 x 521 x 3072 22.0 / 34.8; s8 2898 x 418 x 7936 26.8 / 38.0, 8-byte rows 1083
+// x 950 x 16353 37.8 / 42.6; f8 508 x 1287 x 6400 12.9 / 19.7. Up to one block a unit (results
+// of 2 bytes and 8-byte rows 3/4) K over the waves is 1.11
+// times as fast in the geometric mean of 69 calls, 0.85 at worst; 175 others 1.20 times as
+// fast in these kernels, 0.82 at worst.
+template <Elem E, int RBC>
+bool direct_before_ksplit(const Problem& p) {
+  constexpr bool kInteger = std::is_same<typename ElemTraits<E>::Acc, v4i>::value;
+  if (E == Elem::kF32 || !(RBC >= 16 || (RBC == 8 && kInteger))) return false;
+  const int64_t k_bytes = (int64_t)p.K1 << p.lrb, b64 = workgroups(p, 64, 64), cus = compute_units();
+  if (k_bytes >= 8192 && k_bytes % (64 * ElemTraits<E>::kHalves) == 0) return false;
+  if (ElemTraits<E>::kHalves == 2) return k_bytes < 24576 || 2 * b64 > cus;   // (else in workgroups, too)
+  return 8 * b64 > (ElemTraits<E>::Out::kOutBytes == 2 || RBC == 8 ? 6 : 8) * cus;
+}
+
 // Variant choice for row-bytes class RBC:
 //   big   256x256 workgroup tile, 8 waves of 128x64, software-pipelined, both
 //         operands through LDS-direct loads, any K; f32: RHS straight to
@@ -1070,6 +1090,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if (st >= 0) return st;
   }
   if (choice == 6) {
+  if (forced == 0 && choice == 6 && direct_before_ksplit<E, RBC>(p)) choice = 3;
     // Few 64x64 blocks and a long K: the barrier-free kernel with a 64x64
     // block per workgroup, whose four waves split K.
     if constexpr (RBC >= 8) {

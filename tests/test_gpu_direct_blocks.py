@@ -1,5 +1,6 @@
-"""Which blocks f32 products of few rounds take, and K slices whose workgroups do not divide
-evenly over the XCDs."""
+"""64x64 blocks with the right-hand side straight to registers in the place of a K split
+over waves: which calls take them, K in four parts one after the other (its ends, its
+errors), and K slices whose workgroups do not divide evenly over the XCDs."""
 import pytest
 
 from iree_amd import ukernel as uk
@@ -7,7 +8,9 @@ from iree_amd import ukernel as uk
 pytestmark = pytest.mark.gpu
 
 F16 = (uk.MMT4D_TYPE_F16F16F32, "float16", "float32")
-
+BF16 = (uk.MMT4D_TYPE_BF16BF16F32, "bfloat16", "float32")
+BF16BF16 = (uk.MMT4D_TYPE_BF16BF16BF16 | uk.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS, "bfloat16", "bfloat16")
+S8 = (uk.MMT4D_TYPE_S8S8S32, "int8", "int32")
 F32 = (uk.MMT4D_TYPE_F32F32F32, "float32", "float32")
 
 
@@ -35,6 +38,14 @@ def _small(torch, rows, k, seed):
 
 
 @pytest.mark.parametrize("kind,tile,m,n,k,name", [
+    (F16, (16, 16, 16), 2575, 394, 3273, "64x64_rhs_direct"),      # 287 blocks, K ends inside a step
+    (F16, (16, 16, 8), 1024, 1024, 3200, "64x64_ksplit"),          # one block a unit
+    (F16, (16, 16, 8), 1040, 1024, 3200, "64x64_rhs_direct"),
+    (F16, (16, 16, 8), 1040, 2048, 4096, "64x64_ksplit"),          # 8 KB in whole steps
+    (BF16BF16, (16, 16, 8), 768, 1024, 3200, "64x64_ksplit"),      # 3/4 of a block a unit
+    (BF16BF16, (16, 16, 8), 784, 1024, 3200, "64x64_rhs_direct"),
+    (S8, (16, 16, 16), 2898, 418, 7936, "64x64_rhs_direct"),
+    (S8, (32, 16, 8), 1083, 950, 16353, "64x64_lds_direct"),
     (F32, (16, 16, 4), 41, 12664, 855, "32x32_ksplit"),            # else 32x64 blocks
     (F32, (16, 16, 1), 1879, 1045, 431, "64x64_deep")])
 def test_which_blocks(gpu, kind, tile, m, n, k, name):
@@ -47,6 +58,52 @@ def test_which_blocks(gpu, kind, tile, m, n, k, name):
     assert lib.last_kernel_name() == "mmt4d_mfma_" + name
     want = (a.float() @ b.float().T).to(out.dtype)   # whole numbers below 2^24: exact
     assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("kind", [F16, BF16, BF16BF16])
+def test_every_step_of_the_parts_counts(gpu, kind):
+    """Numbers of steps around the first that are summed in parts (96) and around a multiple
+    of 12, whole steps and a K that ends inside one: equal to the product."""
+    lib, torch = gpu
+    lib.set_kernel_mode(uk.KERNEL_MODE_MFMA_VARIANT + 3)
+    try:
+        a, b = _small(torch, 70, 133 * 32, 3), _small(torch, 130, 133 * 32, 4)
+        for steps in (1, 2, 94, 95, 96, 97, 98, 99, 107, 108, 109, 131, 132):
+            for more in (0, 8):
+                k = steps * 32 + more
+                out = _run(lib, torch, kind, a[:, :k], b[:, :k], 16, 16, 8)
+                assert lib.last_kernel_name() == "mmt4d_mfma_64x64_rhs_direct"
+                assert torch.equal(out, (a[:, :k].float() @ b[:, :k].float().T).to(out.dtype)), (steps, more)
+    finally:
+        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+
+
+@pytest.mark.parametrize("kind", [F16, BF16])
+@pytest.mark.parametrize("k", [3264, 3280, 4008])
+def test_error_of_the_parts(gpu, kind, k):
+    """No larger than that of four chains of sums over a quarter of K each, which four waves
+    that share K have, added in order: the same chains on the CPU, rounded after every eight
+    products (16-bit floats are summed in groups), give the bound, 8 % are left for what is
+    fitted in that number. One chain over all of K has twice the error."""
+    lib, torch = gpu
+    gen = torch.Generator(); gen.manual_seed(k)
+    a, b = (torch.randn(r, k, generator=gen).to(getattr(torch, kind[1])) for r in (96, 128))
+    lib.set_kernel_mode(uk.KERNEL_MODE_MFMA_VARIANT + 3)
+    try:
+        got = _run(lib, torch, kind, a.cuda(), b.cuda(), 16, 16, 8).cpu()
+    finally:
+        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    a, b = a.double(), b.double()
+    want = a @ b.T
+    model = torch.zeros(96, 128)
+    ends = [k * i // 32 // 8 * 8 for i in (0, 8, 16, 24, 32)]
+    for lo, hi in zip(ends, ends[1:]):
+        part = torch.zeros(96, 128)
+        for i in range(lo, hi, 8):
+            part = (part.double() + a[:, i:i + 8] @ b[:, i:i + 8].T).float()
+        model += part
+    error = lambda x: float(((x.double() - want) ** 2).sum() / (want ** 2).sum()) ** 0.5  # noqa: E731
+    assert error(got) <= 1.08 * error(model), (error(got), error(model))
 
 
 @pytest.mark.parametrize("m,n,slices", [(292, 768, 14), (292, 768, 13), (140, 200, 3), (130, 640, 5), (100, 128, 7)])
