@@ -348,7 +348,10 @@ IREE_UK_AMD_EXPORT void iree_uk_amd_set_pointer_mode(int mode);
  *             6 = the 64x64 K-split kernel, 7 = 256x128, 8 = 128x512,
  *             9 / 10 = the persistent kernel in the 128x512 / 256x256 shape,
  *             11 = 64x64 with the deep pipeline, 12..15 = the narrow-row
- *             kernels in the 256x256 / 128x512 / 128x128 / 64x64 shapes)
+ *             kernels in the 256x256 / 128x512 / 128x128 / 64x64 shapes,
+ *             16 / 17 / 18 / 19 / 20 = the LDS-direct pipeline in the 256x256 /
+ *             128x512 / 128x128 / 64x64 / 256x128 shape, 21 = 128x128 blocks
+ *             over as many slices of K as iree_uk_amd_set_k_slices says)
  *             instead of choosing by problem size; pack/unpack as AUTO. */
 enum {
   IREE_UK_AMD_KERNEL_MODE_AUTO = 0,
@@ -397,10 +400,13 @@ IREE_UK_AMD_EXPORT uint64_t iree_uk_amd_mfma_decline_count(void);
 IREE_UK_AMD_EXPORT void iree_uk_amd_mmt4d_no_alloc(const iree_uk_mmt4d_params_t* params);
 IREE_UK_AMD_EXPORT int64_t iree_uk_amd_no_alloc_scratch_bytes(void);
 
-/* Tuning / test knob of the calling thread: into how many slices the M-thin /
- * N-thin mmt4d kernels split K across workgroups (0, the default: chosen from
- * the number of output blocks and compute units; 1: never). The slice count
- * the latest call used is iree_uk_amd_last_k_slices (1 = no split). */
+/* Tuning / test knob of the calling thread: into how many slices mmt4d splits K
+ * across workgroups. 0, the default: chosen from the sizes and the number of
+ * compute units. Any other value is what the M-thin / N-thin kernels, the 64x64
+ * K-split kernel and kernel variant 21 (128x128 blocks) take, where K is long
+ * enough for it (1: no split), and calls that choose by problem size then do not
+ * take those 128x128 blocks. The slice count the latest call used is
+ * iree_uk_amd_last_k_slices (1 = no split). */
 IREE_UK_AMD_EXPORT void iree_uk_amd_set_k_slices(int n);
 IREE_UK_AMD_EXPORT int iree_uk_amd_last_k_slices(void);
 
@@ -503,13 +509,13 @@ IREE_UK_AMD_EXPORT int64_t iree_uk_amd_staging_bytes(void);
 IREE_UK_AMD_EXPORT int iree_uk_amd_release_staging(void);
 
 /* Device buffers that iree_uk_mmt4d and iree_uk_conv_nchwc keep per calling
- * thread and stream beyond a call: the workspace of the thin kernels' K split
- * over workgroups (a few megabytes) and the buffer for operands the library
- * prepares before the matrix-core kernels run (4-bit weights expanded to s8
- * from 512 rows on, the right-hand side of s16 x s8 / s16 x u4 widened to s16,
- * narrow tile rows regrouped along K: as large as the prepared operands, at
- * most 2 GiB), which also holds the partial sums of a convolution whose input
- * channels are split over workgroups (at most 64 MB).
+ * thread and stream beyond a call: the workspace of sums that are split over
+ * workgroups (mmt4d along K, a few megabytes, up to 16 MB for 128x128 blocks in
+ * slices; convolutions with few output pixels along their input channels, up to
+ * 16 MB) and the buffer for operands the library prepares before the matrix-core
+ * kernels run (4-bit weights expanded to s8 from 512 rows on, the right-hand
+ * side of s16 x s8 / s16 x u4 widened to s16, narrow tile rows regrouped along
+ * K: as large as the prepared operands, at most 2 GiB).
  * workspace_bytes reports what the calling thread holds; release_workspaces
  * frees it after waiting for the device (0 or a hipError_t value; a later
  * call allocates again), and so does the thread's end. Calls through

@@ -44,8 +44,8 @@ extern "C" int iree_uk_amd_hip_launch_mmt4d(const iree_uk_mmt4d_params_t* p,
                                             const iree_uk_amd_rowmajor_out_t* rowmajor,
                                             void* stream, int kernel_mode,
                                             const char** kernel_name) {
-  // Every call starts from "one K slice": only the thin matrix-core kernel
-  // ever reports more (iree_uk_amd_last_k_slices).
+  // Every call starts from "one K slice": the barrier-free matrix-core kernels and the
+  // 128x128 blocks in slices report more (iree_uk_amd_last_k_slices).
   uk_mfma::note_k_slices(1);
   // s8 x s4 -> s32 and s16 x s16 -> s32 have an MFMA kernel for some shapes
   // only; the launcher says "not served" (negative) for the rest.

@@ -169,9 +169,9 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
   return go(std::false_type{});
 }
 
-// Workspace of the thin kernel's K split over workgroups: `partial_bytes` of
-// partial accumulators and `n_counters` arrival counters that are zero
-// between launches. Defined in mmt4d_mfma.hip: ordinary calls get a buffer
+// Workspace of a K split over workgroups (the barrier-free kernel's, the K slices' of
+// launch_slices, the split convolution's): `partial_bytes` of partial accumulators and
+// `n_counters` arrival counters that are zero between launches. Defined in mmt4d_mfma.hip: ordinary calls get a buffer
 // the library allocates per host thread and stream (grow-only; none while the
 // stream is being captured into a graph and nothing fits yet), calls through
 // iree_uk_amd_mmt4d_no_alloc get the library's static device array. Returns 0
@@ -760,16 +760,17 @@ bool direct_before_ksplit(const Problem& p) {
 // shape with 256-byte steps three steps ahead (tile rows under 16 bytes),
 // 12 .. 15 the narrow-row kernel (tile rows of 2 or 4 bytes, N0 = 16) in the
 // 256x256 / 128x512 / 128x128 / 64x64 shape, 16 / 17 / 18 / 19 the LDS-direct
-// ping-pong pipeline in the 256x256 / 128x512 / 128x128 / 64x64 shape, 21 the K
-// slices of launch_slices, as many as iree_uk_amd_set_k_slices says;
-// 0 = choose) overrides the
-// size heuristic for tests and tuning.
+// ping-pong pipeline in the 256x256 / 128x512 / 128x128 / 64x64 shape, 20 in the
+// 256x128 shape, 21 the K slices of launch_slices, as many as
+// iree_uk_amd_set_k_slices says; 0 = choose) overrides the size heuristic for tests
+// and tuning.
 //   thin  M-thin (decode-shaped) problems, up to 64 rows, which are bound by
 //         streaming the RHS: the barrier-free kernel of mmt4d_mfma_thin.h (16,
-//         32 or 64 rows x 32 columns per workgroup, K split over its 4 waves)
-//         when rows are at least 8 bytes wide and K is a whole number of
-//         steps, else 32 rows x 64 columns through LDS with loads three steps
-//         ahead.
+//         32 or 64 rows x 16 or 32 columns per workgroup, K split over its 4 or
+//         8 waves: launch_thin_rows) when rows are at least 8 bytes wide and K
+//         is a whole number of steps. Else launch_small_blocks where that serves
+//         (a K that ends inside a step, rows of 2 bytes and more), else 32 rows x 64
+//         columns through LDS with loads three steps ahead.
 template <Elem E, int RBC>
 int launch_class(const Problem& p, int forced, hipStream_t stream, const char** name) {
   constexpr int H = ElemTraits<E>::kHalves;
@@ -1089,8 +1090,8 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
                                                choice == 4 && RBC != 2, stream, name);
     if (st >= 0) return st;
   }
-  if (choice == 6) {
   if (forced == 0 && choice == 6 && direct_before_ksplit<E, RBC>(p)) choice = 3;
+  if (choice == 6) {
     // Few 64x64 blocks and a long K: the barrier-free kernel with a 64x64
     // block per workgroup, whose four waves split K.
     if constexpr (RBC >= 8) {
@@ -1119,7 +1120,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       int st = thin_launch(std::true_type{}, cols_n, rows_m);
       if (st >= 0) { *name = "mmt4d_mfma_thin_transposed"; return st; }
       // (K ends inside a step)
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, true, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, false, stream, name);
       if (st >= 0) return st;
     }
     choice = 3;
@@ -1128,7 +1129,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     if constexpr (RBC >= 8) {
       int st = thin_launch(std::false_type{}, rows_m, cols_n);
       if (st >= 0) { *name = "mmt4d_mfma_thin"; return st; }
-      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, false, stream, name);
+      if (forced == 0) st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, false, false, true, stream, name);
       if (st >= 0) return st;
     }
     // With 2-byte rows a 16-byte piece spans 8 rows and 32 rows do not fill a

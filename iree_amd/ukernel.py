@@ -53,7 +53,7 @@ POINTER_MODE_AUTO = 0
 POINTER_MODE_DEVICE = 1
 KERNEL_MODE_AUTO = 0
 KERNEL_MODE_GENERIC = 1
-KERNEL_MODE_MFMA_VARIANT = 16  # + 1..10: force an mmt4d MFMA workgroup shape
+KERNEL_MODE_MFMA_VARIANT = 16  # + 1..21: force an mmt4d MFMA workgroup shape
 
 # (lhs bits, rhs bits, out bits) per mmt4d type value.
 MMT4D_TYPE_BITS = {
@@ -242,8 +242,9 @@ class UKernelLibrary:
         return int(self.lib.iree_uk_amd_no_alloc_scratch_bytes())
 
     def set_k_slices(self, n: int):
-        """K slices across workgroups of the thin mmt4d kernels on this thread
-        (0 = choose, 1 = never split)."""
+        """K slices across workgroups of mmt4d on this thread (0 = choose, 1 =
+        never split; any value but 0 keeps calls that choose by size off the
+        128x128 blocks in slices)."""
         self.lib.iree_uk_amd_set_k_slices(n)
 
     def set_streamed_weights(self, on: bool):
