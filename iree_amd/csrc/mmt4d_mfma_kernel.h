@@ -59,6 +59,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "uk_float_convert.h"
@@ -266,6 +267,23 @@ __device__ __forceinline__ void static_for(F&& f) {
 // What PIPE 5 loads in place of K-tiles beyond K.
 static __device__ __attribute__((aligned(16))) const uint32_t kZeroPiece[4] = {0, 0, 0, 0};
 
+// Division of numbers below 2^31 by one that is the same for a whole launch: the high
+// half of a product and a shift in place of the some thirty instructions that a vector
+// division is. With 2^(l-1) < d <= 2^l, m = floor(2^(31+l) / d) + 1 and n < 2^31:
+// n * m = n * 2^(31+l) / d + n * e / d with 0 < e <= d <= 2^l, so the second term is
+// below 2^(31+l) / d and n * m >> (31 + l) is the quotient.
+struct Divisor {
+  uint32_t multiplier, shift;  // (d = 1, whose multiplier has 33 bits: 0)
+  static Divisor by(uint32_t d) {
+    uint32_t l = 0;
+    while ((1ull << l) < d) ++l;
+    return l == 0 ? Divisor{0, 0} : Divisor{(uint32_t)((1ull << (31 + l)) / d + 1), l - 1};
+  }
+  __device__ __forceinline__ uint32_t quotient(uint32_t n) const {
+    return multiplier ? __umulhi(n, multiplier) >> shift : n;
+  }
+};
+
 struct Args {
   const char* lhs;
   const char* rhs;
@@ -323,7 +341,29 @@ struct Args {
   uint32_t kslices;
   char* ws_partials;
   uint32_t* ws_counters;
+  // What the kernels divide by (set_divisors): M0, N0, grid_n; the blocks of one slice
+  // of K, those of a rasterization band, and the rows of a band and of the last one.
+  Divisor by_m0, by_n0, by_grid_n, by_blocks, by_band_blocks, by_band, by_last_band;
+  // SLICED instances: steps of a slice, and how many slices have one more.
+  uint32_t slice_steps, longer_slices;
 };
+
+// The last fields of Args from those before.
+inline void set_divisors(Args& a) {
+  a.by_m0 = Divisor::by((uint32_t)a.M0);
+  a.by_n0 = Divisor::by((uint32_t)a.N0);
+  a.by_grid_n = Divisor::by((uint32_t)a.grid_n);
+  const uint32_t slices = a.kslices > 1 ? a.kslices : 1;
+  a.slice_steps = (uint32_t)a.steps / slices;
+  a.longer_slices = (uint32_t)a.steps % slices;
+  if (a.band == 0) return;   // (the barrier-free kernel has no bands)
+  a.by_blocks = Divisor::by((uint32_t)a.grid_m * (uint32_t)a.grid_n);
+  // A band of more rows than there are is the only one.
+  const uint64_t band_blocks = (uint64_t)a.band * (uint32_t)a.grid_n;
+  a.by_band_blocks = Divisor::by((uint32_t)std::min<uint64_t>(band_blocks, 1u << 31));
+  a.by_band = Divisor::by(a.band);
+  a.by_last_band = Divisor::by((uint32_t)a.grid_m % a.band ? (uint32_t)a.grid_m % a.band : a.band);
+}
 
 // Row-slot swizzle for the regrouping loaders (RB < 16): the eight lanes that
 // store together write rows of the same residue mod 8 for different K slices;
@@ -375,14 +415,14 @@ __device__ __forceinline__ void block_of_workgroup(uint32_t wg, const Args& a,
   if (id >= total || (total & 7)) id = wg;  // uneven split: plain order
   if (slice) {
     id = (wg & 7) * (total / 8) + min(wg & 7, total & 7) + (wg >> 3);
-    *slice = id / blocks;
+    *slice = a.by_blocks.quotient(id);
     id -= *slice * blocks;
   }
-  const uint32_t band_blocks = a.band * (uint32_t)a.grid_n;
-  const uint32_t b = id / band_blocks;
-  const uint32_t in_band = id - b * band_blocks;
-  const uint32_t rows = min(a.band, (uint32_t)a.grid_m - b * a.band);
-  const uint32_t col = in_band / rows;
+  const uint32_t b = a.by_band_blocks.quotient(id);
+  const uint32_t in_band = id - b * (a.band * (uint32_t)a.grid_n);
+  const bool whole = a.band <= (uint32_t)a.grid_m - b * a.band;
+  const uint32_t rows = whole ? a.band : (uint32_t)a.grid_m - b * a.band;
+  const uint32_t col = (whole ? a.by_band : a.by_last_band).quotient(in_band);
   *bm = (int)(b * a.band + (in_band - col * rows));
   *bn = (int)col;
 }
@@ -437,9 +477,10 @@ void mmt4d_mfma_kernel(Args a) {
     static_assert(!TAIL, "K in whole steps");
     uint32_t slice;
     block_of_workgroup(blockIdx.x, a, &wg_m, &wg_n, a.kslices, &slice);
-    const uint32_t steps = (uint32_t)a.steps, s0 = (uint32_t)((uint64_t)slice * steps / a.kslices);
+    // (the first `longer_slices` slices have a step more than the others)
+    const uint32_t s0 = slice * a.slice_steps + min(slice, a.longer_slices);
     const int64_t kt = (int64_t)s0 * kts_per_step;
-    a.steps = (int32_t)((uint64_t)(slice + 1) * steps / a.kslices) - (int32_t)s0;
+    a.steps = (int32_t)(a.slice_steps + (slice < a.longer_slices));
     a.K1 = a.steps * kts_per_step;
     a.lhs += kt * a.M0 << lrb;
     a.rhs += kt * a.N0 << lrb;
@@ -471,6 +512,7 @@ void mmt4d_mfma_kernel(Args a) {
     const bool is_b = blk >= BLOCKS_A;
     const int xblk = is_b ? blk - BLOCKS_A : blk;
     const int X0 = is_b ? a.N0 : a.M0;
+    const Divisor by_x0 = is_b ? a.by_n0 : a.by_m0;
     const int X1 = is_b ? a.N1 : a.M1;
     const int px0 = is_b ? pn0 : pm0;
     const int bpx = is_b ? a.bpn : a.bpm;
@@ -485,7 +527,7 @@ void mmt4d_mfma_kernel(Args a) {
       // fetches the piece that belongs there: row r of the block, chunk 4*cb+q.
       const int rbk = xblk / NCHB, cb = xblk - rbk * NCHB;
       const uint32_t row = (uint32_t)rbk * 16 + r;
-      pl = (int)(row / (uint32_t)X0);
+      pl = (int)by_x0.quotient(row);
       const uint32_t m0 = row - (uint32_t)pl * X0;
       const uint32_t kb = (uint32_t)(cb * 4 + q) * 16;  // K byte of the chunk
       const uint32_t ktl = kb >> lrb;
@@ -500,8 +542,8 @@ void mmt4d_mfma_kernel(Args a) {
       // K-tiles g, g + NCH, g + 2*NCH, ... so that one load instruction covers
       // NCH consecutive K-tiles of a panel.
       const uint32_t u = (uint32_t)xblk * 64 + lane;
-      const uint32_t groups = (uint32_t)X0 / R;
-      const uint32_t t1 = u / groups;
+      const uint32_t groups = (uint32_t)X0 / R;   // (R a power of two that divides X0)
+      const uint32_t t1 = by_x0.quotient(u * R);
       const uint32_t mg = u - t1 * groups;
       pl = (int)(t1 / NCH);
       const uint32_t g = t1 - (uint32_t)pl * NCH;
@@ -589,7 +631,7 @@ void mmt4d_mfma_kernel(Args a) {
 #pragma unroll
       for (int tn = 0; tn < TN; ++tn) {
         const int col = (wn * TN + tn) * 16 + 4 * (int)oq;
-        const int pl = col / a.N0, n0 = col - pl * a.N0;
+        const int pl = (int)a.by_n0.quotient(col), n0 = col - pl * a.N0;
         const bool ok = pl < a.bpn && pn0 + pl < a.N1;
         const int left = a.out_cols - (col_origin + col);
         col_n[tn] = ok ? (left >= 4 ? 4 : (left > 0 ? left : 0)) : 0;
@@ -601,7 +643,7 @@ void mmt4d_mfma_kernel(Args a) {
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) {
         const int row = (wm * TM + tm) * 16 + (int)orr;
-        const int pl = row / a.M0, m0 = row - pl * a.M0;
+        const int pl = (int)a.by_m0.quotient(row), m0 = row - pl * a.M0;
         const bool row_ok = pl < a.bpm && pm0 + pl < a.M1 && row_origin + row < a.out_rows;
         const uint32_t row_off = (uint32_t)pl * (uint32_t)s_panel + (uint32_t)m0 * s_m0;
 #pragma unroll
@@ -622,7 +664,7 @@ void mmt4d_mfma_kernel(Args a) {
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm) {
         const int row = (wm * TM + tm) * 16 + (int)orr;
-        const int pl = row / a.M0, m0 = row - pl * a.M0;
+        const int pl = (int)a.by_m0.quotient(row), m0 = row - pl * a.M0;
         const bool row_ok = pl < a.bpm && pm0 + pl < a.M1 && row_origin + row < a.out_rows;
         const uint32_t row_off = (uint32_t)pl * (uint32_t)s_panel + (uint32_t)m0 * s_m0;
 #pragma unroll
@@ -630,7 +672,7 @@ void mmt4d_mfma_kernel(Args a) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int col = (wn * TN + tn) * 16 + 4 * (int)oq + e;
-            const int pc = col / a.N0, n0 = col - pc * a.N0;
+            const int pc = (int)a.by_n0.quotient(col), n0 = col - pc * a.N0;
             if (row_ok && pc < a.bpn && pn0 + pc < a.N1 && col_origin + col < a.out_cols)
               f1(tm, tn, e, out_base + (row_off + (uint32_t)pc * s_pn + (uint32_t)n0 * OB));
           }
@@ -932,7 +974,7 @@ void mmt4d_mfma_kernel(Args a) {
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) {
       const uint32_t row = (uint32_t)(wn * TN + tn) * 16 + r;
-      const uint32_t pl = row / (uint32_t)a.N0;
+      const uint32_t pl = a.by_n0.quotient(row);
       const uint32_t n0 = row - pl * a.N0;
       const bool ok = (int)pl < a.bpn && pn0 + (int)pl < a.N1;
 #pragma unroll
@@ -1031,7 +1073,7 @@ void mmt4d_mfma_kernel(Args a) {
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) {
       const uint32_t row = (uint32_t)(wn * TN + tn) * 16 + r;
-      const uint32_t pl = row / (uint32_t)a.N0;
+      const uint32_t pl = a.by_n0.quotient(row);
       const uint32_t n0 = row - pl * a.N0;
       const bool ok = (int)pl < a.bpn && pn0 + (int)pl < a.N1;
 #pragma unroll
@@ -1243,6 +1285,7 @@ void mmt4d_mfma_kernel(Args a) {
       const int xblk = is_b ? blk - BM / 16 * DCH : blk;   // (row block, 64-byte chunk) of the operand's image
       const int rbk = xblk / DCH, chunk = xblk - rbk * DCH;
       const int X0 = is_b ? a.N0 : a.M0;
+      const Divisor by_x0 = is_b ? a.by_n0 : a.by_m0;
       const int X1 = is_b ? a.N1 : a.M1;
       const int px0 = is_b ? pn0 : pm0;
       const int bpx = is_b ? a.bpn : a.bpm;
@@ -1252,7 +1295,7 @@ void mmt4d_mfma_kernel(Args a) {
       if constexpr (RBC >= 16) {
         // Lane (q, r): row r of the block, bytes 16 q .. 16 q + 15 of the chunk.
         const uint32_t row = (uint32_t)rbk * 16 + r;
-        pl = row / (uint32_t)X0;
+        pl = by_x0.quotient(row);
         const uint32_t x0 = row - pl * (uint32_t)X0;
         const uint32_t kb = (uint32_t)(chunk * 4 + q) * 16;
         d_voff[i] = pl * (uint32_t)xstride + (kb >> lrb) * kt_bytes + (x0 << lrb) + (kb & ((1u << lrb) - 1));
@@ -1260,7 +1303,7 @@ void mmt4d_mfma_kernel(Args a) {
         constexpr int RP = 16 / RBC;   // rows of a K-tile in one 16-byte piece
         constexpr int PPK = 16 / RP;   // pieces per K-tile of a 16-row block
         const uint32_t row0 = (uint32_t)rbk * 16 + ((uint32_t)lane % PPK) * RP;
-        pl = row0 / (uint32_t)X0;
+        pl = by_x0.quotient(row0);
         const uint32_t x0 = row0 - pl * (uint32_t)X0;
         const uint32_t kt_l = (uint32_t)chunk * (64 / RBC) + (uint32_t)lane / PPK;  // K-tile within the step
         d_voff[i] = pl * (uint32_t)xstride + kt_l * kt_bytes + x0 * RBC;

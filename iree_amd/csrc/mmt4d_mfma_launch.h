@@ -150,6 +150,7 @@ int launch_variant(const Problem& p, int kt_begin, int kt_count, bool accumulate
       span_a >= (1ll << 31)) {
     return -1;
   }
+  set_divisors(a);
   auto go = [&](auto tail_c) {
     auto kernel = mmt4d_mfma_kernel<E, RBC, TM, TN, WGM, WGN, NKK, PIPE, decltype(tail_c)::value, SLICED>;
     if (SH::kLdsBytes > 64 * 1024) {
@@ -278,6 +279,7 @@ int launch_persistent(const Problem& p, int kt_count, bool force, hipStream_t st
     return -1;
   }
   constexpr size_t kLds = 4 * (size_t)BM * KS;
+  set_divisors(a);
   auto kernel = mmt4d_mfma_persistent_kernel<E, TM, TN, WGM, WGN>;
   uk::launch(2, kernel, dim3((uint32_t)grid), dim3(WGM * WGN * 64), kLds, stream, a);
   return (int)hipGetLastError();
@@ -325,6 +327,7 @@ int launch_narrow(const Problem& p, int kt_count, hipStream_t stream) {
     return -1;
   }
   constexpr size_t kLds = 3 * (size_t)BM * KS;
+  set_divisors(a);
   uk::launch(2, mmt4d_mfma_narrow_kernel<E, RBC, TM, WGM, WGN>, dim3((uint32_t)(grid_m * grid_n)),
              dim3(WGM * WGN * 64), kLds, stream, a);
   return (int)hipGetLastError();
@@ -443,6 +446,7 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
       kslices = 1;
     }
   }
+  set_divisors(a);
   const dim3 grid((uint32_t)(grid_m * grid_n * kslices)), block(KSPLIT * 64);
   if constexpr (TAIL_OK) {
     // No non-temporal instances: weights that the caller has declared streamed are read
@@ -572,6 +576,7 @@ int launch_slices(const Problem& p, int slices, hipStream_t stream) {
   s.rows = (int32_t)std::min(rows, p.out_rows);
   s.cols = (int32_t)std::min(cols, p.out_cols);
   s.M0 = p.M0; s.N0 = p.N0;
+  s.by_m0 = Divisor::by((uint32_t)p.M0); s.by_n0 = Divisor::by((uint32_t)p.N0);
   s.out = p.out; s.out_stride = p.out_stride;
   s.out_sm0 = (uint32_t)p.out_sm0; s.out_spn = (uint32_t)p.out_spn;
   s.acc = p.accumulate ? p.acc : nullptr; s.acc_stride = p.acc_stride;

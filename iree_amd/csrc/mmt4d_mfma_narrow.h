@@ -182,7 +182,7 @@ void mmt4d_mfma_narrow_kernel(Args a) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
       const int row = (wm * TM + tm) * 16 + (int)orr;
-      const int pl = row / a.M0, m0 = row - pl * a.M0;
+      const int pl = (int)a.by_m0.quotient(row), m0 = row - pl * a.M0;
       const bool ok = col_ok && pl < a.bpm && pm0 + pl < a.M1 && pm0 * a.M0 + row < a.out_rows;
       const uint32_t row_off = (uint32_t)pl * (uint32_t)s_panel + (uint32_t)m0 * s_m0;
 #pragma unroll

@@ -21,6 +21,7 @@ struct SumArgs {
   int64_t slice_bytes, pitch;
   int32_t slices, rows, cols;  // rows, cols: of the result
   int32_t M0, N0;
+  Divisor by_m0, by_n0;
   // Result and initial accumulators (null: none), addressed as in Args.
   char* out;
   int64_t out_stride;
@@ -46,14 +47,14 @@ void mmt4d_sum_slices_kernel(SumArgs a) {
   const int col = (blockIdx.x * kSumThreads + threadIdx.x) * 4;
   const int left = a.cols - col;
   if (left <= 0) return;
-  const int pm = row / a.M0, m0 = row - pm * a.M0;
+  const int pm = (int)a.by_m0.quotient(row), m0 = row - pm * a.M0;
   char* out = a.out + (int64_t)pm * a.out_stride + (int64_t)m0 * a.out_sm0;
   const char* init = a.acc + (int64_t)pm * a.acc_stride + (int64_t)m0 * a.acc_sm0;
   int64_t out_e[4], acc_e[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const int c = min(col + e, a.cols - 1);
-    const int pc = c / a.N0, n0 = c - pc * a.N0;
+    const int pc = (int)a.by_n0.quotient(c), n0 = c - pc * a.N0;
     out_e[e] = (int64_t)pc * a.out_spn + n0 * OB;
     acc_e[e] = (int64_t)pc * a.acc_spn + n0 * OB;
   }

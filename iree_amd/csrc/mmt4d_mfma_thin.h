@@ -9,8 +9,12 @@
 //   * each lane loads its MFMA operands straight from global memory, the RHS
 //     from HBM and the (small, shared) LHS from L2, D steps ahead of the MFMAs
 //     through D register buffers;
-//   * the KSPLIT partial accumulators meet in LDS once, at the end, and wave 0
-//     adds them in wave order and stores;
+//   * the KSPLIT partial accumulators meet in LDS once, at the end; each wave adds
+//     up, in wave order, and stores its share of the output blocks;
+//     what that and the addresses cost bounds the small products and the decode layers
+//     (one K step a wave, f16 512 x 2048 in 64x64 blocks: 6.7 us with the sums and the
+//     stores in one wave and a vector division for each address, 4.6 so; with all of K =
+//     2048 11.3 -> 10.0; s8 16 x 14336 x 4096 14.7 -> 13.7, f16 8 x 4096 x 4096 9.0 -> 8.4);
 //   * when the problem has too few output blocks to occupy the chip (a decode
 //     step against a weight matrix with few rows and a long K), K is split
 //     over several workgroups per block as well: each publishes its partial
@@ -28,8 +32,8 @@
 // bytes and more load one 16-byte piece per operand; 8-byte rows load the two
 // 8-byte halves from two K-tiles (chunk g of a step holds K-tiles g and
 // g + 4), 4- and 2-byte rows likewise from four and eight. A K that
-// ends inside a step (TAIL): the pieces beyond it are read from the operand's
-// first row instead and are zero for the MFMA.
+// ends inside a step (TAIL): the pieces beyond it are zero in both operands (what
+// lies there may be an infinity).
 //
 // s8 x s4 -> s32 (Elem::kS8S4) runs here too. A lane loads 8 RHS bytes (16
 // nibbles, the same 16 K elements as its 16 LHS bytes) and turns them into two
@@ -48,25 +52,32 @@
 namespace uk_mfma {
 
 typedef int v2i __attribute__((ext_vector_type(2)));
-typedef v2i v2i_g __attribute__((aligned(1)));  // as v4i_g: read from global memory at any address
-typedef int int_g __attribute__((aligned(1)));
-typedef short short_g __attribute__((aligned(1)));
 
-// 16, 8 and 4 bytes from any address, non-temporally if NT.
-template <bool NT>
-__device__ __forceinline__ v4i load16(const char* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const v4i_g*>(p));
-  else return *reinterpret_cast<const v4i_g*>(p);
+// Loads from a buffer resource (its base, the same in all lanes), a lane's bytes and a
+// scalar's: a lane's address is one register that the K loop never touches, where an
+// address of its own takes a vector addition for every load, in the pipe that the f32
+// matrix instructions keep busy (f32 16x16x1 in 32x32 blocks: 515 x 1027 x 769 17.0 ->
+// 15.0 us, 700 x 700 x 3000 41.0 -> 34.6, 1500 x 1500 x 1000 52.6 -> 44.9). What lies kBeyond in a lane is outside the resource:
+// such a load returns zeros and reads nothing. NT: non-temporal.
+constexpr uint32_t kBeyond = 0x80000000u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t operand_at(const char* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, (int)kBeyond, 0x00027000);
 }
 template <bool NT>
-__device__ __forceinline__ v2i load8(const char* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const v2i_g*>(p));
-  else return *reinterpret_cast<const v2i_g*>(p);
+__device__ __forceinline__ v4i load16(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
+  return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(from, lane_bytes, bytes, NT ? 2 : 0));
 }
 template <bool NT>
-__device__ __forceinline__ int load4(const char* p) {
-  if constexpr (NT) return __builtin_nontemporal_load(reinterpret_cast<const int_g*>(p));
-  else return *reinterpret_cast<const int_g*>(p);
+__device__ __forceinline__ v2i load8(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
+  return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(from, lane_bytes, bytes, NT ? 2 : 0));
+}
+template <bool NT>
+__device__ __forceinline__ int load4(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
+  return (int)__builtin_amdgcn_raw_buffer_load_b32(from, lane_bytes, bytes, NT ? 2 : 0);
+}
+template <bool NT>
+__device__ __forceinline__ short load2(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
+  return (short)__builtin_amdgcn_raw_buffer_load_b16(from, lane_bytes, bytes, NT ? 2 : 0);
 }
 
 // Sums of floats whose K eight waves share are in several chains, steps i, i + chains, ..
@@ -102,7 +113,10 @@ void mmt4d_thin_kernel(Args a) {
   static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
   static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
 
-  __shared__ v4i partial[KSPLIT > 1 ? KSPLIT - 1 : 1][TM * TN][64];
+  // The blocks that a wave adds up and stores: OWN, or for the last ones fewer.
+  static_assert(KSPLIT > 1, "several waves share K");
+  constexpr int NB = TM * TN, OWN = (NB + KSPLIT - 1) / KSPLIT;
+  __shared__ v4i partial[KSPLIT][NB][64];
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -111,55 +125,55 @@ void mmt4d_thin_kernel(Args a) {
   const uint32_t kslices = a.kslices > 1 ? a.kslices : 1;
   const uint32_t block_id = kslices > 1 ? blockIdx.x / kslices : blockIdx.x;
   const uint32_t slice = kslices > 1 ? blockIdx.x - block_id * kslices : 0;
-  const int bm = (int)(block_id / (uint32_t)a.grid_n);
+  const int bm = (int)a.by_grid_n.quotient(block_id);
   const int bn = (int)(block_id - (uint32_t)bm * a.grid_n);
   // K steps of this workgroup: [step_begin, step_begin + wg_steps).
-  const uint32_t step_begin = (uint32_t)(((uint64_t)slice * (uint32_t)a.steps) / kslices);
-  const int wg_steps = (int)((((uint64_t)(slice + 1) * (uint32_t)a.steps) / kslices) - step_begin);
+  uint32_t step_begin = 0;
+  int wg_steps = a.steps;
+  if (kslices > 1) {
+    step_begin = (uint32_t)(((uint64_t)slice * (uint32_t)a.steps) / kslices);
+    wg_steps = (int)((((uint64_t)(slice + 1) * (uint32_t)a.steps) / kslices) - step_begin);
+  }
   const int lrb = a.lrb;
   const int lrb_b = S4 ? lrb - 1 : lrb;       // log2 of the RHS row bytes
   const uint32_t kt_m = (uint32_t)a.M0 << lrb, kt_n = (uint32_t)a.N0 << lrb_b;
   const uint32_t kts_per_step = KS >> lrb;
   const uint32_t sstep_a = kts_per_step * kt_m, sstep_b = kts_per_step * kt_n;
 
-  // Byte offset of the lane's piece(s) of block row `x` (a row of 16 rows of
-  // the M or N dimension) at K step 0; 0 for rows outside the problem or the
-  // result (tile padding), whose (valid) bytes only reach accumulators that are
-  // never stored: those lanes share the cache lines of the first row.
-  // Offsets are 32-bit and relative to the first panel the workgroup touches.
-  const int pa0 = bm * TM * 16 / a.M0, pb0 = bn * TN * 16 / a.N0;
-  const char* base_a = a.lhs + (int64_t)pa0 * a.lhs_stride;
-  const char* base_b = a.rhs + (int64_t)pb0 * a.rhs_stride;
-  auto operand_offsets = [&](uint32_t (&off)[HALVES][PIECES], int x, int X0, int X1, int rows, int p0,
-                             int64_t stride, uint32_t kt_bytes, int lrb, uint32_t piece_bytes) {
+  // Byte offset of the lane's (first) piece of block row `x` (a row of 16 rows of
+  // the M or N dimension) at K step 0, kBeyond for rows outside the problem or the
+  // result (tile padding), which only reach accumulators that are never stored.
+  // Offsets are relative to the first panel the workgroup touches.
+  const int pa0 = (int)a.by_m0.quotient(bm * TM * 16), pb0 = (int)a.by_n0.quotient(bn * TN * 16);
+  const __amdgpu_buffer_rsrc_t from_a = operand_at(a.lhs + (int64_t)pa0 * a.lhs_stride);
+  const __amdgpu_buffer_rsrc_t from_b = operand_at(a.rhs + (int64_t)pb0 * a.rhs_stride);
+  auto operand_offsets = [&](uint32_t (&off)[HALVES], int x, int X0, const Divisor& by_x0, int X1, int rows,
+                             int p0, int64_t stride, uint32_t kt_bytes, int lrb, uint32_t piece_bytes) {
     const uint32_t row = (uint32_t)x * 16 + r;
-    const uint32_t pabs = row / (uint32_t)X0;
+    const uint32_t pabs = by_x0.quotient(row);
     const uint32_t x0 = row - pabs * X0;
     const bool ok = (int)pabs < X1 && (int)row < rows;
     const uint32_t pl = pabs - (uint32_t)p0;
 #pragma unroll
     for (int h = 0; h < HALVES; ++h) {
       const uint32_t g = (uint32_t)h * 4 + q;
-#pragma unroll
-      for (int t = 0; t < PIECES; ++t) {
-        uint32_t o;
-        if constexpr (RBC >= 16) {
-          const uint32_t kb = g * piece_bytes;
-          o = (kb >> lrb) * kt_bytes + (x0 << lrb) + (kb & ((1u << lrb) - 1));
-        } else {
-          o = (g + (uint32_t)t * NCH) * kt_bytes + x0 * RBC;
-        }
-        off[h][t] = ok ? pl * (uint32_t)stride + o : 0u;
+      uint32_t o;
+      if constexpr (RBC >= 16) {
+        const uint32_t kb = g * piece_bytes;
+        o = (kb >> lrb) * kt_bytes + (x0 << lrb) + (kb & ((1u << lrb) - 1));
+      } else {
+        o = g * kt_bytes + x0 * RBC;
       }
+      off[h] = ok ? pl * (uint32_t)stride + o : kBeyond;
     }
   };
-  uint32_t offa[TM][HALVES][PIECES], offb[TN][HALVES][PIECES];
+  uint32_t offa[TM][HALVES], offb[TN][HALVES];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
-    operand_offsets(offa[tm], bm * TM + tm, a.M0, a.M1, a.out_rows, pa0, a.lhs_stride, kt_m, lrb, 16);
+    operand_offsets(offa[tm], bm * TM + tm, a.M0, a.by_m0, a.M1, a.out_rows, pa0, a.lhs_stride, kt_m, lrb, 16);
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn)
-    operand_offsets(offb[tn], bn * TN + tn, a.N0, a.N1, a.out_cols, pb0, a.rhs_stride, kt_n, lrb_b,
+    operand_offsets(offb[tn], bn * TN + tn, a.N0, a.by_n0, a.N1, a.out_cols, pb0, a.rhs_stride, kt_n, lrb_b,
                     S4 ? 8 : 16);
 
   // Whether piece t of chunk (h, q) of K step s lies inside K.
@@ -170,22 +184,26 @@ void mmt4d_thin_kernel(Args a) {
       return s * kts_per_step + (uint32_t)h * 4 + q + (uint32_t)t * NCH < (uint32_t)a.K1;
     }
   };
-  auto load_operand = [&](auto nontemporal, const char* base, const uint32_t (&off)[PIECES], uint32_t adv,
-                          uint32_t s, int h) {
-    auto at = [&](int t) { return base + (!TAIL || in_k(s, h, t) ? off[t] + adv : 0u); };
+  // One lane operand of step s, `adv` bytes on from step 0. `ends`: K ends inside the
+  // step, and what lies beyond it is zero.
+  auto load_operand = [&](auto nontemporal, auto ends, __amdgpu_buffer_rsrc_t from, uint32_t off, uint32_t adv,
+                          uint32_t kt_bytes, uint32_t s, int h) {
+    auto at = [&](int t) { return !decltype(ends)::value || in_k(s, h, t) ? off : kBeyond; };
     constexpr bool NT = decltype(nontemporal)::value;
+    const uint32_t piece = NCH * kt_bytes;   // from one piece to the next
     if constexpr (RBC >= 16) {
-      return load16<NT>(at(0));
+      return load16<NT>(from, at(0), adv);
     } else if constexpr (RBC == 8) {
-      const v2i lo = load8<NT>(at(0)), hi = load8<NT>(at(1));
+      const v2i lo = load8<NT>(from, at(0), adv), hi = load8<NT>(from, at(1), adv + piece);
       return v4i{lo[0], lo[1], hi[0], hi[1]};
     } else if constexpr (RBC == 4) {
-      return v4i{load4<NT>(at(0)), load4<NT>(at(1)), load4<NT>(at(2)), load4<NT>(at(3))};
+      return v4i{load4<NT>(from, at(0), adv), load4<NT>(from, at(1), adv + piece),
+                 load4<NT>(from, at(2), adv + 2 * piece), load4<NT>(from, at(3), adv + 3 * piece)};
     } else {
       typedef short short8 __attribute__((ext_vector_type(8)));
       short8 v;
 #pragma unroll
-      for (int t = 0; t < 8; ++t) v[t] = *reinterpret_cast<const short_g*>(at(t));
+      for (int t = 0; t < 8; ++t) v[t] = load2<NT>(from, at(t), adv + t * piece);
       return __builtin_bit_cast(v4i, v);
     }
   };
@@ -195,58 +213,68 @@ void mmt4d_thin_kernel(Args a) {
   // Local step i of this wave is K step step_begin + wave + i * KSPLIT.
   auto load_step = [&](int d, int i) {
     const uint32_t s = step_begin + (uint32_t)(wave + i * KSPLIT);
+    auto load = [&](auto ends) {
 #pragma unroll
-    for (int tn = 0; tn < TN; ++tn)
+      for (int tn = 0; tn < TN; ++tn)
 #pragma unroll
-      for (int h = 0; h < HALVES; ++h) {
-        if constexpr (S4) {
-          fb[d][tn][h] = load8<STREAMED>(base_b + (offb[tn][h][0] + s * sstep_b));
-        } else {
-          fb[d][tn][h] = load_operand(std::bool_constant<STREAMED>{}, base_b, offb[tn][h], s * sstep_b, s, h);
+        for (int h = 0; h < HALVES; ++h) {
+          if constexpr (S4) {
+            fb[d][tn][h] = load8<STREAMED>(from_b, offb[tn][h], s * sstep_b);
+          } else {
+            fb[d][tn][h] = load_operand(std::bool_constant<STREAMED>{}, ends, from_b, offb[tn][h], s * sstep_b,
+                                        kt_n, s, h);
+          }
         }
-      }
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
+      for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-      for (int h = 0; h < HALVES; ++h)
-        fa[d][tm][h] = load_operand(std::false_type{}, base_a, offa[tm][h], s * sstep_a, s, h);
+        for (int h = 0; h < HALVES; ++h)
+          fa[d][tm][h] = load_operand(std::false_type{}, ends, from_a, offa[tm][h], s * sstep_a, kt_m, s, h);
+    };
+    if constexpr (TAIL) {
+      if (s == (uint32_t)a.steps - 1) return load(std::true_type{});
+    }
+    load(std::false_type{});
   };
 
   // ---- output addressing (see for_each_output in mmt4d_mfma_kernel.h) ------
-  // Lane (q, r) of block (tm, tn) holds output row r, columns 4q..4q+3.
+  // Lane (q, r) of block b = tm * TN + tn holds output row r, columns 4q..4q+3.
+  // f4(i, p) / f1(i, e, p) for the i-th of this wave's blocks.
+  const int first_own = wave * OWN;
+  auto for_each_own = [&](auto f) {
+#pragma unroll
+    for (int i = 0; i < OWN; ++i)
+      if ((NB % OWN == 0 && first_own < NB) || first_own + i < NB) f(i, (first_own + i) / TN, (first_own + i) % TN);
+  };
   auto for_each_output = [&](const char* base, int64_t s_panel, uint32_t s_m0, uint32_t s_pn,
                              uint32_t s_n0, auto f4, auto f1) {
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
+    for_each_own([&](int i, int tm, int tn) {
       const int row = (bm * TM + tm) * 16 + (int)r;
-      const int pl = row / a.M0, m0 = row - pl * a.M0;
+      const int pl = (int)a.by_m0.quotient(row), m0 = row - pl * a.M0;
       const bool row_ok = pl < a.M1 && row < a.out_rows;
       char* row_base = const_cast<char*>(base) + (int64_t)pl * s_panel + (int64_t)m0 * s_m0;
+      const int col = (bn * TN + tn) * 16 + 4 * (int)q;
+      if (a.vec_out) {
+        const int pc = (int)a.by_n0.quotient(col), n0 = col - pc * a.N0;
+        const int left = a.out_cols - col;
+        char* p = row_base + (int64_t)pc * s_pn + (int64_t)n0 * s_n0;
+        if (row_ok && pc < a.N1 && left >= 4) {
+          f4(i, p);
+        } else if (row_ok && pc < a.N1) {
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        const int col = (bn * TN + tn) * 16 + 4 * (int)q;
-        if (a.vec_out) {
-          const int pc = col / a.N0, n0 = col - pc * a.N0;
-          const int left = a.out_cols - col;
-          char* p = row_base + (int64_t)pc * s_pn + (int64_t)n0 * s_n0;
-          if (row_ok && pc < a.N1 && left >= 4) {
-            f4(tm, tn, p);
-          } else if (row_ok && pc < a.N1) {
+          for (int e = 0; e < 3; ++e)
+            if (e < left) f1(i, e, p + e * s_n0);
+        }
+      } else {
 #pragma unroll
-            for (int e = 0; e < 3; ++e)
-              if (e < left) f1(tm, tn, e, p + e * s_n0);
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int c = col + e;
-            const int pc = c / a.N0, n0 = c - pc * a.N0;
-            if (row_ok && pc < a.N1 && c < a.out_cols)
-              f1(tm, tn, e, row_base + (int64_t)pc * s_pn + (int64_t)n0 * s_n0);
-          }
+        for (int e = 0; e < 4; ++e) {
+          const int c = col + e;
+          const int pc = (int)a.by_n0.quotient(c), n0 = c - pc * a.N0;
+          if (row_ok && pc < a.N1 && c < a.out_cols)
+            f1(i, e, row_base + (int64_t)pc * s_pn + (int64_t)n0 * s_n0);
         }
       }
-    }
+    });
   };
 
   Acc chains[CHAINS][TM][TN];
@@ -263,78 +291,40 @@ void mmt4d_thin_kernel(Args a) {
 #pragma unroll
   for (int d = 0; d < D; ++d)
     if (d < my_steps) load_step(d, d);
-  // Wave 0, which stores, fetches what the store needs now, under the K loop:
-  // the initial accumulators and the scales of the dequantizing store (indices
-  // beyond the matrix are clamped; their elements are never stored).
-  float sm[TM];
-  v4f sn[TN];
+  // The waves that store fetch what the store needs now, under the K loop: the
+  // initial accumulators, which the sums are added to at the end (with K split over
+  // workgroups only to the first slice's), and the scales of the dequantizing store
+  // (indices beyond the matrix are clamped; their elements are never stored).
+  Acc cin[OWN];
+  float sm[OWN];
+  v4f sn[OWN];
 #pragma unroll
-  for (int tm = 0; tm < TM; ++tm) sm[tm] = 1.0f;
-#pragma unroll
-  for (int tn = 0; tn < TN; ++tn) sn[tn] = v4f{1.0f, 1.0f, 1.0f, 1.0f};
-  // With the 4-bit RHS the accumulators hold 16 times the sum, so the
-  // ACCUMULATE input waits in registers of its own. With K split over
-  // workgroups only the first slice starts from the ACCUMULATE input.
-  Acc cin[S4 ? TM : 1][S4 ? TN : 1];
-  if constexpr (S4) {
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) cin[tm][tn] = Acc{0, 0, 0, 0};
+  for (int i = 0; i < OWN; ++i) {
+    cin[i] = Acc{0, 0, 0, 0};
+    sm[i] = 1.0f;
+    sn[i] = v4f{1.0f, 1.0f, 1.0f, 1.0f};
   }
-  if (wave == 0) {
-    if (a.accumulate && slice == 0) {
-      for_each_output(a.acc, a.acc_stride, a.acc_sm0, a.acc_spn, a.acc_sn0,
-                      [&](int tm, int tn, char* p) {
-                        if constexpr (S4) cin[tm][tn] = Out::load4(p);
-                        else acc[tm][tn] = Out::load4(p);
-                      },
-                      [&](int tm, int tn, int e, char* p) {
-                        if constexpr (S4) cin[tm][tn][e] = Out::load1(p);
-                        else acc[tm][tn][e] = Out::load1(p);
-                      });
+  if (a.accumulate && slice == 0) {
+    for_each_output(a.acc, a.acc_stride, a.acc_sm0, a.acc_spn, a.acc_sn0,
+                    [&](int i, char* p) { cin[i] = Out::load4(p); },
+                    [&](int i, int e, char* p) { cin[i][e] = Out::load1(p); });
+  }
+  if (OB == 4 && a.dequant) {
+    if (a.row_scale) {
+      for_each_own([&](int i, int tm, int) {
+        sm[i] = a.row_scale[max(min((bm * TM + tm) * 16 + (int)r, a.out_rows - 1), 0)];
+      });
     }
-    if (OB == 4 && a.dequant) {
-      if (a.row_scale) {
+    if (a.col_scale) {
+      for_each_own([&](int i, int, int tn) {
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-          sm[tm] = a.row_scale[max(min((bm * TM + tm) * 16 + (int)r, a.out_rows - 1), 0)];
-      }
-      if (a.col_scale) {
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            sn[tn][e] =
-                a.col_scale[max(min((bn * TN + tn) * 16 + 4 * (int)q + e, a.out_cols - 1), 0)];
-      }
+        for (int e = 0; e < 4; ++e)
+          sn[i][e] = a.col_scale[max(min((bn * TN + tn) * 16 + 4 * (int)q + e, a.out_cols - 1), 0)];
+      });
     }
   }
-  // The products of step i, whose operands are in registers d, onto chain c.
-  auto compute = [&](int d, int c, int i) {
-    if constexpr (TAIL) {
-      // The step K ends in: nothing beyond it reaches the sums (a zero in both
-      // operands: what was read instead may be an infinity).
-      const uint32_t s = step_begin + (uint32_t)(wave + i * KSPLIT);
-      if (s == (uint32_t)a.steps - 1) {
-        auto cut = [&](v4i& f, int h) {
-#pragma unroll
-          for (int t = 0; t < PIECES; ++t) {
-            const bool in = in_k(s, h, t);
-#pragma unroll
-            for (int w = 0; w < 4 / PIECES; ++w) f[t * (4 / PIECES) + w] = in ? f[t * (4 / PIECES) + w] : 0;
-            if constexpr (PIECES == 8) f[t / 2] = in ? f[t / 2] : f[t / 2] & (t & 1 ? 0xFFFF : (int)0xFFFF0000);
-          }
-        };
-#pragma unroll
-        for (int h = 0; h < HALVES; ++h) {
-#pragma unroll
-          for (int tm = 0; tm < TM; ++tm) cut(fa[d][tm][h], h);
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn) cut(fb[d][tn][h], h);
-        }
-      }
-    }
+  // The products of a step, whose operands are in registers d, onto chain c.
+  auto compute = [&](int d, int c) {
     if constexpr (S4) {
       // LHS: even K bytes, then odd K bytes; RHS: low nibbles, then high ones.
       v4i ea[TM], eb[TN];
@@ -356,6 +346,17 @@ void mmt4d_thin_kernel(Args a) {
       for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = TT::mfma(&eb[tn], &ea[tm], acc[tm][tn]);
+    } else if constexpr (E == Elem::kF32) {
+      // A word of all blocks before the next one: products of one block wait for each other.
+#pragma unroll
+      for (int w = 0; w < 4; ++w)
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn)
+            chains[c][tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(v4f, fb[d][tn][0])[w],
+                                                                     __builtin_bit_cast(v4f, fa[d][tm][0])[w],
+                                                                     chains[c][tm][tn], 0, 0, 0);
     } else {
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm)
@@ -372,7 +373,7 @@ void mmt4d_thin_kernel(Args a) {
   for (; i + U + D <= my_steps; i += U) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      compute(u % D, u % CHAINS, i + u);
+      compute(u % D, u % CHAINS);
       load_step(u % D, i + u + D);
     }
   }
@@ -380,21 +381,21 @@ void mmt4d_thin_kernel(Args a) {
   // after them, and the compiler counts the instructions that have to lie in between
   // along the longer of two paths through `if (compute) { if (load) }` (too few on the
   // shorter one: sums without their last product). So they lie behind the product itself.
-  auto compute_last = [&](int d, int c, int i) {
-    compute(d, c, i);
+  auto compute_last = [&](int d, int c) {
+    compute(d, c);
     if constexpr (CHAINS > 1) settle_products();
   };
   // Fewer than U + D steps left: the same with bounds.
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (i + u < my_steps) {
-      compute_last(u % D, u % CHAINS, i + u);
+      compute_last(u % D, u % CHAINS);
       if (i + u + D < my_steps) load_step(u % D, i + u + D);
     }
   }
 #pragma unroll
   for (int u = U; u < U + D; ++u)
-    if (i + u < my_steps) compute_last(u % D, u % CHAINS, i + u);
+    if (i + u < my_steps) compute_last(u % D, u % CHAINS);
   settle_products();
 #pragma unroll
   for (int c = 1; c < CHAINS; ++c)
@@ -404,69 +405,57 @@ void mmt4d_thin_kernel(Args a) {
       for (int tn = 0; tn < TN; ++tn) acc[tm][tn] += chains[c][tm][tn];
 
   // ---- meet the partial sums ---------------------------------------------------
-  if constexpr (KSPLIT > 1) {
-    if (wave > 0) {
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
+  for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-          partial[wave - 1][tm * TN + tn][lane] = __builtin_bit_cast(v4i, acc[tm][tn]);
-    }
-    __syncthreads();
-    if (wave > 0) return;
+    for (int tn = 0; tn < TN; ++tn) partial[wave][tm * TN + tn][lane] = __builtin_bit_cast(v4i, acc[tm][tn]);
+  __syncthreads();
+  if (kslices <= 1 && first_own >= NB) return;
+  Acc sum[OWN];
+  for_each_own([&](int i, int tm, int tn) {
+    const int b = tm * TN + tn;
+    sum[i] = __builtin_bit_cast(Acc, partial[0][b][lane]);
 #pragma unroll
-    for (int w = 0; w < KSPLIT - 1; ++w)
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-          acc[tm][tn] += __builtin_bit_cast(Acc, partial[w][tm * TN + tn][lane]);
-  }
-
-  if constexpr (S4) {
-    // Every slice holds 16 times its part of the sum (plus, in slice 0, nothing
-    // else: the ACCUMULATE input waits in cin), so the shift is exact per slice.
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = (acc[tm][tn] >> 4) + cin[tm][tn];
-  }
+    for (int w = 1; w < KSPLIT; ++w) sum[i] += __builtin_bit_cast(Acc, partial[w][b][lane]);
+    // (4-bit RHS: every slice holds 16 times its part of the sum, so the shift is
+    // exact per slice.)
+    if constexpr (S4) sum[i] = sum[i] >> 4;
+    sum[i] += cin[i];
+  });
 
   // ---- meet the K slices of the other workgroups -----------------------------------
-  // Only wave 0 is left. It publishes this workgroup's partial block, then
-  // counts itself in; the workgroup that arrives last adds the slices up in
-  // slice order (so a float result does not depend on who arrived when) and
-  // goes on to store. The slices run on different XCDs, each with an L2 of
-  // its own, so partials and counter are moved with device-scope atomic
-  // accesses (relaxed 32-bit stores and loads: they go through to the point
-  // where the XCDs meet and leave the caches alone). A device-scope FENCE
-  // would be correct too and is far too expensive here: it writes back and
-  // invalidates the whole L2, under the feet of every workgroup that streams
-  // weights through it. What the counter increment has to wait for is only
-  // that this wave's own partial stores are complete.
+  // The workgroup publishes its partial blocks, then counts itself in; the
+  // workgroup that arrives last adds the slices up in slice order (so a float
+  // result does not depend on who arrived when) and goes on to store. The slices
+  // run on different XCDs, each with an L2 of its own, so partials and counter are
+  // moved with device-scope atomic accesses (relaxed 32-bit stores and loads: they
+  // go through to the point where the XCDs meet and leave the caches alone). A
+  // device-scope FENCE would be correct too and is far too expensive here: it
+  // writes back and invalidates the whole L2, under the feet of every workgroup
+  // that streams weights through it. What the counter increment has to wait for is
+  // only that the workgroup's own partial stores are complete: every wave waits for
+  // its own before the barrier.
   if (kslices > 1) {
+    __shared__ uint32_t arrived_lds;
     uint32_t* mine = reinterpret_cast<uint32_t*>(a.ws_partials) +
-                     (((size_t)block_id * kslices + slice) * (TM * TN * 64) + lane) * 4;
+                     (((size_t)block_id * kslices + slice) * (NB * 64) + lane) * 4;
+    for_each_own([&](int i, int tm, int tn) {
+      const v4i v = __builtin_bit_cast(v4i, sum[i]);
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        const v4i v = __builtin_bit_cast(v4i, acc[tm][tn]);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          __hip_atomic_store(mine + (tm * TN + tn) * 256 + e, (uint32_t)v[e], __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-      }
-    // All of the wave's stores above have been acknowledged before the count.
+      for (int e = 0; e < 4; ++e)
+        __hip_atomic_store(mine + (tm * TN + tn) * 256 + e, (uint32_t)v[e], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    });
+    // All of the wave's stores above have been acknowledged before the barrier.
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __builtin_amdgcn_s_waitcnt(0);
-    uint32_t arrived = 0;
-    if (lane == 0) {
-      arrived = __hip_atomic_fetch_add(a.ws_counters + block_id, 1u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      arrived_lds = __hip_atomic_fetch_add(a.ws_counters + block_id, 1u, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
     }
-    arrived = (uint32_t)__builtin_amdgcn_readfirstlane((int)arrived);
-    if (arrived != kslices - 1) return;
+    __syncthreads();
+    if (arrived_lds != kslices - 1) return;
     // The reader side of the handoff. What the other slices stored is complete
     // at the point where the XCDs meet before their counter increments (their
     // agent-scope stores are acknowledged from there, and each waited for its
@@ -475,27 +464,22 @@ void mmt4d_thin_kernel(Args a) {
     // loads above the test of the counter (workgroup scope: it costs no cache
     // write-back or invalidation).
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    if (lane == 0) {
+    if (threadIdx.x == 0) {
       __hip_atomic_store(a.ws_counters + block_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     const uint32_t* all = reinterpret_cast<const uint32_t*>(a.ws_partials) +
-                          ((size_t)block_id * kslices * (TM * TN * 64) + lane) * 4;
+                          ((size_t)block_id * kslices * (NB * 64) + lane) * 4;
 #pragma unroll
-    for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = Acc{0, 0, 0, 0};
+    for (int i = 0; i < OWN; ++i) sum[i] = Acc{0, 0, 0, 0};
     for (uint32_t sl = 0; sl < kslices; ++sl) {
+      for_each_own([&](int i, int tm, int tn) {
+        v4i v;
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) {
-          v4i v;
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            v[e] = (int)__hip_atomic_load(all + ((size_t)sl * (TM * TN) + tm * TN + tn) * 256 + e,
-                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          acc[tm][tn] += __builtin_bit_cast(Acc, v);
-        }
+        for (int e = 0; e < 4; ++e)
+          v[e] = (int)__hip_atomic_load(all + ((size_t)sl * NB + tm * TN + tn) * 256 + e,
+                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        sum[i] += __builtin_bit_cast(Acc, v);
+      });
     }
   }
 
@@ -505,28 +489,27 @@ void mmt4d_thin_kernel(Args a) {
       typedef v4f v4f_a4 __attribute__((aligned(4)));
       for_each_output(
           a.out, a.out_stride, a.out_sm0, a.out_spn, a.out_sn0,
-          [&](int tm, int tn, char* p) {
-            v4f v = __builtin_convertvector(acc[tm][tn], v4f);
+          [&](int i, char* p) {
+            v4f v = __builtin_convertvector(sum[i], v4f);
             if (a.col_scale_first) {
-              v = v * sn[tn];
-              v = v * sm[tm];
+              v = v * sn[i];
+              v = v * sm[i];
             } else {
-              v = v * sm[tm];
-              v = v * sn[tn];
+              v = v * sm[i];
+              v = v * sn[i];
             }
             *reinterpret_cast<v4f_a4*>(p) = v;
           },
-          [&](int tm, int tn, int e, char* p) {
-            const float v = (float)acc[tm][tn][e];
-            *reinterpret_cast<float*>(p) =
-                a.col_scale_first ? v * sn[tn][e] * sm[tm] : v * sm[tm] * sn[tn][e];
+          [&](int i, int e, char* p) {
+            const float v = (float)sum[i][e];
+            *reinterpret_cast<float*>(p) = a.col_scale_first ? v * sn[i][e] * sm[i] : v * sm[i] * sn[i][e];
           });
       return;
     }
   }
   for_each_output(a.out, a.out_stride, a.out_sm0, a.out_spn, a.out_sn0,
-                  [&](int tm, int tn, char* p) { Out::store4(p, acc[tm][tn]); },
-                  [&](int tm, int tn, int e, char* p) { Out::store1(p, acc[tm][tn][e]); });
+                  [&](int i, char* p) { Out::store4(p, sum[i]); },
+                  [&](int i, int e, char* p) { Out::store1(p, sum[i][e]); });
 }
 
 }  // namespace uk_mfma
