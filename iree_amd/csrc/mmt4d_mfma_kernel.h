@@ -346,6 +346,8 @@ struct Args {
   Divisor by_m0, by_n0, by_grid_n, by_blocks, by_band_blocks, by_band, by_last_band;
   // SLICED instances: steps of a slice, and how many slices have one more.
   uint32_t slice_steps, longer_slices;
+  // mmt4d_mfma_thin.h only: `band` counts block columns, not rows.
+  uint32_t column_bands;
 };
 
 // The last fields of Args from those before.
@@ -356,13 +358,14 @@ inline void set_divisors(Args& a) {
   const uint32_t slices = a.kslices > 1 ? a.kslices : 1;
   a.slice_steps = (uint32_t)a.steps / slices;
   a.longer_slices = (uint32_t)a.steps % slices;
-  if (a.band == 0) return;   // (the barrier-free kernel has no bands)
   a.by_blocks = Divisor::by((uint32_t)a.grid_m * (uint32_t)a.grid_n);
   // A band of more rows than there are is the only one.
-  const uint64_t band_blocks = (uint64_t)a.band * (uint32_t)a.grid_n;
+  const uint32_t along = (uint32_t)(a.column_bands ? a.grid_n : a.grid_m);
+  const uint32_t across = (uint32_t)(a.column_bands ? a.grid_m : a.grid_n);
+  const uint64_t band_blocks = (uint64_t)a.band * across;
   a.by_band_blocks = Divisor::by((uint32_t)std::min<uint64_t>(band_blocks, 1u << 31));
   a.by_band = Divisor::by(a.band);
-  a.by_last_band = Divisor::by((uint32_t)a.grid_m % a.band ? (uint32_t)a.grid_m % a.band : a.band);
+  a.by_last_band = Divisor::by(along % a.band ? along % a.band : a.band);
 }
 
 // Row-slot swizzle for the regrouping loaders (RB < 16): the eight lanes that

@@ -446,6 +446,9 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
       kslices = 1;
     }
   }
+  // (An XCD's share in as few bands as keep its blocks in a near-square patch.)
+  a.column_bands = grid_n >= grid_m;
+  a.band = (uint32_t)std::min<int64_t>(uk::ceil_div(std::max(grid_m, grid_n), (int64_t)8), 8);
   set_divisors(a);
   const dim3 grid((uint32_t)(grid_m * grid_n * kslices)), block(KSPLIT * 64);
   if constexpr (TAIL_OK) {
@@ -603,6 +606,24 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
   return uk::ceil_div(p.M1, bpm) * uk::ceil_div(p.N1, bpn);
 }
 
+// Steps of loads in flight in a wave of 32x32 to 64x64 blocks: two, three with 8-byte rows
+// (3 % ahead of two in 32x32, 4 % in 32x64, 5 % in 64x64 blocks; else 1 to 20 % behind).
+template <Elem E, int RBC>
+constexpr int steps_ahead() {
+  return RBC == 8 ? 3 : 2;
+}
+
+// What `blocks` workgroups of a kernel take, in us, by the KB of K. A unit's blocks are
+// loaded one beside the other, and a last round of few blocks is not a whole one; below
+// `least` blocks a unit a block's own chain of steps is what it takes.
+struct BlockCost {
+  double launch, round, k, k_block, least;
+};
+inline double block_us(const BlockCost& c, int64_t blocks, double kb) {
+  const double cus = (double)std::max(compute_units(), 1), units = (double)blocks / cus, rounds = std::ceil(units);
+  return c.launch + c.round * rounds + kb * (c.k + c.k_block * std::max(c.least, std::min(rounds, units + 0.6)));
+}
+
 // Problems whose 64x64 blocks leave compute units idle or take a last round that is
 // nearly empty: the barrier-free kernel in 16x16 or 32x32 blocks, several waves of a
 // block sharing K, so that the chain of K steps a wave walks through is short and many
@@ -625,13 +646,18 @@ inline int64_t workgroups(const Problem& p, int BM, int BN) {
 //     1280, 7.1 KB, 1.1 blocks 13.9 / 11.1; 235 x 1631, 11.9 KB, 1.6 blocks 22.2 / 29.0);
 //   f32, whose MFMAs are slow enough to hide the loads of 32x32 blocks, by costs fitted to
 //     1500 products of 64 to 4096 rows and columns, 256 B to 32 KB of K (3 to 10 % off in the
-//     mean; the choice is 1.8 % behind the fastest in the geometric mean, 21 calls are more
-//     than 4 % behind the kernel otherwise): 16x16x1 515 x 1027, 3 KB 22.6 / 17.5, 1500 x 1500
-//     54.3 / 46.2, 3000 x 3000, 8 KB 405 / 322; 16x16x4 1000 x 1500, 3 KB 28.5 / 25.3; but 893 x 4064, 13.5 KB 203 / 245, 16x16x1 1879 x 1045, 1.7 KB 25.0 / 28.0.
+//     mean): first whether at all, by what 32x32 blocks of four and two waves and the kernel
+//     otherwise took (893 x 4064, 13.5 KB 203 otherwise / 245, 16x16x1 1879 x 1045, 1.7 KB
+//     25.0 / 28.0), then which, by what all of these blocks take now: in the larger ones a
+//     unit's L1 and L2 carry fewer bytes a sum. us in 32x32 blocks before / as chosen: 16x16x4
+//     515 x 1027 x 768 13.6 / 11.2 (48x48), 1500 x 1500 x 1000 44.8 / 42.4; 16x16x1 515 x 1027 x
+//     769 17.6 / 12.8 (48x48), 1500 x 1500 x 1000 55.3 / 47.8, 700 x 700 x 3000 36.5 / 29.8.
+//     Geometric means over 400 drawn products: 16-byte rows 1.10, 4-byte rows 1.15.
 template <Elem E, int RBC>
 int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, bool ksplit64, bool parts,
                         bool b32x64, hipStream_t stream, const char** name) {
   constexpr bool F32 = E == Elem::kF32;
+  constexpr int kAhead = steps_ahead<E, RBC>();
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
   const int64_t cus = compute_units();
   if (cus < 1) return -1;   // the device query failed, as the launch will
@@ -648,46 +674,166 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
     }
   }
   if (b16 <= cus && k_bytes >= (RBC < 16 ? 64 : 256)) {
-    st = launch_thin<E, RBC, 1, 1, F32 ? 4 : 8, F32 ? 4 : 2, true>(p, false, stream);
+    st = launch_thin<E, RBC, 1, 1, F32 ? 4 : 8, F32 ? (RBC < 16 ? 8 : 4) : 2, true>(p, false, stream);
     if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
     return st;
   }
   if constexpr (F32) {
     if (k_bytes < (b128 || (RBC >= 16 && b32 > 2 * cus) ? 1024 : 256)) return -1;
     if (b16 <= 3 * cus) {
-      st = launch_thin<E, RBC, 1, 1, 4, 4, true>(p, false, stream);
+      st = launch_thin<E, RBC, 1, 1, 4, RBC < 16 ? 8 : 4, true>(p, false, stream);
       if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
       return st;
     }
-    // us, by the KB of K and the rounds of blocks: of these blocks in four waves, in two (not
-    // as precise as the 64x64 K split, and not in its place), and of the kernel that it would
-    // be otherwise.
-    const double kb = (double)k_bytes / 1024, r32 = (double)uk::ceil_div(b32, cus);
-    const double r64 = (double)uk::ceil_div(workgroups(p, 64, 64), cus);
+    // us of 32x32 blocks in four waves and in two (not as precise as the 64x64 K split, and
+    // not in its place), of 32x48 in four, 48x48 in eight. Where another shape is less than
+    // 6 % ahead, 32x32 blocks. (32x64 and 64x64 blocks were nowhere the fastest.)
+    const double kb = (double)k_bytes / 1024;
+    auto blocks = [&](int bm, int bn) {
+      return uk::ceil_div(rows, (int64_t)bm) * uk::ceil_div(cols, (int64_t)bn);
+    };
+    constexpr bool W = RBC >= 16;
+    constexpr double kOther = 1.06;
+    double us[4] = {
+        block_us(W ? BlockCost{3.14, 0.41, 0.15, 0.93, 1} : BlockCost{3.04, 0.44, 0.35, 0.98, 1}, b32, kb),
+        ksplit64 ? 1e30
+                 : block_us(W ? BlockCost{3.19, 0.30, 1.35, 0.89, 0} : BlockCost{3.14, 0.35, 1.52, 0.94, 0}, b32, kb),
+        kOther * block_us(W ? BlockCost{3.33, 0.58, 0.01, 1.42, 1} : BlockCost{3.24, 0.66, 0.35, 1.43, 1}, blocks(32, 48), kb),
+        kOther * block_us(W ? BlockCost{1.96, 2.55, 0, 2.11, 1} : BlockCost{1.96, 2.77, 0, 2.31, 1}, blocks(48, 48), kb)};
+    if (b32x64) us[2] = us[3] = 1e30;   // (64 rows and fewer)
+    static const char* const names[4] = {"mmt4d_mfma_32x32_ksplit", "mmt4d_mfma_32x32_ksplit", "mmt4d_mfma_32x48_ksplit",
+                                         "mmt4d_mfma_48x48_ksplit"};
+    const int best = (int)(std::min_element(us, us + 4) - us);
+    // And of the kernel that it would be otherwise, against what 32x32 blocks took when its
+    // costs were fitted beside theirs.
+    const double r32 = (double)uk::ceil_div(b32, cus), r64 = (double)uk::ceil_div(workgroups(p, 64, 64), cus);
     const double r128 = (double)uk::ceil_div(workgroups(p, 128, 128), cus);
-    const double four = RBC >= 16 ? 3.6 + 0.5 * r32 + kb * (0.13 + 1.09 * r32)
-                                  : 3.3 + 0.7 * r32 + kb * (0.37 + 1.28 * r32);
-    const double two = ksplit64    ? four
-                       : RBC >= 16 ? 3.75 + 0.33 * r32 + kb * (1.56 + 0.99 * r32)
-                                   : 3.5 + 0.43 * r32 + kb * (2.6 + 1.13 * r32);
-    const double other = b128              ? (RBC < 16 ? 5 + 3.6 * r128 + kb * (4 + 14.7 * r128)
-                                                       : 3 + 3.4 * r128 + kb * (2.4 + 13.65 * r128))
+    const double four = W ? 3.6 + 0.5 * r32 + kb * (0.13 + 1.09 * r32) : 3.3 + 0.7 * r32 + kb * (0.37 + 1.28 * r32);
+    const double two = ksplit64 ? four
+                       : W      ? 3.75 + 0.33 * r32 + kb * (1.56 + 0.99 * r32)
+                                : 3.5 + 0.43 * r32 + kb * (2.6 + 1.13 * r32);
+    const double other = b128              ? (W ? 3 + 3.4 * r128 + kb * (2.4 + 13.65 * r128)
+                                                : 5 + 3.6 * r128 + kb * (4 + 14.7 * r128))
                          : ksplit64        ? 6.7 + 1.1 * r64 + kb * 4 * r64
-                         : RBC >= 16       ? 3.4 + 0.7 * r64 + kb * (0.63 + 3.9 * r64)
+                         : W               ? 3.4 + 0.7 * r64 + kb * (0.63 + 3.9 * r64)
                          : k_bytes <= 8192 ? 2.9 + 1.9 * r64 + kb * (1.2 + 4.56 * r64)
                                            : 4.3 + kb * (2 + 3.95 * r64);
     if (b32x64 ? 2 * b32 > 7 * (int64_t)r64 * cus : std::min(four, two) > 1.02 * other) return -1;
-    st = two < four ? launch_thin<E, RBC, 2, 2, 2, 2, true>(p, false, stream)
-                    : launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
+    switch (best) {
+      case 0: st = launch_thin<E, RBC, 2, 2, 4, kAhead, true>(p, false, stream); break;
+      case 1: st = launch_thin<E, RBC, 2, 2, 2, kAhead, true>(p, false, stream); break;
+      case 2: st = launch_thin<E, RBC, 2, 3, 4, kAhead, true>(p, false, stream); break;
+      default: st = launch_thin<E, RBC, 3, 3, 8, 2, true>(p, false, stream); break;
+    }
+    if (st >= 0) *name = names[best];
+    return st;
   } else {
     // (8-bit floats, two loads an operand: 7/4 blocks a unit, 5/4 with 6 KB of K and more,
     // but in the place of 32x64 blocks. Rows of 2 bytes: one.)
     const int64_t most4 = RBC == 2 ? 4 : ElemTraits<E>::kHalves == 2 && !b32x64 ? (ksplit64 ? 5 : 7) : 8;
     if (4 * b32 > most4 * cus || k_bytes < 1024) return -1;
-    st = launch_thin<E, RBC, 2, 2, 4, 2, true>(p, false, stream);
+    st = launch_thin<E, RBC, 2, 2, 4, kAhead, true>(p, false, stream);
   }
   if (st >= 0) *name = "mmt4d_mfma_32x32_ksplit";
   return st;
+}
+
+// The kernels between the thin ones and 256x256 blocks, by what they take: the barrier-free
+// kernel in blocks of 32x32, 32x64 and 64x64, four waves sharing K; 64x64 blocks with the
+// RHS in registers (rows of 2 bytes: regrouped, 256 bytes of K a step); 64x64 and 128x128
+// blocks of the LDS-direct pipeline. Fitted, for each class of tile rows, to 300 products of
+// 65 to 4096 rows, 65 to 16384 columns, 128 B to 24 KB of K and up to 330 128x128 blocks, each
+// on all of these kernels with operands that are not cached: 5 to 14 % off in the mean, and
+// the choice is 1 to 4 % behind the fastest in the geometric mean (rules by numbers of
+// blocks were 12 to 21 % behind). us by those rules / so: f16 512 x 2048 x 2048 13.4 / 10.3,
+// 700 x 900 x 1504 11.1 / 8.7, 1500 x 1500 x 1504 18.1 / 14.3, but 1000 x 1501 x 777 9.0 /
+// 9.2; f8 900 x 1100 x 1300 8.8 / 7.1; bf16 16x16x2 1000 x 1500 x 784 17.3 / 11.1; s8 16x16x2
+// 2000 x 700 x 2000 17.4 / 13.3. Geometric means over 400 drawn products of 65 to 4096 rows:
+// f16 1.14, s8 1.15, 8-byte rows 1.09, 2-byte rows 1.16, f8 1.10, bf16 4-byte rows 1.13.
+enum BlockKind { k32x32, k32x64, k64x64Split, k64x64, k64x64Lds, k128x128, kBlockKinds };
+template <Elem E, int RBC>
+inline const BlockCost* block_costs() {
+  constexpr double no = 1e30;
+  static constexpr BlockCost f8[kBlockKinds] = {{3.07, 0.28, 0.14, 0.60, 0}, {2.78, 0.87, 0.26, 0.90, 0},
+                                                {1.44, 2.95, 0.21, 1.43, 0}, {3.63, 0.75, 0.20, 1.76, 0},
+                                                {no, 0, 0, 0, 0},            {3.37, 1.53, 2.93, 2.50, 0}};
+  static constexpr BlockCost rows16[kBlockKinds] = {{3.12, 0.20, 0.20, 0.59, 0}, {3.10, 0.49, 0.28, 0.92, 0},
+                                                    {3.07, 1.15, 0.37, 1.26, 0}, {3.34, 0.55, 1.41, 1.40, 0},
+                                                    {no, 0, 0, 0, 0},            {3.48, 1.74, 1.35, 2.74, 0}};
+  static constexpr BlockCost rows8[kBlockKinds] = {{3.08, 0.23, 0.05, 0.92, 1}, {3.09, 0.54, 0.36, 1.31, 0},
+                                                   {3.12, 1.19, 0.59, 1.71, 0}, {no, 0, 0, 0, 0},
+                                                   {1.16, 3.88, 0.39, 1.91, 0}, {3.04, 2.33, 3.08, 1.87, 0}};
+  static constexpr BlockCost rows4[kBlockKinds] = {{3.18, 0.22, 0.03, 0.89, 1}, {3.21, 0.52, 0.04, 1.35, 1},
+                                                   {3.28, 1.22, 0, 1.83, 1},    {no, 0, 0, 0, 0},
+                                                   {1.14, 3.94, 0.41, 1.95, 0}, {3.14, 2.35, 2.98, 2.08, 0}};
+  static constexpr BlockCost rows2[kBlockKinds] = {{2.20, 0.55, 1.31, 1.72, 1.25}, {2.68, 1.18, 0.11, 2.65, 1},
+                                                   {no, 0, 0, 0, 0},               {2.92, 1.19, 0.21, 2.65, 1.25},
+                                                   {1.44, 3.63, 0.06, 1.97, 0},    {3.92, 1.87, 1.62, 2.79, 0}};
+  return ElemTraits<E>::kHalves == 2 ? f8 : RBC >= 16 ? rows16 : RBC == 8 ? rows8 : RBC == 4 ? rows4 : rows2;
+}
+template <Elem E, int RBC>
+double kind_us(const Problem& p, int64_t rows, int64_t cols, int kind) {
+  static constexpr int bm[] = {32, 32, 64, 64, 64, 128}, bn[] = {32, 64, 64, 64, 64, 128};
+  // (LDS blocks hold whole panels, the others need not)
+  const int64_t blocks = kind >= k64x64 ? workgroups(p, bm[kind], bn[kind])
+                                        : uk::ceil_div(rows, (int64_t)bm[kind]) * uk::ceil_div(cols, (int64_t)bn[kind]);
+  if (blocks < 1) return 1e30;
+  return block_us(block_costs<E, RBC>()[kind], blocks, (double)((int64_t)p.K1 << p.lrb) / 1024);
+}
+// `parts`: a float's K stays in four parts, as it is in kernels whose waves share it and in
+// the 64x64 blocks in registers.
+template <Elem E, int RBC>
+int launch_by_cost(const Problem& p, int64_t rows, int64_t cols, bool parts, hipStream_t stream, const char** name) {
+  static_assert(E != Elem::kF32, "launch_small_blocks");
+  constexpr bool kInteger = std::is_same<typename ElemTraits<E>::Acc, v4i>::value;
+  const int64_t k_bytes = (int64_t)p.K1 << p.lrb, cus = compute_units();
+  if (cus < 1) return -1;   // the device query failed, as the launch will
+  if (uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16) <= cus && k_bytes >= (RBC < 16 ? 64 : 256)) {
+    const int st = launch_thin<E, RBC, 1, 1, 8, 2, true>(p, false, stream);
+    if (st >= 0) { *name = "mmt4d_mfma_16x16_ksplit"; return st; }
+  }
+  double us[kBlockKinds];
+  for (int k = 0; k < kBlockKinds; ++k) {
+    us[k] = kind_us<E, RBC>(p, rows, cols, k);
+    // (The 64x64 blocks in registers have a float's K in four parts from 96 steps on. 8-bit
+    // floats: the matrix instructions round to 1.5e-5, however K is divided.)
+    if (parts && !kInteger && ElemTraits<E>::kHalves == 1 && k > k64x64Split &&
+        !(k == k64x64 && RBC >= 16 && k_bytes >= 6144)) {
+      us[k] = 1e30;
+    }
+  }
+  // With less than 1 KB of K a block of 128x128 is its stores, estimated low (f16 3428 x 704 x
+  // 132 in 64x64 blocks 6.3 us, in these 7.6).
+  if (k_bytes < 1024 && workgroups(p, 128, 128) < 192) us[k128x128] = 1e30;
+  // 2-byte results: the LDS-direct 64x64 shape takes K in whole steps.
+  if (ElemTraits<E>::Out::kOutBytes == 2 && k_bytes % 256 != 0) us[k64x64Lds] = 1e30;
+  for (;;) {
+    const int k = (int)(std::min_element(us, us + kBlockKinds) - us);
+    if (us[k] >= 1e30) return -1;
+    us[k] = 1e30;
+    int st = -1;
+    if (k == k32x32) {
+      st = launch_thin<E, RBC, 2, 2, 4, steps_ahead<E, RBC>(), true>(p, false, stream);
+      if (st >= 0) *name = "mmt4d_mfma_32x32_ksplit";
+    } else if (k == k32x64) {
+      st = launch_thin<E, RBC, 2, 4, 4, steps_ahead<E, RBC>(), true>(p, false, stream);
+      if (st >= 0) *name = "mmt4d_mfma_32x64_ksplit";
+    } else if (k == k64x64Split) {
+      if constexpr (RBC >= 4) st = launch_thin<E, RBC, 4, 4, 4, steps_ahead<E, RBC>(), true>(p, false, stream);
+      if (st >= 0) *name = "mmt4d_mfma_64x64_ksplit";
+    } else if (k == k64x64) {
+      if constexpr (RBC >= 16) st = launch_variant<E, RBC, 2, 2, 2, 2, 1, 3>(p, 0, p.K1, p.accumulate, stream);
+      else st = launch_variant<E, RBC, 2, 2, 2, 2, 4 / ElemTraits<E>::kHalves, 4>(p, 0, p.K1, p.accumulate, stream);
+      if (st >= 0) *name = RBC >= 16 ? "mmt4d_mfma_64x64_rhs_direct" : "mmt4d_mfma_64x64_deep";
+    } else if (k == k64x64Lds) {
+      if constexpr (RBC < 16) st = launch_variant<E, RBC, 2, 1, 2, 4, 4, 5>(p, 0, p.K1, p.accumulate, stream);
+      if (st >= 0) *name = "mmt4d_mfma_64x64_lds_direct";
+    } else {
+      st = launch_variant<E, RBC, 4, 2, 2, 4, 1, 5>(p, 0, p.K1, p.accumulate, stream);
+      if (st >= 0) *name = "mmt4d_mfma_128x128_lds_direct";
+    }
+    if (st >= 0) return st;
+  }
 }
 
 // K slices for launch_slices, one workgroup a compute unit or fewer; 0 where the blocks
@@ -1089,11 +1235,31 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
     }
   }
   const bool splits_k = long_k && (E != Elem::kF32 || 2 * workgroups(p, 64, 64) <= compute_units());
-  if (forced == 0 && (choice == 3 || (choice == 6 && (!splits_k || E == Elem::kF32)) || (RBC < 8 && choice == 4) ||
-                      (choice == 2 && E == Elem::kF32))) {
-    const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, choice == 6 && splits_k,
-                                               choice == 4 && RBC != 2, stream, name);
-    if (st >= 0) return st;
+  if constexpr (E == Elem::kF32) {
+    if (forced == 0 && (choice == 2 || choice == 3 || choice == 6 || (RBC < 8 && choice == 4))) {
+      const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, choice == 6 && splits_k,
+                                                 choice == 4 && RBC != 2, stream, name);
+      if (st >= 0) return st;
+    }
+  } else {
+    // (Costs as fitted: up to 330 128x128 blocks; with 24 KB of K and more 64x64 blocks have
+    // it in workgroups, too. Calls that direct_before_ksplit keeps in the kernels that stage
+    // through LDS stay there, and rows under 16 bytes with less than 1 KB of K.)
+    const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
+    const bool by_cost = !long_k && (RBC >= 16 || k_bytes >= 1024) &&
+                         ((choice == 2 && workgroups(p, 128, 128) <= 330) || choice == 3 ||
+                          (choice == 6 && !direct_before_ksplit<E, RBC>(p)) || (RBC == 2 && choice == 4));
+    if (forced == 0 && by_cost) {
+      const int64_t b32 = uk::ceil_div(rows_m, (int64_t)32) * uk::ceil_div(cols_n, (int64_t)32);
+      const bool parts = choice == 6 || (choice != 2 && b32 <= 2 * (int64_t)compute_units() && k_bytes >= 1024) ||
+                         (choice == 3 && RBC >= 16 && k_bytes >= 6144);
+      const int st = launch_by_cost<E, RBC>(p, rows_m, cols_n, parts, stream, name);
+      if (st >= 0) return st;
+    } else if (forced == 0 && (choice == 3 || (choice == 6 && !splits_k) || (RBC < 8 && choice == 4))) {
+      const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, false, choice == 6, false,
+                                                 choice == 4 && RBC != 2, stream, name);
+      if (st >= 0) return st;
+    }
   }
   if (forced == 0 && choice == 6 && direct_before_ksplit<E, RBC>(p)) choice = 3;
   if (choice == 6) {
@@ -1106,7 +1272,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       // 128 x 128 x 65536, four blocks: 177 -> 52 us; 256 x 256 x 32768: 80 ->
       // 35; 512 x 512 x 16384: 44 -> 27; with 8 KB of K per row, 384 x 384 x
       // 4096, it loses: 16 -> 20 us).
-      int st = launch_thin<E, RBC, 4, 4, 4, 2, true>(p, false, stream, long_k, 32);
+      int st = launch_thin<E, RBC, 4, 4, 4, steps_ahead<E, RBC>(), true>(p, false, stream, long_k, 32);
       if (st >= 0) { *name = "mmt4d_mfma_64x64_ksplit"; return st; }
     }
     choice = 3;
