@@ -1253,7 +1253,7 @@ bool launch_stream(const TiledPlan& plan, hipStream_t stream) {
 struct DirectArgs {
   const char* src;
   char* dst;
-  int64_t src_pitch;         // bytes between matrix rows
+  int64_t mat_pitch;         // bytes between matrix rows
   int64_t s0, s1;            // tiled side: bytes from one row tile / column tile to the next
   uint32_t rows, row_bytes;  // the matrix
   uint32_t padded_rows, padded_row_bytes;  // what its tiles hold
@@ -1264,10 +1264,25 @@ struct DirectArgs {
 };
 constexpr int kDirectPieces = 4;
 
+// The first `left` < N bytes of a piece.
+template <int N>
+__device__ __forceinline__ void store_row_end(char* p, const Words<N>& v, int32_t left) {
+  typedef uint32_t u32_a1 __attribute__((aligned(1)));
+  typedef uint16_t u16_a1 __attribute__((aligned(1)));
+  uint32_t rest = v.w[0];  // the word that is not whole
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) {
+    if (left >= 4 * (i + 1)) *reinterpret_cast<u32_a1*>(p + 4 * i) = v.w[i];
+    else if (left > 4 * i) rest = v.w[i];
+  }
+  if (left & 2) *reinterpret_cast<u16_a1*>(p + (left & ~3)) = (uint16_t)rest;
+  if (left & 1) p[left & ~1] = (char)(rest >> (left & 2 ? 16 : 0));
+}
+
 template <int PB>
 __global__ __launch_bounds__(kThreads) void pack_direct_kernel(DirectArgs a) {
   using Piece = typename GBytes<PB>::type;
-  uk::load_arguments_now(a.src, a.dst, a.src_pitch, a.s0, a.s1, a.rows, a.row_bytes, a.padded_rows, a.padded_row_bytes,
+  uk::load_arguments_now(a.src, a.dst, a.mat_pitch, a.s0, a.s1, a.rows, a.row_bytes, a.padded_rows, a.padded_row_bytes,
                          a.tile_row_bytes, a.log2_tile_row_bytes, a.col_groups, a.pad32, a.div_tile_rows.mul);
   const uint32_t rg = blockIdx.x / a.col_groups, cg = blockIdx.x - rg * a.col_groups;
   const uint32_t row = rg * 16 + (threadIdx.x >> 4);
@@ -1275,7 +1290,7 @@ __global__ __launch_bounds__(kThreads) void pack_direct_kernel(DirectArgs a) {
   uint32_t o0, m0;
   a.div_tile_rows.divmod(row, o0, m0);
   const bool row_ok = row < a.rows;
-  const char* srow = a.src + (int64_t)min(row, a.rows - 1) * a.src_pitch;
+  const char* srow = a.src + (int64_t)min(row, a.rows - 1) * a.mat_pitch;
   char* drow = a.dst + (int64_t)o0 * a.s0 + (int64_t)m0 * a.tile_row_bytes;
   const uint32_t col0 = (cg * 64 + (threadIdx.x & 15)) * PB;
   Words<PB> v[kDirectPieces];
@@ -1346,7 +1361,7 @@ bool launch_pack_direct(const iree_uk_pack_params_t* p, const TiledView& v, int 
   }
   DirectArgs a;
   a.src = src; a.dst = dst;
-  a.src_pitch = pitch;
+  a.mat_pitch = pitch;
   a.s0 = s0; a.s1 = s1;
   a.rows = (uint32_t)p->in_size0; a.row_bytes = (uint32_t)row_bytes;
   a.padded_rows = (uint32_t)rows; a.padded_row_bytes = (uint32_t)padded;
@@ -1358,6 +1373,79 @@ bool launch_pack_direct(const iree_uk_pack_params_t* p, const TiledView& v, int 
   a.div_tile_rows = FastDiv((uint32_t)v.tile0);
   uk::launch(0, PB == 16 ? pack_direct_kernel<16> : pack_direct_kernel<8>, dim3((uint32_t)grid), dim3(kThreads), 0,
              stream, a);
+  return true;
+}
+
+// Direct unpack: the same the other way, tile rows of whole pieces to matrix rows.
+// A wave reads, per tile, 4 consecutive tile rows and writes 16 neighbouring pieces
+// of each of 4 matrix rows. A piece beyond the end of its row is loaded from the
+// row's last one and not stored; the piece that the row ends in is stored in parts.
+// Bound by the latency of one pass (launch, load, store) up to some 8 MB of matrix and
+// by the caches it copies between beyond: against the streaming kernel, calls one after
+// the other with the tiles in the caches, f32 from 16x16 1000 x 1501 6.5 -> 4.5 us, 2048
+// x 1024 6.7 -> 4.8, 2047 x 2049 11.8 -> 10.1; 16x4 1500 x 1999 10.1 -> 7.8; f16 2048 x
+// 2048 6.1 -> 4.6 (the host, which takes 4.2 a call, bounds what is smaller).
+template <int PB>
+__global__ __launch_bounds__(kThreads) void unpack_direct_kernel(DirectArgs a) {
+  uk::load_arguments_now(a.src, a.dst, a.mat_pitch, a.s0, a.s1, a.rows, a.row_bytes, a.tile_row_bytes,
+                         a.log2_tile_row_bytes, a.col_groups, a.div_tile_rows.mul);
+  const uint32_t rg = blockIdx.x / a.col_groups, cg = blockIdx.x - rg * a.col_groups;
+  const uint32_t row = rg * 16 + (threadIdx.x >> 4);
+  if (row >= a.rows) return;
+  uint32_t o0, m0;
+  a.div_tile_rows.divmod(row, o0, m0);
+  const char* srow = a.src + (int64_t)o0 * a.s0 + (int64_t)m0 * a.tile_row_bytes;
+  char* drow = a.dst + (int64_t)row * a.mat_pitch;
+  const uint32_t col0 = (cg * 64 + (threadIdx.x & 15)) * PB;
+  const uint32_t last = (a.row_bytes - 1) & ~(uint32_t)(PB - 1);
+  typename GBytes<PB>::type v[kDirectPieces];
+#pragma unroll
+  for (int i = 0; i < kDirectPieces; ++i) {
+    const uint32_t col = min(col0 + i * 16 * PB, last);
+    v[i] = gload<PB>(srow + (int64_t)(col >> a.log2_tile_row_bytes) * a.s1 + (col & (a.tile_row_bytes - 1)));
+  }
+#pragma unroll
+  for (int i = 0; i < kDirectPieces; ++i) {
+    const uint32_t col = col0 + i * 16 * PB;
+    const int32_t left = uk::row_bytes_left(a.row_bytes, col);
+    if (left >= PB) gstore<PB>(drow + col, v[i]);
+    else if (left > 0) store_row_end<PB>(drow + col, __builtin_bit_cast(Words<PB>, v[i]), left);
+  }
+}
+
+// Launches the direct unpack for a call that the streaming kernels would take (`plan`)
+// and that is of its form; false otherwise. Such a call goes by the streaming kernels'
+// name, too.
+bool launch_unpack_direct(const iree_uk_unpack_params_t* p, const TiledPlan& plan, const TiledView& v, int es,
+                          const char* src, char* dst, bool transpose_inner, hipStream_t stream) {
+  if (transpose_inner || plan.VEC != 16 || plan.G < 8) return false;
+  const int64_t trb = v.tile1 * es;
+  if (trb < plan.G || (trb & (trb - 1))) return false;
+  const int64_t rows = v.outer0 * v.tile0, padded = v.outer1 * trb;
+  if (p->out_size0 <= 0 || p->out_size1 <= 0 || p->out_size0 > rows || p->out_size1 * es > padded) return false;
+  // Up to 24 MB, as in the pack: f32 from 16x16 2000 x 2600 12.5 -> 11.7 us, 2500 x 2500
+  // 14.3 -> 13.5 (from 16x4 under TRANSPOSE_OUTER 15.0 -> 14.8), but 3000 x 3001, 34 MB,
+  // 18.9 -> 19.4, 4097 x 6001 38.9 -> 43.4. Tall matrices of few columns, most of whose
+  // lanes have no piece, are level at worst (f32 180000 x 25 from 16x4 14.3 -> 14.4, 400000
+  // x 13 from 1x4 29.3 -> 29.3, 60000 x 30 from 16x16 7.2 -> 5.9); narrower ones are not
+  // the streaming kernels'.
+  if (rows * padded > (24ll << 20) || v.tile0 >= (1 << 20)) return false;
+  const int64_t col_groups = uk::ceil_div(p->out_size1 * es, (int64_t)64 * plan.G);
+  const int64_t grid = uk::ceil_div(p->out_size0, (int64_t)16) * col_groups;
+  DirectArgs a;
+  a.src = src; a.dst = dst;
+  a.mat_pitch = p->out_stride0 * es;
+  a.s0 = v.sl0 * es; a.s1 = v.sl1 * es;
+  a.rows = (uint32_t)p->out_size0; a.row_bytes = (uint32_t)(p->out_size1 * es);
+  a.padded_rows = (uint32_t)rows; a.padded_row_bytes = (uint32_t)padded;
+  a.tile_row_bytes = (uint32_t)trb;
+  a.log2_tile_row_bytes = 0;
+  while ((1u << a.log2_tile_row_bytes) < a.tile_row_bytes) ++a.log2_tile_row_bytes;
+  a.col_groups = (uint32_t)col_groups;
+  a.pad32 = 0;
+  a.div_tile_rows = FastDiv((uint32_t)v.tile0);
+  uk::launch(1, plan.G == 16 ? unpack_direct_kernel<16> : unpack_direct_kernel<8>, dim3((uint32_t)grid),
+             dim3(kThreads), 0, stream, a);
   return true;
 }
 
@@ -1487,7 +1575,9 @@ extern "C" int iree_uk_amd_hip_launch_unpack(const iree_uk_unpack_params_t* p_in
       plan.args.src = src;
       plan.args.dst = dst;
       plan.args.pad32 = 0;
-      if (plan.stream && launch_stream<true>(plan, stream)) {
+      if (plan.stream && ((kernel_mode == IREE_UK_AMD_KERNEL_MODE_AUTO &&
+                           launch_unpack_direct(p, plan, v, es, src, dst, ti, stream)) ||
+                          launch_stream<true>(plan, stream))) {
         *kernel_name = "unpack_stream";
         return (int)hipGetLastError();
       }
