@@ -275,8 +275,7 @@ static __device__ __attribute__((aligned(16))) const uint32_t kZeroPiece[4] = {0
 struct Divisor {
   uint32_t multiplier, shift;  // (d = 1, whose multiplier has 33 bits: 0)
   static Divisor by(uint32_t d) {
-    uint32_t l = 0;
-    while ((1ull << l) < d) ++l;
+    const uint32_t l = d > 1 ? 32 - (uint32_t)__builtin_clz(d - 1) : 0;
     return l == 0 ? Divisor{0, 0} : Divisor{(uint32_t)((1ull << (31 + l)) / d + 1), l - 1};
   }
   __device__ __forceinline__ uint32_t quotient(uint32_t n) const {
