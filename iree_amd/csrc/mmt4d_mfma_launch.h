@@ -451,23 +451,37 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   a.band = (uint32_t)std::min<int64_t>(uk::ceil_div(std::max(grid_m, grid_n), (int64_t)8), 8);
   set_divisors(a);
   const dim3 grid((uint32_t)(grid_m * grid_n * kslices)), block(KSPLIT * 64);
+  // 8-byte rows in twos (PAIRED): 32 x 14336 x 4096, four layers, f16 134 -> 120 us, s8 78 ->
+  // 74, and at 16 rows 115 -> 108 and 68.5 -> 65.8; in 64x64 blocks f16 2000 x 300 x 4099
+  // 19.4 -> 16.8, s8 512 x 2048 x 2048 8.8 -> 8.1, in 32x64 f16 96 x 4096 x 4096 15.0 -> 12.5.
+  // A column tile of an odd number of rows would split such a two.
+  constexpr bool kPairs = RBC == 8 && TN % 2 == 0;
   if constexpr (TAIL_OK) {
     // No non-temporal instances: weights that the caller has declared streamed are read
     // by several row blocks here, which then wait for HBM one after the other (64x64
     // blocks, ordinary / non-temporal us: f16 200 x 8192 x 4096 34.6 / 44.5, s8 80 x 8192 x
     // 8192 21.4 / 25.0, 128 x 4096 x 14336 34.9 / 35.6; at best f8 192 x 4096 x 8192 21.6 / 21.1).
-    if (tail) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, true, CH>, grid, block, 0, stream, a);
-    else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, CH>, grid, block, 0, stream, a);
-    return (int)hipGetLastError();
+    auto go = [&](auto paired_c) {
+      constexpr bool P = decltype(paired_c)::value;
+      if (tail) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, true, CH, P>, grid, block, 0, stream, a);
+      else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, CH, P>, grid, block, 0, stream, a);
+      return (int)hipGetLastError();
+    };
+    if (kPairs && p.N0 % 2 == 0) return go(std::bool_constant<kPairs>{});
+    return go(std::false_type{});
+  } else {
+    // Weights that the caller has declared streamed, when they are too large for
+    // the L2s anyway: loaded non-temporally.
+    const bool streamed = streamed_weights() && (int64_t)p.N1 * p.N0 * k_bytes / (S4 ? 2 : 1) >= (16ll << 20);
+    auto go = [&](auto paired_c) {
+      constexpr bool P = decltype(paired_c)::value;
+      if (streamed) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, true, false, 0, P>, grid, block, 0, stream, a);
+      else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, 0, P>, grid, block, 0, stream, a);
+      return (int)hipGetLastError();
+    };
+    if (kPairs && p.N0 % 2 == 0) return go(std::bool_constant<kPairs>{});
+    return go(std::false_type{});
   }
-  // Weights that the caller has declared streamed, when they are too large for
-  // the L2s anyway: loaded non-temporally.
-  if (streamed_weights() && (int64_t)p.N1 * p.N0 * k_bytes / (S4 ? 2 : 1) >= (16ll << 20)) {
-    uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, true>, grid, block, 0, stream, a);
-    return (int)hipGetLastError();
-  }
-  uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D>, grid, block, 0, stream, a);
-  return (int)hipGetLastError();
 }
 
 // The thin kernel with TM 16-row blocks against `wide_cols` columns (rows of the
@@ -508,8 +522,12 @@ int launch_thin_rows(const Problem& p, bool swapped, int64_t wide_cols, hipStrea
   const int64_t short_k = blocks32 < cus ? kShort : TM == 1 && kInteger ? 1024 : 0;
   if (blocks16 > cus && ((int64_t)p.K1 << p.lrb) <= short_k)
     return launch_thin<E, RBC, TM, 1, 4, 4>(p, swapped, stream, true);
+  // (Not for 8-byte rows in twos, whose loads are half as many in 32 columns: s8, 8-byte rows,
+  // in 16 columns over eight waves / so, four layers, 4 x 11008 x 4096 64.3 / 60.8 us, 16 x
+  // 28672 x 8192 221 / 191. Floats keep the parts of K that eight waves have.)
+  const bool paired = kInteger && RBC == 8 && (swapped ? p.M0 : p.N0) % 2 == 0;
   const bool narrow = blocks16 <= cus ||
-                      (TM == 1 && uk::ceil_div(blocks16, cus) < 2 * uk::ceil_div(blocks32, cus));
+                      (TM == 1 && !paired && uk::ceil_div(blocks16, cus) < 2 * uk::ceil_div(blocks32, cus));
   if (narrow) return launch_thin<E, RBC, TM, 1, 8, TM == 1 && H == 1 ? 4 : 2>(p, swapped, stream, true);
   return launch_thin<E, RBC, TM, 2, 4, TM == 4 ? 3 : 4>(p, swapped, stream, true);
 }

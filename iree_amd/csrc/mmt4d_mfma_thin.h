@@ -116,8 +116,15 @@ __device__ __forceinline__ void block_in_bands(uint32_t wg, const Args& a, int* 
 // (iree_uk_amd_set_streamed_weights): a layer's weights then pass through the
 // caches without displacing what is used again.
 // CH: chains of a wave's sums (0: thin_chains).
-template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false, bool TAIL = false, int CH = 0>
-__global__ __launch_bounds__(KSPLIT * 64)
+// PAIRED: RHS rows of 8 bytes in twos. A lane loads two neighbouring rows of a K-tile as
+// 16 bytes, half as many loads for the same bytes, and what it gets belongs to the same lane
+// of two column blocks: the one then holds the even and the other the odd columns of 32,
+// which the waves that add up and store put back in order. Sums are the same bit for bit.
+// N0 is even. (These blocks are bound by how many loads a unit's L1 and the waves' loops
+// take, the thin ones beside by HBM: launch_thin has the figures.)
+template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false, bool TAIL = false, int CH = 0,
+          bool PAIRED = false>
+__global__ __launch_bounds__(KSPLIT * 64, PAIRED && TM * TN >= 16 ? 2 : 1)   // (else two registers too many for two)
 void mmt4d_thin_kernel(Args a) {
   using TT = ElemTraits<E>;
   using Acc = typename TT::Acc;
@@ -130,6 +137,7 @@ void mmt4d_thin_kernel(Args a) {
   constexpr bool S4 = E == Elem::kS8S4;       // 4-bit RHS: half the bytes per row
   constexpr int CHAINS = CH > 0 ? CH : thin_chains<E, TM, KSPLIT>();
   static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
+  static_assert(!PAIRED || (RBC == 8 && TN % 2 == 0 && HALVES == 1), "two rows in 16 bytes, columns of two blocks");
   static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
 
   // The blocks that a wave adds up and stores: OWN, or for the last ones fewer.
@@ -171,9 +179,8 @@ void mmt4d_thin_kernel(Args a) {
   const int pa0 = (int)a.by_m0.quotient(bm * TM * 16), pb0 = (int)a.by_n0.quotient(bn * TN * 16);
   const __amdgpu_buffer_rsrc_t from_a = operand_at(a.lhs + (int64_t)pa0 * a.lhs_stride);
   const __amdgpu_buffer_rsrc_t from_b = operand_at(a.rhs + (int64_t)pb0 * a.rhs_stride);
-  auto operand_offsets = [&](uint32_t (&off)[HALVES], int x, int X0, const Divisor& by_x0, int X1, int rows,
+  auto operand_offsets = [&](uint32_t (&off)[HALVES], uint32_t row, int X0, const Divisor& by_x0, int X1, int rows,
                              int p0, int64_t stride, uint32_t kt_bytes, int lrb, uint32_t piece_bytes) {
-    const uint32_t row = (uint32_t)x * 16 + r;
     const uint32_t pabs = by_x0.quotient(row);
     const uint32_t x0 = row - pabs * X0;
     const bool ok = (int)pabs < X1 && (int)row < rows;
@@ -194,11 +201,11 @@ void mmt4d_thin_kernel(Args a) {
   uint32_t offa[TM][HALVES], offb[TN][HALVES];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
-    operand_offsets(offa[tm], bm * TM + tm, a.M0, a.by_m0, a.M1, a.out_rows, pa0, a.lhs_stride, kt_m, lrb, 16);
+    operand_offsets(offa[tm], (uint32_t)(bm * TM + tm) * 16 + r, a.M0, a.by_m0, a.M1, a.out_rows, pa0, a.lhs_stride, kt_m, lrb, 16);
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn)
-    operand_offsets(offb[tn], bn * TN + tn, a.N0, a.by_n0, a.N1, a.out_cols, pb0, a.rhs_stride, kt_n, lrb_b,
-                    S4 ? 8 : 16);
+    operand_offsets(offb[tn], (uint32_t)(bn * TN + (PAIRED ? tn & ~1 : tn)) * 16 + (PAIRED ? 2 * r : r), a.N0, a.by_n0,
+                    a.N1, a.out_cols, pb0, a.rhs_stride, kt_n, lrb_b, S4 ? 8 : 16);
 
   // Whether piece t of chunk (h, q) of K step s lies inside K.
   auto in_k = [&](uint32_t s, int h, int t) {
@@ -254,6 +261,11 @@ void mmt4d_thin_kernel(Args a) {
       for (int h = 0; h < HALVES; ++h) {
         if constexpr (S4) {
           fb[d][tn][h] = load8<STREAMED>(from_b, offb[tn][h], at_b);
+        } else if constexpr (PAIRED) {
+          // K-tiles g (even tn) and g + NCH of both columns.
+          const uint32_t off =
+              !decltype(ends)::value || in_k(s, h, tn % 2) ? offb[tn][h] : kBeyond;
+          fb[d][tn][h] = load16<STREAMED>(from_b, off, at_b + (tn % 2) * NCH * kt_n);
         } else {
           fb[d][tn][h] = load_operand(std::bool_constant<STREAMED>{}, ends, from_b, offb[tn][h], at_b, kt_n, s, h);
         }
@@ -276,7 +288,12 @@ void mmt4d_thin_kernel(Args a) {
   // ---- output addressing (see for_each_output in mmt4d_mfma_kernel.h) ------
   // Lane (q, r) of block b = tm * TN + tn holds output row r, columns 4q..4q+3.
   // f4(i, p) / f1(i, e, p) for the i-th of this wave's blocks.
+  // PAIRED: of two neighbouring own blocks the first holds columns 8q..8q+3 of their 32,
+  // the second 8q+4..8q+7.
   const int first_own = wave * OWN;
+  auto first_col = [&](int tn) {
+    return PAIRED ? (bn * TN + (tn & ~1)) * 16 + 8 * (int)q + 4 * (tn & 1) : (bn * TN + tn) * 16 + 4 * (int)q;
+  };
   auto for_each_own = [&](auto f) {
 #pragma unroll
     for (int i = 0; i < OWN; ++i)
@@ -289,7 +306,7 @@ void mmt4d_thin_kernel(Args a) {
       const int pl = (int)a.by_m0.quotient(row), m0 = row - pl * a.M0;
       const bool row_ok = pl < a.M1 && row < a.out_rows;
       char* row_base = const_cast<char*>(base) + (int64_t)pl * s_panel + (int64_t)m0 * s_m0;
-      const int col = (bn * TN + tn) * 16 + 4 * (int)q;
+      const int col = first_col(tn);
       if (a.vec_out) {
         const int pc = (int)a.by_n0.quotient(col), n0 = col - pc * a.N0;
         const int left = a.out_cols - col;
@@ -356,7 +373,7 @@ void mmt4d_thin_kernel(Args a) {
       for_each_own([&](int i, int, int tn) {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          sn[i][e] = a.col_scale[max(min((bn * TN + tn) * 16 + 4 * (int)q + e, a.out_cols - 1), 0)];
+          sn[i][e] = a.col_scale[max(min(first_col(tn) + e, a.out_cols - 1), 0)];
       });
     }
   }
@@ -399,6 +416,19 @@ void mmt4d_thin_kernel(Args a) {
       for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) chains[c][tm][tn] = TT::mfma(&eb[tn], &ea[tm], chains[c][tm][tn]);
+    } else if constexpr (PAIRED) {
+      v4i eb[TN];
+#pragma unroll
+      for (int tn = 0; tn < TN; tn += 2) {
+        const v4i lo = fb[d][tn][0], hi = fb[d][tn + 1][0];
+        eb[tn] = v4i{lo[0], lo[1], hi[0], hi[1]};
+        eb[tn + 1] = v4i{lo[2], lo[3], hi[2], hi[3]};
+      }
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+          chains[c][tm][tn] = TT::mfma(&eb[tn], &fa[d][tm][0], chains[c][tm][tn]);
     } else if constexpr (E == Elem::kF32) {
       // A word of all blocks before the next one: products of one block wait for each other.
 #pragma unroll
@@ -476,9 +506,18 @@ void mmt4d_thin_kernel(Args a) {
   Acc sum[OWN];
   for_each_own([&](int i, int tm, int tn) {
     const int b = tm * TN + tn;
-    sum[i] = __builtin_bit_cast(Acc, partial[0][b][lane]);
+    auto part = [&](int w) {
+      if constexpr (PAIRED) {
+        const v2i even = reinterpret_cast<const v2i*>(&partial[w][b & ~1][lane])[b & 1];
+        const v2i odd = reinterpret_cast<const v2i*>(&partial[w][b | 1][lane])[b & 1];
+        return __builtin_bit_cast(Acc, v4i{even[0], odd[0], even[1], odd[1]});
+      } else {
+        return __builtin_bit_cast(Acc, partial[w][b][lane]);
+      }
+    };
+    sum[i] = part(0);
 #pragma unroll
-    for (int w = 1; w < KSPLIT; ++w) sum[i] += __builtin_bit_cast(Acc, partial[w][b][lane]);
+    for (int w = 1; w < KSPLIT; ++w) sum[i] += part(w);
     // (4-bit RHS: every slice holds 16 times its part of the sum, so the shift is
     // exact per slice.)
     if constexpr (S4) sum[i] = sum[i] >> 4;
