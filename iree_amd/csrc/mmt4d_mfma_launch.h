@@ -451,11 +451,18 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   a.band = (uint32_t)std::min<int64_t>(uk::ceil_div(std::max(grid_m, grid_n), (int64_t)8), 8);
   set_divisors(a);
   const dim3 grid((uint32_t)(grid_m * grid_n * kslices)), block(KSPLIT * 64);
-  // 8-byte rows in twos (PAIRED): 32 x 14336 x 4096, four layers, f16 134 -> 120 us, s8 78 ->
-  // 74, and at 16 rows 115 -> 108 and 68.5 -> 65.8; in 64x64 blocks f16 2000 x 300 x 4099
-  // 19.4 -> 16.8, s8 512 x 2048 x 2048 8.8 -> 8.1, in 32x64 f16 96 x 4096 x 4096 15.0 -> 12.5.
-  // A column tile of an odd number of rows would split such a two.
-  constexpr bool kPairs = RBC == 8 && TN % 2 == 0;
+  // Rows in twos (PAIRED). 8-byte rows, one a load / RHS in twos / both: four layers of 33 x
+  // 14336 x 4096 s8 94.4 / 87.5 / 83.1 us, 16 rows 68.5 / 65.5; f16 32 rows 134 / 120; in 64x64
+  // blocks s8 300 x 4096 x 2000 12.7 / 11.1 / 10.1, 2000 x 300 x 4099 12.6 / 11.1 / 10.6, f16 19.3
+  // / 16.7, 96 x 4096 x 4096 in 32x64 15.0 / 12.5. 4-byte rows of f32, whose products take a
+  // word at a time: 128 x 2048 x 4096 24.0 / 20.0, 96 x 4096 x 4096 38.7 / 33.7, 2000 x
+  // 300 x 4099 53.8 / 50.0, 1000 x 1501 x 777 26.4 / 26.0, six blocks a unit, but 1500 x 1500 x
+  // 1500, nine, 68.5 / 73. Other
+  // types put them together with moves that cost more than the loads: bf16 16x16x2 1000 x
+  // 1501 x 777 11.5 / 14.0, s8 16x16x4 96 x 4096 x 4096 9.5 / 10.7. A tile of an odd number of
+  // rows would split such a two.
+  constexpr bool kPairs = TN % 2 == 0 && (RBC == 8 || (RBC == 4 && E == Elem::kF32 && KSPLIT > 2));
+  const bool pairs = kPairs && (RBC == 8 || grid_m * grid_n <= 6 * (int64_t)compute_units()) && p.N0 % 2 == 0 && (TM % 2 != 0 || p.M0 % 2 == 0);
   if constexpr (TAIL_OK) {
     // No non-temporal instances: weights that the caller has declared streamed are read
     // by several row blocks here, which then wait for HBM one after the other (64x64
@@ -467,7 +474,7 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
       else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, CH, P>, grid, block, 0, stream, a);
       return (int)hipGetLastError();
     };
-    if (kPairs && p.N0 % 2 == 0) return go(std::bool_constant<kPairs>{});
+    if (pairs) return go(std::bool_constant<kPairs>{});
     return go(std::false_type{});
   } else {
     // Weights that the caller has declared streamed, when they are too large for
@@ -479,7 +486,7 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
       else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, 0, P>, grid, block, 0, stream, a);
       return (int)hipGetLastError();
     };
-    if (kPairs && p.N0 % 2 == 0) return go(std::bool_constant<kPairs>{});
+    if (pairs) return go(std::bool_constant<kPairs>{});
     return go(std::false_type{});
   }
 }
@@ -767,7 +774,11 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
 // 700 x 900 x 1504 11.1 / 8.7, 1500 x 1500 x 1504 18.1 / 14.3, but 1000 x 1501 x 777 9.0 /
 // 9.2; f8 900 x 1100 x 1300 8.8 / 7.1; bf16 16x16x2 1000 x 1500 x 784 17.3 / 11.1; s8 16x16x2
 // 2000 x 700 x 2000 17.4 / 13.3. Geometric means over 400 drawn products of 65 to 4096 rows:
-// f16 1.14, s8 1.15, 8-byte rows 1.09, 2-byte rows 1.16, f8 1.10, bf16 4-byte rows 1.13.
+// f16 1.14, s8 1.15, 8-byte rows 1.09, 2-byte rows 1.16, f8 1.10, bf16 4-byte rows 1.13. The
+// barrier-free kinds of 8-byte rows have had their costs by K lowered by what loading rows
+// in twos gave, and serve K from 512 bytes on, where 64x64 blocks through LDS were chosen
+// (s8 957 x 2717 x 634 17.3 / 10.5 us, 502 x 2097 x 658 11.6 / 6.5, 622 x 237 x 973 7.2 / 4.6):
+// 1.12 over 70 products, 3402 x 147 x 2069 in f16 0.95 and s8 2010 x 277 x 2943 0.93 the slowest.
 enum BlockKind { k32x32, k32x64, k64x64Split, k64x64, k64x64Lds, k128x128, kBlockKinds };
 template <Elem E, int RBC>
 inline const BlockCost* block_costs() {
@@ -778,8 +789,8 @@ inline const BlockCost* block_costs() {
   static constexpr BlockCost rows16[kBlockKinds] = {{3.12, 0.20, 0.20, 0.59, 0}, {3.10, 0.49, 0.28, 0.92, 0},
                                                     {3.07, 1.15, 0.37, 1.26, 0}, {3.34, 0.55, 1.41, 1.40, 0},
                                                     {no, 0, 0, 0, 0},            {3.48, 1.74, 1.35, 2.74, 0}};
-  static constexpr BlockCost rows8[kBlockKinds] = {{3.08, 0.23, 0.05, 0.92, 1}, {3.09, 0.54, 0.36, 1.31, 0},
-                                                   {3.12, 1.19, 0.59, 1.71, 0}, {no, 0, 0, 0, 0},
+  static constexpr BlockCost rows8[kBlockKinds] = {{3.08, 0.23, 0.04, 0.71, 1}, {3.09, 0.54, 0.29, 1.06, 0},
+                                                   {3.12, 1.19, 0.48, 1.40, 0}, {no, 0, 0, 0, 0},
                                                    {1.16, 3.88, 0.39, 1.91, 0}, {3.04, 2.33, 3.08, 1.87, 0}};
   static constexpr BlockCost rows4[kBlockKinds] = {{3.18, 0.22, 0.03, 0.89, 1}, {3.21, 0.52, 0.04, 1.35, 1},
                                                    {3.28, 1.22, 0, 1.83, 1},    {no, 0, 0, 0, 0},
@@ -1262,9 +1273,9 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
   } else {
     // (Costs as fitted: up to 330 128x128 blocks; with 24 KB of K and more 64x64 blocks have
     // it in workgroups, too. Calls that direct_before_ksplit keeps in the kernels that stage
-    // through LDS stay there, and rows under 16 bytes with less than 1 KB of K.)
+    // through LDS stay there, and rows under 16 bytes with less than 1 KB of K, 8-byte ones 512 bytes.)
     const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
-    const bool by_cost = !long_k && (RBC >= 16 || k_bytes >= 1024) &&
+    const bool by_cost = !long_k && (RBC >= 16 || k_bytes >= (RBC == 8 ? 512 : 1024)) &&
                          ((choice == 2 && workgroups(p, 128, 128) <= 330) || choice == 3 ||
                           (choice == 6 && !direct_before_ksplit<E, RBC>(p)) || (RBC == 2 && choice == 4));
     if (forced == 0 && by_cost) {

@@ -116,12 +116,13 @@ __device__ __forceinline__ void block_in_bands(uint32_t wg, const Args& a, int* 
 // (iree_uk_amd_set_streamed_weights): a layer's weights then pass through the
 // caches without displacing what is used again.
 // CH: chains of a wave's sums (0: thin_chains).
-// PAIRED: RHS rows of 8 bytes in twos. A lane loads two neighbouring rows of a K-tile as
-// 16 bytes, half as many loads for the same bytes, and what it gets belongs to the same lane
-// of two column blocks: the one then holds the even and the other the odd columns of 32,
-// which the waves that add up and store put back in order. Sums are the same bit for bit.
-// N0 is even. (These blocks are bound by how many loads a unit's L1 and the waves' loops
-// take, the thin ones beside by HBM: launch_thin has the figures.)
+// PAIRED: rows of 8 and 4 bytes in twos, those of the RHS and, with an even number of row
+// blocks, of the LHS. A lane loads two neighbouring rows of a K-tile at once, half as many
+// loads for the same bytes, and what it gets belongs to the same lane of two blocks: the one
+// then holds the even and the other the odd rows or columns of 32. Rows are stored where
+// they belong; columns are put back in order by the waves that add up and store. Sums are
+// the same bit for bit. N0 (M0) is even. (These blocks are bound by how many loads a unit's
+// L1 and the waves' loops take, the thin ones beside by HBM: launch_thin has the figures.)
 template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false, bool TAIL = false, int CH = 0,
           bool PAIRED = false>
 __global__ __launch_bounds__(KSPLIT * 64, PAIRED && TM * TN >= 16 ? 2 : 1)   // (else two registers too many for two)
@@ -137,7 +138,8 @@ void mmt4d_thin_kernel(Args a) {
   constexpr bool S4 = E == Elem::kS8S4;       // 4-bit RHS: half the bytes per row
   constexpr int CHAINS = CH > 0 ? CH : thin_chains<E, TM, KSPLIT>();
   static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
-  static_assert(!PAIRED || (RBC == 8 && TN % 2 == 0 && HALVES == 1), "two rows in 16 bytes, columns of two blocks");
+  static_assert(!PAIRED || ((RBC == 8 || RBC == 4) && TN % 2 == 0 && HALVES == 1), "two rows a load, columns of two blocks");
+  constexpr bool PAIRED_A = PAIRED && TM % 2 == 0;
   static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
 
   // The blocks that a wave adds up and stores: OWN, or for the last ones fewer.
@@ -201,7 +203,8 @@ void mmt4d_thin_kernel(Args a) {
   uint32_t offa[TM][HALVES], offb[TN][HALVES];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
-    operand_offsets(offa[tm], (uint32_t)(bm * TM + tm) * 16 + r, a.M0, a.by_m0, a.M1, a.out_rows, pa0, a.lhs_stride, kt_m, lrb, 16);
+    operand_offsets(offa[tm], (uint32_t)(bm * TM + (PAIRED_A ? tm & ~1 : tm)) * 16 + (PAIRED_A ? 2 * r : r), a.M0, a.by_m0,
+                    a.M1, a.out_rows, pa0, a.lhs_stride, kt_m, lrb, 16);
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn)
     operand_offsets(offb[tn], (uint32_t)(bn * TN + (PAIRED ? tn & ~1 : tn)) * 16 + (PAIRED ? 2 * r : r), a.N0, a.by_n0,
@@ -237,6 +240,31 @@ void mmt4d_thin_kernel(Args a) {
       return v;
     }
   };
+  // PAIRED: half of the pieces of two blocks' lane operands, the first half for the even one.
+  auto load_pair = [&](auto nontemporal, auto ends, __amdgpu_buffer_rsrc_t from, uint32_t off, uint32_t adv,
+                       uint32_t kt_bytes, uint32_t s, int h, int odd) {
+    constexpr int HALF = RBC == 8 ? 1 : 2;
+    auto at = [&](int t) { return !decltype(ends)::value || in_k(s, h, t) ? off : kBeyond; };
+    constexpr bool NT = decltype(nontemporal)::value;
+    const uint32_t piece = NCH * kt_bytes, first = adv + odd * HALF * piece;
+    const int t0 = odd * HALF;
+    if constexpr (RBC == 8) {
+      return load16<NT>(from, at(t0), first);
+    } else {
+      const v2i lo = load8<NT>(from, at(t0), first), hi = load8<NT>(from, at(t0 + 1), first + piece);
+      return v4i{lo[0], lo[1], hi[0], hi[1]};
+    }
+  };
+  // The lane operands of the two blocks from what was loaded so.
+  auto unpair = [&](const v4i& lo, const v4i& hi, v4i& even, v4i& odd) {
+    if constexpr (RBC == 8) {
+      even = v4i{lo[0], lo[1], hi[0], hi[1]};
+      odd = v4i{lo[2], lo[3], hi[2], hi[3]};
+    } else {
+      even = v4i{lo[0], lo[2], hi[0], hi[2]};
+      odd = v4i{lo[1], lo[3], hi[1], hi[3]};
+    }
+  };
   // Rows of 2 bytes: a register for each piece until the step is computed (put together
   // as they come, they would be waited for as they are asked for).
   using AFrag = typename std::conditional<RBC == 2, v8i, v4i>::type;
@@ -262,10 +290,7 @@ void mmt4d_thin_kernel(Args a) {
         if constexpr (S4) {
           fb[d][tn][h] = load8<STREAMED>(from_b, offb[tn][h], at_b);
         } else if constexpr (PAIRED) {
-          // K-tiles g (even tn) and g + NCH of both columns.
-          const uint32_t off =
-              !decltype(ends)::value || in_k(s, h, tn % 2) ? offb[tn][h] : kBeyond;
-          fb[d][tn][h] = load16<STREAMED>(from_b, off, at_b + (tn % 2) * NCH * kt_n);
+          fb[d][tn][h] = load_pair(std::bool_constant<STREAMED>{}, ends, from_b, offb[tn][h], at_b, kt_n, s, h, tn % 2);
         } else {
           fb[d][tn][h] = load_operand(std::bool_constant<STREAMED>{}, ends, from_b, offb[tn][h], at_b, kt_n, s, h);
         }
@@ -273,8 +298,10 @@ void mmt4d_thin_kernel(Args a) {
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-      for (int h = 0; h < HALVES; ++h)
-        fa[d][tm][h] = load_operand(std::false_type{}, ends, from_a, offa[tm][h], at_a, kt_m, s, h);
+      for (int h = 0; h < HALVES; ++h) {
+        if constexpr (PAIRED_A) fa[d][tm][h] = load_pair(std::false_type{}, ends, from_a, offa[tm][h], at_a, kt_m, s, h, tm % 2);
+        else fa[d][tm][h] = load_operand(std::false_type{}, ends, from_a, offa[tm][h], at_a, kt_m, s, h);
+      }
   };
   // Local step i. (Its number is kept from the compiler, which would hold the offsets of all
   // steps of an unrolled round in scalar registers of their own, and spill them, or in
@@ -286,11 +313,15 @@ void mmt4d_thin_kernel(Args a) {
   };
 
   // ---- output addressing (see for_each_output in mmt4d_mfma_kernel.h) ------
-  // Lane (q, r) of block b = tm * TN + tn holds output row r, columns 4q..4q+3.
+  // Lane (q, r) of block b = tm * TN + tn holds output row r, columns 4q..4q+3 (PAIRED_A: row
+  // 2r or 2r + 1 of two blocks' 32).
   // f4(i, p) / f1(i, e, p) for the i-th of this wave's blocks.
   // PAIRED: of two neighbouring own blocks the first holds columns 8q..8q+3 of their 32,
   // the second 8q+4..8q+7.
   const int first_own = wave * OWN;
+  auto row_of = [&](int tm) {
+    return PAIRED_A ? (bm * TM + (tm & ~1)) * 16 + 2 * (int)r + (tm & 1) : (bm * TM + tm) * 16 + (int)r;
+  };
   auto first_col = [&](int tn) {
     return PAIRED ? (bn * TN + (tn & ~1)) * 16 + 8 * (int)q + 4 * (tn & 1) : (bn * TN + tn) * 16 + 4 * (int)q;
   };
@@ -302,7 +333,7 @@ void mmt4d_thin_kernel(Args a) {
   auto for_each_output = [&](const char* base, int64_t s_panel, uint32_t s_m0, uint32_t s_pn,
                              uint32_t s_n0, auto f4, auto f1) {
     for_each_own([&](int i, int tm, int tn) {
-      const int row = (bm * TM + tm) * 16 + (int)r;
+      const int row = row_of(tm);
       const int pl = (int)a.by_m0.quotient(row), m0 = row - pl * a.M0;
       const bool row_ok = pl < a.M1 && row < a.out_rows;
       char* row_base = const_cast<char*>(base) + (int64_t)pl * s_panel + (int64_t)m0 * s_m0;
@@ -366,7 +397,7 @@ void mmt4d_thin_kernel(Args a) {
   if (OB == 4 && a.dequant) {
     if (a.row_scale) {
       for_each_own([&](int i, int tm, int) {
-        sm[i] = a.row_scale[max(min((bm * TM + tm) * 16 + (int)r, a.out_rows - 1), 0)];
+        sm[i] = a.row_scale[max(min(row_of(tm), a.out_rows - 1), 0)];
       });
     }
     if (a.col_scale) {
@@ -400,46 +431,45 @@ void mmt4d_thin_kernel(Args a) {
       for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = TT::mfma(&eb[tn], &ea[tm], acc[tm][tn]);
-    } else if constexpr (RBC == 2) {
-      auto whole = [](const v8i& v) {
-        return v4i{(int)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x05040100u),
-                   (int)__builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x05040100u),
-                   (int)__builtin_amdgcn_perm((uint32_t)v[5], (uint32_t)v[4], 0x05040100u),
-                   (int)__builtin_amdgcn_perm((uint32_t)v[7], (uint32_t)v[6], 0x05040100u)};
+    } else if constexpr (RBC == 2 || PAIRED || E == Elem::kF32) {
+      auto whole = [](const auto& v) {
+        if constexpr (sizeof(v) == sizeof(v8i)) {
+          return v4i{(int)__builtin_amdgcn_perm((uint32_t)v[1], (uint32_t)v[0], 0x05040100u),
+                     (int)__builtin_amdgcn_perm((uint32_t)v[3], (uint32_t)v[2], 0x05040100u),
+                     (int)__builtin_amdgcn_perm((uint32_t)v[5], (uint32_t)v[4], 0x05040100u),
+                     (int)__builtin_amdgcn_perm((uint32_t)v[7], (uint32_t)v[6], 0x05040100u)};
+        } else {
+          return v;
+        }
       };
       v4i ea[TM], eb[TN];
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) ea[tm] = whole(fa[d][tm][0]);
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) eb[tn] = whole(fb[d][tn][0]);
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) chains[c][tm][tn] = TT::mfma(&eb[tn], &ea[tm], chains[c][tm][tn]);
-    } else if constexpr (PAIRED) {
-      v4i eb[TN];
-#pragma unroll
-      for (int tn = 0; tn < TN; tn += 2) {
-        const v4i lo = fb[d][tn][0], hi = fb[d][tn + 1][0];
-        eb[tn] = v4i{lo[0], lo[1], hi[0], hi[1]};
-        eb[tn + 1] = v4i{lo[2], lo[3], hi[2], hi[3]};
+      for (int tm = 0; tm < TM; ++tm) {
+        if constexpr (!PAIRED_A) ea[tm] = whole(fa[d][tm][0]);
+        else if (tm % 2 == 0) unpair(fa[d][tm][0], fa[d][tm + 1][0], ea[tm], ea[tm + 1]);
       }
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
+      for (int tn = 0; tn < TN; ++tn) {
+        if constexpr (!PAIRED) eb[tn] = whole(fb[d][tn][0]);
+        else if (tn % 2 == 0) unpair(fb[d][tn][0], fb[d][tn + 1][0], eb[tn], eb[tn + 1]);
+      }
+      if constexpr (E == Elem::kF32) {
+        // A word of all blocks before the next one: products of one block wait for each other.
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-          chains[c][tm][tn] = TT::mfma(&eb[tn], &fa[d][tm][0], chains[c][tm][tn]);
-    } else if constexpr (E == Elem::kF32) {
-      // A word of all blocks before the next one: products of one block wait for each other.
+        for (int w = 0; w < 4; ++w)
 #pragma unroll
-      for (int w = 0; w < 4; ++w)
+          for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+            for (int tn = 0; tn < TN; ++tn)
+              chains[c][tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(v4f, eb[tn])[w],
+                                                                       __builtin_bit_cast(v4f, ea[tm])[w],
+                                                                       chains[c][tm][tn], 0, 0, 0);
+      } else {
 #pragma unroll
         for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-          for (int tn = 0; tn < TN; ++tn)
-            chains[c][tm][tn] = __builtin_amdgcn_mfma_f32_16x16x4f32(__builtin_bit_cast(v4f, fb[d][tn][0])[w],
-                                                                     __builtin_bit_cast(v4f, fa[d][tm][0])[w],
-                                                                     chains[c][tm][tn], 0, 0, 0);
+          for (int tn = 0; tn < TN; ++tn) chains[c][tm][tn] = TT::mfma(&eb[tn], &ea[tm], chains[c][tm][tn]);
+      }
     } else {
 #pragma unroll
       for (int tm = 0; tm < TM; ++tm)

@@ -32,7 +32,7 @@ def _tiles(torch, x, m0, k0):
     (BF16, (16, 16, 2), 1000, 1500, 783, "32x64_ksplit"),
     (BF16, (16, 16, 2), 530, 2048, 2047, "64x64_ksplit"),
     (BF16, (16, 32, 4), 1011, 777, 1281, "64x64_ksplit"),
-    (S8, (16, 16, 8), 530, 1080, 2047, "64x64_ksplit"),
+    (S8, (16, 16, 8), 530, 1080, 2047, "32x32_ksplit"),
     (S8, (16, 16, 8), 2000, 300, 4099, "64x64_ksplit"),
     (S8, (32, 16, 16), 600, 800, 3001, "32x64_ksplit"),
     (S8, (16, 16, 2), 700, 1000, 1111, "64x64_lds_direct"),

@@ -1,5 +1,5 @@
-"""8-byte rows of the right-hand side loaded in twos: the blocks of two column blocks and more
-that do so, thin and between thin and large, with column tiles of an even number of rows, and of
+"""8-byte rows, and 4-byte rows of f32, loaded in twos: the blocks of two column blocks and more
+that do so, thin and between thin and large, with tiles of an even number of rows, and of
 an odd one, which keep a load a row; results that end at an odd column, inside a tile and inside
 a two; rows and columns swapped; K split over workgroups; K in whole steps and not. Small
 integers, so that every order of the sums gives the product in 64 bits."""
@@ -13,6 +13,7 @@ S8 = (uk.MMT4D_TYPE_S8S8S32, "int8", "int32", 8)
 F16 = (uk.MMT4D_TYPE_F16F16F32, "float16", "float32", 4)
 BF16BF16 = (uk.MMT4D_TYPE_BF16BF16BF16 | uk.MMT4D_SKIP_INTERMEDIATE_ROUNDINGS, "bfloat16", "bfloat16", 4)
 F32 = (uk.MMT4D_TYPE_F32F32F32, "float32", "float32", 2)
+F32_4 = (uk.MMT4D_TYPE_F32F32F32, "float32", "float32", 1)
 
 
 def _tiles(torch, x, m0, k0):
@@ -21,13 +22,13 @@ def _tiles(torch, x, m0, k0):
             .permute(0, 2, 1, 3).contiguous())
 
 
-@pytest.mark.parametrize("kind", [S8, F16, BF16BF16, F32], ids=["s8", "f16", "bf16bf16", "f32"])
+@pytest.mark.parametrize("kind", [S8, F16, BF16BF16, F32, F32_4], ids=["s8", "f16", "bf16bf16", "f32", "f32k1"])
 @pytest.mark.parametrize("m0,n0,m,n,k", [
     (16, 16, 1, 9001, 512), (32, 16, 16, 8211, 1024), (32, 16, 33, 8195, 512), (16, 2, 20, 8205, 256),
     (16, 6, 64, 8193, 512), (16, 7, 16, 8301, 512), (16, 32, 5, 12289, 576), (16, 16, 9001, 17, 512),
     (6, 16, 8201, 33, 512), (16, 16, 64, 200, 8192), (16, 16, 300, 4096, 1000), (16, 16, 513, 2041, 1023),
     (16, 7, 513, 2041, 1023), (48, 48, 96, 4097, 2048), (16, 16, 128, 2049, 2047), (5, 10, 700, 901, 1504),
-    (16, 16, 256, 256, 16384)])
+    (16, 16, 256, 256, 16384), (7, 16, 128, 2049, 2047), (7, 16, 33, 8195, 512)])
 def test_row_pairs(gpu, kind, m0, n0, m, n, k):
     lib, torch = gpu
     flags, tin, tout, k0 = kind
