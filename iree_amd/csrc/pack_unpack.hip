@@ -1414,8 +1414,7 @@ __global__ __launch_bounds__(kThreads) void unpack_direct_kernel(DirectArgs a) {
 }
 
 // Launches the direct unpack for a call that the streaming kernels would take (`plan`)
-// and that is of its form; false otherwise. Such a call goes by the streaming kernels'
-// name, too.
+// and that is of its form; false otherwise.
 bool launch_unpack_direct(const iree_uk_unpack_params_t* p, const TiledPlan& plan, const TiledView& v, int es,
                           const char* src, char* dst, bool transpose_inner, hipStream_t stream) {
   if (transpose_inner || plan.VEC != 16 || plan.G < 8) return false;
@@ -1575,9 +1574,12 @@ extern "C" int iree_uk_amd_hip_launch_unpack(const iree_uk_unpack_params_t* p_in
       plan.args.src = src;
       plan.args.dst = dst;
       plan.args.pad32 = 0;
-      if (plan.stream && ((kernel_mode == IREE_UK_AMD_KERNEL_MODE_AUTO &&
-                           launch_unpack_direct(p, plan, v, es, src, dst, ti, stream)) ||
-                          launch_stream<true>(plan, stream))) {
+      if (plan.stream && kernel_mode == IREE_UK_AMD_KERNEL_MODE_AUTO &&
+          launch_unpack_direct(p, plan, v, es, src, dst, ti, stream)) {
+        *kernel_name = "unpack_direct";
+        return (int)hipGetLastError();
+      }
+      if (plan.stream && launch_stream<true>(plan, stream)) {
         *kernel_name = "unpack_stream";
         return (int)hipGetLastError();
       }

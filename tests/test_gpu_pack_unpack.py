@@ -109,7 +109,8 @@ def test_pack_block_spanning_shapes(gpu, oracle, mode):
         assert tiled == 0
 
 
-@pytest.mark.parametrize("mode", MODES)
+# (MFMA_VARIANT + 1 keeps unpack on the LDS-staged kernels.)
+@pytest.mark.parametrize("mode", MODES + [uk.KERNEL_MODE_MFMA_VARIANT + 1])
 def test_unpack_block_spanning_shapes(gpu, oracle, mode):
     lib, torch = gpu
     lib.set_kernel_mode(mode)
@@ -126,8 +127,8 @@ def test_unpack_block_spanning_shapes(gpu, oracle, mode):
         G.run_unpack_case(oracle, c, inp, want)
         got = T.gpu_unpack(lib, torch, c, inp, out0)
         assert np.array_equal(got, want), (c.label(), lib.last_kernel_name())
-        tiled += lib.last_kernel_name() in ("unpack_tiled", "unpack_stream")
-    if mode == uk.KERNEL_MODE_AUTO:
+        tiled += lib.last_kernel_name() in ("unpack_tiled", "unpack_stream", "unpack_direct")
+    if mode != uk.KERNEL_MODE_GENERIC:
         assert tiled >= 40, tiled
 
 
@@ -405,8 +406,8 @@ def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
         assert np.array_equal(got, want), c.label()
         want_kernel = "pack_tiled" if narrow or cols * es < 16 else "pack_stream"
         assert lib.last_kernel_name() == want_kernel, (c.label(), lib.last_kernel_name())
-        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
         if es == 1:
+            lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
             continue
         u = T.UnpackCase(tf | flags, so0, so1, s2, s3, rows, cols, so1 * s2 * s3, pitch, 1, 0, 0)
         inp, out0 = T.make_unpack_buffers(u, rng)
@@ -416,6 +417,9 @@ def test_narrow_matrices_take_the_tiled_kernels(gpu, oracle, tf, t0, t1, flags):
         assert np.array_equal(got, want), u.label()
         want_kernel = "unpack_tiled" if narrow else "unpack_stream"
         assert lib.last_kernel_name() == want_kernel, (u.label(), lib.last_kernel_name())
+        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+        got = T.gpu_unpack(lib, torch, u, inp, out0)
+        assert np.array_equal(got, want), (u.label(), lib.last_kernel_name())
 
 
 @pytest.mark.parametrize("tf,s2,s3,flags", [
@@ -577,7 +581,7 @@ def test_pack_unpack_round_trip_and_numpy_identity(gpu):
         d_y = torch.full((x.size * x.itemsize,), 0x5A, dtype=torch.uint8, device="cuda")
         lib.unpack(d_p.data_ptr(), 0, o1 * o2 * o3, o2 * o3, d_y.data_ptr(), 0,
                    shape[1], 1, o0, o1, o2, o3, shape[0], shape[1], flags)
-        assert lib.last_kernel_name() in ("unpack_stream", "unpack_tiled")
+        assert lib.last_kernel_name() in ("unpack_stream", "unpack_tiled", "unpack_direct")
         assert np.array_equal(d_y.cpu().numpy().view(dtype).reshape(shape), x)
 
 

@@ -122,16 +122,23 @@ def test_pack_random_sweep_element_transpositions(gpu, oracle):
 def test_unpack_random_sweep(gpu, oracle):
     lib, torch = gpu
     rng = np.random.default_rng(2025)
-    kernels = set()
-    for ci in range(160):
-        c = _unpack_case(rng, UNPACK_TYPES[ci % len(UNPACK_TYPES)])
-        inp, out = T.make_unpack_buffers(c, np.random.default_rng(ci))
-        want = out.copy()
-        G.run_unpack_case(oracle, c, inp, want)
-        got = T.gpu_unpack(lib, torch, c, inp, out)
-        assert np.array_equal(got, want), (ci, c, lib.last_kernel_name())
-        kernels.add(lib.last_kernel_name())
-    assert {"unpack_stream", "unpack_generic"} <= kernels, kernels
+    staged = uk.KERNEL_MODE_MFMA_VARIANT + 1   # (past the kernel that moves pieces through registers)
+    kernels = {uk.KERNEL_MODE_AUTO: set(), staged: set()}
+    try:
+        for ci in range(160):
+            c = _unpack_case(rng, UNPACK_TYPES[ci % len(UNPACK_TYPES)])
+            inp, out = T.make_unpack_buffers(c, np.random.default_rng(ci))
+            want = out.copy()
+            G.run_unpack_case(oracle, c, inp, want)
+            for mode, names in kernels.items():
+                lib.set_kernel_mode(mode)
+                got = T.gpu_unpack(lib, torch, c, inp, out)
+                assert np.array_equal(got, want), (ci, c, lib.last_kernel_name())
+                names.add(lib.last_kernel_name())
+    finally:
+        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    assert {"unpack_direct", "unpack_stream", "unpack_generic"} <= kernels[uk.KERNEL_MODE_AUTO], kernels
+    assert {"unpack_stream", "unpack_generic"} <= kernels[staged] and "unpack_direct" not in kernels[staged], kernels
 
 
 MMT4D_TYPES = [uk.MMT4D_TYPE_S8S8S32, uk.MMT4D_TYPE_F16F16F32, uk.MMT4D_TYPE_BF16BF16F32,

@@ -34,9 +34,11 @@ def test_unpack_direct(gpu, oracle, tf, t0, t1, flags):
         G.run_unpack_case(oracle, c, inp, want)
         got = T.gpu_unpack(lib, torch, c, inp, out0)
         assert np.array_equal(got, want), (c.label(), lib.last_kernel_name())
+        assert lib.last_kernel_name() == "unpack_direct", c.label()
         lib.set_kernel_mode(uk.KERNEL_MODE_MFMA_VARIANT + 1)   # the LDS-staged kernels on the same call
         try:
             staged = T.gpu_unpack(lib, torch, c, inp, out0)
         finally:
             lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
         assert np.array_equal(staged, want), (c.label(), "staged")
+        assert lib.last_kernel_name() == "unpack_stream", c.label()
