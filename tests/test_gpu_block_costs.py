@@ -49,8 +49,6 @@ def _tiles(torch, x, m0, k0):
     (F32, (48, 16, 4), 1030, 1050, 1301, "32x48_ksplit")])
 def test_blocks_by_cost(gpu, kind, tile, m, n, k, name):
     lib, torch = gpu
-    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
-        pytest.skip("the costs are of 256 compute units")
     flags, tin, tout = kind
     (m0, n0, k0), tin, tout = tile, getattr(torch, tin), getattr(torch, tout)
     gen = torch.Generator(device="cuda"); gen.manual_seed(m + n)
@@ -71,4 +69,6 @@ def test_blocks_by_cost(gpu, kind, tile, m, n, k, name):
     assert torch.equal(mat[:m], want.to(tout)) and bool((mat[m] == 7).all())
     want = torch.nn.functional.pad(want, (0, n1 * n0 - n, 0, m1 * m0 - m)).view(m1, m0, n1, n0).permute(0, 2, 1, 3)
     assert torch.equal(out, (want + acc.float()).to(tout))
-    assert tiled_name == lib.last_kernel_name() == "mmt4d_mfma_" + name
+    assert tiled_name == lib.last_kernel_name()
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:   # (which the costs are of)
+        assert tiled_name == "mmt4d_mfma_" + name

@@ -65,3 +65,26 @@ def test_row_pairs(gpu, kind, m0, n0, m, n, k):
         got, exact = scaled[:m].double(), sums.double() * row.double()[:, None] * col.double()
         # Two roundings to 24 bits.
         assert bool(((got - exact).abs() <= exact.abs() * 2.0 ** -22).all()) and bool((scaled[m] == 7.0).all())
+
+
+@pytest.mark.parametrize("kind", [S8, F16, F32, F32_4], ids=["s8", "f16", "f32", "f32k1"])
+@pytest.mark.parametrize("m,n,k", [(5, 12289, 576), (16, 8211, 1024), (33, 8195, 512), (500, 500, 1000),
+                                   (513, 2041, 1023)])
+def test_row_pairs_at_odd_addresses(gpu, kind, m, n, k):
+    """Rows in twos that begin at an odd byte (8-bit types) or at an odd element."""
+    lib, torch = gpu
+    flags, tin, tout, k0 = kind
+    tin, tout = getattr(torch, tin), getattr(torch, tout)
+    gen = torch.Generator(device="cuda"); gen.manual_seed(m + n)
+    a, b = (torch.randint(-1, 2, (r, k), generator=gen, device="cuda").float() for r in (m, n))
+    lhs, rhs = (_tiles(torch, x, 16, k0).to(tin) for x in (a, b))
+    m1, n1, k1 = lhs.shape[0], rhs.shape[0], lhs.shape[1]
+    d_lhs, d_rhs = (torch.cat([x.new_zeros(3), x.reshape(-1)]) for x in (lhs, rhs))
+    mat = torch.zeros(m, n, device="cuda", dtype=tout)
+    torch.cuda.synchronize()
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    lib.mmt4d_unpack(d_lhs.data_ptr(), 3, k1 * 16 * k0, d_rhs.data_ptr(), 3, k1 * 16 * k0, mat.data_ptr(), 0, n, m, n,
+                     m1, n1, k1, 16, 16, k0, flags)
+    lib.synchronize()
+    assert "thin" in lib.last_kernel_name() or "ksplit" in lib.last_kernel_name(), lib.last_kernel_name()
+    assert torch.equal(mat, (a @ b.T).to(tout)), lib.last_kernel_name()
