@@ -638,6 +638,23 @@ constexpr int steps_ahead() {
   return RBC == 8 ? 3 : 2;
 }
 
+// 16x16 blocks, K over their waves, with two steps in flight, with rows of 2 and 4 bytes four
+// (s8 16x16x2 12 %, bf16 16x16x2 3 % ahead of two in the mean; 8-byte rows 2 % behind). f32,
+// whose products are slower: four, with rows under 16 bytes three (eight 5 to 7 % behind in the
+// mean, up to 17 %), of 4 bytes from 20 KB of K on, which the L2s hold no longer, eight (98 x 270 x
+// 10742 in three 32.5 us, so 25.2, 84 x 484 x 5767 18.8 / 16.1; but 90 x 265 x 3392 10.0 / 10.4).
+template <Elem E, int RBC, int KSPLIT>
+int launch_16x16(const Problem& p, hipStream_t stream) {
+  if constexpr (E == Elem::kF32) {
+    if constexpr (RBC == 4) {
+      if (((int64_t)p.K1 << p.lrb) >= 20480) return launch_thin<E, RBC, 1, 1, KSPLIT, 8, true>(p, false, stream);
+    }
+    return launch_thin<E, RBC, 1, 1, KSPLIT, RBC < 16 ? 3 : 4, true>(p, false, stream);
+  } else {
+    return launch_thin<E, RBC, 1, 1, KSPLIT, RBC < 8 ? 4 : 2, true>(p, false, stream);
+  }
+}
+
 // What `blocks` workgroups of a kernel take, in us, by the KB of K. A unit's blocks are
 // loaded one beside the other, and a last round of few blocks is not a whole one; below
 // `least` blocks a unit a block's own chain of steps is what it takes.
@@ -699,14 +716,14 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
     }
   }
   if (b16 <= cus && k_bytes >= (RBC < 16 ? 64 : 256)) {
-    st = launch_thin<E, RBC, 1, 1, F32 ? 4 : 8, F32 ? (RBC < 16 ? 8 : 4) : 2, true>(p, false, stream);
+    st = launch_16x16<E, RBC, F32 ? 4 : 8>(p, stream);
     if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
     return st;
   }
   if constexpr (F32) {
     if (k_bytes < (b128 || (RBC >= 16 && b32 > 2 * cus) ? 1024 : 256)) return -1;
     if (b16 <= 3 * cus) {
-      st = launch_thin<E, RBC, 1, 1, 4, RBC < 16 ? 8 : 4, true>(p, false, stream);
+      st = launch_16x16<E, RBC, 4>(p, stream);
       if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
       return st;
     }
@@ -818,7 +835,7 @@ int launch_by_cost(const Problem& p, int64_t rows, int64_t cols, bool parts, hip
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb, cus = compute_units();
   if (cus < 1) return -1;   // the device query failed, as the launch will
   if (uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16) <= cus && k_bytes >= (RBC < 16 ? 64 : 256)) {
-    const int st = launch_thin<E, RBC, 1, 1, 8, 2, true>(p, false, stream);
+    const int st = launch_16x16<E, RBC, 8>(p, stream);
     if (st >= 0) { *name = "mmt4d_mfma_16x16_ksplit"; return st; }
   }
   double us[kBlockKinds];

@@ -60,24 +60,28 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 // 15.0 us, 700 x 700 x 3000 41.0 -> 34.6, 1500 x 1500 x 1000 52.6 -> 44.9). What lies kBeyond in a lane is outside the resource:
 // such a load returns zeros and reads nothing. NT: non-temporal.
 constexpr uint32_t kBeyond = 0x80000000u;
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t operand_at(const char* base) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, (int)kBeyond, 0x00027000);
+struct Operand {
+  __amdgpu_buffer_rsrc_t buffer;
+  const char* base;
+};
+__device__ __forceinline__ Operand operand_at(const char* base) {
+  return {__builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base), 0, (int)kBeyond, 0x00027000), base};
 }
 template <bool NT>
-__device__ __forceinline__ v4i load16(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
-  return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(from, lane_bytes, bytes, NT ? 2 : 0));
+__device__ __forceinline__ v4i load16(const Operand& from, uint32_t lane_bytes, uint32_t bytes) {
+  return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(from.buffer, lane_bytes, bytes, NT ? 2 : 0));
 }
 template <bool NT>
-__device__ __forceinline__ v2i load8(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
-  return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(from, lane_bytes, bytes, NT ? 2 : 0));
+__device__ __forceinline__ v2i load8(const Operand& from, uint32_t lane_bytes, uint32_t bytes) {
+  return __builtin_bit_cast(v2i, __builtin_amdgcn_raw_buffer_load_b64(from.buffer, lane_bytes, bytes, NT ? 2 : 0));
 }
 template <bool NT>
-__device__ __forceinline__ int load4(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
-  return (int)__builtin_amdgcn_raw_buffer_load_b32(from, lane_bytes, bytes, NT ? 2 : 0);
+__device__ __forceinline__ int load4(const Operand& from, uint32_t lane_bytes, uint32_t bytes) {
+  return (int)__builtin_amdgcn_raw_buffer_load_b32(from.buffer, lane_bytes, bytes, NT ? 2 : 0);
 }
 template <bool NT>
-__device__ __forceinline__ int load2(__amdgpu_buffer_rsrc_t from, uint32_t lane_bytes, uint32_t bytes) {
-  return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from, lane_bytes, bytes, NT ? 2 : 0);
+__device__ __forceinline__ int load2(const Operand& from, uint32_t lane_bytes, uint32_t bytes) {
+  return (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(from.buffer, lane_bytes, bytes, NT ? 2 : 0);
 }
 
 // Sums of floats whose K eight waves share are in several chains, steps i, i + chains, ..
@@ -138,6 +142,13 @@ void mmt4d_thin_kernel(Args a) {
   constexpr bool S4 = E == Elem::kS8S4;       // 4-bit RHS: half the bytes per row
   constexpr int CHAINS = CH > 0 ? CH : thin_chains<E, TM, KSPLIT>();
   static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
+  // Rows of 2 and 4 bytes in 16x16 blocks, which are bound by how many loads a unit takes, load
+  // from addresses: a unit takes more narrow loads of these than from a buffer resource, and
+  // the vector addition that each costs is hidden here. us from resources / so, four steps
+  // ahead: s8 16x16x2 100 x 128 x 20480 21.0 / 12.6 (14.4 with the addition in scalar
+  // registers), 16x16x4 126 x 408 x 19584 11.9 / 9.9; bf16 16x16x2 100 x 128 x 10240 11.9 / 9.9;
+  // f32 16x16x1 540 x 115 x 7400 30.1 / 25.8. (Rows of 8 bytes: level; sixteen chains: 15 to 22 % behind.)
+  constexpr bool BY_ADDRESS = RBC <= 4 && TM * TN == 1 && CHAINS < 16;
   static_assert(!PAIRED || ((RBC == 8 || RBC == 4) && TN % 2 == 0 && HALVES == 1), "two rows a load, columns of two blocks");
   constexpr bool PAIRED_A = PAIRED && TM % 2 == 0;
   static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
@@ -179,8 +190,8 @@ void mmt4d_thin_kernel(Args a) {
   // result (tile padding), which only reach accumulators that are never stored.
   // Offsets are relative to the first panel the workgroup touches.
   const int pa0 = (int)a.by_m0.quotient(bm * TM * 16), pb0 = (int)a.by_n0.quotient(bn * TN * 16);
-  const __amdgpu_buffer_rsrc_t from_a = operand_at(a.lhs + (int64_t)pa0 * a.lhs_stride);
-  const __amdgpu_buffer_rsrc_t from_b = operand_at(a.rhs + (int64_t)pb0 * a.rhs_stride);
+  const Operand from_a = operand_at(a.lhs + (int64_t)pa0 * a.lhs_stride);
+  const Operand from_b = operand_at(a.rhs + (int64_t)pb0 * a.rhs_stride);
   auto operand_offsets = [&](uint32_t (&off)[HALVES], uint32_t row, int X0, const Divisor& by_x0, int X1, int rows,
                              int p0, int64_t stride, uint32_t kt_bytes, int lrb, uint32_t piece_bytes) {
     const uint32_t pabs = by_x0.quotient(row);
@@ -220,12 +231,26 @@ void mmt4d_thin_kernel(Args a) {
   };
   // One lane operand of step s, `adv` bytes on from step 0. `ends`: K ends inside the
   // step, and what lies beyond it is zero.
-  auto load_operand = [&](auto nontemporal, auto ends, __amdgpu_buffer_rsrc_t from, uint32_t off, uint32_t adv,
+  auto load_operand = [&](auto nontemporal, auto ends, const Operand& from, uint32_t off, uint32_t adv,
                           uint32_t kt_bytes, uint32_t s, int h) {
     auto at = [&](int t) { return !decltype(ends)::value || in_k(s, h, t) ? off : kBeyond; };
     constexpr bool NT = decltype(nontemporal)::value;
     const uint32_t piece = NCH * kt_bytes;   // from one piece to the next
-    if constexpr (RBC >= 16) {
+    if constexpr (BY_ADDRESS && !decltype(ends)::value) {
+      // (Rows outside the problem: the first one's bytes, whose sums are not stored either.)
+      auto address = [&](int t) { return from.base + ((off == kBeyond ? 0u : off + t * piece) + adv); };
+      if constexpr (RBC == 4) {
+        typedef int int_g __attribute__((aligned(1)));
+        auto load = [&](int t) { return *reinterpret_cast<const int_g*>(address(t)); };
+        return v4i{load(0), load(1), load(2), load(3)};
+      } else {
+        typedef uint16_t u16_g __attribute__((aligned(1)));
+        v8i v;
+#pragma unroll
+        for (int t = 0; t < 8; ++t) v[t] = *reinterpret_cast<const u16_g*>(address(t));
+        return v;
+      }
+    } else if constexpr (RBC >= 16) {
       return load16<NT>(from, at(0), adv);
     } else if constexpr (RBC == 8) {
       const v2i lo = load8<NT>(from, at(0), adv), hi = load8<NT>(from, at(1), adv + piece);
@@ -241,7 +266,7 @@ void mmt4d_thin_kernel(Args a) {
     }
   };
   // PAIRED: half of the pieces of two blocks' lane operands, the first half for the even one.
-  auto load_pair = [&](auto nontemporal, auto ends, __amdgpu_buffer_rsrc_t from, uint32_t off, uint32_t adv,
+  auto load_pair = [&](auto nontemporal, auto ends, const Operand& from, uint32_t off, uint32_t adv,
                        uint32_t kt_bytes, uint32_t s, int h, int odd) {
     constexpr int HALF = RBC == 8 ? 1 : 2;
     auto at = [&](int t) { return !decltype(ends)::value || in_k(s, h, t) ? off : kBeyond; };
@@ -308,7 +333,7 @@ void mmt4d_thin_kernel(Args a) {
   // vector registers, and loop over the lanes at every load.)
   auto load_step = [&](int d, int i) {
     uint32_t s = __builtin_amdgcn_readfirstlane(first_step + (uint32_t)(i * KSPLIT));
-    asm volatile("" : "+s"(s));
+    if constexpr (!BY_ADDRESS) asm volatile("" : "+s"(s));
     load_at(d, s * sstep_a, s * sstep_b, s, std::false_type{});
   };
 

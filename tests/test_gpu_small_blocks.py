@@ -108,6 +108,32 @@ def test_infinities_stay_in_their_row(gpu, dtype, k0, m, n):
     assert not torch.isfinite(got[~whole[0]]).any() and not torch.isfinite(got[:, ~whole[1]]).any()
 
 
+@pytest.mark.parametrize("dtype,k0", [("s8", 2), ("s8", 4), ("bf16", 1), ("bf16", 2), ("f16", 4), ("f32", 1), ("f32", 2)])
+def test_16x16_blocks_with_every_number_of_steps(gpu, dtype, k0):
+    """Rows under 16 bytes: every number of steps that four and eight waves can begin and end
+    with, three, four or eight in flight, in whole steps and with one tile more."""
+    lib, torch = gpu
+    lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    flags, tin, tout = TYPES[dtype]
+    tin, tout = getattr(torch, tin), getattr(torch, tout)
+    m, n, step = 100, 130, 64 // tin.itemsize
+    many = [320 + s for s in range(70)] if (dtype, k0) == ("f32", 1) else []   # (20 KB and more)
+    most = (max(many or [100]) + 1) * step + k0
+    gen = torch.Generator(device="cuda"); gen.manual_seed(k0)
+    a, b = (torch.randint(-2, 3, (r, most), generator=gen, device="cuda").float() for r in (m, n))
+    for steps in list(range(1, 100)) + many:
+        k = steps * step + (k0 if steps % 2 else 0)
+        lhs, rhs = (torch.nn.functional.pad(x[:, :k], (0, 0, 0, -x.shape[0] % 16)).view(-1, 16, k // k0, k0)
+                    .permute(0, 2, 1, 3).contiguous().to(tin) for x in (a, b))
+        out = torch.zeros(m, n, device="cuda", dtype=tout)
+        torch.cuda.synchronize()
+        lib.mmt4d_unpack(lhs.data_ptr(), 0, 16 * k, rhs.data_ptr(), 0, 16 * k, out.data_ptr(), 0, n, m, n, lhs.shape[0],
+                         rhs.shape[0], k // k0, 16, 16, k0, flags)
+        lib.synchronize()
+        assert "16x16_ksplit" in lib.last_kernel_name()
+        assert torch.equal(out, (a[:, :k] @ b[:, :k].T).to(tout)), (k, lib.last_kernel_name())
+
+
 @pytest.mark.parametrize("k0", [1, 2, 4])
 @pytest.mark.parametrize("m,n", [(100, 130), (128, 1000)])   # up to one 16x16 block a unit, up to three
 def test_f32_sixteen_chains_with_every_number_of_steps(gpu, k0, m, n):
