@@ -569,6 +569,7 @@ extern "C" int iree_uk_amd_hip_launch_mmt4d_mfma(const iree_uk_mmt4d_params_t* p
   pr.lrb = 0;
   while ((1 << pr.lrb) < pr.rb) ++pr.lrb;
   pr.accumulate = (p->flags & IREE_UK_FLAG_MMT4D_ACCUMULATE) != 0;
+  pr.cus = uk_mfma::compute_units();
   switch (e) {
     case Elem::kS8S4: return uk_mfma::launch_s8s4(pr, stream, kernel_name);
     case Elem::kS16: return uk_mfma::launch_s16(pr, forced_variant, stream, kernel_name);

@@ -43,6 +43,7 @@ struct Problem {
   int32_t M1, N1, K1, M0, N0;
   int32_t rb, lrb;  // bytes per tile row and its log2
   bool accumulate;
+  int32_t cus;      // compute units of the device, 0: the query failed, as the launch will (asked for once a call)
 };
 
 // Whether a shape has an instance for a K that ends inside a step (TAIL of the
@@ -244,7 +245,7 @@ int launch_persistent(const Problem& p, int kt_count, bool force, hipStream_t st
   if (k_bytes % (4 * KS) || k_bytes / KS < 8 || k_bytes / KS >= (1 << 24)) return -1;
   const int64_t grid_m = p.M1 / bpm, grid_n = p.N1 / bpn;
   const int64_t total = grid_m * grid_n;
-  int cus = compute_units() & ~7;  // a multiple of the 8 XCDs keeps blocks on their XCD
+  int cus = p.cus & ~7;  // a multiple of the 8 XCDs keeps blocks on their XCD
   if (persistent_workgroups_override() > 0) cus = persistent_workgroups_override();
   if (cus < 1 || total >= (1ll << 30)) return -1;
   if (!force && total < 2 * (int64_t)cus) return -1;
@@ -421,7 +422,7 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   int64_t kslices = 1;
   if (allow_k_slices) {
     const int64_t blocks = grid_m * grid_n;
-    const int cus = compute_units();
+    const int cus = p.cus;
     if (k_slices_override() > 0) {
       kslices = k_slices_override();
     } else if (cus > 0 && 2 * blocks <= cus) {
@@ -462,7 +463,7 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   // 1501 x 777 11.5 / 14.0, s8 16x16x4 96 x 4096 x 4096 9.5 / 10.7. A tile of an odd number of
   // rows would split such a two.
   constexpr bool kPairs = TN % 2 == 0 && (RBC == 8 || (RBC == 4 && E == Elem::kF32 && KSPLIT > 2));
-  const bool pairs = kPairs && (RBC == 8 || grid_m * grid_n <= 6 * (int64_t)compute_units()) && p.N0 % 2 == 0 && (TM % 2 != 0 || p.M0 % 2 == 0);
+  const bool pairs = kPairs && (RBC == 8 || grid_m * grid_n <= 6 * (int64_t)p.cus) && p.N0 % 2 == 0 && (TM % 2 != 0 || p.M0 % 2 == 0);
   if constexpr (TAIL_OK) {
     // No non-temporal instances: weights that the caller has declared streamed are read
     // by several row blocks here, which then wait for HBM one after the other (64x64
@@ -517,7 +518,7 @@ int launch_thin_rows(const Problem& p, bool swapped, int64_t wide_cols, hipStrea
   const int64_t rows = swapped ? std::min<int64_t>((int64_t)p.N1 * p.N0, p.out_cols)
                                : std::min<int64_t>((int64_t)p.M1 * p.M0, p.out_rows);
   const int64_t row_blocks = std::max<int64_t>(1, uk::ceil_div(rows, (int64_t)(TM * 16)));
-  const int64_t cus = std::max(compute_units(), 1);
+  const int64_t cus = std::max(p.cus, 1);
   const int64_t blocks16 = row_blocks * uk::ceil_div(wide_cols, (int64_t)16);
   const int64_t blocks32 = row_blocks * uk::ceil_div(wide_cols, (int64_t)32);
   constexpr bool kInteger = std::is_same<typename ElemTraits<E>::Acc, v4i>::value;
@@ -545,7 +546,7 @@ int launch_thin_rows(const Problem& p, bool swapped, int64_t wide_cols, hipStrea
 // 64-row block / two of 32: 10.9 / 7.5; s8 64 x 300 x 4 KB in one / four of 16: 8.3 / 4.1).
 template <Elem E, int RBC>
 int launch_thin_any(const Problem& p, bool swapped, int64_t thin_rows, int64_t wide_cols, hipStream_t stream) {
-  const int64_t cus = compute_units(), cols16 = uk::ceil_div(wide_cols, (int64_t)16);
+  const int64_t cus = p.cus, cols16 = uk::ceil_div(wide_cols, (int64_t)16);
   const bool cached = wide_cols * ((int64_t)p.K1 << p.lrb) <= (16ll << 20);
   if (thin_rows <= 16 || (cached && uk::ceil_div(thin_rows, (int64_t)16) * cols16 <= cus))
     return launch_thin_rows<E, RBC, 1>(p, swapped, wide_cols, stream);
@@ -661,8 +662,8 @@ int launch_16x16(const Problem& p, hipStream_t stream) {
 struct BlockCost {
   double launch, round, k, k_block, least;
 };
-inline double block_us(const BlockCost& c, int64_t blocks, double kb) {
-  const double cus = (double)std::max(compute_units(), 1), units = (double)blocks / cus, rounds = std::ceil(units);
+inline double block_us(const BlockCost& c, int64_t cus, int64_t blocks, double kb) {
+  const double units = (double)blocks / (double)cus, rounds = std::ceil(units);
   return c.launch + c.round * rounds + kb * (c.k + c.k_block * std::max(c.least, std::min(rounds, units + 0.6)));
 }
 
@@ -701,8 +702,8 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
   constexpr bool F32 = E == Elem::kF32;
   constexpr int kAhead = steps_ahead<E, RBC>();
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb;
-  const int64_t cus = compute_units();
-  if (cus < 1) return -1;   // the device query failed, as the launch will
+  const int64_t cus = p.cus;
+  if (cus < 1) return -1;
   const int64_t b16 = uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16);
   const int64_t b32 = uk::ceil_div(rows, (int64_t)32) * uk::ceil_div(cols, (int64_t)32);
   int st = -1;
@@ -737,11 +738,11 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
     constexpr bool W = RBC >= 16;
     constexpr double kOther = 1.06;
     double us[4] = {
-        block_us(W ? BlockCost{3.14, 0.41, 0.15, 0.93, 1} : BlockCost{3.04, 0.44, 0.35, 0.98, 1}, b32, kb),
+        block_us(W ? BlockCost{3.14, 0.41, 0.15, 0.93, 1} : BlockCost{3.04, 0.44, 0.35, 0.98, 1}, cus, b32, kb),
         ksplit64 ? 1e30
-                 : block_us(W ? BlockCost{3.19, 0.30, 1.35, 0.89, 0} : BlockCost{3.14, 0.35, 1.52, 0.94, 0}, b32, kb),
-        kOther * block_us(W ? BlockCost{3.33, 0.58, 0.01, 1.42, 1} : BlockCost{3.24, 0.66, 0.35, 1.43, 1}, blocks(32, 48), kb),
-        kOther * block_us(W ? BlockCost{1.96, 2.55, 0, 2.11, 1} : BlockCost{1.96, 2.77, 0, 2.31, 1}, blocks(48, 48), kb)};
+                 : block_us(W ? BlockCost{3.19, 0.30, 1.35, 0.89, 0} : BlockCost{3.14, 0.35, 1.52, 0.94, 0}, cus, b32, kb),
+        kOther * block_us(W ? BlockCost{3.33, 0.58, 0.01, 1.42, 1} : BlockCost{3.24, 0.66, 0.35, 1.43, 1}, cus, blocks(32, 48), kb),
+        kOther * block_us(W ? BlockCost{1.96, 2.55, 0, 2.11, 1} : BlockCost{1.96, 2.77, 0, 2.31, 1}, cus, blocks(48, 48), kb)};
     if (b32x64) us[2] = us[3] = 1e30;   // (64 rows and fewer)
     static const char* const names[4] = {"mmt4d_mfma_32x32_ksplit", "mmt4d_mfma_32x32_ksplit", "mmt4d_mfma_32x48_ksplit",
                                          "mmt4d_mfma_48x48_ksplit"};
@@ -824,7 +825,7 @@ double kind_us(const Problem& p, int64_t rows, int64_t cols, int kind) {
   const int64_t blocks = kind >= k64x64 ? workgroups(p, bm[kind], bn[kind])
                                         : uk::ceil_div(rows, (int64_t)bm[kind]) * uk::ceil_div(cols, (int64_t)bn[kind]);
   if (blocks < 1) return 1e30;
-  return block_us(block_costs<E, RBC>()[kind], blocks, (double)((int64_t)p.K1 << p.lrb) / 1024);
+  return block_us(block_costs<E, RBC>()[kind], p.cus, blocks, (double)((int64_t)p.K1 << p.lrb) / 1024);
 }
 // `parts`: a float's K stays in four parts, as it is in kernels whose waves share it and in
 // the 64x64 blocks in registers.
@@ -832,8 +833,8 @@ template <Elem E, int RBC>
 int launch_by_cost(const Problem& p, int64_t rows, int64_t cols, bool parts, hipStream_t stream, const char** name) {
   static_assert(E != Elem::kF32, "launch_small_blocks");
   constexpr bool kInteger = std::is_same<typename ElemTraits<E>::Acc, v4i>::value;
-  const int64_t k_bytes = (int64_t)p.K1 << p.lrb, cus = compute_units();
-  if (cus < 1) return -1;   // the device query failed, as the launch will
+  const int64_t k_bytes = (int64_t)p.K1 << p.lrb, cus = p.cus;
+  if (cus < 1) return -1;
   if (uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16) <= cus && k_bytes >= (RBC < 16 ? 64 : 256)) {
     const int st = launch_16x16<E, RBC, 8>(p, stream);
     if (st >= 0) { *name = "mmt4d_mfma_16x16_ksplit"; return st; }
@@ -904,7 +905,7 @@ int launch_by_cost(const Problem& p, int64_t rows, int64_t cols, bool parts, hip
 // 8-bit floats, whose matrix instructions round to 1.5e-5, stay at 16 steps and 2 KB).
 template <Elem E, int RBC>
 int slices_that_pay(const Problem& p, int64_t rows, int64_t cols, bool long_k) {
-  const int64_t cus = compute_units();
+  const int64_t cus = p.cus;
   const int64_t k_bytes = (int64_t)p.K1 << p.lrb, b128 = workgroups(p, 128, 128);
   const int64_t b64 = workgroups(p, 64, 64);
   const int64_t b32 = uk::ceil_div(rows, (int64_t)32) * uk::ceil_div(cols, (int64_t)32);
@@ -937,7 +938,7 @@ template <Elem E, int RBC>
 bool direct_before_ksplit(const Problem& p) {
   constexpr bool kInteger = std::is_same<typename ElemTraits<E>::Acc, v4i>::value;
   if (E == Elem::kF32 || !(RBC >= 16 || (RBC == 8 && kInteger))) return false;
-  const int64_t k_bytes = (int64_t)p.K1 << p.lrb, b64 = workgroups(p, 64, 64), cus = compute_units();
+  const int64_t k_bytes = (int64_t)p.K1 << p.lrb, b64 = workgroups(p, 64, 64), cus = p.cus;
   if (k_bytes >= 8192 && k_bytes % (64 * ElemTraits<E>::kHalves) == 0) return false;
   if (ElemTraits<E>::kHalves == 2) return k_bytes < 24576 || 2 * b64 > cus;   // (else in workgroups, too)
   return 8 * b64 > (ElemTraits<E>::Out::kOutBytes == 2 || RBC == 8 ? 6 : 8) * cus;
@@ -1068,7 +1069,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       // the last 4096 columns in 256x128 blocks).
       const int bpm_w = 128 / p.M0, bpn_w = 512 / p.N0;
       if (!split_m && !split_n && bpm_w >= 1 && bpn_w >= 1 && p.M1 % bpm_w == 0 && p.N1 % bpn_w == 0) {
-        const int64_t gm = p.M1 / bpm_w, gn = p.N1 / bpn_w, cus = compute_units();
+        const int64_t gm = p.M1 / bpm_w, gn = p.N1 / bpn_w, cus = p.cus;
         const int64_t rem = cus > 0 ? (gm * gn) % cus : 0;
         if (gm * gn > cus && rem > 0 && 2 * rem <= cus && rem % gm == 0) {
           split_n = 1;
@@ -1280,7 +1281,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
       if (st >= 0) { *name = "mmt4d_mfma_128x128_kslices"; return st; }
     }
   }
-  const bool splits_k = long_k && (E != Elem::kF32 || 2 * workgroups(p, 64, 64) <= compute_units());
+  const bool splits_k = long_k && (E != Elem::kF32 || 2 * workgroups(p, 64, 64) <= p.cus);
   if constexpr (E == Elem::kF32) {
     if (forced == 0 && (choice == 2 || choice == 3 || choice == 6 || (RBC < 8 && choice == 4))) {
       const int st = launch_small_blocks<E, RBC>(p, rows_m, cols_n, choice == 2, choice == 6, choice == 6 && splits_k,
@@ -1297,7 +1298,7 @@ int launch_class(const Problem& p, int forced, hipStream_t stream, const char** 
                           (choice == 6 && !direct_before_ksplit<E, RBC>(p)) || (RBC == 2 && choice == 4));
     if (forced == 0 && by_cost) {
       const int64_t b32 = uk::ceil_div(rows_m, (int64_t)32) * uk::ceil_div(cols_n, (int64_t)32);
-      const bool parts = choice == 6 || (choice != 2 && b32 <= 2 * (int64_t)compute_units() && k_bytes >= 1024) ||
+      const bool parts = choice == 6 || (choice != 2 && b32 <= 2 * (int64_t)p.cus && k_bytes >= 1024) ||
                          (choice == 3 && RBC >= 16 && k_bytes >= 6144);
       const int st = launch_by_cost<E, RBC>(p, rows_m, cols_n, parts, stream, name);
       if (st >= 0) return st;
