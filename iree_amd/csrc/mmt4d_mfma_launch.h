@@ -784,48 +784,36 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
 // The kernels between the thin ones and 256x256 blocks, by what they take: the barrier-free
 // kernel in blocks of 32x32, 32x64 and 64x64, four waves sharing K; 64x64 blocks with the
 // RHS in registers (rows of 2 bytes: regrouped, 256 bytes of K a step); 64x64 and 128x128
-// blocks of the LDS-direct pipeline. Fitted, for each class of tile rows, to 300 products of
-// 65 to 4096 rows, 65 to 16384 columns, 128 B to 24 KB of K and up to 330 128x128 blocks, each
-// on all of these kernels with operands that are not cached: 5 to 14 % off in the mean, and
-// the choice is 1 to 4 % behind the fastest in the geometric mean (rules by numbers of
-// blocks were 12 to 21 % behind). us by those rules / so: f16 512 x 2048 x 2048 13.4 / 10.3,
-// 700 x 900 x 1504 11.1 / 8.7, 1500 x 1500 x 1504 18.1 / 14.3, but 1000 x 1501 x 777 9.0 /
-// 9.2; f8 900 x 1100 x 1300 8.8 / 7.1; bf16 16x16x2 1000 x 1500 x 784 17.3 / 11.1; s8 16x16x2
-// 2000 x 700 x 2000 17.4 / 13.3. Geometric means over 400 drawn products of 65 to 4096 rows:
-// f16 1.14, s8 1.15, 8-byte rows 1.09, 2-byte rows 1.16, f8 1.10, bf16 4-byte rows 1.13. The
-// barrier-free kinds of 8-byte rows have had their costs by K lowered by what loading rows
-// in twos gave, and serve K from 512 bytes on, where 64x64 blocks through LDS were chosen
-// (s8 957 x 2717 x 634 17.3 / 10.5 us, 502 x 2097 x 658 11.6 / 6.5, 622 x 237 x 973 7.2 / 4.6):
-// 1.12 over 70 products, 3402 x 147 x 2069 in f16 0.95 and s8 2010 x 277 x 2943 0.93 the slowest.
+// blocks of the LDS-direct pipeline. Fitted, for each class of tile rows, to 1000 products a
+// type of 65 to 4096 rows, 65 to 16384 columns, 64 B to 24 KB of K, each on all of these kernels
+// with operands that are not cached, for a choice near the fastest (0.1 to 0.6 % behind in the
+// geometric mean; single kernels are estimated 4 to 11 % off). us by numbers of blocks / so: f16
+// 512 x 2048 x 2048 17.5 / 11.8, 700 x 900 x 1504 11.2 / 8.7, 1500 x 1500 x 1504 20.1 / 18.1; f8
+// 900 x 1100 x 1300 8.8 / 6.9; 8-byte rows s8 957 x 2717 x 634 17.5 / 9.2, 2010 x 277 x 2943 13.7 /
+// 8.7, f16 3402 x 147 x 2069 19.8 / 13.1; bf16 16x16x2 1000 x 1500 x 784 17.2 / 10.8; s8 16x16x2
+// 2000 x 700 x 2000 17.5 / 13.4, 155 x 799 x 1919 7.6 / 6.5. Geometric means of 250 other
+// products where the choice differs: 16-byte rows f16 1.25, s8 1.29, bf16 -> bf16 1.35, f8 1.30,
+// 8-byte rows 1.58, 4-byte 1.30, 2-byte 1.55; 7 of 2500 are 4 % and more behind, 8 % at worst.
 enum BlockKind { k32x32, k32x64, k64x64Split, k64x64, k64x64Lds, k128x128, kBlockKinds };
 template <Elem E, int RBC>
 inline const BlockCost* block_costs() {
   constexpr double no = 1e30;
-  static constexpr BlockCost f8[kBlockKinds] = {{3.07, 0.28, 0.14, 0.60, 0}, {2.78, 0.87, 0.26, 0.90, 0},
-                                                {1.44, 2.95, 0.21, 1.43, 0}, {3.63, 0.75, 0.20, 1.76, 0},
-                                                {no, 0, 0, 0, 0},            {3.37, 1.53, 2.93, 2.50, 0}};
-  static constexpr BlockCost rows16[kBlockKinds] = {{3.12, 0.20, 0.20, 0.59, 0}, {3.10, 0.49, 0.28, 0.92, 0},
-                                                    {3.07, 1.15, 0.37, 1.26, 0}, {3.34, 0.55, 1.41, 1.40, 0},
-                                                    {no, 0, 0, 0, 0},            {3.48, 1.74, 1.35, 2.74, 0}};
-  static constexpr BlockCost rows8[kBlockKinds] = {{3.08, 0.23, 0.04, 0.71, 1}, {3.09, 0.54, 0.29, 1.06, 0},
-                                                   {3.12, 1.19, 0.48, 1.40, 0}, {no, 0, 0, 0, 0},
-                                                   {1.16, 3.88, 0.39, 1.91, 0}, {3.04, 2.33, 3.08, 1.87, 0}};
-  static constexpr BlockCost rows4[kBlockKinds] = {{3.18, 0.22, 0.03, 0.89, 1}, {3.21, 0.52, 0.04, 1.35, 1},
-                                                   {3.28, 1.22, 0, 1.83, 1},    {no, 0, 0, 0, 0},
-                                                   {1.14, 3.94, 0.41, 1.95, 0}, {3.14, 2.35, 2.98, 2.08, 0}};
-  static constexpr BlockCost rows2[kBlockKinds] = {{2.20, 0.55, 1.31, 1.72, 1.25}, {2.68, 1.18, 0.11, 2.65, 1},
-                                                   {no, 0, 0, 0, 0},               {2.92, 1.19, 0.21, 2.65, 1.25},
-                                                   {1.44, 3.63, 0.06, 1.97, 0},    {3.92, 1.87, 1.62, 2.79, 0}};
+  static constexpr BlockCost f8[kBlockKinds] = {{2.62, 0.23, 0.12, 0.67, 1.10}, {2.56, 0.94, 0.29, 0.87, 0},
+                                                {1.42, 3.00, 0.16, 1.45, 0.72}, {3.58, 0.57, 0.24, 1.77, 0},
+                                                {no, 0, 0, 0, 0}, {3.25, 1.03, 3.53, 2.46, 0.09}};
+  static constexpr BlockCost rows16[kBlockKinds] = {{3.06, 0.20, 0.13, 0.59, 0.94}, {3.20, 0.51, 0.32, 0.90, 0.62},
+                                                    {3.53, 1.11, 0.18, 1.26, 0.89}, {3.37, 0.54, 1.37, 1.45, 0.38},
+                                                    {no, 0, 0, 0, 0}, {5.14, 1.01, 1.20, 2.75, 0.24}};
+  static constexpr BlockCost rows8[kBlockKinds] = {{2.74, 0.35, 0.05, 0.71, 1.13}, {3.35, 0.40, 0.29, 1.07, 0.26},
+                                                   {3.13, 1.22, 0.50, 1.40, 0.37}, {no, 0, 0, 0, 0},
+                                                   {1.09, 4.57, 0.13, 2.02, 0.81}, {3.04, 2.63, 3.02, 1.91, 0.69}};
+  static constexpr BlockCost rows4[kBlockKinds] = {{2.94, 0.10, 0.12, 0.93, 0.13}, {3.26, 0.47, 0.10, 1.35, 0.90},
+                                                   {3.23, 1.22, 0, 1.82, 1.07}, {no, 0, 0, 0, 0},
+                                                   {0.85, 5.24, 0.16, 1.92, 0.84}, {2.93, 2.54, 2.92, 2.10, 0.71}};
+  static constexpr BlockCost rows2[kBlockKinds] = {{1.90, 0.96, 0.38, 1.58, 0.96}, {2.97, 0.97, 0.20, 2.66, 0.89},
+                                                   {no, 0, 0, 0, 0}, {3.10, 0.83, 0.25, 2.58, 1.40},
+                                                   {1.96, 3.68, 0.12, 1.97, 0.07}, {3.84, 0.82, 1.87, 2.83, 0.11}};
   return ElemTraits<E>::kHalves == 2 ? f8 : RBC >= 16 ? rows16 : RBC == 8 ? rows8 : RBC == 4 ? rows4 : rows2;
-}
-template <Elem E, int RBC>
-double kind_us(const Problem& p, int64_t rows, int64_t cols, int kind) {
-  static constexpr int bm[] = {32, 32, 64, 64, 64, 128}, bn[] = {32, 64, 64, 64, 64, 128};
-  // (LDS blocks hold whole panels, the others need not)
-  const int64_t blocks = kind >= k64x64 ? workgroups(p, bm[kind], bn[kind])
-                                        : uk::ceil_div(rows, (int64_t)bm[kind]) * uk::ceil_div(cols, (int64_t)bn[kind]);
-  if (blocks < 1) return 1e30;
-  return block_us(block_costs<E, RBC>()[kind], p.cus, blocks, (double)((int64_t)p.K1 << p.lrb) / 1024);
 }
 // `parts`: a float's K stays in four parts, as it is in kernels whose waves share it and in
 // the 64x64 blocks in registers.
@@ -839,9 +827,15 @@ int launch_by_cost(const Problem& p, int64_t rows, int64_t cols, bool parts, hip
     const int st = launch_16x16<E, RBC, 8>(p, stream);
     if (st >= 0) { *name = "mmt4d_mfma_16x16_ksplit"; return st; }
   }
+  // (LDS blocks hold whole panels, the others need not)
+  const int64_t r32 = uk::ceil_div(rows, (int64_t)32), r64 = uk::ceil_div(rows, (int64_t)64);
+  const int64_t c32 = uk::ceil_div(cols, (int64_t)32), c64 = uk::ceil_div(cols, (int64_t)64);
+  const int64_t b64 = workgroups(p, 64, 64), b128 = workgroups(p, 128, 128);
+  const int64_t blocks[kBlockKinds] = {r32 * c32, r32 * c64, r64 * c64, b64, b64, b128};
+  const double kb = (double)k_bytes / 1024;
   double us[kBlockKinds];
   for (int k = 0; k < kBlockKinds; ++k) {
-    us[k] = kind_us<E, RBC>(p, rows, cols, k);
+    us[k] = blocks[k] < 1 ? 1e30 : block_us(block_costs<E, RBC>()[k], cus, blocks[k], kb);
     // (The 64x64 blocks in registers have a float's K in four parts from 96 steps on. 8-bit
     // floats: the matrix instructions round to 1.5e-5, however K is divided.)
     if (parts && !kInteger && ElemTraits<E>::kHalves == 1 && k > k64x64Split &&
@@ -851,7 +845,13 @@ int launch_by_cost(const Problem& p, int64_t rows, int64_t cols, bool parts, hip
   }
   // With less than 1 KB of K a block of 128x128 is its stores, estimated low (f16 3428 x 704 x
   // 132 in 64x64 blocks 6.3 us, in these 7.6).
-  if (k_bytes < 1024 && workgroups(p, 128, 128) < 192) us[k128x128] = 1e30;
+  if (k_bytes < 1024 && b128 < 192) us[k128x128] = 1e30;
+  // With 256 bytes of K, of which some waves of the barrier-free blocks get no step, and more than
+  // four 32x32 blocks a unit, launching and adding up those is what they take: f8 1090 x 1412 x
+  // 105 6.3 us, so 4.9, s8 716 x 2957 x 256 7.8 / 6.5. (16-bit results, of which the 64x64
+  // blocks store half as much at a time, from some nine blocks a unit on: estimated.)
+  if (RBC >= 16 && ElemTraits<E>::Out::kOutBytes == 4 && k_bytes <= 256 && r32 * c32 > 4 * cus)
+    us[k32x32] = us[k32x64] = us[k64x64Split] = 1e30;
   // 2-byte results: the LDS-direct 64x64 shape takes K in whole steps.
   if (ElemTraits<E>::Out::kOutBytes == 2 && k_bytes % 256 != 0) us[k64x64Lds] = 1e30;
   for (;;) {

@@ -25,7 +25,11 @@ def _tiles(torch, x, m0, k0):
 
 @pytest.mark.parametrize("kind,tile,m,n,k,name", [
     (F16, (16, 16, 8), 700, 900, 1504, "64x64_ksplit"),
-    (F16, (16, 16, 8), 513, 2041, 1020, "32x64_ksplit"),
+    (F16, (16, 16, 8), 513, 2041, 1020, "32x32_ksplit"),
+    (F16, (16, 16, 8), 1000, 1501, 777, "32x64_ksplit"),
+    (F8, (16, 16, 16), 1090, 1412, 105, "64x64_rhs_direct"),   # (256 bytes of K and less: not by costs)
+    (S8, (16, 16, 16), 716, 2957, 256, "64x64_rhs_direct"),
+    (BF16, (16, 16, 1), 131, 521, 2003, "32x32_ksplit"),
     (F16, (16, 16, 16), 300, 4096, 530, "32x32_ksplit"),
     (F16, (48, 16, 8), 1500, 1490, 1504, "128x128_lds_direct"),
     (BF16BF16, (16, 16, 8), 777, 1011, 643, "64x64_ksplit"),
