@@ -658,44 +658,63 @@ int launch_16x16(const Problem& p, hipStream_t stream) {
 
 // What `blocks` workgroups of a kernel take, in us, by the KB of K. A unit's blocks are
 // loaded one beside the other, and a last round of few blocks is not a whole one; below
-// `least` blocks a unit a block's own chain of steps is what it takes.
+// `least` blocks a unit a block's own chain of steps is what it takes. Where a unit holds
+// `resident` blocks at a time (0: all), those of a last turn take as long as `last` of them.
 struct BlockCost {
-  double launch, round, k, k_block, least;
+  double launch, round, k, k_block, least, resident = 0, last = 0;
 };
 inline double block_us(const BlockCost& c, int64_t cus, int64_t blocks, double kb) {
   const double units = (double)blocks / (double)cus, rounds = std::ceil(units);
-  return c.launch + c.round * rounds + kb * (c.k + c.k_block * std::max(c.least, std::min(rounds, units + 0.6)));
+  const double whole = c.resident > 0 && units > c.resident ? c.resident * (std::ceil(units / c.resident) - 1) : 0;
+  const double rest = std::max(whole > 0 ? c.last : c.least, std::min(rounds, units + 0.6) - whole);
+  return c.launch + c.round * rounds + kb * (c.k + c.k_block * (whole + rest));
+}
+
+// f32: the barrier-free kernel in 32x32 blocks, K over four waves and over two, in 32x48
+// blocks over four, 48x48 over eight; and those it is weighed against: 128x128 blocks, the 64x64
+// K split, 64x64 blocks, with rows of 4 bytes and more than 8 KB of K the regrouping ones. Fitted,
+// like block_costs below, to 600 to 725 products of 65 to 4096 rows and 256 B to 24 KB of K a class of
+// rows (16, 8, 4 bytes); the choice is 0.2 to 0.3 % behind the fastest in the geometric mean.
+enum F32Kind { kF32x32, kF32x32Two, kF32x48, kF48x48, kF128x128, kF64x64Split, kF64x64, kF64x64Long, kF32Kinds };
+template <int RBC>
+inline const BlockCost* f32_costs() {
+  static constexpr BlockCost rows16[kF32Kinds] = {{2.80, 0.34, 0.18, 0.93, 1.31, 6, 2.80}, {1.02, 0.23, 0.47, 1.08, 4.15, 10, 4.66},
+                                                  {3.60, 0.41, 0.03, 1.40, 0.00, 4, 2.53}, {1.66, 2.80, 0.02, 2.06, 1.02, 1, 1.00},
+                                                  {3.06, 3.39, 1.22, 13.32, 0.57}, {4.23, 1.94, 0.06, 3.60, 0.95},
+                                                  {3.36, 0.73, 0.63, 3.90, 0.95}, {1e30, 0, 0, 0, 0}};
+  static constexpr BlockCost rows8[kF32Kinds] = {{3.04, 0.27, 0.30, 0.96, 0.00, 5, 3.04}, {2.28, 0.29, 1.00, 0.93, 4.51, 8, 3.00},
+                                                 {3.44, 0.69, 0.21, 1.53, 0.56, 5, 1.30}, {1.92, 2.73, 0, 2.25, 0.96, 9, 1.62},
+                                                 {2.87, 4.49, 4.10, 14.36, 0.35}, {4.68, 0.15, 0, 3.84, 0.95},
+                                                 {3.64, 1.26, 1.11, 4.63, 1.01}, {1e30, 0, 0, 0, 0}};
+  static constexpr BlockCost rows4[kF32Kinds] = {{2.73, 0.44, 0.31, 0.98, 1.05, 5, 2.22}, {2.76, 0.38, 1.23, 0.86, 0.00, 10, 4.47},
+                                                 {3.24, 0.63, 0.30, 1.43, 1.08, 4, 1.61}, {2.02, 2.51, 0, 2.31, 0.97, 9, 1.91},
+                                                 {2.62, 4.69, 3.94, 14.31, 0.80}, {1e30, 0, 0, 0, 0},
+                                                 {3.49, 1.23, 1.23, 4.51, 0.98}, {3.82, 1.91, 2.86, 3.20, 1.01}};
+  return RBC >= 16 ? rows16 : RBC == 8 ? rows8 : rows4;
 }
 
 // Problems whose 64x64 blocks leave compute units idle or take a last round that is
-// nearly empty: the barrier-free kernel in 16x16 or 32x32 blocks, several waves of a
-// block sharing K, so that the chain of K steps a wave walks through is short and many
-// more loads are in flight than one workgroup a unit keeps. `b128`, `ksplit64`, `b32x64`:
-// whether it would be the 128x128 kernels, the 64x64 K split (or what takes its place) or
-// 32x64 blocks through LDS otherwise (else 64x64). Any K, any tile rows. Returns a HIP
-// status, or -1 where those kernels are the better ones. `parts` (f32): that K split would have K in workgroups too, up to 128 parts; up to three 16x16
-// blocks a unit then have it in four or eight waves of sixteen chains, and as small an error
-// (128 x 128 x 6144 41 us, 1.77e-7 / 11.3, 1.56e-7; 128 x 1024 x 6144 31.8 / 22.5). us
-// before / in these blocks, same buffers:
-//   one 16x16 block a unit or fewer, from 256 bytes of K (rows under 16 bytes: 64):
-//     f16 220 x 215, K 512 B 4.5 / 4.2, 2 KB 6.8 / 4.2, 7.6 KB 14.9 / 5.4; s8 16x16x2
-//     128 x 512, 100 B 4.4 / 3.8, 1 KB 6.5 / 4.0; f32 16x16x1 220 x 215, 3 KB 22.1 /
-//     5.9 (there up to three blocks a unit: 374 x 391, 1 KB 11.1 / 5.5);
-//   two 32x32 blocks a unit or fewer, from 1 KB (f32: 256 B): s8 500 x 500, 3.8 KB
-//     9.6 / 6.5; f16 512 x 1024, 1 KB 5.5 / 5.3, 7.6 KB 15.7 / 13.6; bf16 16x16x2 500 x
-//     500, 1 KB 6.8 / 5.3 (rows of 2 bytes load an element at a time: one block a unit,
-//     s8 16x16x2 500 x 500, 3.8 KB 13.9 / 10.6, 512 x 1024 14.1 / 13.7); 8-bit floats up to
-//     7/4 blocks a unit (139 x 3012, 4 KB, 1.86 blocks 9.2 / 12.3), 5/4 from 6 KB on (212 x
-//     1280, 7.1 KB, 1.1 blocks 13.9 / 11.1; 235 x 1631, 11.9 KB, 1.6 blocks 22.2 / 29.0);
-//   f32, whose MFMAs are slow enough to hide the loads of 32x32 blocks, by costs fitted to
-//     1500 products of 64 to 4096 rows and columns, 256 B to 32 KB of K (3 to 10 % off in the
-//     mean): first whether at all, by what 32x32 blocks of four and two waves and the kernel
-//     otherwise took (893 x 4064, 13.5 KB 203 otherwise / 245, 16x16x1 1879 x 1045, 1.7 KB
-//     25.0 / 28.0), then which, by what all of these blocks take now: in the larger ones a
-//     unit's L1 and L2 carry fewer bytes a sum. us in 32x32 blocks before / as chosen: 16x16x4
-//     515 x 1027 x 768 13.6 / 11.2 (48x48), 1500 x 1500 x 1000 44.8 / 42.4; 16x16x1 515 x 1027 x
-//     769 17.6 / 12.8 (48x48), 1500 x 1500 x 1000 55.3 / 47.8, 700 x 700 x 3000 36.5 / 29.8.
-//     Geometric means over 400 drawn products: 16-byte rows 1.10, 4-byte rows 1.15.
+// nearly empty: the barrier-free kernel in small blocks, several waves of a block sharing K,
+// so that the chain of K steps a wave walks through is short and many more loads are in flight
+// than one workgroup a unit keeps. f32, and what launch_by_cost does not choose for. `b128`,
+// `ksplit64`, `b32x64`: whether it would be the 128x128 kernels, the 64x64 K split (or what
+// takes its place) or 32x64 blocks through LDS otherwise (else 64x64). Any K, any tile rows.
+// Returns a HIP status, or -1 where those kernels are the better ones. `parts` (f32): that K split
+// would have K in workgroups too, up to 128 parts; up to three 16x16 blocks a unit then have it in
+// four or eight waves of sixteen chains, and as small an error (128 x 128 x 6144 41 us, 1.77e-7 /
+// 11.3, 1.56e-7; 128 x 1024 x 6144 31.8 / 22.5). us otherwise / in these blocks:
+//   one 16x16 block a unit or fewer, from 256 bytes of K (rows under 16 bytes: 64): f16 220 x
+//     215, K 512 B 4.5 / 4.2, 7.6 KB 14.9 / 5.4; s8 16x16x2 128 x 512, 100 B 4.4 / 3.8; f32
+//     16x16x1 220 x 215, 3 KB 22.1 / 5.9 (there up to three blocks a unit: 374 x 391, 1 KB 11.1
+//     / 5.5);
+//   f32, whose MFMAs are slow enough to hide the loads of 32x32 blocks, by f32_costs: in the
+//     larger blocks a unit's L1 and L2 carry fewer bytes a sum. 16x16x4 515 x 1027 x 768 11.2 (48x48;
+//     13.8 in 32x32 blocks before), 3140 x 237 x 2088 35.9 / 28.3 (32x48); 16x16x2 2173 x 674 x 3168
+//     95.7 / 77.3 (32x48); 16x16x1 515 x 1027 x 769 12.1 (48x48), 958 x 810 x 690 20.4 / 13.5, 1500 x
+//     1500 x 1000 42.8 (32x48), 3582 x 3328 x 1792 382 / 331 (32x32); but 1564 x 1150 x 2621, seven
+//     32x32 blocks a unit, of which it holds six at a time, 80 / 91 (64x64);
+//   other types, where K ends inside a step of a thin product: two 32x32 blocks a unit or fewer,
+//     from 1 KB (8-bit floats, two loads an operand: 7/4; rows of 2 bytes: one).
 template <Elem E, int RBC>
 int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128, bool ksplit64, bool parts,
                         bool b32x64, hipStream_t stream, const char** name) {
@@ -722,46 +741,42 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
     return st;
   }
   if constexpr (F32) {
-    if (k_bytes < (b128 || (RBC >= 16 && b32 > 2 * cus) ? 1024 : 256)) return -1;
+    // (Below 1 KB of K not with many blocks: rows of 16 bytes more than two 32x32 blocks a unit,
+    // others in the place of 128x128 blocks, unless those are more than two a unit: 16x16x2 2988 x
+    // 3666 x 218 62.7 us, so 53.6, 16x16x1 63.5 / 55.2, but 2048 x 4096 x 240 42.5 / 45.6.)
+    if (k_bytes < ((RBC >= 16 ? b32 > 2 * cus : b128 && workgroups(p, 128, 128) <= 2 * cus) ? 1024 : 256)) return -1;
     if (b16 <= 3 * cus) {
       st = launch_16x16<E, RBC, 4>(p, stream);
       if (st >= 0) *name = "mmt4d_mfma_16x16_ksplit";
       return st;
     }
-    // us of 32x32 blocks in four waves and in two (not as precise as the 64x64 K split, and
-    // not in its place), of 32x48 in four, 48x48 in eight. Where another shape is less than
-    // 6 % ahead, 32x32 blocks. (32x64 and 64x64 blocks were nowhere the fastest.)
     const double kb = (double)k_bytes / 1024;
     auto blocks = [&](int bm, int bn) {
       return uk::ceil_div(rows, (int64_t)bm) * uk::ceil_div(cols, (int64_t)bn);
     };
-    constexpr bool W = RBC >= 16;
-    constexpr double kOther = 1.06;
-    double us[4] = {
-        block_us(W ? BlockCost{3.14, 0.41, 0.15, 0.93, 1} : BlockCost{3.04, 0.44, 0.35, 0.98, 1}, cus, b32, kb),
-        ksplit64 ? 1e30
-                 : block_us(W ? BlockCost{3.19, 0.30, 1.35, 0.89, 0} : BlockCost{3.14, 0.35, 1.52, 0.94, 0}, cus, b32, kb),
-        kOther * block_us(W ? BlockCost{3.33, 0.58, 0.01, 1.42, 1} : BlockCost{3.24, 0.66, 0.35, 1.43, 1}, cus, blocks(32, 48), kb),
-        kOther * block_us(W ? BlockCost{1.96, 2.55, 0, 2.11, 1} : BlockCost{1.96, 2.77, 0, 2.31, 1}, cus, blocks(48, 48), kb)};
+    const BlockCost* costs = f32_costs<RBC>();
+    auto us_of = [&](int kind, int64_t n) { return n < 1 ? 1e30 : block_us(costs[kind], cus, n, kb); };
+    double us[4] = {us_of(kF32x32, b32), 1e30, us_of(kF32x48, blocks(32, 48)), us_of(kF48x48, blocks(48, 48))};
+    // K in two parts instead of four only with many rounds of blocks and few steps, where it
+    // was in two before, and not in the place of the 64x64 K split: the error is larger.
+    const double rounds = (double)uk::ceil_div(b32, cus), turns = std::min(rounds, (double)b32 / (double)cus + 0.6);
+    if (!ksplit64 && (RBC >= 16 ? 0.11 * rounds + 0.04 * kb * turns > 0.05 + 1.2 * kb
+                                : 0.09 * rounds + 0.04 * kb * turns > 0.1 + 1.17 * kb)) {
+      us[1] = us_of(kF32x32Two, b32);
+    }
     if (b32x64) us[2] = us[3] = 1e30;   // (64 rows and fewer)
     static const char* const names[4] = {"mmt4d_mfma_32x32_ksplit", "mmt4d_mfma_32x32_ksplit", "mmt4d_mfma_32x48_ksplit",
                                          "mmt4d_mfma_48x48_ksplit"};
     const int best = (int)(std::min_element(us, us + 4) - us);
-    // And of the kernel that it would be otherwise, against what 32x32 blocks took when its
-    // costs were fitted beside theirs.
-    const double r32 = (double)uk::ceil_div(b32, cus), r64 = (double)uk::ceil_div(workgroups(p, 64, 64), cus);
-    const double r128 = (double)uk::ceil_div(workgroups(p, 128, 128), cus);
-    const double four = W ? 3.6 + 0.5 * r32 + kb * (0.13 + 1.09 * r32) : 3.3 + 0.7 * r32 + kb * (0.37 + 1.28 * r32);
-    const double two = ksplit64 ? four
-                       : W      ? 3.75 + 0.33 * r32 + kb * (1.56 + 0.99 * r32)
-                                : 3.5 + 0.43 * r32 + kb * (2.6 + 1.13 * r32);
-    const double other = b128              ? (W ? 3 + 3.4 * r128 + kb * (2.4 + 13.65 * r128)
-                                                : 5 + 3.6 * r128 + kb * (4 + 14.7 * r128))
-                         : ksplit64        ? 6.7 + 1.1 * r64 + kb * 4 * r64
-                         : W               ? 3.4 + 0.7 * r64 + kb * (0.63 + 3.9 * r64)
-                         : k_bytes <= 8192 ? 2.9 + 1.9 * r64 + kb * (1.2 + 4.56 * r64)
-                                           : 4.3 + kb * (2 + 3.95 * r64);
-    if (b32x64 ? 2 * b32 > 7 * (int64_t)r64 * cus : std::min(four, two) > 1.02 * other) return -1;
+    if (b32x64) {
+      if (2 * b32 > 7 * uk::ceil_div(workgroups(p, 64, 64), cus) * cus) return -1;
+    } else {
+      const double other = b128                            ? us_of(kF128x128, workgroups(p, 128, 128))
+                           : ksplit64                      ? us_of(kF64x64Split, workgroups(p, 64, 64))
+                           : RBC >= 16 || k_bytes <= 8192  ? us_of(kF64x64, workgroups(p, 64, 64))
+                                                           : us_of(kF64x64Long, workgroups(p, 64, 64));
+      if (us[best] > other) return -1;
+    }
     switch (best) {
       case 0: st = launch_thin<E, RBC, 2, 2, 4, kAhead, true>(p, false, stream); break;
       case 1: st = launch_thin<E, RBC, 2, 2, 2, kAhead, true>(p, false, stream); break;

@@ -49,7 +49,12 @@ def _tiles(torch, x, m0, k0):
     (F32, (16, 16, 4), 515, 1027, 770, "48x48_ksplit"),
     (F32, (16, 16, 1), 1027, 515, 771, "48x48_ksplit"),
     (F32, (16, 16, 1), 600, 700, 300, "32x32_ksplit"),
-    (F32, (16, 16, 4), 1100, 1300, 2001, "32x32_ksplit"),
+    (F32, (16, 16, 4), 1100, 1300, 2001, "32x48_ksplit"),
+    (F32, (16, 16, 4), 1500, 1500, 1000, "32x32_ksplit"),
+    (F32, (16, 16, 4), 3140, 237, 2088, "32x48_ksplit"),     # (64x64 blocks by older costs)
+    (F32, (16, 16, 1), 958, 810, 690, "32x48_ksplit"),
+    (F32, (16, 16, 2), 2988, 3666, 218, "32x32_ksplit"),     # (under 1 KB of K)
+    (F32, (16, 16, 2), 2048, 4096, 240, "128x128"),
     (F32, (48, 16, 4), 1030, 1050, 1301, "32x48_ksplit")])
 def test_blocks_by_cost(gpu, kind, tile, m, n, k, name):
     lib, torch = gpu

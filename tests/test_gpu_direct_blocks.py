@@ -47,7 +47,7 @@ def _small(torch, rows, k, seed):
     (S8, (16, 16, 16), 2898, 418, 7936, "64x64_rhs_direct"),
     (S8, (32, 16, 8), 1083, 950, 16353, "64x64_lds_direct"),
     (F32, (16, 16, 4), 41, 12664, 855, "32x32_ksplit"),            # else 32x64 blocks
-    (F32, (16, 16, 1), 1879, 1045, 431, "64x64_deep")])
+    (F32, (16, 16, 1), 1879, 1045, 431, "32x32_ksplit")])
 def test_which_blocks(gpu, kind, tile, m, n, k, name):
     lib, torch = gpu
     if torch.cuda.get_device_properties(0).multi_processor_count != 256:

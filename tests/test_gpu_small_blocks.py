@@ -73,7 +73,7 @@ def test_small_blocks_against_the_exact_product(gpu, dtype, m0, n0, k0, m, n, k,
 def test_f32_blocks_against_full_rounds(gpu, k0, m, n, k):
     names = _run(gpu, "f32", m, n, k, 16, 16, k0, seed=n)
     if k0 == 1 or k >= 256:
-        assert all("32x32_ksplit" in x for x in names), names
+        assert all("32x32_ksplit" in x or "32x48_ksplit" in x for x in names), names
 
 
 @pytest.mark.parametrize("dtype,k0,m,n", [("f16", 16, 100, 90), ("f32", 1, 100, 90), ("bf16", 2, 100, 90),
