@@ -556,8 +556,9 @@ extern "C" int iree_uk_amd_hip_launch_mmt4d_mfma(const iree_uk_mmt4d_params_t* p
       pr.acc_stride < 0) {
     return -1;
   }
-  // Operands need no alignment beyond their element's: the kernels read them
-  // with vector loads that take any address (v4i_g in the kernel header).
+  // Operands need no alignment beyond their element's: the kernels read them with
+  // vector and buffer loads that take any address (v4i_g in the kernel header, load16
+  // and the others of the barrier-free kernel).
   if (((uintptr_t)pr.lhs | (uintptr_t)pr.rhs) & (uintptr_t)(s8s4 ? 0 : eb - 1)) return -1;
   if ((uintptr_t)pr.out & (uintptr_t)(ob - 1)) return -1;
   pr.M1 = (int32_t)p->M;

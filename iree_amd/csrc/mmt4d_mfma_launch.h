@@ -456,40 +456,37 @@ int launch_thin(const Problem& caller, bool swapped, hipStream_t stream, bool al
   // 14336 x 4096 s8 94.4 / 87.5 / 83.1 us, 16 rows 68.5 / 65.5; f16 32 rows 134 / 120; in 64x64
   // blocks s8 300 x 4096 x 2000 12.7 / 11.1 / 10.1, 2000 x 300 x 4099 12.6 / 11.1 / 10.6, f16 19.3
   // / 16.7, 96 x 4096 x 4096 in 32x64 15.0 / 12.5. 4-byte rows of f32, whose products take a
-  // word at a time: 128 x 2048 x 4096 24.0 / 20.0, 96 x 4096 x 4096 38.7 / 33.7, 2000 x
-  // 300 x 4099 53.8 / 50.0, 1000 x 1501 x 777 26.4 / 26.0, six blocks a unit, but 1500 x 1500 x
-  // 1500, nine, 68.5 / 73. Other
-  // types put them together with moves that cost more than the loads: bf16 16x16x2 1000 x
-  // 1501 x 777 11.5 / 14.0, s8 16x16x4 96 x 4096 x 4096 9.5 / 10.7. A tile of an odd number of
-  // rows would split such a two.
-  constexpr bool kPairs = TN % 2 == 0 && (RBC == 8 || (RBC == 4 && E == Elem::kF32 && KSPLIT > 2));
-  const bool pairs = kPairs && (RBC == 8 || grid_m * grid_n <= 6 * (int64_t)p.cus) && p.N0 % 2 == 0 && (TM % 2 != 0 || p.M0 % 2 == 0);
-  if constexpr (TAIL_OK) {
-    // No non-temporal instances: weights that the caller has declared streamed are read
-    // by several row blocks here, which then wait for HBM one after the other (64x64
-    // blocks, ordinary / non-temporal us: f16 200 x 8192 x 4096 34.6 / 44.5, s8 80 x 8192 x
-    // 8192 21.4 / 25.0, 128 x 4096 x 14336 34.9 / 35.6; at best f8 192 x 4096 x 8192 21.6 / 21.1).
-    auto go = [&](auto paired_c) {
-      constexpr bool P = decltype(paired_c)::value;
-      if (tail) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, true, CH, P>, grid, block, 0, stream, a);
-      else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, CH, P>, grid, block, 0, stream, a);
-      return (int)hipGetLastError();
-    };
-    if (pairs) return go(std::bool_constant<kPairs>{});
-    return go(std::false_type{});
-  } else {
-    // Weights that the caller has declared streamed, when they are too large for
-    // the L2s anyway: loaded non-temporally.
-    const bool streamed = streamed_weights() && (int64_t)p.N1 * p.N0 * k_bytes / (S4 ? 2 : 1) >= (16ll << 20);
-    auto go = [&](auto paired_c) {
-      constexpr bool P = decltype(paired_c)::value;
-      if (streamed) uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, true, false, 0, P>, grid, block, 0, stream, a);
-      else uk::launch(2, mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, 0, P>, grid, block, 0, stream, a);
-      return (int)hipGetLastError();
-    };
-    if (pairs) return go(std::bool_constant<kPairs>{});
-    return go(std::false_type{});
+  // word at a time: 128 x 2048 x 4096 24.0 / 20.0, 96 x 4096 x 4096 38.7 / 33.7, 2000 x 300 x
+  // 4099 53.8 / 50.0, 1000 x 1501 x 777 26.4 / 26.0, six blocks a unit, but 1500 x 1500 x 1500,
+  // nine, 68.5 / 73. Other types put them together with moves that cost more than the loads:
+  // bf16 16x16x2 1000 x 1501 x 777 11.5 / 14.0, s8 16x16x4 96 x 4096 x 4096 9.5 / 10.7. (Tiles
+  // of an odd number of such rows are regrouped to rows of 16 bytes before they come here.)
+  constexpr bool kPairs8 = TN % 2 == 0 && RBC == 8;
+  constexpr bool kPairs4 = TN % 2 == 0 && RBC == 4 && E == Elem::kF32 && KSPLIT > 2;
+  // No non-temporal instances where K may end inside a step: weights that the caller has
+  // declared streamed are read by several row blocks there, which then wait for HBM one after
+  // the other (64x64 blocks, ordinary / non-temporal us: f16 200 x 8192 x 4096 34.6 / 44.5, s8
+  // 80 x 8192 x 8192 21.4 / 25.0, 128 x 4096 x 14336 34.9 / 35.6; at best f8 192 x 4096 x 8192
+  // 21.6 / 21.1). Else where they are too large for the L2s anyway.
+  const bool streamed =
+      !TAIL_OK && streamed_weights() && (int64_t)p.N1 * p.N0 * k_bytes / (S4 ? 2 : 1) >= (16ll << 20);
+  auto go = [&](auto paired_c) {
+    constexpr bool P = decltype(paired_c)::value;
+    if constexpr (TAIL_OK) {
+      auto kernel = tail ? mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, true, CH, P>
+                         : mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, CH, P>;
+      uk::launch(2, kernel, grid, block, 0, stream, a);
+    } else {
+      auto kernel = streamed ? mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, true, false, 0, P>
+                             : mmt4d_thin_kernel<E, RBC, TM, TN, KSPLIT, D, false, false, 0, P>;
+      uk::launch(2, kernel, grid, block, 0, stream, a);
+    }
+    return (int)hipGetLastError();
+  };
+  if constexpr (kPairs4) {
+    if (grid_m * grid_n <= 6 * (int64_t)p.cus) return go(std::true_type{});
   }
+  return go(std::bool_constant<kPairs8>{});
 }
 
 // The thin kernel with TM 16-row blocks against `wide_cols` columns (rows of the
@@ -533,7 +530,7 @@ int launch_thin_rows(const Problem& p, bool swapped, int64_t wide_cols, hipStrea
   // (Not for 8-byte rows in twos, whose loads are half as many in 32 columns: s8, 8-byte rows,
   // in 16 columns over eight waves / so, four layers, 4 x 11008 x 4096 64.3 / 60.8 us, 16 x
   // 28672 x 8192 221 / 191. Floats keep the parts of K that eight waves have.)
-  const bool paired = kInteger && RBC == 8 && (swapped ? p.M0 : p.N0) % 2 == 0;
+  constexpr bool paired = kInteger && RBC == 8;
   const bool narrow = blocks16 <= cus ||
                       (TM == 1 && !paired && uk::ceil_div(blocks16, cus) < 2 * uk::ceil_div(blocks32, cus));
   if (narrow) return launch_thin<E, RBC, TM, 1, 8, TM == 1 && H == 1 ? 4 : 2>(p, swapped, stream, true);
@@ -678,18 +675,21 @@ inline double block_us(const BlockCost& c, int64_t cus, int64_t blocks, double k
 enum F32Kind { kF32x32, kF32x32Two, kF32x48, kF48x48, kF128x128, kF64x64Split, kF64x64, kF64x64Long, kF32Kinds };
 template <int RBC>
 inline const BlockCost* f32_costs() {
-  static constexpr BlockCost rows16[kF32Kinds] = {{2.80, 0.34, 0.18, 0.93, 1.31, 6, 2.80}, {1.02, 0.23, 0.47, 1.08, 4.15, 10, 4.66},
-                                                  {3.60, 0.41, 0.03, 1.40, 0.00, 4, 2.53}, {1.66, 2.80, 0.02, 2.06, 1.02, 1, 1.00},
-                                                  {3.06, 3.39, 1.22, 13.32, 0.57}, {4.23, 1.94, 0.06, 3.60, 0.95},
-                                                  {3.36, 0.73, 0.63, 3.90, 0.95}, {1e30, 0, 0, 0, 0}};
-  static constexpr BlockCost rows8[kF32Kinds] = {{3.04, 0.27, 0.30, 0.96, 0.00, 5, 3.04}, {2.28, 0.29, 1.00, 0.93, 4.51, 8, 3.00},
-                                                 {3.44, 0.69, 0.21, 1.53, 0.56, 5, 1.30}, {1.92, 2.73, 0, 2.25, 0.96, 9, 1.62},
-                                                 {2.87, 4.49, 4.10, 14.36, 0.35}, {4.68, 0.15, 0, 3.84, 0.95},
-                                                 {3.64, 1.26, 1.11, 4.63, 1.01}, {1e30, 0, 0, 0, 0}};
-  static constexpr BlockCost rows4[kF32Kinds] = {{2.73, 0.44, 0.31, 0.98, 1.05, 5, 2.22}, {2.76, 0.38, 1.23, 0.86, 0.00, 10, 4.47},
-                                                 {3.24, 0.63, 0.30, 1.43, 1.08, 4, 1.61}, {2.02, 2.51, 0, 2.31, 0.97, 9, 1.91},
-                                                 {2.62, 4.69, 3.94, 14.31, 0.80}, {1e30, 0, 0, 0, 0},
-                                                 {3.49, 1.23, 1.23, 4.51, 0.98}, {3.82, 1.91, 2.86, 3.20, 1.01}};
+  static constexpr BlockCost rows16[kF32Kinds] = {
+      {2.80, 0.34, 0.18, 0.93, 1.31, 6, 2.80}, {1.02, 0.23, 0.47, 1.08, 4.15, 10, 4.66},
+      {3.60, 0.41, 0.03, 1.40, 0.00, 4, 2.53}, {1.66, 2.80, 0.02, 2.06, 1.02, 1, 1.00},
+      {3.06, 3.39, 1.22, 13.32, 0.57}, {4.23, 1.94, 0.06, 3.60, 0.95},
+      {3.36, 0.73, 0.63, 3.90, 0.95}, {1e30, 0, 0, 0, 0}};
+  static constexpr BlockCost rows8[kF32Kinds] = {
+      {3.04, 0.27, 0.30, 0.96, 0.00, 5, 3.04}, {2.28, 0.29, 1.00, 0.93, 4.51, 8, 3.00},
+      {3.44, 0.69, 0.21, 1.53, 0.56, 5, 1.30}, {1.92, 2.73, 0, 2.25, 0.96, 9, 1.62},
+      {2.87, 4.49, 4.10, 14.36, 0.35}, {4.68, 0.15, 0, 3.84, 0.95},
+      {3.64, 1.26, 1.11, 4.63, 1.01}, {1e30, 0, 0, 0, 0}};
+  static constexpr BlockCost rows4[kF32Kinds] = {
+      {2.73, 0.44, 0.31, 0.98, 1.05, 5, 2.22}, {2.76, 0.38, 1.23, 0.86, 0.00, 10, 4.47},
+      {3.24, 0.63, 0.30, 1.43, 1.08, 4, 1.61}, {2.02, 2.51, 0, 2.31, 0.97, 9, 1.91},
+      {2.62, 4.69, 3.94, 14.31, 0.80}, {1e30, 0, 0, 0, 0},
+      {3.49, 1.23, 1.23, 4.51, 0.98}, {3.82, 1.91, 2.86, 3.20, 1.01}};
   return RBC >= 16 ? rows16 : RBC == 8 ? rows8 : rows4;
 }
 
@@ -726,7 +726,7 @@ int launch_small_blocks(const Problem& p, int64_t rows, int64_t cols, bool b128,
   const int64_t b16 = uk::ceil_div(rows, (int64_t)16) * uk::ceil_div(cols, (int64_t)16);
   const int64_t b32 = uk::ceil_div(rows, (int64_t)32) * uk::ceil_div(cols, (int64_t)32);
   int st = -1;
-  if constexpr (F32) {
+  if constexpr (F32 && RBC >= 8) {   // (choice 6 only)
     if (parts) {
       if (b16 > 3 * cus) return -1;
       st = b16 <= cus ? launch_thin<E, RBC, 1, 1, 8, 4, true, 16>(p, false, stream)

@@ -57,8 +57,9 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 // scalar's: a lane's address is one register that the K loop never touches, where an
 // address of its own takes a vector addition for every load, in the pipe that the f32
 // matrix instructions keep busy (f32 16x16x1 in 32x32 blocks: 515 x 1027 x 769 17.0 ->
-// 15.0 us, 700 x 700 x 3000 41.0 -> 34.6, 1500 x 1500 x 1000 52.6 -> 44.9). What lies kBeyond in a lane is outside the resource:
-// such a load returns zeros and reads nothing. NT: non-temporal.
+// 15.0 us, 700 x 700 x 3000 41.0 -> 34.6, 1500 x 1500 x 1000 52.6 -> 44.9). What lies
+// kBeyond in a lane is outside the resource: such a load returns zeros and reads nothing.
+// NT: non-temporal.
 constexpr uint32_t kBeyond = 0x80000000u;
 struct Operand {
   __amdgpu_buffer_rsrc_t buffer;
@@ -124,9 +125,10 @@ __device__ __forceinline__ void block_in_bands(uint32_t wg, const Args& a, int* 
 // blocks, of the LHS. A lane loads two neighbouring rows of a K-tile at once, half as many
 // loads for the same bytes, and what it gets belongs to the same lane of two blocks: the one
 // then holds the even and the other the odd rows or columns of 32. Rows are stored where
-// they belong; columns are put back in order by the waves that add up and store. Sums are
-// the same bit for bit. N0 (M0) is even. (These blocks are bound by how many loads a unit's
-// L1 and the waves' loops take, the thin ones beside by HBM: launch_thin has the figures.)
+// they belong; columns are put back in order by the waves that add up and store. Each sum
+// has the same products in the same order. N0 (M0) is even: others come here with rows of 16
+// bytes. (These blocks are bound by how many loads a unit's L1 and the waves' loops take, the
+// thin ones beside by HBM: launch_thin has the figures.)
 template <Elem E, int RBC, int TM, int TN, int KSPLIT, int D, bool STREAMED = false, bool TAIL = false, int CH = 0,
           bool PAIRED = false>
 __global__ __launch_bounds__(KSPLIT * 64, PAIRED && TM * TN >= 16 ? 2 : 1)   // (else two registers too many for two)
@@ -138,7 +140,6 @@ void mmt4d_thin_kernel(Args a) {
   constexpr int HALVES = TT::kHalves;
   constexpr int NCH = 4 * HALVES;             // 16-byte chunks per row per step
   constexpr int KS = NCH * 16;                // bytes of K per row per step
-  constexpr int PIECES = RBC >= 16 ? 1 : 16 / RBC;   // loads per 16-byte operand
   constexpr bool S4 = E == Elem::kS8S4;       // 4-bit RHS: half the bytes per row
   constexpr int CHAINS = CH > 0 ? CH : thin_chains<E, TM, KSPLIT>();
   static_assert(RBC >= 2, "rows narrower than 2 bytes take the LDS kernels");
@@ -147,8 +148,8 @@ void mmt4d_thin_kernel(Args a) {
   // the vector addition that each costs is hidden here. us from resources / so, four steps
   // ahead: s8 16x16x2 100 x 128 x 20480 21.0 / 12.6 (14.4 with the addition in scalar
   // registers), 16x16x4 126 x 408 x 19584 11.9 / 9.9; bf16 16x16x2 100 x 128 x 10240 11.9 / 9.9;
-  // f32 16x16x1 540 x 115 x 7400 30.1 / 25.8. (Rows of 8 bytes: level; sixteen chains: 15 to 22 % behind.)
-  constexpr bool BY_ADDRESS = RBC <= 4 && TM * TN == 1 && CHAINS < 16;
+  // f32 16x16x1 540 x 115 x 7400 30.1 / 25.8. (Rows of 8 bytes: level.)
+  constexpr bool BY_ADDRESS = RBC <= 4 && TM * TN == 1;
   static_assert(!PAIRED || ((RBC == 8 || RBC == 4) && TN % 2 == 0 && HALVES == 1), "two rows a load, columns of two blocks");
   constexpr bool PAIRED_A = PAIRED && TM % 2 == 0;
   static_assert(!S4 || (RBC >= 16 && !TAIL), "4-bit RHS: LHS rows of at least 16 bytes, K in whole steps");
@@ -324,8 +325,10 @@ void mmt4d_thin_kernel(Args a) {
     for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
       for (int h = 0; h < HALVES; ++h) {
-        if constexpr (PAIRED_A) fa[d][tm][h] = load_pair(std::false_type{}, ends, from_a, offa[tm][h], at_a, kt_m, s, h, tm % 2);
-        else fa[d][tm][h] = load_operand(std::false_type{}, ends, from_a, offa[tm][h], at_a, kt_m, s, h);
+        if constexpr (PAIRED_A)
+          fa[d][tm][h] = load_pair(std::false_type{}, ends, from_a, offa[tm][h], at_a, kt_m, s, h, tm % 2);
+        else
+          fa[d][tm][h] = load_operand(std::false_type{}, ends, from_a, offa[tm][h], at_a, kt_m, s, h);
       }
   };
   // Local step i. (Its number is kept from the compiler, which would hold the offsets of all

@@ -1,6 +1,6 @@
 """8-byte rows, and 4-byte rows of f32, loaded in twos: the blocks of two column blocks and more
-that do so, thin and between thin and large, with tiles of an even number of rows, and of
-an odd one, which keep a load a row; results that end at an odd column, inside a tile and inside
+that do so, thin and between thin and large; tiles of an odd number of rows, which are regrouped
+to 16-byte rows and give the same; results that end at an odd column, inside a tile and inside
 a two; rows and columns swapped; K split over workgroups; K in whole steps and not. Small
 integers, so that every order of the sums gives the product in 64 bits."""
 import pytest
