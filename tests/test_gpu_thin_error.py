@@ -89,3 +89,43 @@ def test_the_last_products_of_every_chain_count(gpu, flags, t, tout, k0, rows):
         lib.synchronize()
         want = (a[:, :k].float() @ b[:, :k].float().T).to(tout)
         assert torch.equal(out, want), (steps, lib.last_kernel_name())
+
+
+# No more than that of 64x64 blocks whose four waves share K: other blocks with four waves have
+# the same chains, 48x48 blocks, with eight, 0.56 of it. 8-bit floats, whose matrix instructions round
+# to 1.5e-5 however K is divided, also in one chain and in slices: at most 1.000003 of it measured.
+@pytest.mark.parametrize("dtype,k0,m,n,k,block", [
+    ("f16", 8, 97, 2406, 7048, "32x32_ksplit"), ("f16", 8, 300, 1500, 1504, "32x64_ksplit"),
+    ("f16", 8, 200, 4096, 2048, "64x64_ksplit"), ("f16", 4, 300, 1500, 1500, "32x64_ksplit"),
+    ("f16", 4, 300, 4096, 1000, "32x64_ksplit"), ("bf16", 8, 700, 900, 1504, "64x64_ksplit"),
+    ("f32", 4, 515, 1027, 768, "48x48_ksplit"), ("f32", 4, 3140, 237, 2088, "32x48_ksplit"),
+    ("f32", 2, 2173, 674, 3168, "32x48_ksplit"), ("f32", 4, 1564, 1150, 2624, "64x64_ksplit"),
+    ("f8", 16, 687, 2008, 1280, "32x64_ksplit"), ("f8", 16, 2153, 1308, 3840, "64x64_rhs_direct"),
+    ("f8", 16, 508, 1287, 8192, ""), ("f8", 16, 1500, 700, 16384, "")])
+def test_error_of_blocks_chosen_by_cost(gpu, dtype, k0, m, n, k, block):
+    lib, torch = gpu
+    flags, t = (uk.MMT4D_TYPE_F8E4M3FNF8E4M3FNF32, torch.float8_e4m3fn) if dtype == "f8" else \
+        (TYPES[dtype][0], getattr(torch, TYPES[dtype][1]))
+    gen = torch.Generator(device="cuda"); gen.manual_seed(m + k)
+    a, b = ((torch.randn(r, k, generator=gen, device="cuda") * (60 if dtype == "f8" else 1)).clamp(-448, 448).to(t)
+            for r in (m, n))
+    lhs, rhs = (torch.nn.functional.pad(x.float(), (0, 0, 0, -x.shape[0] % 16)).view(-1, 16, k // k0, k0)
+                .permute(0, 2, 1, 3).contiguous().to(t) for x in (a, b))
+    want = a.double() @ b.double().T
+    errors = []
+    try:
+        for mode in (uk.KERNEL_MODE_AUTO, uk.KERNEL_MODE_MFMA_VARIANT + 6):
+            lib.set_kernel_mode(mode)
+            out = torch.zeros(m, n, device="cuda")
+            torch.cuda.synchronize()
+            lib.mmt4d_unpack(lhs.data_ptr(), 0, 16 * k, rhs.data_ptr(), 0, 16 * k, out.data_ptr(), 0, n, m, n,
+                             lhs.shape[0], rhs.shape[0], k // k0, 16, 16, k0, flags)
+            lib.synchronize()
+            if mode == uk.KERNEL_MODE_AUTO and torch.cuda.get_device_properties(0).multi_processor_count == 256:
+                assert lib.last_kernel_name().endswith(block), lib.last_kernel_name()
+            if mode != uk.KERNEL_MODE_AUTO:
+                assert lib.last_kernel_name() == "mmt4d_mfma_64x64_ksplit"
+            errors.append(_error(out, want))
+    finally:
+        lib.set_kernel_mode(uk.KERNEL_MODE_AUTO)
+    assert errors[0] <= (1.0001 if dtype == "f8" else 1.0) * errors[1], errors
