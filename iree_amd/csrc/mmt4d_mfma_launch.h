@@ -863,9 +863,12 @@ int launch_by_cost(const Problem& p, int64_t rows, int64_t cols, bool parts, hip
   if (k_bytes < 1024 && b128 < 192) us[k128x128] = 1e30;
   // With 256 bytes of K, of which some waves of the barrier-free blocks get no step, and more than
   // four 32x32 blocks a unit, launching and adding up those is what they take: f8 1090 x 1412 x
-  // 105 6.3 us, so 4.9, s8 716 x 2957 x 256 7.8 / 6.5. (16-bit results, of which the 64x64
-  // blocks store half as much at a time, from some nine blocks a unit on: estimated.)
-  if (RBC >= 16 && ElemTraits<E>::Out::kOutBytes == 4 && k_bytes <= 256 && r32 * c32 > 4 * cus)
+  // 105 6.3 us, so 4.9, s8 716 x 2957 x 256 7.8 / 6.5. (16-bit results, of which the 64x64 blocks
+  // store half as much at a time, only from eight to twelve blocks a unit on. 16-bit floats, whose
+  // sums of 64 to 128 products in one chain are 1.05 to 1.26 times as far off as in four, with one
+  // step only.)
+  constexpr int64_t kShort = kInteger || ElemTraits<E>::kHalves == 2 ? 256 : 64;
+  if (RBC >= 16 && ElemTraits<E>::Out::kOutBytes == 4 && k_bytes <= kShort && r32 * c32 > 4 * cus)
     us[k32x32] = us[k32x64] = us[k64x64Split] = 1e30;
   // 2-byte results: the LDS-direct 64x64 shape takes K in whole steps.
   if (ElemTraits<E>::Out::kOutBytes == 2 && k_bytes % 256 != 0) us[k64x64Lds] = 1e30;

@@ -98,6 +98,7 @@ def test_the_last_products_of_every_chain_count(gpu, flags, t, tout, k0, rows):
     ("f16", 8, 97, 2406, 7048, "32x32_ksplit"), ("f16", 8, 300, 1500, 1504, "32x64_ksplit"),
     ("f16", 8, 200, 4096, 2048, "64x64_ksplit"), ("f16", 4, 300, 1500, 1500, "32x64_ksplit"),
     ("f16", 4, 300, 4096, 1000, "32x64_ksplit"), ("bf16", 8, 700, 900, 1504, "64x64_ksplit"),
+    ("f16", 8, 1100, 1200, 112, "32x32_ksplit"), ("bf16", 8, 716, 2957, 128, "32x32_ksplit"),
     ("f32", 4, 515, 1027, 768, "48x48_ksplit"), ("f32", 4, 3140, 237, 2088, "32x48_ksplit"),
     ("f32", 2, 2173, 674, 3168, "32x48_ksplit"), ("f32", 4, 1564, 1150, 2624, "64x64_ksplit"),
     ("f8", 16, 687, 2008, 1280, "32x64_ksplit"), ("f8", 16, 2153, 1308, 3840, "64x64_rhs_direct"),
